@@ -11,8 +11,8 @@
  *
  * All entry points return 0 on success or a negative KIFMM_E* code, never
  * exit.  A handle is not thread-safe; several handles may coexist.  Each
- * handle owns three HIP streams at default priority on its device: the
- * main one, a second compute stream and a copy stream.
+ * handle owns two HIP streams at default priority on its device: the main
+ * one and a second compute stream.
  */
 #ifndef KIFMM_HIP_H
 #define KIFMM_HIP_H
@@ -36,9 +36,9 @@ enum {
 enum {
   KIFMM_GPU_GRAPH = 1, /* capture the far-field launch sequence (fills, up, V, W, X, down)
                           in one HIP graph at the first full evaluate and replay it
-                          afterwards; the U-list chunks and their copies back, which run
-                          beside one another on three streams, stay outside the graph
-                          (phase times then report the U-list, the copy and the total) */
+                          afterwards; the U-list, whose early chunks may run on the second
+                          stream, stays outside the graph (phase times then report the
+                          U-list, the copy and the total) */
   KIFMM_GPU_NO_CLOSE_LIST = 2, /* do not list the U-list pairs closer than 1/8 of the target
                                   leaf's half-width at create time: the mixed path then tests
                                   for them inside its loop, the FP64 path forms r^2 from
@@ -50,8 +50,8 @@ enum {
                            priority) alongside up, V, W, X and down, into a buffer of its own
                            that one pass adds to the far field at the end
                            (kifmm_gpu_tuning.overlap; the autotuner may change it).  The
-                           potentials are bit-identical to the default layout, but the copy
-                           back can no longer overlap the U-list.  Phase times then overlap:
+                           potentials are bit-identical to the default layout, but they reach
+                           the host only with that pass.  Phase times then overlap:
                            ulist is the U-list's own span. */
 };
 
@@ -71,14 +71,13 @@ typedef struct kifmm_gpu_tuning {
                         STATIC or SPLIT on the mixed path */
   int hadamard_fb;   /* frequencies per V-list Hadamard block: 4, 8 (default) or 16 */
   int hadamard_form; /* KIFMM_HAD_*: V-list Hadamard on MFMA (default) or on the VALU */
-  int overlap;       /* stream layout of the U-list's copy-out chunks: 0 all of them last,
-                        after the far field, on the two streams in turn, their copies back
-                        overlapping the later chunks; 1 all of them on the handle's second
-                        stream from the start, alongside the far field (initially 1 with
-                        KIFMM_GPU_OVERLAP); 2, 3 the first one or two chunks there, the
-                        rest last; 4 all of them last, one after another on the main stream
-                        (the first copies start sooner: pays when the copy back is long
-                        against the U-list); 5, 6 as 2, 3 with the rest one after another */
+  int overlap;       /* stream layout of the U-list: 0 all of it last, after the far field;
+                        1 all of it on the handle's second stream from the start, alongside
+                        the far field (initially 1 with KIFMM_GPU_OVERLAP); 2, 3 its first
+                        one or two chunks there, the rest last; 4 as 0 and 5, 6 as 2, 3, but
+                        where the last part runs chunk by chunk (a result buffer other than
+                        kifmm_gpu_output()'s) the chunks run one after another on the main
+                        stream instead of on the two streams in turn */
   int up_form;       /* KIFMM_LEVEL_*: how each level's M2M (UE2UC stack, then UC2UE) runs */
   int down_form;     /* KIFMM_LEVEL_*: how each level's L2L + DC2DE runs */
   int reserved[2];
@@ -119,9 +118,9 @@ typedef struct kifmm_phase_times {
   double xlist;
   double down;      /* L2L + DC2DE + L2T                  */
   double copy;      /* device -> host potentials: the part left after the last
-                       kernel (the copies of earlier U-list chunks overlap the later
-                       chunks), plus the host pass into a caller buffer that is not
-                       kifmm_gpu_output()'s */
+                       kernel (the U-list, or the join of its early chunks, writes
+                       them to the host itself), plus the host pass into a caller
+                       buffer that is not kifmm_gpu_output()'s */
   double total;     /* first event to last event (+ that host pass) */
   double p2p_kernel;/* the U-list kernel alone            */
   double reserved[3];
@@ -142,7 +141,7 @@ typedef struct kifmm_work_counts {
   double close_pairs;  /* U-list pairs closer than 1/8 of the target leaf's half-width,
                           listed at create time; -1 when not listed (KIFMM_GPU_NO_CLOSE_LIST
                           or too many) */
-  double copy_chunks;  /* U-list chunks whose copies back overlap the later chunks */
+  double copy_chunks;  /* U-list chunks whose host passes into a caller buffer overlap the later chunks */
   double pair_items;   /* sibling-leaf pairs among the mixed U-list's work items */
   double reserved[2];
 } kifmm_work_counts;
@@ -151,10 +150,10 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops,
                      const kifmm_gpu_options* opts, kifmm_gpu** out);
 /* Evaluate the potentials.  pot_leaf (host, n_trg doubles, gathered target
  * order) may be NULL: the result then stays in device memory and the copy
- * phase is skipped.  The copy goes to the handle's pinned host buffer,
- * chunk by chunk while the U-list (the last phase) still computes; with
- * pot_leaf == kifmm_gpu_output(g) that is all, any other pot_leaf gets one
- * host pass from it (pipelined chunk by chunk in eager mode).  times may be
+ * phase is skipped.  The U-list (the last phase) writes the potentials to
+ * the handle's pinned host buffer as it finishes them; with pot_leaf ==
+ * kifmm_gpu_output(g) that is all, any other pot_leaf gets one host pass
+ * from it, chunk by chunk while the U-list still computes.  times may be
  * NULL. */
 int kifmm_gpu_evaluate(kifmm_gpu* g, double* pot_leaf, kifmm_phase_times* times);
 int kifmm_gpu_destroy(kifmm_gpu* g);

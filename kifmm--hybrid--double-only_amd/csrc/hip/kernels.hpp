@@ -110,6 +110,37 @@ __device__ __forceinline__ void eval8_lds(const double4* __restrict__ src, int n
 
 /* ------------------------------------------------------------------ U-list */
 
+/* A launch's U-list items per XCD.  Workgroups go round-robin to the 8 XCDs:
+ * giving XCD x (blocks b with b % 8 = x) the contiguous run beg[x] ..
+ * beg[x + 1] - 1 keeps neighbouring leaves, which share sources, in one L2.
+ * The runs are cut at equal cost (xcd_runs on the host), not equal count: on
+ * clustered inputs the items of a run cost up to several times those of
+ * another, and the launch ends with its slowest XCD (U-list of 1M ellipsoid
+ * points, one launch: 0.905 -> 0.503 ms). */
+struct XcdRuns {
+  int beg[9];
+};
+/* this block's item, -1 past its XCD's run */
+__device__ __forceinline__ int xcd_item(const XcdRuns& r) {
+  const int x = (int)(blockIdx.x & 7), k = r.beg[x] + (int)(blockIdx.x >> 3);
+  return k < r.beg[x + 1] ? k : -1;
+}
+
+/* A target's potential v, complete: to the device array and, with host set,
+ * to the pinned host buffer (device-mapped, posted PCIe writes that overlap
+ * the rest of the launch; neighbouring lanes hold neighbouring targets, so
+ * that they leave as whole lines).  Against a launch per copy-out chunk with
+ * a copy behind each: no partly empty last round of blocks per chunk (4M
+ * points mixed 2.98 -> 2.70 ms, 16M FP64 20.08 -> 19.66 ms) and, on small
+ * inputs, no copy launch and cross-stream waits (4 thousand points 334 ->
+ * 285 us per evaluation). */
+__device__ __forceinline__ void put_pot(double* __restrict__ pot, double* __restrict__ host, int t, double v,
+                                        int accum) {
+  if (accum) v = v + pot[t];
+  pot[t] = v;
+  if (host) __builtin_nontemporal_store(v, host + t);
+}
+
 /* U-list work item = {source range set, first target, target count, leaf},
  * up to 4 * 8 * G targets of one target leaf.  A block of 4 waves takes one
  * item: target group g (8 targets) belongs to wave g % 4, so a wave carries
@@ -213,9 +244,10 @@ __device__ __forceinline__ void eval8_gram(const double4* __restrict__ src, cons
   }
 }
 
-/* Scratch of the Gram form: the scaled source weights of a tile, the close-
- * pair sums of an item's targets (LDS), and the per-target records
- * (-2t', |t'|^2) with the close-pair CSR list (device memory). */
+/* The item's potentials on their way out, in the Gram form first its close-
+ * pair sums (sc_sum, LDS); and for the Gram form the scaled source weights of
+ * a tile (LDS) and the per-target records (-2t', |t'|^2) with the close-pair
+ * CSR list (device memory). */
 struct GramArgs {
   double* sw;
   double* sc_sum;
@@ -229,7 +261,7 @@ template <bool MASK, int G, bool GRAM>
 __device__ __forceinline__ void p2p_item(double4* tile, const int4 it, int rot, const int* __restrict__ rng_ptr,
                                          const int2* __restrict__ rng, const double4* __restrict__ src4,
                                          const double4* __restrict__ trg4, double* __restrict__ pot,
-                                         const GramArgs& ga, int accum) {
+                                         double* __restrict__ host, const GramArgs& ga, int accum) {
   const int tid = threadIdx.x, lane = tid & 63;
   /* groups g = wave' + 4k with wave' the wave index rotated by the item:
    * when the group count is not a multiple of 4 the short wave moves from
@@ -353,33 +385,33 @@ __device__ __forceinline__ void p2p_item(double4* tile, const int4 it, int rot, 
     if (grp < ngroups) {
       const double sum = wave_reduce8(acc[k], lane);
       const int t = 8 * grp + (lane >> 3);
-      if ((lane & 7) == 0 && t < it.z) {
-        const double v = GRAM ? (HALF_OOFP_R * sc) * (sum + ga.sc_sum[t]) : HALF_OOFP_R * sum;
-        pot[it.y + t] = accum ? v + pot[it.y + t] : v;
-      }
+      if ((lane & 7) == 0 && t < it.z)
+        ga.sc_sum[t] = GRAM ? (HALF_OOFP_R * sc) * (sum + ga.sc_sum[t]) : HALF_OOFP_R * sum;
     }
   }
+  /* the item's potentials leave as one run (and writing them here, with the
+   * accumulators dead, keeps the kernel's registers free of spills) */
+  __syncthreads();
+  for (int t = tid; t < it.z; t += 256) put_pot(pot, host, it.y + t, ga.sc_sum[t], accum);
 }
 
 /* One block per item of at most 32 G targets. */
 template <bool MASK, int G, bool GRAM>
-__global__ __launch_bounds__(256) void k_p2p_ulist(const int4* __restrict__ items, int n_items, int per_xcd,
+__global__ __launch_bounds__(256) void k_p2p_ulist(const int4* __restrict__ items, const XcdRuns runs,
                                                    const int* __restrict__ rng_ptr, const int2* __restrict__ rng,
                                                    const double4* __restrict__ src4,
                                                    const double4* __restrict__ trg4, double* __restrict__ pot,
-                                                   const double4* __restrict__ geo,
+                                                   double* __restrict__ host, const double4* __restrict__ geo,
                                                    const double4* __restrict__ trg_gram,
                                                    const int* __restrict__ cptr, const int* __restrict__ cidx,
                                                    int accum) {
   __shared__ double4 tile[P2P_TILE];
   __shared__ double sw[GRAM ? P2P_TILE : 1];
-  __shared__ double sc_sum[GRAM ? 32 * G : 1];
-  /* workgroups go round-robin to the 8 XCDs: give each XCD a contiguous run
-   * of items (neighbouring leaves) so their shared sources stay in its L2 */
-  const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= n_items) return; /* whole block, before any barrier */
+  __shared__ double sc_sum[32 * G];
+  const int item = xcd_item(runs);
+  if (item < 0) return; /* whole block, before any barrier */
   const GramArgs ga{sw, sc_sum, geo, trg_gram, cptr, cidx};
-  p2p_item<MASK, G, GRAM>(tile, items[item], item, rng_ptr, rng, src4, trg4, pot, ga, accum);
+  p2p_item<MASK, G, GRAM>(tile, items[item], item, rng_ptr, rng, src4, trg4, pot, host, ga, accum);
 }
 
 /* The same with items of at most 64 targets (G = 2 groups per wave): the
@@ -390,17 +422,17 @@ __global__ __launch_bounds__(256) void k_p2p_ulist(const int4* __restrict__ item
  * 5.61 for 4 x 4.) */
 template <bool MASK, bool GRAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_p2p_ulist64(
-    const int4* __restrict__ items, int n_items, int per_xcd, const int* __restrict__ rng_ptr,
+    const int4* __restrict__ items, const XcdRuns runs, const int* __restrict__ rng_ptr,
     const int2* __restrict__ rng, const double4* __restrict__ src4, const double4* __restrict__ trg4,
-    double* __restrict__ pot, const double4* __restrict__ geo, const double4* __restrict__ trg_gram,
-    const int* __restrict__ cptr, const int* __restrict__ cidx, int accum) {
+    double* __restrict__ pot, double* __restrict__ host, const double4* __restrict__ geo,
+    const double4* __restrict__ trg_gram, const int* __restrict__ cptr, const int* __restrict__ cidx, int accum) {
   __shared__ double4 tile[P2P_TILE];
   __shared__ double sw[GRAM ? P2P_TILE : 1];
-  __shared__ double sc_sum[GRAM ? P2P_MAXT : 1];
-  const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= n_items) return; /* whole block, before any barrier */
+  __shared__ double sc_sum[P2P_MAXT / 2];
+  const int item = xcd_item(runs);
+  if (item < 0) return; /* whole block, before any barrier */
   const GramArgs ga{sw, sc_sum, geo, trg_gram, cptr, cidx};
-  p2p_item<MASK, P2P_G / 2, GRAM>(tile, items[item], item, rng_ptr, rng, src4, trg4, pot, ga, accum);
+  p2p_item<MASK, P2P_G / 2, GRAM>(tile, items[item], item, rng_ptr, rng, src4, trg4, pot, host, ga, accum);
 }
 
 /* Persistent form over the same items (<= 32 G targets): a fixed grid
@@ -409,22 +441,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
  * so uneven items even out inside each XCD.  Every block leaves the loop
  * at its first draw past the run's end; the counters only grow. */
 template <bool MASK, int G, bool GRAM>
-__global__ __launch_bounds__(256) void k_p2p_ulist_persist(const int4* __restrict__ items, int n_items, int per_xcd,
+__global__ __launch_bounds__(256) void k_p2p_ulist_persist(const int4* __restrict__ items, const XcdRuns runs,
                                                            const int* __restrict__ rng_ptr,
                                                            const int2* __restrict__ rng,
                                                            const double4* __restrict__ src4,
                                                            const double4* __restrict__ trg4, double* __restrict__ pot,
-                                                           int* __restrict__ counters,
+                                                           double* __restrict__ host, int* __restrict__ counters,
                                                            const double4* __restrict__ geo,
                                                            const double4* __restrict__ trg_gram,
                                                            const int* __restrict__ cptr, const int* __restrict__ cidx,
                                                            int accum) {
   __shared__ double4 tile[P2P_TILE];
   __shared__ double sw[GRAM ? P2P_TILE : 1];
-  __shared__ double sc_sum[GRAM ? 32 * G : 1];
+  __shared__ double sc_sum[32 * G];
   __shared__ int draw;
   const int x = (int)(blockIdx.x & 7);
-  const int lo = x * per_xcd, n = min(n_items - lo, per_xcd);
+  const int lo = runs.beg[x], n = runs.beg[x + 1] - lo;
   const GramArgs ga{sw, sc_sum, geo, trg_gram, cptr, cidx};
   for (;;) {
     if (threadIdx.x == 0) draw = atomicAdd(counters + x, 1);
@@ -432,7 +464,7 @@ __global__ __launch_bounds__(256) void k_p2p_ulist_persist(const int4* __restric
     const int k = draw;
     __syncthreads(); /* every thread has read draw before the next draw overwrites it */
     if (k >= n) break;
-    p2p_item<MASK, G, GRAM>(tile, items[lo + k], lo + k, rng_ptr, rng, src4, trg4, pot, ga, accum);
+    p2p_item<MASK, G, GRAM>(tile, items[lo + k], lo + k, rng_ptr, rng, src4, trg4, pot, host, ga, accum);
   }
 }
 
@@ -476,6 +508,24 @@ typedef float v4f __attribute__((ext_vector_type(4)));
  * contribution below 1e-6 of a target's U-list sum. */
 constexpr float MIX_TAU2 = 0.01f;
 constexpr double MIX_FAR = 1.0e6;
+
+/* acc[e] of the 16 lanes of each lane row summed (fixed order): lane l gets
+ * the row's sum of element l & 3, so the lanes with (l & 15) < 4 hold the
+ * wave's 16 targets in order (target 4 (l / 16) + (l & 3)) and write them
+ * with one store */
+__device__ __forceinline__ double row_sum16(const double (&acc)[4], int lane) {
+  double s[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    double v = acc[e];
+    v += __shfl_xor(v, 8, 64);
+    v += __shfl_xor(v, 4, 64);
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 1, 64);
+    s[e] = v;
+  }
+  return lane & 2 ? (lane & 1 ? s[3] : s[2]) : (lane & 1 ? s[1] : s[0]);
+}
 
 template <bool MASK, int G>
 __device__ __forceinline__ void mixed_chunks(const float4* __restrict__ sB, const float* __restrict__ sW,
@@ -529,19 +579,20 @@ __device__ __forceinline__ void mixed_chunks(const float4* __restrict__ sB, cons
 }
 
 template <bool MASK>
-__global__ __launch_bounds__(256) void k_p2p_ulist_mixed(const int4* __restrict__ items, int n_items, int per_xcd,
+__global__ __launch_bounds__(256) void k_p2p_ulist_mixed(const int4* __restrict__ items, const XcdRuns runs,
                                                          const int* __restrict__ rng_ptr,
                                                          const int2* __restrict__ rng,
                                                          const double4* __restrict__ geo,
                                                          const double4* __restrict__ src4,
                                                          const double4* __restrict__ trg4,
-                                                         double* __restrict__ pot, int accum) {
+                                                         double* __restrict__ pot, double* __restrict__ host,
+                                                         int accum) {
   __shared__ float4 sB[P2P_TILE];
   __shared__ float sW[P2P_TILE];
   __shared__ double4 sS[P2P_TILE];
   __shared__ double4 sT[P2P_MAXT];
-  const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= n_items) return; /* whole block, before any barrier */
+  const int item = xcd_item(runs);
+  if (item < 0) return; /* whole block, before any barrier */
   const int4 it = items[item];
   const double4 g = geo[it.w];
   const double ih = 1.0 / g.w;
@@ -608,19 +659,9 @@ __global__ __launch_bounds__(256) void k_p2p_ulist_mixed(const int4* __restrict_
   for (int q = 0; q < 2; q++) {
     const int grp = wave + 4 * q;
     if (grp < ngroups) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        double v = acc[q][e];
-        v += __shfl_xor(v, 8, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 1, 64);
-        const int t = 16 * grp + 4 * (lane >> 4) + e;
-        if ((lane & 15) == 0 && t < it.z) {
-          const double u = OOFP_R * ih * v;
-          pot[it.y + t] = accum ? u + pot[it.y + t] : u;
-        }
-      }
+      const double v = row_sum16(acc[q], lane);
+      const int t = 16 * grp + 4 * (lane >> 4) + (lane & 3);
+      if ((lane & 15) < 4 && t < it.z) put_pot(pot, host, it.y + t, OOFP_R * ih * v, accum);
     }
   }
 }
@@ -867,7 +908,7 @@ __device__ __forceinline__ void mixed_tau_range(const v8bf (*sB)[P2P_TILE], cons
   }
 }
 template <bool MASK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_p2p_ulist_mixed_tau(const int4* __restrict__ items, int n_items, int per_xcd,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_p2p_ulist_mixed_tau(const int4* __restrict__ items, const XcdRuns runs,
                                                              const int* __restrict__ rng_ptr,
                                                              const int2* __restrict__ rng,
                                                              const double4* __restrict__ geo,
@@ -875,12 +916,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                                                              const double4* __restrict__ trg4,
                                                              const int* __restrict__ cptr,
                                                              const int* __restrict__ cidx,
-                                                             double* __restrict__ pot, int accum) {
+                                                             double* __restrict__ pot, double* __restrict__ host,
+                                                             int accum) {
   __shared__ v8bf sB[4][P2P_TILE];
   __shared__ float sW[P2P_TILE];
   __shared__ double4 sT[P2P_MAXT5];
-  const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= n_items) return; /* whole block, before any barrier */
+  const int item = xcd_item(runs);
+  if (item < 0) return; /* whole block, before any barrier */
   const int4 it = items[item];
   /* a leaf (nB = 0) or two sibling leaves A = it.w and B = it.w + 1 whose
    * targets follow each other: groups 0 .. gA - 1 are A's, the rest B's,
@@ -994,21 +1036,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
   for (int q = 0; q < MIX_G; q++) {
     const int grp = wave + 4 * q;
     if (grp < ngroups) {
-      const int first = grp_first(grp), cnt = grp_count(grp);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        double v = acc[q][e];
-        v += __shfl_xor(v, 8, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 1, 64);
-        const int r = 4 * (lane >> 4) + e; /* the target's row in the group */
-        if ((lane & 15) == 0 && r < cnt) {
-          const double u = scale * (v + sC[16 * grp + r]);
-          double* const o = pot + it.y + first + r;
-          *o = accum ? u + *o : u;
-        }
-      }
+      const double v = row_sum16(acc[q], lane);
+      const int r = 4 * (lane >> 4) + (lane & 3); /* the target's row in the group */
+      if ((lane & 15) < 4 && r < grp_count(grp))
+        put_pot(pot, host, it.y + grp_first(grp) + r, scale * (v + sC[16 * grp + r]), accum);
     }
   }
 }
@@ -1030,15 +1061,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 constexpr int MIXS_G = 2;
 template <bool MASK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_p2p_ulist_mixed_split(
-    const int4* __restrict__ items, int n_items, int per_xcd, const int* __restrict__ rng_ptr,
+    const int4* __restrict__ items, const XcdRuns runs, const int* __restrict__ rng_ptr,
     const int2* __restrict__ rng, const double4* __restrict__ geo, const double4* __restrict__ src4,
     const double4* __restrict__ trg4, const int* __restrict__ cptr, const int* __restrict__ cidx,
-    double* __restrict__ pot, int accum) {
+    double* __restrict__ pot, double* __restrict__ host, int accum) {
   __shared__ v8bf sB[4][P2P_TILE];
   __shared__ float sW[P2P_TILE];
   __shared__ double4 sT[P2P_MAXT];
-  const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= n_items) return; /* whole block, before any barrier */
+  const int item = xcd_item(runs);
+  if (item < 0) return; /* whole block, before any barrier */
   const int4 it = items[item];
   const double4 g = geo[it.w];
   const double sc = (1.0 / MIX_CLOSE) / g.w; /* 1 / (tau h), a power of two */
@@ -1107,16 +1138,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 #pragma unroll
   for (int q = 0; q < MIXS_G; q++) {
     if (q < gn) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        double v = acc[q][e];
-        v += __shfl_xor(v, 8, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 1, 64);
-        const int t = 16 * (g0 + q) + 4 * (lane >> 4) + e;
-        if ((lane & 15) == 0) red[part * P2P_MAXT + t] = v;
-      }
+      const double v = row_sum16(acc[q], lane);
+      if ((lane & 15) < 4) red[part * P2P_MAXT + 16 * (g0 + q) + 4 * (lane >> 4) + (lane & 3)] = v;
     }
   }
   /* FP64 close-pair terms, group grp by wave grp % 4 (as in the tau kernel) */
@@ -1128,8 +1151,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
   for (int t = tid; t < it.z; t += 256) {
     double v = red[t]; /* the target's set: its waves' partial sums in wave order */
     for (int p_ = 1; p_ < wps; p_++) v += red[p_ * P2P_MAXT + t];
-    const double u = scale * (v + sC[t]);
-    pot[it.y + t] = accum ? u + pot[it.y + t] : u;
+    put_pot(pot, host, it.y + t, scale * (v + sC[t]), accum);
   }
 }
 
@@ -2901,11 +2923,12 @@ static __global__ void k_fill(double* __restrict__ p, size_t n, double v) {
 
 /* pot = u + pot over [0, n): the U-list sums (u) written on the second
  * stream joined with the far field (W, X, L2T) accumulated in pot, in the
- * same operand order as the U-list kernels' own accumulating write */
-static __global__ void k_join_pot(double* __restrict__ pot, const double* __restrict__ u, size_t n) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) pot[i] = u[i] + pot[i];
+ * same operand order as the U-list kernels' own accumulating write (and to
+ * the pinned host buffer, when host is set) */
+static __global__ void k_join_pot(double* __restrict__ pot, double* __restrict__ host, const double* __restrict__ u,
+                                  int n) {
+  const int stride = gridDim.x * blockDim.x;
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) put_pot(pot, host, (int)i, u[i], 1);
 }
 
 /* (x, y, z, w) records from coordinate arrays; w = 0 without a density array */

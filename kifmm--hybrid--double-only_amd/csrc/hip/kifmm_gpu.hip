@@ -133,21 +133,24 @@ struct kifmm_gpu {
   /* wall ms of kifmm_gpu_create: host plan, upload, close-pair search,
    * other device set-up (translation spectra, Gram records), whole call */
   double create_ms[5] = {0, 0, 0, 0, 0};
-  /* pinned host staging of the potentials (device -> host copy at PCIe rate) */
+  /* pinned host buffer of the potentials, and its device address: the last
+   * kernels of an evaluation write it themselves */
   double* pinned = nullptr;
+  double* pinned_dev = nullptr;
   /* HIP graph of the whole launch sequence (KIFMM_GPU_GRAPH) */
   int use_graph = 0;
   bool capturing = false;
   hipGraph_t graph[2] = {nullptr, nullptr}; /* [0]: the far-field sequence */
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   /* copy-out: target cuts of the U-list chunks (leaf starts, 0 .. n_trg),
-   * the first item of each chunk per item list, the copy stream (default
-   * priority) and the events that order chunks, copies and joins */
+   * the first item of each chunk per item list, whether the items cover every
+   * target, and the events that mark a chunk's potentials as on the host */
   std::vector<int> cuts;
   std::vector<int> chunk_beg[4];
-  hipStream_t cstream = nullptr;
-  std::vector<hipEvent_t> ch_ev, cd_ev;
-  hipEvent_t far_ev = nullptr, sdone_ev = nullptr, cdone_ev = nullptr;
+  std::vector<double> u_cost[4]; /* prefix sums of the items' costs, per list */
+  bool tiled = false;
+  std::vector<hipEvent_t> cd_ev;
+  hipEvent_t far_ev = nullptr, sdone_ev = nullptr;
   /* the U-list's own sums when it runs on the second stream (overlap layout) */
   double* potU = nullptr;
   /* staging of kifmm_gpu_set_densities */
@@ -304,6 +307,8 @@ struct Plan {
    * first item of each chunk */
   std::vector<int> cuts;
   std::vector<int> chunk_beg[4];
+  std::vector<double> u_cost[4];
+  bool tiled = false;
   std::vector<int> rng_ptr;
   std::vector<int2> rng;
   std::vector<int4> s2m_items;
@@ -407,6 +412,30 @@ int pair_items(const kifmm_tree_view* t, Plan& P) {
   return KIFMM_OK;
 }
 
+/* What a U-list item costs its CU, in steps of 64 sources (16 x 16 tiles on
+ * the mixed path) by one target group: its longest wave's steps, and a fixed
+ * part (item and range loads, first tile, close pairs, reductions) of about
+ * 4 such steps.  set_src: the sources of each range set. */
+double item_cost(const int4& it, int group, const std::vector<int>& set_src) {
+  const int groups = ((it.z & 0xffff) + group - 1) / group + ((it.z >> 16) + group - 1) / group;
+  double src = set_src[it.x];
+  if (it.z >> 16) src += 0.5 * ((double)set_src[it.x + 1] + set_src[it.x + 2]); /* of a pair: half the groups each */
+  return (groups + 3) / 4 * (src / 64.0 + 1.0) + 4.0;
+}
+
+/* Items [b, e) of a list cut into 8 runs of about equal cost. */
+XcdRuns xcd_runs(const std::vector<double>& cost, int b, int e) {
+  XcdRuns r;
+  r.beg[0] = b;
+  for (int x = 1; x < 8; x++) {
+    const double want = cost[b] + (cost[e] - cost[b]) * x / 8;
+    const int k = (int)(std::lower_bound(cost.begin() + b, cost.begin() + e, want) - cost.begin());
+    r.beg[x] = std::max(k, r.beg[x - 1]);
+  }
+  r.beg[8] = e;
+  return r;
+}
+
 int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
   TRY(check_view(t));
   const int np = t->np;
@@ -485,6 +514,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
       }
       if (next != t->n_trg) tiled = false;
     }
+    P.tiled = tiled;
     P.cuts.assign(1, 0);
     if (tiled && t->n_trg >= (1 << 18)) {
       static const double frac[] = {0.30, 0.55, 0.75, 0.88, 0.95};
@@ -502,8 +532,14 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
       }
     }
     P.cuts.push_back(t->n_trg);
+    std::vector<int> set_src(P.rng_ptr.size(), 0); /* sources of each range set */
+    for (size_t k = 0; k + 1 < P.rng_ptr.size(); k++)
+      for (int r = P.rng_ptr[k]; r < P.rng_ptr[k + 1]; r++) set_src[k] += P.rng[r].y;
     for (int l = 0; l < 4; l++) {
       const std::vector<int4>& L = *lists[l];
+      std::vector<double>& cost = P.u_cost[l];
+      cost.assign(1, 0.0);
+      for (const int4& it : L) cost.push_back(cost.back() + item_cost(it, l == 3 ? 16 : 8, set_src));
       P.chunk_beg[l].clear();
       size_t k = 0;
       for (size_t c = 0; c + 1 < P.cuts.size(); c++) {
@@ -909,7 +945,11 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
   TRY(dev_upload(g, &g->p2p_itemsP, P.p2p_itemsP.data(), P.p2p_itemsP.size()));
   TRY(dev_zero(g, &g->p2p_counters, 8 * std::max<size_t>(P.cuts.size(), 1)));
   g->cuts = P.cuts;
-  for (int l = 0; l < 4; l++) g->chunk_beg[l] = P.chunk_beg[l];
+  g->tiled = P.tiled;
+  for (int l = 0; l < 4; l++) {
+    g->chunk_beg[l] = P.chunk_beg[l];
+    g->u_cost[l] = P.u_cost[l];
+  }
   TRY(dev_zero(g, &g->potU, (size_t)t->n_trg));
   TRY(dev_zero(g, &g->den_stage, (size_t)t->n_src));
   {
@@ -1226,67 +1266,80 @@ int vlist_phase(kifmm_gpu* g, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3) {
  * pairs and single leaves (list 3), the FP64 Gram-form kernels items of
  * <= P2P_MAXT5 targets (list 2), the STATIC64 shape items of <= 64 (list
  * 1), the difference form, the mixed source-split form and the mixed
- * in-loop test items of <= P2P_MAXT (list 0). */
+ * in-loop test items of <= P2P_MAXT (list 0).  The STATIC Gram form also
+ * takes the <= 64 list where leaves are small, U_SMALL targets or fewer per
+ * item of list 2: its kernel holds 6 waves per SIMD instead of 4, which on
+ * short items outweighs the second source walk of the few large leaves.
+ * Measured, list 2 -> list 1: 0.503 -> 0.455 ms at 50 targets per item (1M
+ * ellipsoid), 0.160 -> 0.137 at 37 (300 thousand, NP 6), 13.16 -> 12.89 at
+ * 64 (16M uniform); 5.36 -> 5.59 at 128 (4M uniform).  The sums are the same
+ * bit for bit. */
+constexpr double U_SMALL = 96.0;
 int u_list_index(const kifmm_gpu* g) {
   if (g->precision == KIFMM_PREC_MIXED) return g->close_listed && g->p2p_form != KIFMM_P2P_SPLIT ? 3 : 0;
   if (g->p2p_form == KIFMM_P2P_STATIC64) return 1;
+  if (g->p2p_form == KIFMM_P2P_STATIC && g->trg_gram && g->n_trg <= U_SMALL * g->n_p2p5) return 1;
   return g->trg_gram ? 2 : 0;
 }
 
 /* U-list over the items of copy-out chunks [c0, c1) on stream st, writing
- * out[t] = u (accum = 0) or out[t] = u + out[t] (accum = 1).  The
+ * out[t] = u (accum = 0) or out[t] = u + out[t] (accum = 1), and to host[t]
+ * (device address of the pinned buffer) when host is set.  The
  * persistent form's per-XCD counters of the launch are slot c0. */
 template <bool MASK>
-int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, int accum) {
+int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum) {
   const int l = u_list_index(g);
   const int4* list = l == 0 ? g->p2p_items : l == 1 ? g->p2p_items64 : l == 2 ? g->p2p_items5 : g->p2p_itemsP;
   const int beg = g->chunk_beg[l][c0], end = g->chunk_beg[l][c1];
   const int chunk = c0;
-  const int n = end - beg, per = (n + 7) / 8;
-  if (n <= 0) return KIFMM_OK;
-  const int4* items = list + beg;
+  if (end <= beg) return KIFMM_OK;
+  const XcdRuns runs = xcd_runs(g->u_cost[l], beg, end);
+  int per = 0;
+  for (int x = 0; x < 8; x++) per = std::max(per, runs.beg[x + 1] - runs.beg[x]);
+  const int4* items = list;
   if (g->precision == KIFMM_PREC_MIXED) {
     if (g->close_listed && g->p2p_form == KIFMM_P2P_SPLIT)
-      hipLaunchKernelGGL(k_p2p_ulist_mixed_split<MASK>, dim3(8 * per), dim3(256), 0, st, items, n, per, g->rng_ptr,
-                         g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, accum);
+      hipLaunchKernelGGL(k_p2p_ulist_mixed_split<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+                         g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, host, accum);
     else if (g->close_listed)
-      hipLaunchKernelGGL(k_p2p_ulist_mixed_tau<MASK>, dim3(8 * per), dim3(256), 0, st, items, n, per, g->rng_ptr,
-                         g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, accum);
+      hipLaunchKernelGGL(k_p2p_ulist_mixed_tau<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+                         g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, host, accum);
     else
-      hipLaunchKernelGGL(k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), 0, st, items, n, per, g->rng_ptr, g->rng,
-                         g->geo, g->src4, g->trg4, out, accum);
-  } else if (g->p2p_form == KIFMM_P2P_STATIC64) {
+      hipLaunchKernelGGL(k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr, g->rng,
+                         g->geo, g->src4, g->trg4, out, host, accum);
+  } else if (l == 1) {
     if (g->trg_gram)
-      hipLaunchKernelGGL((k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), 0, st, items, n, per, g->rng_ptr,
-                         g->rng, g->src4, g->trg4, out, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
+      hipLaunchKernelGGL((k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+                         g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
-      hipLaunchKernelGGL((k_p2p_ulist64<MASK, false>), dim3(8 * per), dim3(256), 0, st, items, n, per, g->rng_ptr,
-                         g->rng, g->src4, g->trg4, out, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
+      hipLaunchKernelGGL((k_p2p_ulist64<MASK, false>), dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+                         g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
   } else if (g->p2p_form == KIFMM_P2P_PERSISTENT) {
     int* counters = g->p2p_counters + 8 * std::max(chunk, 0);
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, counters, 8, 0);
     if (g->trg_gram)
       hipLaunchKernelGGL((k_p2p_ulist_persist<MASK, P2P_G5, true>), dim3(g->persist_grid[1]), dim3(256), 0, st, items,
-                         n, per, g->rng_ptr, g->rng, g->src4, g->trg4, out, counters, g->geo, g->trg_gram, g->cptr,
+                         runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
     else
       hipLaunchKernelGGL((k_p2p_ulist_persist<MASK, P2P_G, false>), dim3(g->persist_grid[0]), dim3(256), 0, st, items,
-                         n, per, g->rng_ptr, g->rng, g->src4, g->trg4, out, counters, g->geo, g->trg_gram, g->cptr,
+                         runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
   } else {
     if (g->trg_gram)
-      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G5, true>), dim3(8 * per), dim3(256), 0, st, items, n, per,
-                         g->rng_ptr, g->rng, g->src4, g->trg4, out, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
+      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G5, true>), dim3(8 * per), dim3(256), 0, st, items, runs,
+                         g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
-      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G, false>), dim3(8 * per), dim3(256), 0, st, items, n, per,
-                         g->rng_ptr, g->rng, g->src4, g->trg4, out, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
+      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G, false>), dim3(8 * per), dim3(256), 0, st, items, runs,
+                         g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
   }
   LAUNCH_CHECK();
   return KIFMM_OK;
 }
 
-int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, int accum) {
-  return g->coincident ? launch_u<true>(g, st, c0, c1, out, accum) : launch_u<false>(g, st, c0, c1, out, accum);
+int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum) {
+  return g->coincident ? launch_u<true>(g, st, c0, c1, out, host, accum)
+                       : launch_u<false>(g, st, c0, c1, out, host, accum);
 }
 
 /* Copy-out chunks whose U-list runs on the second stream from the start of
@@ -1333,13 +1386,6 @@ int point_phases_wx(kifmm_gpu* g, unsigned mask, hipEvent_t ew) {
  * sequence, then one after each phase in launch order. */
 enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_W, E_X, E_DOWN, E_U, E_END };
 
-/* device -> host copy of potentials [b, e) to dst + b */
-int copy_out(kifmm_gpu* g, hipStream_t st, double* dst, int b, int e) {
-  if (e > b)
-    HIP_TRY(hipMemcpyAsync(dst + b, g->pot + b, sizeof(double) * (size_t)(e - b), hipMemcpyDeviceToHost, st));
-  return KIFMM_OK;
-}
-
 /* One evaluation is three launch sequences on the handle's streams:
  *   enqueue_side  the U-list of the early copy-out chunks (early_chunks) on
  *                 the second stream from the start, into potU, alongside
@@ -1347,10 +1393,12 @@ int copy_out(kifmm_gpu* g, hipStream_t st, double* dst, int b, int e) {
  *   enqueue_far   the fills, up, V, W, X and down on the main stream (what a
  *                 graph handle captures and replays);
  *   enqueue_near  the join pot = potU + pot of the early chunks, then the
- *                 U-list of the other chunks, alternating between the two
- *                 compute streams, each chunk's potentials copied to the
- *                 host (dst, when non-null) on the copy stream while the
- *                 later chunks compute.
+ *                 U-list of the others; both write the finished potentials
+ *                 to the host as well (host, the pinned buffer's device
+ *                 address, when non-null).  One U-list launch, or with
+ *                 chunked (a caller buffer filled by host passes) one per
+ *                 chunk, each followed by its event, so that the host copies
+ *                 a chunk while the later ones compute.
  * The U-list's accumulating write (u + pot) and the join (potU + pot) add
  * the same two terms, so every layout gives the same bits. */
 int enqueue_side(kifmm_gpu* g, unsigned mask) {
@@ -1359,7 +1407,7 @@ int enqueue_side(kifmm_gpu* g, unsigned mask) {
   HIP_TRY(hipEventRecord(g->fork_ev, g->stream)); /* after the previous evaluation's join read potU */
   HIP_TRY(hipStreamWaitEvent(g->side, g->fork_ev, 0));
   HIP_TRY(hipEventRecord(g->su0, g->side));
-  TRY(launch_u(g, g->side, 0, e, g->potU, 0));
+  TRY(launch_u(g, g->side, 0, e, g->potU, nullptr, 0));
   HIP_TRY(hipEventRecord(g->su1, g->side));
   HIP_TRY(hipEventRecord(g->join_ev, g->side));
   return KIFMM_OK;
@@ -1457,33 +1505,23 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
   return KIFMM_OK;
 }
 
-int enqueue_near(kifmm_gpu* g, unsigned mask, double* dst) {
-  const int n = g->n_trg;
-  if (!(mask & KIFMM_PHASE_U)) {
-    HIP_TRY(hipEventRecord(g->ev[E_U], g->stream));
-    if (dst) TRY(copy_out(g, g->stream, dst, 0, n));
-    return KIFMM_OK;
-  }
+int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
   const int nch = (int)g->cuts.size() - 1, e = early_chunks(g, mask);
-  if (e > 0) { /* the early chunks: join, then their copy */
-    const size_t m = (size_t)g->cuts[e];
+  if (e > 0) { /* the early chunks: join */
+    const int m = g->cuts[e];
     HIP_TRY(hipStreamWaitEvent(g->stream, g->join_ev, 0));
-    const int blocks = (int)std::min<size_t>(4096, (m + 255) / 256);
-    if (m > 0) hipLaunchKernelGGL(k_join_pot, dim3(std::max(blocks, 1)), dim3(256), 0, g->stream, g->pot, g->potU, m);
+    const int blocks = std::min(4096, (m + 255) / 256);
+    if (m > 0)
+      hipLaunchKernelGGL(k_join_pot, dim3(std::max(blocks, 1)), dim3(256), 0, g->stream, g->pot, host, g->potU, m);
     LAUNCH_CHECK();
-    if (dst) {
-      HIP_TRY(hipEventRecord(g->ch_ev[0], g->stream));
-      HIP_TRY(hipStreamWaitEvent(g->cstream, g->ch_ev[0], 0));
-      TRY(copy_out(g, g->cstream, dst, 0, (int)m));
-      for (int c = 0; c < e; c++) HIP_TRY(hipEventRecord(g->cd_ev[c], g->cstream));
-    }
+    if (chunked)
+      for (int c = 0; c < e; c++) HIP_TRY(hipEventRecord(g->cd_ev[c], g->stream));
   }
-  if (e < nch) { /* the other chunks after the far field */
-    const int late = dst ? nch - e : 1; /* without a copy: one launch */
-    /* on the two streams in turn (one chunk's last blocks run beside the
-     * next chunk's first), or in layouts 4 - 6 one after another on the
-     * main stream: the first copies then start sooner, which pays when the
-     * copy back is long against the U-list */
+  if ((mask & KIFMM_PHASE_U) && e < nch) { /* the other chunks after the far field */
+    const int late = chunked ? nch - e : 1;
+    /* chunk launches on the two streams in turn (one chunk's last blocks run
+     * beside the next chunk's first), or in layouts 4 - 6 one after another
+     * on the main stream */
     const bool pairs = late > 1 && g->overlap < 4;
     if (pairs) {
       HIP_TRY(hipEventRecord(g->far_ev, g->stream));
@@ -1492,13 +1530,8 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* dst) {
     for (int k = 0; k < late; k++) {
       const int c = e + k;
       hipStream_t st = (pairs && (k & 1)) ? g->side : g->stream;
-      TRY(launch_u(g, st, c, dst ? c + 1 : nch, g->pot, 1));
-      if (dst) {
-        HIP_TRY(hipEventRecord(g->ch_ev[c], st));
-        HIP_TRY(hipStreamWaitEvent(g->cstream, g->ch_ev[c], 0));
-        TRY(copy_out(g, g->cstream, dst, g->cuts[c], g->cuts[c + 1]));
-        HIP_TRY(hipEventRecord(g->cd_ev[c], g->cstream));
-      }
+      TRY(launch_u(g, st, c, chunked ? c + 1 : nch, g->pot, host, 1));
+      if (chunked) HIP_TRY(hipEventRecord(g->cd_ev[c], st));
     }
     if (pairs) {
       HIP_TRY(hipEventRecord(g->sdone_ev, g->side));
@@ -1506,10 +1539,6 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* dst) {
     }
   }
   HIP_TRY(hipEventRecord(g->ev[E_U], g->stream));
-  if (dst) {
-    HIP_TRY(hipEventRecord(g->cdone_ev, g->cstream));
-    HIP_TRY(hipStreamWaitEvent(g->stream, g->cdone_ev, 0));
-  }
   return KIFMM_OK;
 }
 
@@ -1537,10 +1566,15 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
    * stream, so the U-list chunks and their copies, whose point is to run
    * beside one another, stay outside it */
   const bool graph = g->use_graph && mask == KIFMM_PHASE_ALL;
-  /* the copy lands in the handle's pinned buffer (the caller's own buffer
-   * when it is that one; otherwise one host pass follows), or without
-   * pinned memory straight into the caller's buffer */
-  double* dst = pot_leaf ? (g->pinned ? g->pinned : pot_leaf) : nullptr;
+  /* the potentials land in the handle's pinned buffer (the caller's own
+   * buffer when it is that one; otherwise one host pass follows), or without
+   * pinned memory straight in the caller's buffer.  The U-list writes them
+   * there itself (or the join, in the overlap layouts); without a U-list, or
+   * when its items do not cover every target, a copy follows */
+  double* const dst = pot_leaf ? (g->pinned ? g->pinned : pot_leaf) : nullptr;
+  const bool direct = pot_leaf && g->pinned_dev && g->tiled && (mask & KIFMM_PHASE_U);
+  const bool host_pass = pot_leaf && g->pinned && pot_leaf != g->pinned;
+  const bool pipelined = direct && host_pass && g->cuts.size() > 2; /* the host pass chunk by chunk */
   if (graph && !g->gexec[0]) {
     g->capturing = true;
     HIP_TRY(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
@@ -1564,12 +1598,13 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
   } else {
     TRY(enqueue_far(g, mask));
   }
-  TRY(enqueue_near(g, mask, dst));
+  TRY(enqueue_near(g, mask, direct ? g->pinned_dev : nullptr, pipelined));
+  if (dst && !direct && g->n_trg > 0)
+    HIP_TRY(hipMemcpyAsync(dst, g->pot, sizeof(double) * (size_t)g->n_trg, hipMemcpyDeviceToHost, g->stream));
   HIP_TRY(hipEventRecord(ev[E_END], g->stream));
   double host_copy_ms = 0.0;
-  if (pot_leaf && dst == g->pinned && pot_leaf != g->pinned) {
+  if (host_pass) {
     const int nch = (int)g->cuts.size() - 1;
-    const bool pipelined = (mask & KIFMM_PHASE_U) && nch > 1; /* cd_ev recorded for every chunk */
     double t0 = 0.0;
     if (pipelined) { /* each chunk as soon as its copy is done */
       for (int c = 0; c < nch; c++) {
@@ -1611,7 +1646,7 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
       times->ulist += mu;
       times->p2p_kernel = early_chunks(g, mask) == (int)g->cuts.size() - 1 ? mu : times->ulist;
     }
-    /* the copy left after the last kernel (the rest overlaps the U-list) */
+    /* the copy left after the last kernel (it overlaps the U-list) */
     times->copy = ms[E_END] + host_copy_ms;
     times->total = tot + host_copy_ms;
   }
@@ -1693,14 +1728,12 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
   g->overlap = opts ? (opts->flags & KIFMM_GPU_OVERLAP) != 0 : 0;
   /* the second stream exists on every handle: the layout is a tuning choice */
   if (hipStreamCreateWithFlags(&g->side, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&g->cstream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&g->fork_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->join_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->far_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->sdone_ev, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&g->cdone_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&g->su0) != hipSuccess || hipEventCreate(&g->su1) != hipSuccess) {
-    set_error("kifmm_gpu_create: second stream, copy stream or their events could not be created");
+    set_error("kifmm_gpu_create: second stream or its events could not be created");
     kifmm_gpu_destroy(g);
     return KIFMM_EDEVICE;
   }
@@ -1708,11 +1741,9 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
     kifmm_gpu_destroy(g);
     return KIFMM_EDEVICE;
   }
-  g->ch_ev.assign(P.cuts.size(), nullptr);
   g->cd_ev.assign(P.cuts.size(), nullptr);
   for (size_t c = 0; c < P.cuts.size(); c++)
-    if (hipEventCreateWithFlags(&g->ch_ev[c], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->cd_ev[c], hipEventDisableTiming) != hipSuccess) {
+    if (hipEventCreateWithFlags(&g->cd_ev[c], hipEventDisableTiming) != hipSuccess) {
       set_error("kifmm_gpu_create: copy-out events could not be created");
       kifmm_gpu_destroy(g);
       return KIFMM_EDEVICE;
@@ -1739,10 +1770,11 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
     kifmm_gpu_destroy(g);
     return r;
   }
-  /* pinned staging for the potentials; without it the copy goes straight
-   * to the caller's (pageable) buffer */
+  /* pinned buffer of the potentials; without it the copy goes straight to
+   * the caller's (pageable) buffer */
   if (hipHostMalloc((void**)&g->pinned, sizeof(double) * std::max(g->n_trg, 1), hipHostMallocDefault) != hipSuccess)
     g->pinned = nullptr;
+  if (g->pinned && hipHostGetDevicePointer((void**)&g->pinned_dev, g->pinned, 0) != hipSuccess) g->pinned_dev = nullptr;
   if (hipDeviceSynchronize() != hipSuccess) {
     set_error("device synchronisation failed after upload");
     kifmm_gpu_destroy(g);
@@ -1775,7 +1807,6 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   if (g->pinned) (void)hipHostFree(g->pinned);
   if (g->side) (void)hipStreamSynchronize(g->side);
-  if (g->cstream) (void)hipStreamSynchronize(g->cstream);
   for (int k = 0; k < 2; k++) {
     if (g->gexec[k]) (void)hipGraphExecDestroy(g->gexec[k]);
     if (g->graph[k]) (void)hipGraphDestroy(g->graph[k]);
@@ -1783,13 +1814,10 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   for (void* p : g->allocs) (void)hipFree(p);
   for (auto& e : g->ev)
     if (e) (void)hipEventDestroy(e);
-  for (hipEvent_t e : {g->fork_ev, g->join_ev, g->su0, g->su1, g->far_ev, g->sdone_ev, g->cdone_ev})
-    if (e) (void)hipEventDestroy(e);
-  for (hipEvent_t e : g->ch_ev)
+  for (hipEvent_t e : {g->fork_ev, g->join_ev, g->su0, g->su1, g->far_ev, g->sdone_ev})
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : g->cd_ev)
     if (e) (void)hipEventDestroy(e);
-  if (g->cstream) (void)hipStreamDestroy(g->cstream);
   if (g->side) (void)hipStreamDestroy(g->side);
   if (g->stream) (void)hipStreamDestroy(g->stream);
   delete g;

@@ -67,6 +67,28 @@ def test_copy_out_is_the_device_result(prec):
         ev.evaluate()
 
 
+@pytest.mark.parametrize("n,dist,q,c", [(5, "uniform", 64, 0), (70, "uniform", 16, 1), (900, "gaussmix", 100, 0),
+                                         (3000, "ellipsoid", 1, 1), (20000, "ellipsoid", 200, 0)])
+@pytest.mark.parametrize("prec", [K.PREC_FP64, K.PREC_MIXED], ids=["fp64", "mixed"])
+def test_few_items_per_xcd(n, dist, q, c, prec):
+    """Fewer U-list items than XCDs, empty XCD runs, items of very unequal
+    cost: every target's potential is written once, on the device and on the
+    host, the same by every item list and launch form."""
+    prob = K.Problem.create(n, dist, q, np_=3, seed=21, coincide=c)
+    ev = K.GpuEvaluator(prob, precision=prec)
+    ev.evaluate(copy=False)
+    dev = ev.intermediate("pot")
+    for f in (K.P2P_STATIC, K.P2P_STATIC64, K.P2P_PERSISTENT) if prec == K.PREC_FP64 else (K.P2P_STATIC,):
+        for ov in (0, 1, 2):
+            ev.set_tuning(f, 8, K.HAD_MFMA, ov)
+            ev.output()[:] = np.nan
+            view, _ = ev.evaluate(copy="view")
+            assert np.array_equal(view, dev) and np.array_equal(ev.intermediate("pot"), dev), (f, ov)
+            own = np.full(ev.n_trg, np.nan)
+            ev.evaluate_into(own)
+            assert np.array_equal(own, dev), (f, ov)
+
+
 def test_phase_subsets_copy_out():
     """A subset of phases copies back what it computed (U-list last or absent)."""
     prob = K.Problem.create(280000, "ellipsoid", 64, np_=4, seed=12)
