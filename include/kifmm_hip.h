@@ -114,7 +114,7 @@ typedef struct kifmm_phase_times {
                        create time, so ~0 here               */
   double v_hadamard;/* spectral multiply-accumulate       */
   double v_ifft;    /* inverse DFT + check-surface gather */
-  double wlist;
+  double wlist;     /* W and X run in one launch, whose time is split by their pair counts */
   double xlist;
   double down;      /* L2L + DC2DE + L2T                  */
   double copy;      /* device -> host potentials: the part left after the last

@@ -11,15 +11,15 @@
  *   k_trans ........... compute_fft_trans__gpu_eval + D2Z x343  (874-963)
  *   k_hadamard ........ vlist_calc__gpu_eval                    (1200-1240)
  *   k_dft_inv ......... scale_nrmfc + cuFFT Z2D + regVal2SamVal (965-1196)
- *   k_wx<., false> .... wlist_eval__gpu                         (2070-2197)
- *   k_wx<., true> ..... xlist_eval__gpu                         (2380-2493)
+ *   k_wx .............. wlist_eval__gpu, xlist_eval__gpu        (2070-2197, 2380-2493)
  *   k_l2t ............. down_eval__gpu_leaves                   (1804-1872)
  *
  * The FP64 U-list gives a wave 8 targets held in scalar registers, its 64
  * lanes stride over a source tile staged in LDS, and the 8 per-lane partial
  * sums are combined by a 6-step butterfly (recursive halving) across the
- * wave.  The W / X lists and the L2T give each lane a target and read the
- * sources as wave-wide broadcasts.  Sources are (x, y, z, w) double4
+ * wave; the W / X lists do the same with the sources in registers.  The L2T
+ * gives each lane a target and reads the surface points as wave-wide
+ * broadcasts.  Sources are (x, y, z, w) double4
  * records; tiles are padded with zero-weight points far outside the root
  * box so no per-pair bounds checks are needed.
  */
@@ -2682,158 +2682,265 @@ __global__ __launch_bounds__(512) void k_dft_inv(const int* __restrict__ blocks,
 /* ------------------------------------------------- W, X and L2T evaluation */
 
 /* W- and X-list evaluation (wlist_eval__gpu, fmm/cuda.cu:2070-2197;
- * xlist_eval__gpu, fmm/cuda.cu:2380-2493): one wave per item, a lane per
- * target point, the point in registers for the whole item and its sum in
- * four lane-private accumulators (an item of at most 32 or 16 points runs
- * 2 or 4 source phases, one per lane group, added by a lane shuffle at the
- * end).  Item = two int4:
- *   a = {node t, first point, count <= 64, kind}: kind 0 the targets of
- *       leaf t (trg4 from tbeg[t]), kind 1 the DC check surface c + r SP of
- *       node t, results into dchk (X-list nodes with n_e or more targets);
- *   b = {first entry, end entry, partial slot or -1, 0}: a chunk of t's
- *       list (lidx), cut at entry boundaries.
- * The sources of entry s are leaf points (every X-list entry; W-list leaves
- * with fewer than n_e sources) or the UE surface c_s + r_s SP with the
- * densities uden[s] (other W-list nodes), staged WX_TILE at a time in LDS
- * and read as wave-wide broadcasts, the next tile loaded into registers
- * while the current one is summed.  A list longer than one chunk is split:
- * its chunks write their sums to part[slot][lane] and k_wx_reduce adds them
- * to the output in chunk order (deterministic). */
-constexpr int WX_TILE = 256;
-constexpr int WX_PER = WX_TILE / 64;
-constexpr int WX_CHUNK_SRC = 1024; /* sources per chunk (an entry is never split) */
+ * xlist_eval__gpu, fmm/cuda.cu:2380-2493), both in one launch of one-wave
+ * items.  An item is up to WX_T points of one node t, either targets of the
+ * leaf t or points of t's DC check surface (X-list nodes with n_e or more
+ * targets), times a chunk of its list.  A chunk is a run of ranges {code, n}:
+ * code >= 0 is n leaf sources from index code (every X-list entry; W-list
+ * leaves with fewer than n_e sources), code < 0 the n = n_e points of the UE
+ * surface of node ~code with its upward densities (other W-list entries).
+ *
+ * As in the U-list, the lanes hold sources and the points are wave-uniform
+ * (their Gram records come through scalar registers): the ranges, 35 - 56
+ * sources long on average, are laid out back to back over the lanes, so all
+ * 64 work whatever the entry sizes, where a lane per point left a third of
+ * them idle (41 points per list on average) and walked the list entry by
+ * entry, four dependent loads each.  A lane loads WX_P sources, moves them to t's frame and
+ * runs them against all points of the item; a butterfly sums the lanes at the
+ * end.  Per pair the Gram form of the U-list (9 VALU instructions; no clamp,
+ * no close pairs: gram items are at least CLOSE_FRAC h away).  A list entry
+ * nearer than that, a box more than four levels below t, goes into items of
+ * its own with WX_DIFF set, which use coordinate differences.
+ *
+ * Every item writes its sums to its own slot of part; k_wx_reduce adds the
+ * slots of a point in list order (deterministic, and W and X sums of the same
+ * target never race).  The plan picks the chunk size by the work in hand:
+ * short chunks where there is too little to fill the chip.
+ * Measured, W + X with their reductions, against a lane per point: 203 -> 171
+ * us at 1M ellipsoid points NP 4 (1.5e12 pairs/s; the padding of ~200-source
+ * lists to 64 lanes and of ~41 points to groups of 8 takes a third of the
+ * lane slots), 132 -> 81 at 300 thousand NP 6, 109 -> 25 at 16 thousand NP 6,
+ * 99 -> 12 at 4 thousand NP 3.  Two sources per lane (106 registers) or five
+ * waves per SIMD by force (20 bytes of spills) changed nothing. */
+constexpr int WX_T = 32, WX_G = WX_T / 8; /* points per item, groups of 8 */
+constexpr int WX_P = 4;                   /* sources per lane and pass */
+constexpr int WX_CAP = 1024;              /* sources per chunk at most */
+enum { WX_SURF = 1, WX_DIFF = 2, WX_W = 4, WX_X = 8 }; /* item flags; WX_W / WX_X also select lists in a launch */
 
-struct WxWalk {
-  int k, kend, base; /* entry, end of the chunk, offset within the entry */
-};
-
-/* Loads the next tile (up to WX_TILE sources of one entry, padded with
- * zero-weight far points) into registers; returns its count, 0 at the end. */
-template <bool XL>
-__device__ __forceinline__ int wx_fetch(WxWalk& w, const int* __restrict__ lidx, const int* __restrict__ child,
-                                        const int* __restrict__ snum, const int* __restrict__ sbeg,
-                                        const double4* __restrict__ geo, const double* __restrict__ surf_ue,
-                                        int ld_surf, int n_e, const double* __restrict__ uden, int ld_e,
-                                        const double4* __restrict__ src4, int lane, double4 (&pre)[WX_PER]) {
-  int s = 0, n = 0;
-  bool direct = true;
-  for (; w.k < w.kend; w.k++, w.base = 0) { /* skips entries without sources */
-    s = lidx[w.k];
-    direct = XL || (child[s] == -1 && snum[s] < n_e);
-    n = direct ? snum[s] : n_e;
-    if (w.base < n) break;
+static __global__ __launch_bounds__(64) void k_wx(const int4* __restrict__ items, /* {first range, end range, first point, points}, {node, slot, flags, sources} */
+                                                  const int2* __restrict__ rng, int lists,
+                                                  const double4* __restrict__ geo, const double* __restrict__ surf_ue,
+                                                  const double* __restrict__ surf_dc, int ld_surf,
+                                                  const double* __restrict__ uden, int ld_e,
+                                                  const double4* __restrict__ src4, const double4* __restrict__ trg4,
+                                                  const double4* __restrict__ trg_gram,
+                                                  const double4* __restrict__ dc_gram, double* __restrict__ part) {
+  __shared__ int2 map[WX_CAP]; /* source k: {-1, source index} or {node, surface point} */
+  const int4 a = items[2 * blockIdx.x], b = items[2 * blockIdx.x + 1];
+  if (!(b.z & lists)) return; /* whole block */
+  const int lane = threadIdx.x;
+  const double4 c = geo[b.x];
+  const double sc = GRAM_SC / c.w;
+  for (int rb = a.x, off = 0; rb < a.y; rb += 64) {
+    const int2 r = rng[min(rb + lane, a.y - 1)];
+    const int nr = min(64, a.y - rb);
+    for (int i = 0; i < nr; i++) {
+      const int code = __builtin_amdgcn_readlane(r.x, i), n = __builtin_amdgcn_readlane(r.y, i);
+      for (int l = lane; l < n; l += 64) map[off + l] = code >= 0 ? make_int2(-1, code + l) : make_int2(~code, l);
+      off += n;
+    }
   }
-  if (w.k >= w.kend) return 0;
-  const int cnt = min(WX_TILE, n - w.base);
-  if (direct) {
-    const double4* __restrict__ p = src4 + sbeg[s] + w.base;
+  __syncthreads();
+  double acc[WX_G][8];
 #pragma unroll
-    for (int m = 0; m < WX_PER; m++) {
+  for (int g = 0; g < WX_G; g++)
+#pragma unroll
+    for (int t = 0; t < 8; t++) acc[g][t] = 0.0;
+  const int ngroups = (a.w + 7) >> 3;
+  /* source k in absolute coordinates with its weight */
+  auto source = [&](int k) {
+    const int2 m = map[k];
+    if (m.x < 0) return src4[m.y];
+    const double4 g = geo[m.x];
+    return make_double4(g.x + g.w * surf_ue[m.y], g.y + g.w * surf_ue[ld_surf + m.y],
+                        g.z + g.w * surf_ue[2 * ld_surf + m.y], uden[(size_t)m.x * ld_e + m.y]);
+  };
+  if (!(b.z & WX_DIFF)) {
+    const double4* __restrict__ rec = (b.z & WX_SURF ? dc_gram : trg_gram) + a.z;
+    for (int base = 0; base < b.w; base += 64 * WX_P) {
+      double4 s[WX_P];
+      double w[WX_P];
+#pragma unroll
+      for (int p = 0; p < WX_P; p++) {
+        const int k = base + 64 * p + lane;
+        s[p] = make_double4(GRAM_FAR, GRAM_FAR, GRAM_FAR, 3.0 * GRAM_FAR * GRAM_FAR);
+        w[p] = 0.0;
+        if (k < b.w) {
+          const double4 q = source(k);
+          s[p] = gram_src(q, c, sc);
+          w[p] = q.w;
+        }
+      }
+      const int np = min(WX_P, (b.w - base + 63) >> 6); /* wave-uniform */
+#pragma unroll
+      for (int g = 0; g < WX_G; g++) {
+        if (g < ngroups) {
+          double4 r[8];
+#pragma unroll
+          for (int t = 0; t < 8; t++) r[t] = rec[min(8 * g + t, a.w - 1)];
+#pragma unroll
+          for (int p = 0; p < WX_P; p++) {
+            if (p < np) {
+#pragma unroll
+              for (int t = 0; t < 8; t++) {
+                const double r2 = __builtin_fma(r[t].x, s[p].x, __builtin_fma(r[t].y, s[p].y,
+                                                __builtin_fma(r[t].z, s[p].z, r[t].w + s[p].w)));
+                acc[g][t] = __builtin_fma(w[p], rsqrt2_fp64(r2), acc[g][t]);
+              }
+            }
+          }
+        }
+      }
+    }
+  } else {
+    /* lane l holds point l; each is broadcast to the wave in turn */
+    const int pt = a.z + min(lane, a.w - 1);
+    double4 q = trg4[b.z & WX_SURF ? 0 : pt];
+    if (b.z & WX_SURF)
+      q = make_double4(c.x + c.w * surf_dc[pt], c.y + c.w * surf_dc[ld_surf + pt], c.z + c.w * surf_dc[2 * ld_surf + pt], 0.0);
+    for (int base = 0; base < b.w; base += 64) {
+      double4 s = make_double4(FAR, FAR, FAR, 0.0);
+      if (base + lane < b.w) s = source(base + lane);
+#pragma unroll
+      for (int g = 0; g < WX_G; g++) {
+        if (g < ngroups) {
+#pragma unroll
+          for (int t = 0; t < 8; t++) {
+            const double dx = __shfl(q.x, 8 * g + t, 64) - s.x, dy = __shfl(q.y, 8 * g + t, 64) - s.y,
+                         dz = __shfl(q.z, 8 * g + t, 64) - s.z;
+            acc[g][t] = __builtin_fma(s.w, inv_r2<true>(__builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx))), acc[g][t]);
+          }
+        }
+      }
+    }
+  }
+  const double scale = b.z & WX_DIFF ? HALF_OOFP_R : HALF_OOFP_R * sc;
+#pragma unroll
+  for (int g = 0; g < WX_G; g++) {
+    if (g < ngroups) {
+      const double v = wave_reduce8(acc[g], lane);
+      if ((lane & 7) == 0) part[(size_t)b.y * WX_T + 8 * g + (lane >> 3)] = scale * v;
+    }
+  }
+}
+
+/* Adds the chunk sums of up to WX_T points to their outputs, W before X, each
+ * in list order.  Item = {output offset, points, 0 potentials / 1 check
+ * values, 0} and {first W slot, W slots, first X slot, X slots}; two items per
+ * wave. */
+static __global__ __launch_bounds__(64) void k_wx_reduce(const int4* __restrict__ items, int n_items, int lists,
+                                                         const double* __restrict__ part, double* __restrict__ pot,
+                                                         double* __restrict__ dchk) {
+  const int item = 2 * blockIdx.x + (threadIdx.x >> 5), l = threadIdx.x & 31;
+  if (item >= n_items) return;
+  const int4 a = items[2 * item], b = items[2 * item + 1];
+  if (l >= a.y) return;
+  double* const o = (a.z ? dchk : pot) + a.x + l;
+  double v = *o;
+  if (lists & WX_W) {
+    double s = 0.0;
+    for (int k = 0; k < b.y; k++) s += part[(size_t)(b.x + k) * WX_T + l];
+    v += s;
+  }
+  if (lists & WX_X) {
+    double s = 0.0;
+    for (int k = 0; k < b.w; k++) s += part[(size_t)(b.z + k) * WX_T + l];
+    v += s;
+  }
+  *o = v;
+}
+
+/* X-list sums onto DC check surfaces on the mixed path: one wave per item, a
+ * lane per surface point, the sources of one list entry at a time staged in
+ * LDS and read as wave-wide broadcasts, the next tile loaded meanwhile.  These
+ * sums pass through the pseudo-inverse into densities that the FP32 L2T
+ * rounds; another order of summation (k_wx's) flips roundings there, moving
+ * single potentials by 4e-8 of their size at 465 thousand points, so the
+ * mixed path keeps this one.  Item = {node t, first point, points <= 64, 0},
+ * {first range, end range, partial slot or -1, 0}; an item of at most 32 (16)
+ * points splits the wave into 2 (4) source phases, added by a lane shuffle. */
+__device__ __forceinline__ void add_scaled(double& o, double sum) { /* two roundings, not an FMA */
+#pragma clang fp contract(off)
+  const double v = HALF_OOFP_R * sum;
+  o = o + v;
+}
+constexpr int XS_TILE = 256, XS_PER = XS_TILE / 64;
+constexpr int XS_CHUNK = 1024; /* sources per chunk (an entry is never split) */
+static __global__ __launch_bounds__(64) void k_x_surf(const int4* __restrict__ items, const int2* __restrict__ rng,
+                                                      const double4* __restrict__ geo,
+                                                      const double* __restrict__ surf_dc, int ld_surf,
+                                                      const double4* __restrict__ src4, double* __restrict__ dchk,
+                                                      int ld_e, double* __restrict__ part) {
+  __shared__ double4 tile[XS_TILE];
+  const int4 a = items[2 * blockIdx.x], b = items[2 * blockIdx.x + 1];
+  const int lane = threadIdx.x;
+  const int lg = a.z <= 16 ? 2 : a.z <= 32 ? 1 : 0; /* log2 of the source phases, item-uniform */
+  const int tl = lane & ((64 >> lg) - 1), ph = lane >> (6 - lg);
+  const int pt = a.y + min(tl, a.z - 1);
+  const double4 g = geo[a.x];
+  const double tx = g.x + g.w * surf_dc[pt], ty = g.y + g.w * surf_dc[ld_surf + pt],
+               tz = g.z + g.w * surf_dc[2 * ld_surf + pt];
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  int k = b.x, base = 0;
+  int2 r = rng[k];
+  double4 pre[XS_PER];
+  /* the next tile (up to XS_TILE sources of one entry); 0 at the end */
+  auto fetch = [&] {
+    if (k >= b.y) return 0;
+    const int cnt = min(XS_TILE, r.y - base);
+    const double4* __restrict__ p = src4 + r.x + base;
+#pragma unroll
+    for (int m = 0; m < XS_PER; m++) {
       const int i = lane + 64 * m;
       pre[m] = i < cnt ? p[i] : make_double4(FAR, FAR, FAR, 0.0);
     }
-  } else {
-    const double4 g = geo[s];
-    const double* __restrict__ d = uden + (size_t)s * ld_e + w.base;
-#pragma unroll
-    for (int m = 0; m < WX_PER; m++) {
-      const int i = lane + 64 * m, j = w.base + i;
-      pre[m] = i < cnt ? make_double4(g.x + g.w * surf_ue[j], g.y + g.w * surf_ue[ld_surf + j],
-                                      g.z + g.w * surf_ue[2 * ld_surf + j], d[i])
-                       : make_double4(FAR, FAR, FAR, 0.0);
+    base += cnt;
+    if (base >= r.y) {
+      k++;
+      base = 0;
+      if (k < b.y) r = rng[k];
     }
-  }
-  w.base += cnt;
-  if (w.base >= n) {
-    w.k++;
-    w.base = 0;
-  }
-  return cnt;
-}
-
-/* acc[u] += 2 w / |x - p| over the staged sources j0 + u, j0 = first,
- * first + stride, ... < n4 (n4, first and stride multiples of 4) */
-template <bool MASK>
-__device__ __forceinline__ void wx_sum_tile(const double4* tile, int n4, int first, int stride, double tx, double ty,
-                                            double tz, double (&acc)[4]) {
-  for (int j = first; j < n4; j += stride) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const double4 p = tile[j + u];
-      const double dx = tx - p.x, dy = ty - p.y, dz = tz - p.z;
-      const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-      acc[u] = __builtin_fma(p.w, inv_r2<MASK>(r2), acc[u]);
-    }
-  }
-}
-
-/* XL = false: W-list (lidx = w_idx), XL = true: X-list (lidx = x_idx) */
-template <bool MASK, bool XL>
-__global__ __launch_bounds__(64) void k_wx(const int4* __restrict__ items, const int* __restrict__ lidx,
-                                           const int* __restrict__ child, const int* __restrict__ snum,
-                                           const int* __restrict__ sbeg, const int* __restrict__ tbeg,
-                                           const double4* __restrict__ geo, const double* __restrict__ surf_ue,
-                                           const double* __restrict__ surf_dc, int ld_surf, int n_e,
-                                           const double* __restrict__ uden, int ld_e,
-                                           const double4* __restrict__ src4, const double4* __restrict__ trg4,
-                                           double* __restrict__ pot, double* __restrict__ dchk,
-                                           double* __restrict__ part) {
-  __shared__ double4 tile[WX_TILE];
-  const int4 a = items[2 * blockIdx.x], b = items[2 * blockIdx.x + 1];
-  const int lane = threadIdx.x;
-  /* an item of at most 32 (16) points splits the wave into 2 (4) source
-   * phases of 64 / G lanes: lane = phase * (64 / G) + point, phase ph takes
-   * the source quads 4 (ph + G i); the phases' sums meet in a lane shuffle */
-  const int lg = a.z <= 16 ? 2 : a.z <= 32 ? 1 : 0; /* log2 G, item-uniform */
-  const int tl = lane & ((64 >> lg) - 1), ph = lane >> (6 - lg);
-  const int pt = a.y + min(tl, a.z - 1);
-  double tx, ty, tz;
-  if (a.w) {
-    const double4 g = geo[a.x];
-    tx = g.x + g.w * surf_dc[pt];
-    ty = g.y + g.w * surf_dc[ld_surf + pt];
-    tz = g.z + g.w * surf_dc[2 * ld_surf + pt];
-  } else {
-    const double4 q = trg4[tbeg[a.x] + pt];
-    tx = q.x; ty = q.y; tz = q.z;
-  }
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  WxWalk w{b.x, b.y, 0};
-  double4 pre[WX_PER];
-  int cnt = wx_fetch<XL>(w, lidx, child, snum, sbeg, geo, surf_ue, ld_surf, n_e, uden, ld_e, src4, lane, pre);
+    return cnt;
+  };
+  int cnt = fetch();
   while (cnt > 0) {
     __syncthreads(); /* the previous tile's reads are done (one wave: an LDS ordering point) */
 #pragma unroll
-    for (int m = 0; m < WX_PER; m++) tile[lane + 64 * m] = pre[m];
+    for (int m = 0; m < XS_PER; m++) tile[lane + 64 * m] = pre[m];
     __syncthreads();
-    const int next = wx_fetch<XL>(w, lidx, child, snum, sbeg, geo, surf_ue, ld_surf, n_e, uden, ld_e, src4, lane, pre);
-    if (a.w) wx_sum_tile<false>(tile, (cnt + 3) & ~3, 4 * ph, 4 << lg, tx, ty, tz, acc);
-    else wx_sum_tile<MASK>(tile, (cnt + 3) & ~3, 4 * ph, 4 << lg, tx, ty, tz, acc);
+    const int next = fetch();
+    for (int j = 4 * ph; j < ((cnt + 3) & ~3); j += 4 << lg) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const double4 p = tile[j + u];
+        const double dx = tx - p.x, dy = ty - p.y, dz = tz - p.z;
+        const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+        acc[u] = __builtin_fma(p.w, inv_r2<false>(r2), acc[u]);
+      }
+    }
     cnt = next;
   }
   double sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   for (int m = 64 >> lg; m < 64; m <<= 1) sum += __shfl_xor(sum, m, 64);
   if (ph == 0 && tl < a.z) {
     if (b.z >= 0) part[(size_t)b.z * 64 + tl] = sum;
-    else if (a.w) dchk[(size_t)a.x * ld_e + a.y + tl] += HALF_OOFP_R * sum;
-    else pot[tbeg[a.x] + a.y + tl] += HALF_OOFP_R * sum;
+    else add_scaled(dchk[(size_t)a.x * ld_e + a.y + tl], sum);
   }
 }
 
-/* Adds the chunk sums of a split W / X item to its output, in chunk order.
- * Item = {node t, first point, count, kind} and {first slot, slots, 0, 0}. */
-static __global__ __launch_bounds__(64) void k_wx_reduce(const int4* __restrict__ items,
-                                                        const int* __restrict__ tbeg, int ld_e,
-                                                        const double* __restrict__ part,
-                                                        double* __restrict__ pot, double* __restrict__ dchk) {
+/* The chunk sums of a split k_x_surf item, in chunk order.  Item = {node,
+ * first point, points, 0} and {first slot, slots, 0, 0}. */
+static __global__ __launch_bounds__(64) void k_x_surf_reduce(const int4* __restrict__ items, int ld_e,
+                                                            const double* __restrict__ part,
+                                                            double* __restrict__ dchk) {
   const int4 a = items[2 * blockIdx.x], b = items[2 * blockIdx.x + 1];
   const int lane = threadIdx.x;
   if (lane >= a.z) return;
   double s = 0.0;
   for (int c = 0; c < b.y; c++) s += part[(size_t)(b.x + c) * 64 + lane];
-  if (a.w) dchk[(size_t)a.x * ld_e + a.y + lane] += HALF_OOFP_R * s;
-  else pot[tbeg[a.x] + a.y + lane] += HALF_OOFP_R * s;
+  add_scaled(dchk[(size_t)a.x * ld_e + a.y + lane], s);
 }
+
 /* L2T (down_eval__gpu_leaves, fmm/cuda.cu:1804-1872): item = {leaf, first
  * target, count <= 64}, one wave; lane = target, the leaf's DE surface
  * points c + r * SP_DE[j] with densities dden[leaf][j] are wave-uniform. */

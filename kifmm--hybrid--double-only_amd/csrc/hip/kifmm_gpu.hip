@@ -90,8 +90,7 @@ struct kifmm_gpu {
   float *surf_uc32 = nullptr, *surf_de32 = nullptr;
   float4* src32 = nullptr;
   int *cube2surf = nullptr, *surf2cube = nullptr;
-  int *child = nullptr, *snum = nullptr, *sbeg = nullptr, *tbeg = nullptr, *depth = nullptr, *tag = nullptr;
-  int *widx = nullptr, *xidx = nullptr;
+  int *snum = nullptr, *sbeg = nullptr, *depth = nullptr, *tag = nullptr;
   int *u_ptr = nullptr, *u_idx = nullptr; /* U-list CSR (node ids), for the close-pair search */
   /* work lists */
   int4* p2p_items = nullptr; int n_p2p = 0;
@@ -110,7 +109,9 @@ struct kifmm_gpu {
   /* mixed path: per target, the U-list sources closer than MIX_CLOSE h */
   int* cptr = nullptr; int* cidx = nullptr;
   int close_listed = 0;
-  double4* trg_gram = nullptr; /* FP64 Gram-form U-list: (-2t', |t'|^2) per target, when close_listed */
+  int gram_u = 0;              /* the U-list runs on the FP64 Gram form: close pairs listed, FP64 path */
+  double4* trg_gram = nullptr; /* (-2t', |t'|^2) per target, for gram_u and the W / X lists */
+  double4* dc_gram = nullptr;  /* the same of the DC check surface in its node's frame */
   long long n_close = 0;
   int4* s2m_items = nullptr; int n_s2m = 0;
   GemmList s2m_gemm;
@@ -120,11 +121,13 @@ struct kifmm_gpu {
   int4* hgroups = nullptr; int n_hgroups = 0;
   int* huslots = nullptr;
   unsigned char* hloc = nullptr;
-  int4* witems = nullptr; int n_witems = 0; /* k_wx items, two int4 each */
-  int4* xitems = nullptr; int n_xitems = 0;
-  int4* wred = nullptr; int n_wred = 0;     /* k_wx_reduce items of split lists */
-  int4* xred = nullptr; int n_xred = 0;
-  double* wxpart = nullptr;                 /* chunk sums of split lists, 64 per slot */
+  int4* wx_items = nullptr; int n_wx = 0;   /* k_wx items, two int4 each */
+  int4* wx_red = nullptr; int n_wxred = 0;  /* k_wx_reduce items, two int4 each */
+  int2* wx_rng = nullptr;                   /* their source ranges */
+  int4* xs_items = nullptr; int n_xs = 0;   /* mixed path: k_x_surf items, two int4 each */
+  int4* xs_red = nullptr; int n_xsred = 0;  /* and the reductions of split ones */
+  double* wxpart = nullptr;                 /* chunk sums, WX_T per slot (k_x_surf: 64) */
+  bool wx_targets = false;                  /* some item's points are targets */
   int4* l2t_items = nullptr; int n_l2t = 0;
   size_t chk_cols = 0;
   double* ws = nullptr;
@@ -316,9 +319,11 @@ struct Plan {
   std::vector<HostLevel> lv;
   size_t chk_cols = 0;
   size_t ws_len = 0;
-  std::vector<int> vblocks, vslot, hnbr, hslot, wleaves, xnodes, l2t;
-  std::vector<int4> witems, xitems, wred, xred; /* two int4 per item */
-  int wx_slots = 0, w_slots = 0, x_slots = 0;     /* partial slots of split W / X lists */
+  std::vector<int> vblocks, vslot, hnbr, hslot, l2t;
+  std::vector<int4> wx_items, wx_red, xs_items, xs_red; /* two int4 per item */
+  std::vector<int2> wx_rng;
+  int wx_slots = 0, xs_slots = 0;
+  bool wx_targets = false; /* some W / X item's points are targets */
   std::vector<int4> l2t_items;
   std::vector<int4> hgroups;
   std::vector<int> huslots;
@@ -436,7 +441,204 @@ XcdRuns xcd_runs(const std::vector<double>& cost, int b, int e) {
   return r;
 }
 
-int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
+/* The W / X items (k_wx) and their reductions.  Per target node and list,
+ * the entries' sources as ranges, far ones (Gram form) before near ones,
+ * cut into chunks; the node's points in blocks of WX_T; an item per block and
+ * chunk with a slot of its own, the slots of a block's chunks consecutive.
+ * Chunks hold WX_CAP sources on inputs with plenty of work; below, as many
+ * as leave about WX_ITEMS items (16 waves on each of 256 CUs), at least 128:
+ * a 4 thousand point input has 33 W blocks, and walking 1024 sources each
+ * took 82 us on an otherwise idle chip.  Items run largest first.  On the
+ * mixed path the X sums onto check surfaces are k_x_surf's: blocks of 64
+ * points, chunks of XS_CHUNK sources cut at entry boundaries. */
+int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
+  constexpr long WX_ITEMS = 4096;
+  const int nn = t->n_nodes;
+  auto w_of = [&](int i) { return t->child[i] == -1 && (t->tag[i] & KIFMM_TRGNODE) && t->w_ptr[i + 1] > t->w_ptr[i]; };
+  auto x_of = [&](int i) { return (t->tag[i] & KIFMM_TRGNODE) && t->x_ptr[i + 1] > t->x_ptr[i]; };
+  /* a list entry as a range, {0, 0} if it has no sources */
+  auto range = [&](int s, bool xl) {
+    if (xl || (t->child[s] == -1 && t->src_num[s] < ne))
+      return t->src_num[s] > 0 ? make_int2(t->src_beg[s], t->src_num[s]) : make_int2(0, 0);
+    return make_int2(~s, ne);
+  };
+  auto points = [&](int i, bool xl, bool& surf) {
+    surf = xl && !(t->child[i] == -1 && t->trg_num[i] < ne);
+    return surf ? ne : t->trg_num[i];
+  };
+  /* whether box s stays CLOSE_FRAC h away from box i (h = i's half-width) */
+  auto far = [&](int i, int s) {
+    const double hi = 1.0 / (1 << t->depth[i]), hs = 1.0 / (1 << t->depth[s]);
+    double d2 = 0.0;
+    for (int k = 0; k < 3; k++) {
+      const double gap = std::fabs((2 * t->path[3 * i + k] + 1) * hi - (2 * t->path[3 * s + k] + 1) * hs) - (hi + hs);
+      if (gap > 0.0) d2 += gap * gap;
+    }
+    return d2 >= CLOSE_FRAC * CLOSE_FRAC * hi * hi;
+  };
+  long total = 0; /* sources x blocks */
+  for (int i = 0; i < nn; i++)
+    for (int xl = 0; xl < 2; xl++) {
+      if (!(xl ? x_of(i) : w_of(i))) continue;
+      bool surf;
+      const long blocks = (points(i, xl, surf) + WX_T - 1) / WX_T;
+      if (mixed && surf) continue;
+      const int *ptr = xl ? t->x_ptr : t->w_ptr, *idx = xl ? t->x_idx : t->w_idx;
+      for (int k = ptr[i]; k < ptr[i + 1]; k++) total += blocks * range(idx[k], xl).y;
+    }
+  const int chunk = (int)std::min<long>(WX_CAP, std::max<long>(128, (total / WX_ITEMS + 63) / 64 * 64));
+  struct Chunk {
+    int rb, re, n, flags;
+  };
+  std::vector<Chunk> chunks;
+  std::vector<int2> lists[2]; /* far, near */
+  std::vector<std::pair<long, std::array<int4, 2>>> work, xs_work;
+  auto sorted = [](std::vector<std::pair<long, std::array<int4, 2>>>& w, std::vector<int4>& out) {
+    std::stable_sort(w.begin(), w.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+    for (const auto& e : w) {
+      out.push_back(e.second[0]);
+      out.push_back(e.second[1]);
+    }
+  };
+  for (int i = 0; i < nn; i++) {
+    size_t wred_at = 0; /* the node's W reductions, to which X sums of the same targets are added */
+    bool wred = false;
+    for (int xl = 0; xl < 2; xl++) {
+      if (!(xl ? x_of(i) : w_of(i))) continue;
+      bool surf;
+      const int npts = points(i, xl, surf);
+      const int *ptr = xl ? t->x_ptr : t->w_ptr, *idx = xl ? t->x_idx : t->w_idx;
+      if (mixed && surf) { /* one range per entry, chunks as rng index ranges */
+        chunks.clear();
+        Chunk c{(int)P.wx_rng.size(), 0, 0, 0};
+        for (int k = ptr[i]; k < ptr[i + 1]; k++) {
+          const int2 r = range(idx[k], true);
+          if (r.y <= 0) continue;
+          if (c.n > 0 && c.n + r.y > XS_CHUNK) {
+            c.re = (int)P.wx_rng.size();
+            chunks.push_back(c);
+            c = Chunk{(int)P.wx_rng.size(), 0, 0, 0};
+          }
+          P.wx_rng.push_back(r);
+          c.n += r.y;
+        }
+        c.re = (int)P.wx_rng.size();
+        if (c.n > 0) chunks.push_back(c);
+        const int nch = (int)chunks.size();
+        for (int p = 0; p < npts && nch > 0; p += 64) {
+          const int4 a = make_int4(i, p, std::min(64, npts - p), 0);
+          for (int h = 0; h < nch; h++)
+            xs_work.push_back({chunks[h].n, {a, make_int4(chunks[h].rb, chunks[h].re, nch > 1 ? P.xs_slots + h : -1, 0)}});
+          if (nch > 1) {
+            P.xs_red.push_back(a);
+            P.xs_red.push_back(make_int4(P.xs_slots, nch, 0, 0));
+            P.xs_slots += nch;
+          }
+        }
+        continue;
+      }
+      lists[0].clear();
+      lists[1].clear();
+      for (int k = ptr[i]; k < ptr[i + 1]; k++) {
+        const int2 r = range(idx[k], xl);
+        if (r.y <= 0) continue;
+        std::vector<int2>& L = lists[far(i, idx[k]) ? 0 : 1];
+        if (r.x >= 0 && !L.empty() && L.back().x >= 0 && L.back().x + L.back().y == r.x) L.back().y += r.y;
+        else L.push_back(r);
+      }
+      chunks.clear();
+      for (int near = 0; near < 2; near++) {
+        Chunk c{(int)P.wx_rng.size(), 0, 0, near ? WX_DIFF : 0};
+        auto close = [&] {
+          if (c.n > 0) {
+            c.re = (int)P.wx_rng.size();
+            chunks.push_back(c);
+          }
+          c.rb = (int)P.wx_rng.size();
+          c.n = 0;
+        };
+        for (int2 r : lists[near]) {
+          if (r.x < 0) { /* a surface is never split */
+            if (c.n > 0 && c.n + r.y > chunk) close();
+            P.wx_rng.push_back(r);
+            c.n += r.y;
+            continue;
+          }
+          while (r.y > 0) {
+            if (c.n >= chunk) close();
+            const int take = std::min(r.y, chunk - c.n);
+            P.wx_rng.push_back(make_int2(r.x, take));
+            c.n += take;
+            r.x += take;
+            r.y -= take;
+          }
+        }
+        close();
+      }
+      if (chunks.empty() || npts <= 0) continue;
+      if (!surf) P.wx_targets = true;
+      const int out0 = surf ? i * lde : t->trg_beg[i];
+      const bool join = xl && !surf && wred;
+      if (!xl) {
+        wred = true;
+        wred_at = P.wx_red.size();
+      }
+      for (int p = 0, m = 0; p < npts; p += WX_T, m++) {
+        const int cnt = std::min(WX_T, npts - p), slot0 = P.wx_slots;
+        for (const Chunk& c : chunks)
+          work.push_back({(long)((c.n + 63) / 64) * ((cnt + 7) / 8),
+                          {make_int4(c.rb, c.re, surf ? p : t->trg_beg[i] + p, cnt),
+                           make_int4(i, P.wx_slots++, c.flags | (surf ? WX_SURF : 0) | (xl ? WX_X : WX_W), c.n)}});
+        const int nch = P.wx_slots - slot0;
+        if (join) {
+          int4& b = P.wx_red[wred_at + 2 * m + 1];
+          b.z = slot0;
+          b.w = nch;
+        } else {
+          P.wx_red.push_back(make_int4(out0 + p, cnt, surf ? 1 : 0, 0));
+          P.wx_red.push_back(xl ? make_int4(0, 0, slot0, nch) : make_int4(slot0, nch, 0, 0));
+        }
+      }
+    }
+  }
+  sorted(work, P.wx_items);
+  sorted(xs_work, P.xs_items);
+  /* what k_wx, k_x_surf and their reductions index */
+  bool ok = true;
+  for (const int2& r : P.wx_rng)
+    ok = ok && (r.x >= 0 ? r.y >= 1 && (long)r.x + r.y <= t->n_src : ~r.x < nn && r.y == ne);
+  for (size_t m = 0; m < P.wx_items.size(); m += 2) {
+    const int4 a = P.wx_items[m], b = P.wx_items[m + 1];
+    int n = 0;
+    for (int k = a.x; k < a.y; k++) n += P.wx_rng[k].y;
+    ok = ok && a.x >= 0 && a.y <= (int)P.wx_rng.size() && a.w >= 1 && a.w <= WX_T && a.z >= 0 &&
+         (long)a.z + a.w <= (b.z & WX_SURF ? ne : t->n_trg) && b.x >= 0 && b.x < nn && b.y >= 0 && b.y < P.wx_slots &&
+         b.w == n && n >= 1 && n <= WX_CAP;
+  }
+  for (size_t m = 0; m < P.wx_red.size(); m += 2) {
+    const int4 a = P.wx_red[m], b = P.wx_red[m + 1];
+    ok = ok && a.x >= 0 && a.y >= 1 && a.y <= WX_T && (long)a.x + a.y <= (a.z ? (long)nn * lde : (long)t->n_trg) &&
+         b.x >= 0 && b.x + b.y <= P.wx_slots && b.z >= 0 && b.z + b.w <= P.wx_slots;
+  }
+  for (size_t m = 0; m < P.xs_items.size(); m += 2) {
+    const int4 a = P.xs_items[m], b = P.xs_items[m + 1];
+    ok = ok && a.x >= 0 && a.x < nn && a.y >= 0 && a.z >= 1 && a.z <= 64 && a.y + a.z <= ne && b.x >= 0 && b.x < b.y &&
+         b.y <= (int)P.wx_rng.size() && b.z < P.xs_slots;
+    for (int k = b.x; ok && k < b.y; k++) ok = P.wx_rng[k].x >= 0;
+  }
+  for (size_t m = 0; m < P.xs_red.size(); m += 2) {
+    const int4 a = P.xs_red[m], b = P.xs_red[m + 1];
+    ok = ok && a.x >= 0 && a.x < nn && a.y >= 0 && a.z >= 1 && a.z <= 64 && a.y + a.z <= ne && b.x >= 0 && b.y >= 2 &&
+         b.x + b.y <= P.xs_slots;
+  }
+  if (!ok) {
+    set_error("internal: W / X work item out of range");
+    return KIFMM_EINVAL;
+  }
+  return KIFMM_OK;
+}
+
+int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, Plan& P) {
   TRY(check_view(t));
   const int np = t->np;
   P.np = np;
@@ -699,7 +901,6 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
     const bool leaf = t->child[i] == -1;
     const bool trg = (t->tag[i] & KIFMM_TRGNODE) != 0;
     if (trg && leaf && t->w_ptr[i + 1] > t->w_ptr[i]) {
-      P.wleaves.push_back(i);
       for (int k = t->w_ptr[i]; k < t->w_ptr[i + 1]; k++) {
         const int s = t->w_idx[k];
         const bool direct = t->child[s] == -1 && t->src_num[s] < ne;
@@ -707,7 +908,6 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
       }
     }
     if (trg && t->x_ptr[i + 1] > t->x_ptr[i]) {
-      P.xnodes.push_back(i);
       const bool direct = leaf && t->trg_num[i] < ne;
       for (int k = t->x_ptr[i]; k < t->x_ptr[i + 1]; k++)
         wc.x_pairs += (double)t->src_num[t->x_idx[k]] * (direct ? t->trg_num[i] : ne);
@@ -719,73 +919,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, Plan& P) {
         P.l2t_items.push_back(make_int4(i, t->trg_beg[i] + c, std::min(64, t->trg_num[i] - c), 0));
     }
   }
-  /* W / X items (k_wx): per target node, its list cut at entry boundaries
-   * into chunks of at most WX_CHUNK_SRC sources (an entry larger than that is
-   * a chunk of its own), and its points into blocks of 64; one item per
-   * (block, chunk).  A node with several chunks gets a partial slot per item
-   * and a reduce item per block.  Items run longest chunk first. */
-  auto wx_plan = [&](const std::vector<int>& nodes, const int* ptr, const int* idx, bool xl, std::vector<int4>& items,
-                     std::vector<int4>& red) {
-    std::vector<std::pair<long, std::array<int4, 2>>> work;
-    for (int i : nodes) {
-      const int kind = xl && !(t->child[i] == -1 && t->trg_num[i] < ne) ? 1 : 0;
-      const int npts = kind ? ne : t->trg_num[i];
-      std::vector<int> cut{ptr[i]};
-      std::vector<long> cost;
-      long acc = 0;
-      for (int k = ptr[i]; k < ptr[i + 1]; k++) {
-        const int s_ = idx[k];
-        const long n = xl || (t->child[s_] == -1 && t->src_num[s_] < ne) ? t->src_num[s_] : ne;
-        if (acc > 0 && acc + n > WX_CHUNK_SRC) {
-          cut.push_back(k);
-          cost.push_back(acc);
-          acc = 0;
-        }
-        acc += n;
-      }
-      cut.push_back(ptr[i + 1]);
-      cost.push_back(acc);
-      const int nch = (int)cost.size();
-      for (int c = 0; c < npts; c += 64) {
-        const int4 a = make_int4(i, c, std::min(64, npts - c), kind);
-        const int slot0 = nch > 1 ? P.wx_slots : -1;
-        for (int h = 0; h < nch; h++)
-          work.push_back({cost[h], {a, make_int4(cut[h], cut[h + 1], nch > 1 ? P.wx_slots + h : -1, 0)}});
-        if (nch > 1) {
-          red.push_back(a);
-          red.push_back(make_int4(slot0, nch, 0, 0));
-          P.wx_slots += nch;
-        }
-      }
-    }
-    std::stable_sort(work.begin(), work.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
-    for (const auto& w : work) {
-      items.push_back(w.second[0]);
-      items.push_back(w.second[1]);
-    }
-  };
-  P.wx_slots = 0;
-  wx_plan(P.wleaves, t->w_ptr, t->w_idx, false, P.witems, P.wred);
-  P.w_slots = P.wx_slots;
-  P.wx_slots = 0;
-  wx_plan(P.xnodes, t->x_ptr, t->x_idx, true, P.xitems, P.xred);
-  P.x_slots = P.wx_slots;
-  /* k_wx clamps point indices to [first, first + count - 1] of its item and
-   * reads trg4 from tbeg[t] (kind 0) or the n_e-point DC surface (kind 1) */
-  auto wx_check = [&](const std::vector<int4>& v, const int* ptr, int slots, bool reduce) {
-    for (size_t m = 0; m < v.size(); m += 2) {
-      const int4 a = v[m], b = v[m + 1];
-      if (a.x < 0 || a.x >= nn || a.z < 1 || a.z > 64 || a.y < 0 || a.y + a.z > (a.w ? ne : t->trg_num[a.x]))
-        return false;
-      if (!reduce && (b.x < ptr[a.x] || b.y > ptr[a.x + 1] || b.x >= b.y || b.z >= slots)) return false;
-      if (reduce && (b.x < 0 || b.y < 2 || b.x + b.y > slots)) return false;
-    }
-    return true;
-  };
-  if (!wx_check(P.witems, t->w_ptr, P.w_slots, false) || !wx_check(P.wred, t->w_ptr, P.w_slots, true))
-    return fail("W-list item out of range");
-  if (!wx_check(P.xitems, t->x_ptr, P.x_slots, false) || !wx_check(P.xred, t->x_ptr, P.x_slots, true))
-    return fail("X-list item out of range");
+  TRY(wx_plan(t, ne, lde, mixed, P));
   for (int i : P.l2t)
     if (t->trg_num[i] < 1) return fail("L2T leaf without targets");
   /* k_l2t reads trg4[it.y .. it.y + it.z - 1] and the leaf's DE densities */
@@ -860,14 +994,10 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
                             -1.0 + (2.0 * 1.0) * (t->path[3 * i + 2] + 0.5) / sc, 1.0 / sc);
     }
     TRY(dev_upload(g, &g->geo, geo.data(), geo.size()));
-    TRY(dev_upload(g, &g->child, t->child, nn));
     TRY(dev_upload(g, &g->snum, t->src_num, nn));
     TRY(dev_upload(g, &g->sbeg, t->src_beg, nn));
-    TRY(dev_upload(g, &g->tbeg, t->trg_beg, nn));
     TRY(dev_upload(g, &g->depth, t->depth, nn));
     TRY(dev_upload(g, &g->tag, t->tag, nn));
-    TRY(dev_upload(g, &g->widx, t->w_idx, t->w_ptr[nn]));
-    TRY(dev_upload(g, &g->xidx, t->x_idx, t->x_ptr[nn]));
     TRY(dev_upload(g, &g->u_ptr, t->u_ptr, (size_t)nn + 1));
     TRY(dev_upload(g, &g->u_idx, t->u_idx, t->u_ptr[nn]));
     TRY(dev_zero(g, &g->uden, (size_t)nn * lde));
@@ -916,6 +1046,13 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
     }
     std::fill(s.begin(), s.end(), 0.0);
     host_surface(np, 1.0, s, ls); TRY(dev_upload(g, &g->surf_dc, s.data(), s.size()));
+    {
+      std::vector<double4> r(ne);
+      for (int j = 0; j < ne; j++)
+        r[j] = make_double4(-2.0 * GRAM_SC * s[j], -2.0 * GRAM_SC * s[ls + j], -2.0 * GRAM_SC * s[2 * ls + j],
+                            GRAM_SC * GRAM_SC * s[3 * ls + j]);
+      TRY(dev_upload(g, &g->dc_gram, r.data(), r.size()));
+    }
     const int N = g->N;
     std::vector<double2> w(N);
     for (int m = 0; m < N; m++) {
@@ -996,16 +1133,18 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
     TRY(dev_zero(g, &g->Y, spec));
     TRY(dev_zero(g, &g->T, (size_t)g->F * 343));
   }
-  g->n_witems = (int)P.witems.size() / 2;
-  g->n_xitems = (int)P.xitems.size() / 2;
-  g->n_wred = (int)P.wred.size() / 2;
-  g->n_xred = (int)P.xred.size() / 2;
+  g->n_wx = (int)P.wx_items.size() / 2;
+  g->n_wxred = (int)P.wx_red.size() / 2;
+  g->wx_targets = P.wx_targets;
+  g->n_xs = (int)P.xs_items.size() / 2;
+  g->n_xsred = (int)P.xs_red.size() / 2;
   g->n_l2t = (int)P.l2t_items.size();
-  TRY(dev_upload(g, &g->witems, P.witems.data(), P.witems.size()));
-  TRY(dev_upload(g, &g->xitems, P.xitems.data(), P.xitems.size()));
-  TRY(dev_upload(g, &g->wred, P.wred.data(), P.wred.size()));
-  TRY(dev_upload(g, &g->xred, P.xred.data(), P.xred.size()));
-  TRY(dev_zero(g, &g->wxpart, (size_t)std::max(P.w_slots, P.x_slots) * 64));
+  TRY(dev_upload(g, &g->wx_items, P.wx_items.data(), P.wx_items.size()));
+  TRY(dev_upload(g, &g->wx_red, P.wx_red.data(), P.wx_red.size()));
+  TRY(dev_upload(g, &g->wx_rng, P.wx_rng.data(), P.wx_rng.size()));
+  TRY(dev_upload(g, &g->xs_items, P.xs_items.data(), P.xs_items.size()));
+  TRY(dev_upload(g, &g->xs_red, P.xs_red.data(), P.xs_red.size()));
+  TRY(dev_zero(g, &g->wxpart, std::max((size_t)P.wx_slots * WX_T, (size_t)P.xs_slots * 64)));
   TRY(dev_upload(g, &g->l2t_items, P.l2t_items.data(), P.l2t_items.size()));
   return KIFMM_OK;
 }
@@ -1109,9 +1248,11 @@ int trans_setup(kifmm_gpu* g) {
   }
 }
 
-/* FP64 path with listed close pairs: the U-list runs on the Gram form
- * (k_p2p_ulist<., ., true>), whose per-target records are written here. */
+/* The per-target records of the Gram form, for the FP64 U-list with listed
+ * close pairs (k_p2p_ulist<., ., true>) and the W / X items on targets. */
 int gram_setup(kifmm_gpu* g) {
+  g->gram_u = g->precision == KIFMM_PREC_FP64 && g->close_listed;
+  if (!g->gram_u && !g->wx_targets) return KIFMM_OK;
   TRY(dev_zero(g, &g->trg_gram, (size_t)std::max(g->n_trg, 1)));
   if (g->n_p2p > 0)
     hipLaunchKernelGGL(k_trg_gram, dim3(g->n_p2p), dim3(128), 0, g->stream, g->p2p_items, g->geo, g->trg4,
@@ -1278,8 +1419,8 @@ constexpr double U_SMALL = 96.0;
 int u_list_index(const kifmm_gpu* g) {
   if (g->precision == KIFMM_PREC_MIXED) return g->close_listed && g->p2p_form != KIFMM_P2P_SPLIT ? 3 : 0;
   if (g->p2p_form == KIFMM_P2P_STATIC64) return 1;
-  if (g->p2p_form == KIFMM_P2P_STATIC && g->trg_gram && g->n_trg <= U_SMALL * g->n_p2p5) return 1;
-  return g->trg_gram ? 2 : 0;
+  if (g->p2p_form == KIFMM_P2P_STATIC && g->gram_u && g->n_trg <= U_SMALL * g->n_p2p5) return 1;
+  return g->gram_u ? 2 : 0;
 }
 
 /* U-list over the items of copy-out chunks [c0, c1) on stream st, writing
@@ -1308,7 +1449,7 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
       hipLaunchKernelGGL(k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr, g->rng,
                          g->geo, g->src4, g->trg4, out, host, accum);
   } else if (l == 1) {
-    if (g->trg_gram)
+    if (g->gram_u)
       hipLaunchKernelGGL((k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
                          g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
@@ -1317,7 +1458,7 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
   } else if (g->p2p_form == KIFMM_P2P_PERSISTENT) {
     int* counters = g->p2p_counters + 8 * std::max(chunk, 0);
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, counters, 8, 0);
-    if (g->trg_gram)
+    if (g->gram_u)
       hipLaunchKernelGGL((k_p2p_ulist_persist<MASK, P2P_G5, true>), dim3(g->persist_grid[1]), dim3(256), 0, st, items,
                          runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
@@ -1326,7 +1467,7 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
                          runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
   } else {
-    if (g->trg_gram)
+    if (g->gram_u)
       hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G5, true>), dim3(8 * per), dim3(256), 0, st, items, runs,
                          g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
@@ -1358,33 +1499,33 @@ int early_chunks(const kifmm_gpu* g, unsigned mask) {
   }
 }
 
-template <bool MASK>
-int point_phases_wx(kifmm_gpu* g, unsigned mask, hipEvent_t ew) {
-  if ((mask & KIFMM_PHASE_W) && g->n_witems > 0) {
-    hipLaunchKernelGGL((k_wx<MASK, false>), dim3(g->n_witems), dim3(64), 0, g->stream, g->witems, g->widx, g->child,
-                       g->snum, g->sbeg, g->tbeg, g->geo, g->surf_ue, g->surf_dc, g->ld_surf, g->n_e, g->uden,
-                       g->ld_e, g->src4, g->trg4, g->pot, g->dchk, g->wxpart);
-    if (g->n_wred > 0)
-      hipLaunchKernelGGL(k_wx_reduce, dim3(g->n_wred), dim3(64), 0, g->stream, g->wred, g->tbeg, g->ld_e, g->wxpart,
-                         g->pot, g->dchk);
+/* W and X in one launch (lists: which of the two) and the sums of their
+ * chunks; on the mixed path the X sums onto check surfaces on their own */
+int wx_phase(kifmm_gpu* g, unsigned mask) {
+  const int lists = (mask & KIFMM_PHASE_W ? WX_W : 0) | (mask & KIFMM_PHASE_X ? WX_X : 0);
+  if (lists && g->n_wx > 0) {
+    hipLaunchKernelGGL(k_wx, dim3(g->n_wx), dim3(64), 0, g->stream, g->wx_items, g->wx_rng, lists, g->geo, g->surf_ue,
+                       g->surf_dc, g->ld_surf, g->uden, g->ld_e, g->src4, g->trg4, g->trg_gram, g->dc_gram, g->wxpart);
+    LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_wx_reduce, dim3((g->n_wxred + 1) / 2), dim3(64), 0, g->stream, g->wx_red, g->n_wxred, lists,
+                       g->wxpart, g->pot, g->dchk);
+    LAUNCH_CHECK();
   }
-  LAUNCH_CHECK();
-  REC(ew);
-  if ((mask & KIFMM_PHASE_X) && g->n_xitems > 0) {
-    hipLaunchKernelGGL((k_wx<MASK, true>), dim3(g->n_xitems), dim3(64), 0, g->stream, g->xitems, g->xidx, g->child,
-                       g->snum, g->sbeg, g->tbeg, g->geo, g->surf_ue, g->surf_dc, g->ld_surf, g->n_e, g->uden,
-                       g->ld_e, g->src4, g->trg4, g->pot, g->dchk, g->wxpart);
-    if (g->n_xred > 0)
-      hipLaunchKernelGGL(k_wx_reduce, dim3(g->n_xred), dim3(64), 0, g->stream, g->xred, g->tbeg, g->ld_e, g->wxpart,
-                         g->pot, g->dchk);
+  if ((lists & WX_X) && g->n_xs > 0) {
+    hipLaunchKernelGGL(k_x_surf, dim3(g->n_xs), dim3(64), 0, g->stream, g->xs_items, g->wx_rng, g->geo, g->surf_dc,
+                       g->ld_surf, g->src4, g->dchk, g->ld_e, g->wxpart);
+    LAUNCH_CHECK();
+    if (g->n_xsred > 0)
+      hipLaunchKernelGGL(k_x_surf_reduce, dim3(g->n_xsred), dim3(64), 0, g->stream, g->xs_red, g->ld_e, g->wxpart,
+                         g->dchk);
+    LAUNCH_CHECK();
   }
-  LAUNCH_CHECK();
   return KIFMM_OK;
 }
 
 /* Phase events (recorded outside graph capture): E_START before the
  * sequence, then one after each phase in launch order. */
-enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_W, E_X, E_DOWN, E_U, E_END };
+enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_WX, E_DOWN, E_U, E_END };
 
 /* One evaluation is three launch sequences on the handle's streams:
  *   enqueue_side  the U-list of the early copy-out chunks (early_chunks) on
@@ -1476,11 +1617,8 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
   }
   REC(ev[E_IFFT]);
   /* W and X */
-  if (mask & (KIFMM_PHASE_W | KIFMM_PHASE_X))
-    TRY(g->coincident ? point_phases_wx<true>(g, mask, ev[E_W]) : point_phases_wx<false>(g, mask, ev[E_W]));
-  else
-    REC(ev[E_W]);
-  REC(ev[E_X]);
+  TRY(wx_phase(g, mask));
+  REC(ev[E_WX]);
   /* down: DC2DE at depth 2, then per level the fused L2L + DC2DE
    * (k_l2l_dc2de over the parents at depth d - 1), then L2T */
   for (int d = 2; d <= g->max_depth && (mask & KIFMM_PHASE_DOWN); d++) {
@@ -1633,8 +1771,10 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
       times->v_hadamard = ms[E_HAD];
       times->v_ifft = ms[E_IFFT];
       times->vlist = ms[E_FFT] + ms[E_TRANS] + ms[E_HAD] + ms[E_IFFT];
-      times->wlist = ms[E_W];
-      times->xlist = ms[E_X];
+      /* one launch: its time split by the lists' pairs */
+      const double w = mask & KIFMM_PHASE_W ? g->counts.w_pairs : 0.0, x = mask & KIFMM_PHASE_X ? g->counts.x_pairs : 0.0;
+      times->wlist = w + x > 0.0 ? ms[E_WX] * w / (w + x) : ms[E_WX];
+      times->xlist = ms[E_WX] - times->wlist;
       times->down = ms[E_DOWN];
     }
     /* the U-list: its chunks after the far field, plus the span of the
@@ -1686,7 +1826,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
   const double t_plan0 = kifmm::wall_seconds();
   Plan P;
   try {
-    const int pr = make_plan(tree, ops, P);
+    const int pr = make_plan(tree, ops, opts && opts->precision == KIFMM_PREC_MIXED, P);
     if (pr != KIFMM_OK) return pr;
   } catch (const std::bad_alloc&) {
     set_error("host allocation failed in kifmm_gpu_create");
@@ -1757,7 +1897,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
     const double t2 = kifmm::wall_seconds();
     if (r == KIFMM_OK) r = trans_setup(g);
     if (r == KIFMM_OK && g->precision == KIFMM_PREC_MIXED) r = mixed_setup(g);
-    if (r == KIFMM_OK && g->precision == KIFMM_PREC_FP64 && g->close_listed) r = gram_setup(g);
+    if (r == KIFMM_OK) r = gram_setup(g);
     const double t3 = kifmm::wall_seconds();
     g->create_ms[1] = (t1 - t0) * 1e3;
     g->create_ms[2] = (t2 - t1) * 1e3;
@@ -1919,7 +2059,7 @@ int kifmm_gpu_plan(const kifmm_tree_view* tree, const kifmm_operators* ops, kifm
   Plan P;
   int r = KIFMM_OK;
   try {
-    r = make_plan(tree, ops, P);
+    r = make_plan(tree, ops, false, P);
   } catch (const std::bad_alloc&) {
     set_error("host allocation failed in kifmm_gpu_plan");
     return KIFMM_ENOMEM;
