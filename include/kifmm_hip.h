@@ -69,8 +69,9 @@ enum {
 typedef struct kifmm_gpu_tuning {
   int p2p_form;      /* KIFMM_P2P_*: STATIC, PERSISTENT or STATIC64 on the FP64 path;
                         STATIC or SPLIT on the mixed path */
-  int hadamard_fb;   /* frequencies per V-list Hadamard block: 4, 8 (default) or 16 */
-  int hadamard_form; /* KIFMM_HAD_*: V-list Hadamard on MFMA (default) or on the VALU */
+  int hadamard_fb;   /* frequencies per V-list Hadamard block: 4, 8 (default) or 16; fewer
+                        where that many leave CUs without a block */
+  int hadamard_form; /* KIFMM_HAD_*: how the V-list Hadamard forms its products */
   int overlap;       /* stream layout of the U-list: 0 all of it last, after the far field;
                         1 all of it on the handle's second stream from the start, alongside
                         the far field (initially 1 with KIFMM_GPU_OVERLAP); 2, 3 its first
@@ -92,8 +93,10 @@ enum {
                             block, the intermediate vectors kept in LDS */
 };
 enum {
-  KIFMM_HAD_VALU = 0, /* a lane per parent, two waves per 64 parents */
-  KIFMM_HAD_MFMA = 1  /* 16 parents per 16x16x4 MFMA tile, four waves per 64 parents (default) */
+  KIFMM_HAD_VALU = 0, /* the 64 child products per neighbour on the VALU, a lane per parent */
+  KIFMM_HAD_MFMA = 1  /* default: FP32 spectra (mixed path) on MFMA, 16 parents per 16x16x4
+                         tile; FP64 spectra, whose MFMAs run at the VALU's rate, as 36
+                         products per neighbour (Toeplitz factors) on the VALU */
 };
 
 typedef struct kifmm_gpu_options {

@@ -2392,10 +2392,10 @@ __global__ __launch_bounds__(128) void k_hadamard(const int4* __restrict__ group
   }
 }
 
-/* MFMA form of the Hadamard.  For one frequency and one neighbour
- * direction o every parent applies the same 8 x 8 complex matrix
- * T_o[c][c'] = T[f][2o + 3 + c' - c] (target child c, source child c') to
- * its neighbour's 8 child spectra.  In real form [[Tr, -Ti], [Ti, Tr]]
+/* MFMA form of the Hadamard, FP32 spectra (mixed path).  For one frequency
+ * and one neighbour direction o every parent applies the same 8 x 8 complex
+ * matrix T_o[c][c'] = T[f][2o + 3 + c' - c] (target child c, source child c')
+ * to its neighbour's 8 child spectra.  In real form [[Tr, -Ti], [Ti, Tr]]
  * (16 x 16, rows: Re Y[c] then Im Y[c]; columns: Re X[c'] then Im X[c'])
  * over 16 parents that is four 16x16x4 MFMAs, k = 4m + kk with source
  * child (4m + kk) & 7, real parts for m < 2 and imaginary for m >= 2.
@@ -2406,53 +2406,29 @@ __global__ __launch_bounds__(128) void k_hadamard(const int4* __restrict__ group
  * translation values are staged per frequency, the next frequency's
  * prefetched into registers meanwhile.  A lane's A operand is Re or Im of a
  * translation value for the real-part MFMAs and -Im or Re for the
- * imaginary-part ones, by the lane's row.  In FP32 the translation values
- * are staged twice, as (Re, Im) in TA and (-Im, Re) in TB, so that the
- * operand is one LDS read at a lane-fixed offset, with no select or negation
- * on the VALU, whose issue adds to the 35-cycle FP32 MFMAs' (-15 % at 16M
- * points, NP 4).  The FP64 form keeps one (Re, Im) copy and selects: its
- * fully unrolled direction loop prefetches the LDS reads of later directions
- * at 128 VGPRs, which the 64-cycle FP64 MFMAs need more than the saved VALU
- * slots (the staged-twice form measured 5 % slower there).  MFMA operand
- * layouts as pinned by test_mfma_f64_operand_layout /
- * test_mfma_f32_operand_layout. */
-__device__ __forceinline__ v4d mfma4(double a, double b, v4d c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-template <typename R>
-struct Acc4;
-template <>
-struct Acc4<double> {
-  typedef v4d T;
-};
-template <>
-struct Acc4<float> {
-  typedef v4f T;
-};
-
-template <int NP, typename ST, int FB>
+ * imaginary-part ones, by the lane's row: the translation values are staged
+ * twice, as (Re, Im) in TA and (-Im, Re) in TB, so that the operand is one
+ * LDS read at a lane-fixed offset, with no select or negation on the VALU,
+ * whose issue adds to the 35-cycle FP32 MFMAs' (-15 % at 16M points, NP 4).
+ * MFMA operand layout as pinned by test_mfma_f32_operand_layout.  (FP64
+ * spectra take k_hadamard_fact: the FP64 MFMA runs at the VALU's rate.) */
+template <int NP, int FB>
 __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ groups,
                                                        const int* __restrict__ uslots,
                                                        const unsigned char* __restrict__ loc,
-                                                       const int* __restrict__ yslot, const ST* __restrict__ T,
-                                                       const ST* __restrict__ X, ST* __restrict__ Y, int n_groups,
-                                                       int per_xcd) {
-  typedef typename Spec<ST>::R R;
-  typedef typename Acc4<R>::T V;
+                                                       const int* __restrict__ yslot, const float2* __restrict__ T,
+                                                       const float2* __restrict__ X, float2* __restrict__ Y,
+                                                       int n_groups, int per_xcd) {
   using G = Grid<NP>;
   constexpr int F = G::F;
   static_assert(F % FB == 0, "frequency blocks");
   constexpr int PER = (HAD_CAP * 8 + 255) / 256;
   constexpr int PERT = (343 + 255) / 256;
-  __shared__ ST Xs[HAD_CAP][9];
-  constexpr bool F32 = sizeof(R) == 4;
-  /* FP32: TA = (Re, Im) then TB = (-Im, Re), 2 x 343 float2; FP64: Ts = (Re, Im) */
-  __shared__ ST Tsh[F32 ? 2 * 343 : 343];
-  R* const TA = reinterpret_cast<R*>(Tsh);
-  R* const TB = TA + 2 * 343;
+  __shared__ float2 Xs[HAD_CAP][9];
+  /* TA = (Re, Im) then TB = (-Im, Re) */
+  __shared__ float2 Tsh[2 * 343];
+  float* const TA = reinterpret_cast<float*>(Tsh);
+  float* const TB = TA + 2 * 343;
   __shared__ unsigned char sloc[27][64];
   const int v = had_block(n_groups, F / FB, per_xcd);
   if (v < 0) return; /* whole block, before any barrier */
@@ -2467,17 +2443,17 @@ __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ 
     const int e = tid + 256 * k;
     us[k] = e < ne8 ? uslots[g.z + (e >> 3)] : 0;
   }
-  ST pre[PER], pret[PERT];
+  float2 pre[PER], pret[PERT];
   auto fetch = [&](int f) {
 #pragma unroll
     for (int k = 0; k < PER; k++) {
       const int e = tid + 256 * k;
-      pre[k] = e < ne8 ? X[((size_t)us[k] * F + f) * 8 + (e & 7)] : Spec<ST>::mk(0.0, 0.0);
+      pre[k] = e < ne8 ? X[((size_t)us[k] * F + f) * 8 + (e & 7)] : make_float2(0.0f, 0.0f);
     }
 #pragma unroll
     for (int k = 0; k < PERT; k++) {
       const int e = tid + 256 * k;
-      pret[k] = e < 343 ? T[(size_t)f * 343 + e] : Spec<ST>::mk(0.0, 0.0);
+      pret[k] = e < 343 ? T[(size_t)f * 343 + e] : make_float2(0.0f, 0.0f);
     }
   };
   fetch(f0);
@@ -2493,17 +2469,15 @@ __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ 
   /* row i = j of A: target child c = j & 7, real part for j < 8; the two
    * source children this lane supplies are kk and kk + 4 */
   const int c = j & 7;
-  const bool rrow = j < 8;
-  const int sel = rrow ? 0 : 1; /* rows 0-7: Re Y (A = Re T, -Im T); rows 8-15: Im Y (A = Im T, Re T) */
+  const int sel = j < 8 ? 0 : 1; /* rows 0-7: Re Y (A = Re T, -Im T); rows 8-15: Im Y (A = Im T, Re T) */
   auto base = [&](int cs) {
     return (3 + ((cs >> 2) & 1) - ((c >> 2) & 1)) + 7 * (3 + ((cs >> 1) & 1) - ((c >> 1) & 1)) +
            49 * (3 + (cs & 1) - (c & 1));
   };
-  const int b0 = base(kk), b1 = base(kk + 4);
-  /* FP32: this lane's A operands for source children kk and kk + 4, before
-   * the direction offset */
-  const R* const a0r = TA + 2 * b0 + sel;
-  const R* const a1r = TA + 2 * b1 + sel;
+  /* this lane's A operands for source children kk and kk + 4, before the
+   * direction offset */
+  const float* const a0r = TA + 2 * base(kk) + sel;
+  const float* const a1r = TA + 2 * base(kk + 4) + sel;
   const int ys = yslot[g.x + min(pj, g.y - 1)];
   for (int fi = 0; fi < FB; fi++) {
     const int f = f0 + fi;
@@ -2517,14 +2491,10 @@ __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ 
     for (int k = 0; k < PERT; k++) {
       const int e = tid + 256 * k;
       if (e < 343) {
-        if constexpr (F32) {
-          TA[2 * e] = pret[k].x;
-          TA[2 * e + 1] = pret[k].y;
-          TB[2 * e] = -pret[k].y;
-          TB[2 * e + 1] = pret[k].x;
-        } else {
-          Tsh[e] = pret[k];
-        }
+        TA[2 * e] = pret[k].x;
+        TA[2 * e + 1] = pret[k].y;
+        TB[2 * e] = -pret[k].y;
+        TB[2 * e + 1] = pret[k].x;
       }
     }
     __syncthreads();
@@ -2532,21 +2502,7 @@ __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ 
     if (!active) continue;
     /* four independent accumulator chains: no MFMA waits on the one just
      * issued */
-    V accr0 = {0, 0, 0, 0}, acci0 = {0, 0, 0, 0}, accr1 = {0, 0, 0, 0}, acci1 = {0, 0, 0, 0};
-    if constexpr (!F32) {
-#pragma unroll 2
-      for (int o = 0; o < 27; o++) {
-        if (o == 13) continue; /* the parent itself: its children are all adjacent */
-        const int os = 2 * (o / 9 - 1) + 14 * ((o / 3) % 3 - 1) + 98 * (o % 3 - 1);
-        const ST t0 = Tsh[b0 + os], t1 = Tsh[b1 + os];
-        const ST* xs = Xs[sloc[o][pj]];
-        const ST x0 = xs[kk], x1 = xs[kk + 4];
-        accr0 = mfma4(rrow ? t0.x : t0.y, x0.x, accr0);
-        acci0 = mfma4(rrow ? -t0.y : t0.x, x0.y, acci0);
-        accr1 = mfma4(rrow ? t1.x : t1.y, x1.x, accr1);
-        acci1 = mfma4(rrow ? -t1.y : t1.x, x1.y, acci1);
-      }
-    } else {
+    v4f accr0 = {0, 0, 0, 0}, acci0 = {0, 0, 0, 0}, accr1 = {0, 0, 0, 0}, acci1 = {0, 0, 0, 0};
     /* the 26 directions (ox, oy, oz) in the order o = 9 (ox + 1) + 3 (oy +
      * 1) + oz + 1; only the z loop is unrolled: unrolling all of them would
      * hoist the LDS reads of many directions into registers and halve the
@@ -2556,39 +2512,219 @@ __global__ __launch_bounds__(256) void k_hadamard_mfma(const int4* __restrict__ 
 #pragma unroll 1
       for (int oy = -1; oy <= 1; oy++) {
         const int oxy = 9 * (ox + 1) + 3 * (oy + 1);
-        const int osxy = 2 * (2 * ox + 14 * oy); /* in R elements */
+        const int osxy = 2 * (2 * ox + 14 * oy); /* in floats */
 #pragma unroll
         for (int oz = -1; oz <= 1; oz++) {
           if (ox == 0 && oy == 0 && oz == 0) continue; /* the parent itself: its children are all adjacent */
-          const ST* xs = Xs[sloc[oxy + oz + 1][pj]];
-          const ST x0 = xs[kk], x1 = xs[kk + 4];
-          const R* const p0 = a0r + osxy + 2 * 98 * oz;
-          const R* const p1 = a1r + osxy + 2 * 98 * oz;
-          accr0 = mfma4(p0[0], x0.x, accr0);
-          acci0 = mfma4(p0[2 * 343], x0.y, acci0);
-          accr1 = mfma4(p1[0], x1.x, accr1);
-          acci1 = mfma4(p1[2 * 343], x1.y, acci1);
+          const float2* xs = Xs[sloc[oxy + oz + 1][pj]];
+          const float2 x0 = xs[kk], x1 = xs[kk + 4];
+          const float* const p0 = a0r + osxy + 2 * 98 * oz;
+          const float* const p1 = a1r + osxy + 2 * 98 * oz;
+          accr0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[0], x0.x, accr0, 0, 0, 0);
+          acci0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[2 * 343], x0.y, acci0, 0, 0, 0);
+          accr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[0], x1.x, accr1, 0, 0, 0);
+          acci1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[2 * 343], x1.y, acci1, 0, 0, 0);
         }
       }
-    }
-    const V acc = (accr0 + accr1) + (acci0 + acci1);
-    ST* yb = Y + ((size_t)ys * F + f) * 8;
-    if constexpr (sizeof(R) == 8) {
-      /* D[i][j] in lane j + 16(i % 4), element i / 4: rows kk, kk+4 (Re)
-       * and kk+8, kk+12 (Im) = children kk and kk + 4 */
-      if (pj < g.y) {
-        yb[kk] = Spec<ST>::mk(acc[0], acc[2]);
-        yb[kk + 4] = Spec<ST>::mk(acc[1], acc[3]);
+    const v4f acc = (accr0 + accr1) + (acci0 + acci1);
+    float2* yb = Y + ((size_t)ys * F + f) * 8;
+    /* D[i][j] in lane j + 16(i / 4), element i % 4: lanes kk < 2 hold Re
+     * of children 4kk + e, lanes kk + 2 (the same column j) their Im */
+    float im[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) im[e] = __shfl_xor(acc[e], 32, 64);
+    if (pj < g.y && kk < 2)
+#pragma unroll
+      for (int e = 0; e < 4; e++) yb[4 * kk + e] = make_float2(acc[e], im[e]);
+  }
+}
+
+/* Factored form of the Hadamard, FP64 spectra.  Along each axis the matrix
+ * T[2o + c' - c] between source child c' and target child c is 2 x 2
+ * Toeplitz in the child bits, and three products do instead of four:
+ *   m0 = t(2o) (x0 + x1),  m1 = (t(2o+1) - t(2o)) x1,
+ *   m2 = (t(2o-1) - t(2o)) x0,   y0 = m0 + m1,  y1 = m0 + m2.
+ * Applied along y and z (component k = 3 ky + kz; along x the four products
+ * stay) the 64 complex products of a neighbour become 36.  The sums over x
+ * are formed once per source slot and the sums into y once per parent, after
+ * the 26 directions have been accumulated, so only the 36 products are paid
+ * per direction.  An FP64 MFMA has no more throughput than VALU FMAs here,
+ * and the factored products are no matrix product: they run as FMAs, a lane
+ * per parent.  The factors That (k_trans_fact, once per handle) are then
+ * wave-uniform and come through scalar registers, 7 per (oy, oz): dx = 2 ox +
+ * c'x - cx in -3 .. 3.  (All three axes factored would be 27 products but one
+ * 16-byte LDS read for each instead of one for two: the LDS pipe, level with
+ * the FMAs here, would bound it.)
+ *
+ * Per frequency the block stages the sums over x of its slot union, row 2 k
+ * + x bit, 68 KB (2 blocks per CU), from spectra prefetched into registers
+ * during the previous frequency's products.  Wave k of 8 takes component k
+ * in all 26 directions, its neighbours' LDS addresses in registers, and 3 or
+ * 4 directions of component 8.  (A ninth wave for it leaves one block per
+ * CU: 4.8 ms at 16M points against 2.8 for the eight.)  The LDS serves a
+ * wave's 64 16-byte reads in as many cycles as the busiest of its 8 bank
+ * groups has reads, 8 at best (measured): the plan puts a slot of octant r
+ * (within its own siblings) at an index of residue r mod 8, and the 64
+ * neighbours of a full group fall 8 to a bank group in every direction.  The
+ * components of a parent meet through the same LDS in a fixed order.
+ * Bound by the LDS pipe: 651 reads and writes of 8 cycles per frequency and
+ * group, 74 % of the time it takes (VALU 60 %).
+ * Measured against the FP64 MFMA form of 4 MFMAs per direction and 16 parents:
+ * 3.50 -> 2.13 ms at 16M points NP 4, 1.22 -> 0.87 at 4M NP 6, 0.42 -> 0.38
+ * at 1M ellipsoid NP 4, 0.42 -> 0.37 at 300 thousand NP 6.  Error against the
+ * oracle as before (2.4e-13 at NP 4, 1.5e-11 at NP 6: the pseudo-inverse). */
+constexpr int HAD_FACT = 9 * 9 * 7; /* factors per frequency: [k][oy oz][dx + 3] */
+
+/* the factors from T[f][343]; near-field entries are zero in T */
+static __global__ __launch_bounds__(256) void k_trans_fact(const double2* __restrict__ T, int n,
+                                                          double2* __restrict__ That) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  const int f = e / HAD_FACT, r = e % HAD_FACT, k = r / 63, oyz = (r / 7) % 9, dx = r % 7;
+  const int ky = k / 3, kz = k % 3, dy = 2 * (oyz / 3 - 1) + 3, dz = 2 * (oyz % 3 - 1) + 3; /* + 3 */
+  const double2* __restrict__ t = T + (size_t)f * 343 + dx;
+  const int sy = ky == 1 ? 1 : -1, sz = kz == 1 ? 1 : -1; /* 1: t(2o + 1) - t(2o), 2: t(2o - 1) - t(2o) */
+  auto along_z = [&](int y) {
+    const double2 a = t[7 * y + 49 * dz];
+    if (kz == 0) return a;
+    const double2 b = t[7 * y + 49 * (dz + sz)];
+    return make_double2(b.x - a.x, b.y - a.y);
+  };
+  double2 v = along_z(dy);
+  if (ky > 0) {
+    const double2 b = along_z(dy + sy);
+    v = make_double2(b.x - v.x, b.y - v.y);
+  }
+  That[e] = v;
+}
+
+__device__ __forceinline__ double2 add2(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+/* a += t x */
+__device__ __forceinline__ void cmac(double2& a, double2 t, double2 x) {
+  a.x = __builtin_fma(t.x, x.x, __builtin_fma(-t.y, x.y, a.x));
+  a.y = __builtin_fma(t.x, x.y, __builtin_fma(t.y, x.x, a.y));
+}
+
+template <int NP, int FB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_hadamard_fact(
+    const int4* __restrict__ groups, const int* __restrict__ uslots, const unsigned char* __restrict__ loc,
+    const int* __restrict__ yslot, const double2* __restrict__ That, const double2* __restrict__ X,
+    double2* __restrict__ Y, int n_groups, int per_xcd) {
+  constexpr int F = Grid<NP>::F;
+  static_assert(F % FB == 0, "frequency blocks");
+  static_assert(2 * HAD_CAP <= 512, "one staging thread per slot and x bit");
+  constexpr int ROW = HAD_CAP + 4; /* = 4 mod 8: the two x bits staged by a wave spread over the banks */
+  static_assert(ROW % 8 == 4, "row stride");
+  constexpr int YLD = 65; /* row stride of the exchange: the 8 children of a parent read different banks */
+  __shared__ double2 S[18 * ROW];
+  static_assert(18 * ROW >= 32 * YLD, "the exchange reuses the staging area");
+  const int v = had_block(n_groups, F / FB, per_xcd);
+  if (v < 0) return; /* whole block, before any barrier */
+  const int4 g = groups[v % n_groups];
+  const int f0 = (v / n_groups) * FB;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int k = __builtin_amdgcn_readfirstlane(tid >> 6);
+  /* staging: thread 2 u + cx takes the 4 (y, z) children at x bit cx of union slot u */
+  const int su = tid >> 1, cx = tid & 1;
+  const bool stages = su < g.w;
+  const double2* __restrict__ xp = X + (size_t)(stages ? uslots[g.z + su] : 0) * F * 8 + 4 * cx;
+  double2 pre[4];
+  auto fetch = [&](int f) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) pre[c] = xp[(size_t)f * 8 + c]; /* threads past the union: slot 0 */
+  };
+  fetch(f0);
+  /* this lane's neighbours: LDS addresses at component k, x bit 0 (lanes past
+   * the group's count repeat its last parent) */
+  const double2* nb[27];
+  const unsigned char* __restrict__ l = loc + (size_t)(g.x + min(lane, g.y - 1)) * 27;
+#pragma unroll
+  for (int o = 0; o < 27; o++) nb[o] = S + 2 * k * ROW + l[o];
+  /* and of the wave's directions k, k + 8, ... of component 8 */
+  const double2* nb8[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int i = min(k + 8 * j, 25);
+    nb8[j] = S + 16 * ROW + l[i + (i >= 13)];
+  }
+  const int yp = tid >> 3, yc = tid & 7; /* output: parent, child */
+  double2* __restrict__ yo = Y + (size_t)yslot[g.x + min(yp, g.y - 1)] * F * 8 + yc;
+  for (int fi = 0; fi < FB; fi++) {
+    const int f = f0 + fi;
+    __syncthreads(); /* the previous frequency's exchange has been read */
+    if (stages) {
+      const double2 z0[3] = {add2(pre[0], pre[1]), pre[1], pre[0]}, z1[3] = {add2(pre[2], pre[3]), pre[3], pre[2]};
+      double2* const d = S + cx * ROW + su;
+#pragma unroll
+      for (int kz = 0; kz < 3; kz++) {
+        d[2 * kz * ROW] = add2(z0[kz], z1[kz]);
+        d[2 * (3 + kz) * ROW] = z1[kz];
+        d[2 * (6 + kz) * ROW] = z0[kz];
       }
-    } else {
-      /* D[i][j] in lane j + 16(i / 4), element i % 4: lanes kk < 2 hold Re
-       * of children 4kk + e, lanes kk + 2 (the same column j) their Im */
-      R im[4];
+    }
+    __syncthreads();
+    if (fi + 1 < FB) fetch(f + 1);
+    const double2* __restrict__ tf = That + (size_t)f * HAD_FACT + k * 63;
+    double2 y[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)}, y8[2] = {y[0], y[0]}; /* [target x bit] */
+    /* one (oy, oz) at a time, the next one's spectra and factors under way
+     * meanwhile; the scheduling barriers keep the compiler from hoisting the
+     * LDS reads of all directions into (spilled) registers */
+    double2 xc[6], xn[6], tc[7], tn[7];
+    auto load = [&](double2 (&x)[6], double2 (&t)[7], int oyz) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) im[e] = __shfl_xor(acc[e], 32, 64);
-      if (pj < g.y && kk < 2)
+      for (int m = 0; m < 7; m++) t[m] = tf[7 * oyz + m];
 #pragma unroll
-        for (int e = 0; e < 4; e++) yb[4 * kk + e] = Spec<ST>::mk(acc[e], im[e]);
+      for (int ox = 0; ox < 3; ox++) {
+        x[2 * ox] = nb[9 * ox + oyz][0];
+        x[2 * ox + 1] = nb[9 * ox + oyz][ROW];
+      }
+    };
+    load(xc, tc, 0);
+#pragma unroll
+    for (int oyz = 0; oyz < 9; oyz++) {
+      if (oyz < 8) load(xn, tn, oyz + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ox = 0; ox < 3; ox++) {
+        if (oyz == 4 && ox == 1) continue; /* the parent itself: its children are all adjacent */
+        cmac(y[0], tc[2 * ox + 1], xc[2 * ox]); /* dx + 3 = 2 ox' + 3 + c'x - cx with ox' = ox - 1 */
+        cmac(y[1], tc[2 * ox], xc[2 * ox]);
+        cmac(y[0], tc[2 * ox + 2], xc[2 * ox + 1]);
+        cmac(y[1], tc[2 * ox + 1], xc[2 * ox + 1]);
+      }
+      __asm__ volatile("" : "+v"(y[0].x), "+v"(y[0].y), "+v"(y[1].x), "+v"(y[1].y));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < 6; m++) xc[m] = xn[m];
+#pragma unroll
+      for (int m = 0; m < 7; m++) tc[m] = tn[m];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int i = k + 8 * j, o = i + (i >= 13);
+      if (i >= 26) break; /* wave-uniform */
+      const double2 x0 = nb8[j][0], x1 = nb8[j][ROW];
+      const double2* __restrict__ t = That + (size_t)f * HAD_FACT + 8 * 63 + 7 * (o % 9) + 2 * (o / 9) + 1;
+      cmac(y8[0], t[0], x0);
+      cmac(y8[1], t[-1], x0);
+      cmac(y8[0], t[1], x1);
+      cmac(y8[1], t[0], x1);
+    }
+    __syncthreads(); /* every wave is done with the staged sums */
+#pragma unroll
+    for (int sx = 0; sx < 2; sx++) {
+      S[(2 * k + sx) * YLD + lane] = y[sx];
+      S[(16 + 2 * k + sx) * YLD + lane] = y8[sx];
+    }
+    __syncthreads();
+    if (yp < g.y) {
+      const int sx = yc >> 2, ky = 1 + ((yc >> 1) & 1), kz = 1 + (yc & 1);
+      auto at = [&](int c) { return S[(2 * c + sx) * YLD + yp]; };
+      double2 m = at(3 * ky + kz); /* component 8: its first partial sum */
+      if (3 * ky + kz == 8)
+#pragma unroll
+        for (int p = 1; p < 8; p++) m = add2(m, at(8 + p));
+      yo[(size_t)f * 8] = add2(add2(at(0), at(kz)), add2(at(3 * ky), m));
     }
   }
 }

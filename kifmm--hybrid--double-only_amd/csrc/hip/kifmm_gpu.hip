@@ -84,7 +84,7 @@ struct kifmm_gpu {
   double *pot = nullptr, *uden = nullptr, *dchk = nullptr, *dden = nullptr, *chk = nullptr;
   double *UC2UE = nullptr, *UE2UC = nullptr, *DC2DE = nullptr, *DE2DC = nullptr;
   double *surf_ue = nullptr, *surf_uc = nullptr, *surf_de = nullptr, *surf_dc = nullptr;
-  double2 *X = nullptr, *Y = nullptr, *T = nullptr, *tw = nullptr;
+  double2 *X = nullptr, *Y = nullptr, *T = nullptr, *That = nullptr, *tw = nullptr;
   /* mixed path: FP32 spectra, FP32 unit surfaces, FP32 leaf-local sources */
   float2 *Xf = nullptr, *Yf = nullptr, *Tf = nullptr;
   float *surf_uc32 = nullptr, *surf_de32 = nullptr;
@@ -327,7 +327,7 @@ struct Plan {
   std::vector<int4> l2t_items;
   std::vector<int4> hgroups;
   std::vector<int> huslots;
-  std::vector<unsigned char> hloc;
+  std::vector<unsigned char> hloc, hoct; /* union index; octant of the neighbour's position */
   kifmm_work_counts wc{};
 };
 
@@ -638,6 +638,116 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
   return KIFMM_OK;
 }
 
+/* Hadamard groups: runs of at most 64 consecutive parents (a lane each) whose
+ * neighbour-slot union fits the LDS staging area.  The runs are put together
+ * from whole 4 x 4 x 4 blocks of parents (the same box two levels up) where
+ * they fit: such a block's union is at most 6 x 6 x 6, while 64 parents
+ * across two blocks overrun the area.  (Runs cut blindly every 64 parents
+ * are out of step with the blocks from the second level on: 876 groups
+ * instead of 586 at 16M uniform points.)  A block too large by itself is
+ * cut between siblings.
+ * The union is laid out by octant, a position of octant r (of its own
+ * sibling group) at an index of residue r mod 8, missing neighbours (slot 0)
+ * included, so that a group's neighbours in any direction spread evenly over
+ * the LDS banks (k_hadamard_fact). */
+int had_groups(const kifmm_tree_view* t, Plan& P) {
+  const int np_ = (int)P.hslot.size();
+  P.hloc.assign((size_t)np_ * 27, 0);
+  std::vector<int> node(np_); /* the parents' nodes */
+  for (int p = 0; p < np_; p++) node[p] = t->parent[P.vblocks[p]];
+  auto same_box = [&](int p, int q, int up) {
+    if (t->depth[node[p]] != t->depth[node[q]]) return false;
+    for (int k = 0; k < 3; k++)
+      if ((t->path[3 * node[p] + k] >> up) != (t->path[3 * node[q] + k] >> up)) return false;
+    return true;
+  };
+  /* per class (octant) the slots in the open group; mark[slot] = the group
+   * that holds it, index[slot] its place among its class.  A slot has one
+   * octant, but for slot 0, which each class holds once when it needs it. */
+  std::vector<int> mark(P.nblk + 1, -1), index(P.nblk + 1, 0), cls[8];
+  int zero[8], group = 0, first = 0, cnt = 0;
+  auto open = [&](int p) {
+    first = p;
+    cnt = 0;
+    group++;
+    for (int r = 0; r < 8; r++) {
+      cls[r].clear();
+      zero[r] = -1;
+    }
+  };
+  /* adds the parents [p, e) if they fit; else leaves the group as it was */
+  auto add = [&](int p, int e) {
+    if (cnt + (e - p) > 64) return false;
+    size_t was[8];
+    int wz[8];
+    for (int r = 0; r < 8; r++) {
+      was[r] = cls[r].size();
+      wz[r] = zero[r];
+    }
+    size_t most = 0;
+    for (size_t k = (size_t)p * 27; k < (size_t)e * 27; k++) {
+      const int slot = P.hnbr[k], r = P.hoct[k];
+      if (slot == 0 ? zero[r] >= 0 : mark[slot] == group) continue;
+      if (slot == 0) {
+        zero[r] = (int)cls[r].size();
+      } else {
+        mark[slot] = group;
+        index[slot] = (int)cls[r].size();
+      }
+      cls[r].push_back(slot);
+      most = std::max(most, cls[r].size());
+    }
+    if (8 * most > (size_t)HAD_CAP) {
+      for (int r = 0; r < 8; r++) {
+        for (size_t j = was[r]; j < cls[r].size(); j++)
+          if (cls[r][j] != 0) mark[cls[r][j]] = -1;
+        cls[r].resize(was[r]);
+        zero[r] = wz[r];
+      }
+      return false;
+    }
+    cnt += e - p;
+    return true;
+  };
+  auto close = [&] {
+    if (cnt == 0) return;
+    size_t most = 0;
+    for (auto& c : cls) most = std::max(most, c.size());
+    P.hgroups.push_back(make_int4(first, cnt, (int)P.huslots.size(), (int)(8 * most)));
+    for (size_t k = (size_t)first * 27; k < (size_t)(first + cnt) * 27; k++)
+      P.hloc[k] = (unsigned char)(8 * (P.hnbr[k] ? index[P.hnbr[k]] : zero[P.hoct[k]]) + P.hoct[k]);
+    for (size_t j = 0; j < most; j++)
+      for (int r = 0; r < 8; r++) P.huslots.push_back(j < cls[r].size() ? cls[r][j] : 0);
+  };
+  open(0);
+  for (int p = 0; p < np_;) {
+    int e = p + 1;
+    while (e < np_ && same_box(p, e, 2)) e++;
+    if (!add(p, e)) {
+      close();
+      open(p);
+      if (!add(p, e)) { /* a block larger than a group: sibling sets one by one */
+        for (int a = p; a < e;) {
+          int b = a + 1;
+          while (b < e && b - a < 8 && same_box(a, b, 1)) b++;
+          if (!add(a, b)) {
+            close();
+            open(a);
+            if (!add(a, b)) {
+              set_error("internal: Hadamard neighbour union exceeds the LDS capacity");
+              return KIFMM_EINVAL;
+            }
+          }
+          a = b;
+        }
+      }
+    }
+    p = e;
+  }
+  close();
+  return KIFMM_OK;
+}
+
 int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, Plan& P) {
   TRY(check_view(t));
   const int np = t->np;
@@ -853,6 +963,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
         if (t->depth[c] == d && t->child[c] != -1) slot = (t->child[c] - 1) / 8 + 1;
       }
       P.hnbr.push_back(slot);
+      P.hoct.push_back((unsigned char)(((w[0] & 1) << 2) | ((w[1] & 1) << 1) | (w[2] & 1)));
     }
   }
   for (size_t k = 0; k < P.vblocks.size(); k++)
@@ -861,31 +972,9 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
       return fail("V-list block out of range");
   for (int v : P.hnbr)
     if (v < 0 || v > P.nblk) return fail("V-list neighbour slot out of range");
-  /* Hadamard groups: runs of consecutive parents whose neighbour-slot union
-   * fits the LDS staging area; 64 parents (one lane each) when possible */
+  TRY(had_groups(t, P));
   {
     const int np_ = (int)P.hslot.size();
-    P.hloc.assign((size_t)np_ * 27, 0);
-    std::vector<int> uni;
-    int first = 0;
-    while (first < np_) {
-      int cnt = std::min(64, np_ - first);
-      for (;;) {
-        uni.assign(P.hnbr.begin() + (size_t)first * 27, P.hnbr.begin() + (size_t)(first + cnt) * 27);
-        std::sort(uni.begin(), uni.end());
-        uni.erase(std::unique(uni.begin(), uni.end()), uni.end());
-        if ((int)uni.size() <= HAD_CAP || cnt == 1) break;
-        cnt = std::max(1, cnt / 2);
-      }
-      if ((int)uni.size() > HAD_CAP) return fail("Hadamard neighbour union exceeds the LDS capacity");
-      P.hgroups.push_back(make_int4(first, cnt, (int)P.huslots.size(), (int)uni.size()));
-      for (int k = 0; k < cnt * 27; k++) {
-        const int slot = P.hnbr[(size_t)first * 27 + k];
-        P.hloc[(size_t)first * 27 + k] = (unsigned char)(std::lower_bound(uni.begin(), uni.end(), slot) - uni.begin());
-      }
-      P.huslots.insert(P.huslots.end(), uni.begin(), uni.end());
-      first += cnt;
-    }
     for (const int4& gq : P.hgroups)
       if (gq.y < 1 || gq.y > 64 || gq.x + gq.y > np_ || gq.w > HAD_CAP || gq.z + gq.w > (int)P.huslots.size())
         return fail("Hadamard group out of range");
@@ -1132,6 +1221,7 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
     TRY(dev_zero(g, &g->X, spec));
     TRY(dev_zero(g, &g->Y, spec));
     TRY(dev_zero(g, &g->T, (size_t)g->F * 343));
+    TRY(dev_zero(g, &g->That, (size_t)g->F * HAD_FACT));
   }
   g->n_wx = (int)P.wx_items.size() / 2;
   g->n_wxred = (int)P.wx_red.size() / 2;
@@ -1227,14 +1317,18 @@ int close_list(kifmm_gpu* g) {
 }
 
 /* The 343 translation spectra (k_trans; compute_fft_trans__gpu_eval,
- * fmm/cuda.cu:874-963, which the reference recomputes every run): they
- * depend only on NP, so they are formed once per handle. */
+ * fmm/cuda.cu:874-963, which the reference recomputes every run) and, FP64,
+ * their factored form: they depend only on NP, so they are formed once per
+ * handle. */
 template <int NP>
 int trans_setup_np(kifmm_gpu* g) {
-  if (g->precision == KIFMM_PREC_MIXED)
+  if (g->precision == KIFMM_PREC_MIXED) {
     hipLaunchKernelGGL((k_trans<NP, float2>), dim3(343), dim3(256), 0, g->stream, g->tw, g->Tf);
-  else
+  } else {
     hipLaunchKernelGGL((k_trans<NP, double2>), dim3(343), dim3(256), 0, g->stream, g->tw, g->T);
+    const int n = g->F * HAD_FACT;
+    hipLaunchKernelGGL(k_trans_fact, dim3((n + 255) / 256), dim3(256), 0, g->stream, g->T, n, g->That);
+  }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(g->stream));
   return KIFMM_OK;
@@ -1356,8 +1450,21 @@ int fill(kifmm_gpu* g, double* p, size_t n) {
   return KIFMM_OK;
 }
 
-template <int NP, typename ST>
-int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, ST* T, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3) {
+/* Frequencies per Hadamard block: had_fb, halved (to 2 at least) while the
+ * launch has fewer than two blocks per CU.  A block runs its frequencies one
+ * after another: 4 thousand points NP 3 took 29 us in blocks of 8, 17 of 4
+ * and 12 of 2; above that the prefetch across frequencies pays (4M NP 6: 0.88
+ * ms in blocks of 4, 0.87 of 8).  The sums are the same. */
+int had_block_size(const kifmm_gpu* g) {
+  int fb = g->had_fb;
+  while (fb > 2 && (long)g->n_hgroups * (g->F / fb) < 512) fb /= 2;
+  return fb;
+}
+
+/* The V-list's four sub-phases; had launches the Hadamard in 8 per_xcd blocks
+ * of fb frequencies in XCD-contiguous order (had_block). */
+template <int NP, typename ST, typename HAD>
+int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3, HAD had) {
   if (g->n_vblocks > 0)
     hipLaunchKernelGGL((k_dft_fwd<NP, ST>), dim3(g->n_vblocks), dim3(512), 0, g->stream, g->vblocks, g->vslot,
                        g->depth, g->uden, g->ld_e, g->tw, g->cube2surf, X);
@@ -1366,29 +1473,11 @@ int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, ST* T, hipEvent_t e1, hipEvent_t e2,
   /* the translation spectra T depend only on NP: computed once at create
    * time (trans_setup), so this sub-phase is empty */
   REC(e2);
-  /* XCD-contiguous block order (had_block): 8 per_xcd blocks for the
-   * n_hgroups x F / fb (group, frequency block) pairs */
-  const int had_per_xcd = (int)(((long)g->n_hgroups * (g->F / g->had_fb) + 7) / 8);
-  if (g->n_hgroups > 0)
-    switch (g->had_fb * 2 + g->had_form) {
-#define KIFMM_HAD_CASE(FBV)                                                                                    \
-  case 2 * FBV:                                                                                                \
-    hipLaunchKernelGGL((k_hadamard<NP, ST, FBV>), dim3(8 * had_per_xcd), dim3(128), 0, g->stream, g->hgroups,  \
-                       g->huslots, g->hloc, g->hslot, T, X, Y, g->n_hgroups, had_per_xcd);                    \
-    break;                                                                                                     \
-  case 2 * FBV + 1:                                                                                            \
-    hipLaunchKernelGGL((k_hadamard_mfma<NP, ST, FBV>), dim3(8 * had_per_xcd), dim3(256), 0, g->stream,         \
-                       g->hgroups, g->huslots, g->hloc, g->hslot, T, X, Y, g->n_hgroups, had_per_xcd);        \
-    break;
-      KIFMM_HAD_CASE(4)
-      KIFMM_HAD_CASE(8)
-      KIFMM_HAD_CASE(16)
-#undef KIFMM_HAD_CASE
-      default:
-        set_error("internal: unknown Hadamard shape");
-        return KIFMM_EINVAL;
-    }
-  LAUNCH_CHECK();
+  if (g->n_hgroups > 0) {
+    const int fb = had_block_size(g);
+    TRY(had(fb, (int)(((long)g->n_hgroups * (g->F / fb) + 7) / 8)));
+    LAUNCH_CHECK();
+  }
   REC(e3);
   if (g->n_vblocks > 0)
     hipLaunchKernelGGL((k_dft_inv<NP, ST>), dim3(g->n_vblocks), dim3(512), 0, g->stream, g->vblocks, g->vslot, Y,
@@ -1397,11 +1486,45 @@ int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, ST* T, hipEvent_t e1, hipEvent_t e2,
   return KIFMM_OK;
 }
 
+/* A Hadamard kernel by its block size fb: KERNEL(FB) is the instantiation, T
+ * its translation values */
+#define KIFMM_HAD_LAUNCH(KERNEL, THREADS, T, X, Y)                                                                 \
+  switch (fb) {                                                                                                    \
+    case 2: hipLaunchKernelGGL(KERNEL(2), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+                               g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
+    case 4: hipLaunchKernelGGL(KERNEL(4), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+                               g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
+    case 8: hipLaunchKernelGGL(KERNEL(8), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+                               g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
+    case 16: hipLaunchKernelGGL(KERNEL(16), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,     \
+                                g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                             \
+    default: set_error("internal: unknown Hadamard shape"); return KIFMM_EINVAL;                                   \
+  }
+#define HAD_V32(FB) (k_hadamard<NP, float2, FB>)
+#define HAD_V64(FB) (k_hadamard<NP, double2, FB>)
+#define HAD_M32(FB) (k_hadamard_mfma<NP, FB>)
+#define HAD_F64(FB) (k_hadamard_fact<NP, FB>)
 template <int NP>
 int vlist_phase(kifmm_gpu* g, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3) {
-  if (g->precision == KIFMM_PREC_MIXED) return vlist_phase<NP, float2>(g, g->Xf, g->Yf, g->Tf, e1, e2, e3);
-  return vlist_phase<NP, double2>(g, g->X, g->Y, g->T, e1, e2, e3);
+  if constexpr (NP <= 4) {
+    if (g->precision == KIFMM_PREC_MIXED)
+      return vlist_phase<NP>(g, g->Xf, g->Yf, e1, e2, e3, [&](int fb, int per) {
+        if (g->had_form == KIFMM_HAD_VALU) KIFMM_HAD_LAUNCH(HAD_V32, 128, g->Tf, g->Xf, g->Yf)
+        else KIFMM_HAD_LAUNCH(HAD_M32, 256, g->Tf, g->Xf, g->Yf)
+        return KIFMM_OK;
+      });
+  }
+  return vlist_phase<NP>(g, g->X, g->Y, e1, e2, e3, [&](int fb, int per) {
+    if (g->had_form == KIFMM_HAD_VALU) KIFMM_HAD_LAUNCH(HAD_V64, 128, g->T, g->X, g->Y)
+    else KIFMM_HAD_LAUNCH(HAD_F64, 512, g->That, g->X, g->Y)
+    return KIFMM_OK;
+  });
 }
+#undef HAD_V32
+#undef HAD_V64
+#undef HAD_M32
+#undef HAD_F64
+#undef KIFMM_HAD_LAUNCH
 
 /* The item list the U-list launch uses: the mixed tau kernel takes sibling
  * pairs and single leaves (list 3), the FP64 Gram-form kernels items of

@@ -175,3 +175,37 @@ def test_level_forms_match_oracle(n, dist, q, np_, c):
     for w in ("uden", "dden"):
         a, b = inter[K.LEVEL_FUSED][w], inter[K.LEVEL_GEMM][w]
         assert np.linalg.norm(a - b) <= 1e3 * O.PARITY_RTOL[np_] * np.linalg.norm(b), w
+
+
+def shell(n, seed):
+    """Points near a sphere and a dense knot on it: parents with most
+    neighbours missing, sibling sets with one or two parents, deep levels."""
+    rng = np.random.default_rng(seed)
+    v = rng.standard_normal((3, n))
+    p = 0.7 * v / np.linalg.norm(v, axis=0) * (1.0 + 1e-3 * rng.standard_normal(n))
+    p[:, : n // 4] = np.array([[0.7], [1e-3], [1e-3]]) + 0.01 * rng.standard_normal((3, n // 4))
+    return np.clip(p, -1.0, 1.0), rng.random(n)
+
+
+@pytest.mark.parametrize("n,q,np_", [(70, 2, 3), (400, 1, 4), (9, 1, 6), (5000, 3, 4), (20000, 9, 6), (40000, 30, 3)])
+@pytest.mark.parametrize("kind", ["uniform", "shell"])
+def test_hadamard_groups_and_forms(n, q, np_, kind):
+    """The factored Hadamard against the 64-product form over groups of one
+    parent to 64, unions cut inside a block of parents, and missing
+    neighbours; every block size gives the same bits."""
+    pts, den = shell(n, 3) if kind == "shell" else (np.random.default_rng(3).uniform(-1, 1, (3, n)),
+                                                     np.random.default_rng(4).random(n))
+    prob = K.Problem.from_points(*pts, den, pts_max=q, np_=np_)
+    ev = K.GpuEvaluator(prob)
+    ev.set_tuning(K.P2P_STATIC, 8, K.HAD_VALU)
+    ref, _ = ev.evaluate()
+    assert np.all(np.isfinite(ref))
+    first = None
+    for fb in (4, 8, 16):
+        ev.set_tuning(K.P2P_STATIC, fb, K.HAD_MFMA)
+        got, _ = ev.evaluate()
+        first = got if first is None else first
+        assert np.array_equal(got, first), fb
+    r = rel(first, ref)
+    print(f"  {kind} n={n} q={q} NP={np_}: {r:.2e}", flush=True)
+    assert r <= O.PARITY_RTOL[np_]
