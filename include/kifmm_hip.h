@@ -84,13 +84,13 @@ typedef struct kifmm_gpu_tuning {
   int reserved[2];
 } kifmm_gpu_tuning;
 enum {
-  KIFMM_LEVEL_AUTO = 0,  /* default: the fused kernel for L2L + DC2DE, and for M2M at NP <= 4
-                            (column GEMMs for M2M at NP = 6): the faster forms measured on
+  KIFMM_LEVEL_AUTO = 0,  /* default: as FUSED, the faster form measured at every NP on
                             uniform and clustered inputs */
   KIFMM_LEVEL_GEMM = 1,  /* two column GEMMs per level (K split over blocks when the level has
                             few columns, then a reduction launch) */
-  KIFMM_LEVEL_FUSED = 2  /* one kernel per level: both operator applies of 16 columns per
-                            block, the intermediate vectors kept in LDS */
+  KIFMM_LEVEL_FUSED = 2  /* no reductions: M2M as two launches whose blocks share a column
+                            tile's rows; L2L + DC2DE as one kernel that keeps the intermediate
+                            vectors in LDS, on short levels at NP = 6 as two launches */
 };
 enum {
   KIFMM_HAD_VALU = 0, /* the 64 child products per neighbour on the VALU, a lane per parent */

@@ -1790,102 +1790,122 @@ __global__ __launch_bounds__(256) void k_l2l_dc2de(int ne, int lde, const double
   }
 }
 
-/* One level of the upward pass with its two operator applies fused
- * (up_eval__gpu_non_leaf + up_calc__gpu_reduction, fmm/cuda.cu:430-566): a
- * block owns up to 16 parents at depth d (in_off[j] = their 8 children's
- * upward densities, 8 * lde contiguous doubles; out_off[j] = their own).
- *   phase 1  chk = 2^(d+1) UE2UC_stack (children's densities)   (UC check values)
- *   phase 2  uden[parent] = 2^-d UC2UE chk
- * v_mfma_f64_16x16x4f64 over the 16 parent columns, K in steps of 4 in
- * order (the column GEMM's order, so its sums are bit-identical to two
- * unsplit k_gemm_cols launches), the children's densities staged through LDS
- * 64 k at a time (the next chunk loaded during the current one) and chk kept
- * in LDS between the phases.  RT1 / RT2: row
- * tiles of the two operators (lda_uc / 16, lda_e / 16). */
-constexpr int M2M_KC = 64;
-template <int RT1, int RT2>
-__global__ __launch_bounds__(256) void k_m2m(int ne, int lde, int lduc, const double* __restrict__ UE2UC, int lda_uc,
-                                             const double* __restrict__ UC2UE, int lda_e, int npar,
-                                             const int* __restrict__ in_off, const int* __restrict__ out_off, int d,
-                                             double* __restrict__ uden) {
-  constexpr int LDC = 16 * RT1 + 1; /* odd: conflict-free column reads */
-  __shared__ double Bs[16][M2M_KC + 1];
-  __shared__ double C[16][LDC];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j0 = blockIdx.x * 16, jn = min(16, npar - j0);
+/* One operator apply of a level, spread over blocks by row: 16 columns and 4
+ * row tiles (a wave each) per block, for part z = blockIdx.z
+ *   out[off(j) + z out_z + row] (= or +=) 2^e(j) (A + z a_z)[row][k] x(j)[z in_z + k],
+ * off(j) = out_off[j], or j ldo where out_off is null; x(j) at in_off[j], or
+ * j ldi where that is null, the sum of NIN slices (the parts of a product
+ * split along K), added in order while staged.  Every sum runs over k in
+ * steps of 4 in order, as k_l2l_dc2de's do: the same bits.
+ * A level of a few dozen columns is bound by latency.  One block per 16
+ * columns, both applies in it, put the 10 x 112 MFMAs of the NP 4 UE2UC
+ * stack (64 cycles each, 7.5 us of one CU's four matrix pipes) and its chain
+ * of operator loads on one CU: 27 - 30 us per level.  Here three blocks share
+ * it, a pipe has one row tile, and the operator's next LVL_KB steps load while
+ * the current ones multiply (8 steps ahead: 12 us, 16: 10); the check values
+ * make a trip through L2 and a second launch applies the other operator.
+ * Per level, M2M at NP 4: 28 -> 15 us (up to 2 thousand columns), 160 -> 141
+ * (32768); at NP 6, whose 304 steps are split along K in 4 parts on short
+ * levels, two split column GEMMs with their reductions -> this: 35 - 45
+ * -> 18 us up to 300 parents, 62 -> 40 at 990, 140 -> 89 at 4096; L2L + DC2DE
+ * at NP 6, fused -> this: 25 -> 13, 39 -> 35 at 990 parents. */
+constexpr int LVL_KC = 256, LVL_KB = 16; /* k staged in LDS at a time; steps of 4 k loaded ahead */
+struct LevelOp {
+  int M, K;             /* rows; k (a multiple of 8) */
+  const double* A;
+  int lda;
+  size_t a_z;
+  int ncols;
+  const int* in_off;    /* null: column j at j ldi */
+  int ldi;
+  int in_z;
+  const double* in;
+  size_t slice;         /* between input slices */
+  const int* out_off;   /* null: column j at j ldo */
+  int ldo;
+  size_t out_z;
+  double* out;
+  const int* sexp;      /* scales 2^sexp[j], or null: 2^e */
+  int e, accumulate;
+};
+template <int NIN>
+__global__ __launch_bounds__(256) void k_level_op(const LevelOp op) {
+  constexpr int PER = LVL_KC / 32, CHUNK = LVL_KC / 4;
+  static_assert(LVL_KC % 32 == 0 && CHUNK % LVL_KB == 0, "whole batches per staged chunk");
+  __shared__ double Bs[16][LVL_KC + 1]; /* odd: conflict-free column reads */
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int z = blockIdx.z, col0 = blockIdx.x * 16, tile = blockIdx.y * 4 + wave;
+  const bool active = 16 * tile < op.M; /* wave-uniform */
   const int jl = lane & 15, kl = lane >> 4;
-  const int K = 8 * lde;
-  constexpr int TPW1 = (RT1 + 3) / 4, TPW2 = (RT2 + 3) / 4;
-  v4d acc[TPW1];
+  /* staging: 16 threads per column, each the k pairs 2 (tid & 15) + 32 m of a chunk */
+  const int sj = tid >> 4, sk = 2 * (tid & 15), scol = min(col0 + sj, op.ncols - 1); /* past the end: not used */
+  const double* __restrict__ ip =
+      op.in + (op.in_off ? (size_t)op.in_off[scol] : (size_t)scol * op.ldi) + (size_t)z * op.in_z;
+  double r0[PER], r1[PER];
+  auto fetch = [&](int k0) {
 #pragma unroll
-  for (int u = 0; u < TPW1; u++) acc[u] = (v4d){0.0, 0.0, 0.0, 0.0};
-  /* the children's densities of the next K chunk are loaded into
-   * registers while the current chunk is multiplied */
-  constexpr int BPT = 16 * M2M_KC / 256;
-  double rb[BPT];
-  size_t boff[BPT];
+    for (int m = 0; m < PER; m++) {
+      const int k = min(k0 + sk + 32 * m, op.K - 2); /* past the end: not used */
+      r0[m] = ip[k];
+      r1[m] = ip[k + 1];
 #pragma unroll
-  for (int m = 0; m < BPT; m++) {
-    const int j = (tid + 256 * m) / M2M_KC;
-    boff[m] = j < jn ? (size_t)in_off[j0 + j] : 0;
-  }
-  auto load_b = [&](int kc) {
-    const int kn = min(M2M_KC, K - kc);
-#pragma unroll
-    for (int m = 0; m < BPT; m++) {
-      const int e = tid + 256 * m, j = e / M2M_KC, k = e % M2M_KC;
-      rb[m] = (j < jn && k < kn) ? uden[boff[m] + kc + k] : 0.0;
+      for (int q = 1; q < NIN; q++) {
+        r0[m] += ip[q * op.slice + k];
+        r1[m] += ip[q * op.slice + k + 1];
+      }
     }
   };
-  load_b(0);
-  for (int kc = 0; kc < K; kc += M2M_KC) {
-    const int kn = min(M2M_KC, K - kc); /* a multiple of 4 (8 lde) */
-    __syncthreads(); /* the previous chunk's readers are done */
+  const int nsteps = op.K / 4;
+  const double* __restrict__ a = op.A + z * op.a_z + (size_t)kl * op.lda + min(16 * tile + jl, op.M - 1);
+  double av[2][LVL_KB];
+  auto load = [&](double (&v)[LVL_KB], int sb) { /* steps past the end repeat the last: loaded, not used */
 #pragma unroll
-    for (int m = 0; m < BPT; m++) {
-      const int e = tid + 256 * m;
-      Bs[e / M2M_KC][e % M2M_KC] = rb[m];
+    for (int st = 0; st < LVL_KB; st++) v[st] = a[(size_t)(4 * min(sb + st, nsteps - 1)) * op.lda];
+  };
+  v4d acc = (v4d){0.0, 0.0, 0.0, 0.0};
+  auto mul = [&](const double (&v)[LVL_KB], int sb) {
+    const double* b = &Bs[jl][4 * (sb % CHUNK) + kl];
+#pragma unroll
+    for (int st = 0; st < LVL_KB; st++) {
+      if (sb + st >= nsteps) break;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v[st], b[4 * st], acc, 0, 0, 0);
+    }
+  };
+  auto stage = [&](int sb) { /* at a chunk's first step: its inputs to LDS, the next chunk's loads under way */
+    if (sb % CHUNK != 0) return;
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < PER; m++) {
+      Bs[sj][sk + 32 * m] = r0[m];
+      Bs[sj][sk + 32 * m + 1] = r1[m];
     }
     __syncthreads();
-    if (kc + M2M_KC < K) load_b(kc + M2M_KC);
-    mfma_chain<8>(
-        kn / 4,
-        [&](int st, int u) {
-          const int row_a = min(16 * (wave + 4 * u) + (lane & 15), lda_uc - 1); /* rows past RT1 tiles: unused */
-          return UE2UC[(size_t)(kc + 4 * st + kl) * lda_uc + row_a];
-        },
-        [&](int st) { return Bs[jl][4 * st + kl]; }, acc);
-  }
-  const double s1 = ldexp(1.0, d + 1), s2 = ldexp(1.0, -d);
-#pragma unroll
-  for (int u = 0; u < TPW1; u++) {
-    const int r = wave + 4 * u;
-    if (r >= RT1) continue;
-#pragma unroll
-    for (int i = 0; i < 4; i++) C[jl][16 * r + kl + 4 * i] = s1 * acc[u][i];
-  }
-  __syncthreads();
-  v4d acc2[TPW2];
-#pragma unroll
-  for (int u = 0; u < TPW2; u++) acc2[u] = (v4d){0.0, 0.0, 0.0, 0.0};
-  mfma_chain<8>(
-      lduc / 4,
-      [&](int st, int u) {
-        const int row_a = min(16 * (wave + 4 * u) + (lane & 15), lda_e - 1);
-        return UC2UE[(size_t)(4 * st + kl) * lda_e + row_a];
-      },
-      [&](int st) { return C[jl][4 * st + kl]; }, acc2);
-  if (jl >= jn) return;
-  double* const out = uden + out_off[j0 + jl];
-#pragma unroll
-  for (int u = 0; u < TPW2; u++) {
-    const int r = wave + 4 * u;
-    if (r >= RT2) continue;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int row = 16 * r + kl + 4 * i;
-      if (row < ne) out[row] = s2 * acc2[u][i];
+    if (4 * (sb + CHUNK) < op.K) fetch(4 * (sb + CHUNK));
+  };
+  fetch(0);
+  if (active) load(av[0], 0);
+  for (int sb = 0; sb < nsteps; sb += 2 * LVL_KB) {
+    stage(sb);
+    if (active) {
+      if (sb + LVL_KB < nsteps) load(av[1], sb + LVL_KB);
+      mul(av[0], sb);
     }
+    if (sb + LVL_KB < nsteps) {
+      stage(sb + LVL_KB);
+      if (active) {
+        if (sb + 2 * LVL_KB < nsteps) load(av[0], sb + 2 * LVL_KB);
+        mul(av[1], sb + LVL_KB);
+      }
+    }
+  }
+  const int col = col0 + jl;
+  if (!active || col >= op.ncols) return;
+  const double sc = ldexp(1.0, op.sexp ? op.sexp[col] : op.e);
+  double* const o = op.out + (op.out_off ? (size_t)op.out_off[col] : (size_t)col * op.ldo) + z * op.out_z;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int row = 16 * tile + kl + 4 * i;
+    if (row < op.M) o[row] = op.accumulate ? o[row] + sc * acc[i] : sc * acc[i];
   }
 }
 

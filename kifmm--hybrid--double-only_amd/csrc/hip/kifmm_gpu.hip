@@ -293,6 +293,13 @@ int check_view(const kifmm_tree_view* t) {
   return KIFMM_OK;
 }
 
+/* Parts along K of a level's UE2UC stack: at NP 6 (304 MFMA steps, FP64 only)
+ * short levels split it over more blocks; at NP <= 4, where the mixed path
+ * needs one order of summation, never. */
+constexpr int M2M_PARTS = 4;
+inline int m2m_parts(int np, int ncols) { return np == 6 && ncols < 1024 ? M2M_PARTS : 1; }
+constexpr int LEAF_SPLIT = 8192; /* leaves below which the FP64 leaf UC2UE is a k_level_op */
+
 /* Everything the device needs, derived on the host from the tree view.
  * make_plan() touches no device; upload() copies a checked plan. */
 struct HostGemm {
@@ -902,7 +909,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
         wc.gemm_flops += 2.0 * ne * ne;
       }
     }
-    P.chk_cols = std::max(P.chk_cols, (size_t)col);
+    P.chk_cols = std::max(P.chk_cols, (size_t)col * m2m_parts(np, col));
   }
   /* the fused downward kernel (k_l2l_dc2de) of depth d >= 3 runs over the
    * L2L parents at d - 1 and writes the densities of their target
@@ -1387,39 +1394,15 @@ int gemm(kifmm_gpu* g, const GemmList& L, int M, int K, const double* A, int lda
   return KIFMM_OK;
 }
 
-/* Per level, M2M (UE2UC stack, then UC2UE) and L2L + DC2DE run either as
- * two column GEMMs or as one fused kernel.  A fused block runs every k step
- * of both operators for its 16 columns with 4 waves: fine for the square
- * n_e x n_e operators of the downward pass and for the UE2UC stack (K =
- * 8 n_e) up to NP = 4, but at NP = 6 (K = 1216) that serial chain per block
- * is longer than the column GEMMs (64 columns a block, K split over blocks
- * on short levels).  The automatic choice is fused down, fused up at
- * NP <= 4 and GEMMs up at NP = 6; KIFMM_LEVEL_GEMM / _FUSED force one form. */
-bool fused_up(const kifmm_gpu* g) {
-  return g->up_form == KIFMM_LEVEL_FUSED || (g->up_form == KIFMM_LEVEL_AUTO && g->np <= 4);
-}
-bool fused_down(const kifmm_gpu* g) {
-  return g->down_form != KIFMM_LEVEL_GEMM; /* AUTO: the fused kernel at every NP */
-}
-
-int m2m(kifmm_gpu* g, const GemmList& A, const GemmList& B, int d) {
-  const dim3 grid((A.n + 15) / 16);
-  const int rt1 = g->lda_uc / 16, rt2 = g->lda_e / 16;
-#define KIFMM_M2M_CASE(R1, R2)                                                                                    \
-  if (rt1 == R1 && rt2 == R2)                                                                                     \
-    hipLaunchKernelGGL((k_m2m<R1, R2>), grid, dim3(256), 0, g->stream, g->n_e, g->ld_e, g->ld_uc, g->UE2UC,        \
-                       g->lda_uc, g->UC2UE, g->lda_e, A.n, A.in_off, B.out_off, d, g->uden);
-  KIFMM_M2M_CASE(7, 2)
-  else KIFMM_M2M_CASE(10, 4)
-  else KIFMM_M2M_CASE(19, 10)
-  else {
-    set_error("internal: no fused upward kernel for these operator sizes");
-    return KIFMM_EINVAL;
-  }
-#undef KIFMM_M2M_CASE
-  LAUNCH_CHECK();
-  return KIFMM_OK;
-}
+/* KIFMM_LEVEL_GEMM runs a level's applies as column GEMMs; otherwise (AUTO,
+ * FUSED) M2M is two launches of k_level_op, and L2L + DC2DE is the fused
+ * kernel, or at NP 6 on levels of up to L2L_SPLIT parents two launches of
+ * k_level_op as well (13 us against 25 up to 200 parents, 35 against 39 at 990,
+ * 119 against 119 at 4096; at NP 4 the fused kernel's 9 us beat two launches'
+ * 11).  The two orders of summation are the same bit for bit. */
+bool level_gemm_up(const kifmm_gpu* g) { return g->up_form == KIFMM_LEVEL_GEMM; }
+bool level_gemm_down(const kifmm_gpu* g) { return g->down_form == KIFMM_LEVEL_GEMM; }
+constexpr int L2L_SPLIT = 2048;
 
 /* L2L of the parents at depth d - 1 and DC2DE of their children, fused */
 int l2l_dc2de(kifmm_gpu* g, const GemmList& L, int d) {
@@ -1441,6 +1424,56 @@ int l2l_dc2de(kifmm_gpu* g, const GemmList& L, int d) {
   }
   LAUNCH_CHECK();
   return KIFMM_OK;
+}
+
+int level_op(kifmm_gpu* g, const LevelOp& op, int parts, int nin) {
+  if (op.ncols == 0) return KIFMM_OK;
+  const dim3 grid((op.ncols + 15) / 16, (op.M + 63) / 64, parts);
+  if (nin == 1) hipLaunchKernelGGL(k_level_op<1>, grid, dim3(256), 0, g->stream, op);
+  else hipLaunchKernelGGL(k_level_op<M2M_PARTS>, grid, dim3(256), 0, g->stream, op);
+  LAUNCH_CHECK();
+  return KIFMM_OK;
+}
+
+/* UC2UE: check values (lduc apart, in nin slices) to upward densities */
+int uc2ue(kifmm_gpu* g, const GemmList& B, int nin) {
+  LevelOp op{};
+  op.M = g->n_e; op.K = g->ld_uc; op.A = g->UC2UE; op.lda = g->lda_e;
+  op.ncols = B.n; op.ldi = g->ld_uc; op.in = g->chk; op.slice = (size_t)B.n * g->ld_uc;
+  op.out_off = B.out_off; op.out = g->uden; op.sexp = B.sexp;
+  return level_op(g, op, 1, nin);
+}
+
+/* M2M of one level in two launches: the UE2UC stack into check values, in
+ * m2m_parts slices along K, then UC2UE */
+int m2m(kifmm_gpu* g, const GemmList& A, const GemmList& B, int d) {
+  const int parts = m2m_parts(g->np, A.n);
+  LevelOp op{};
+  op.M = g->n_uc; op.K = 8 * g->ld_e / parts; op.A = g->UE2UC; op.lda = g->lda_uc;
+  op.a_z = (size_t)op.K * g->lda_uc; op.in_z = op.K;
+  op.ncols = A.n; op.in_off = A.in_off; op.in = g->uden;
+  op.ldo = g->ld_uc; op.out_z = (size_t)A.n * g->ld_uc; op.out = g->chk; op.e = d + 1;
+  TRY(level_op(g, op, parts, 1));
+  return uc2ue(g, B, parts);
+}
+
+/* DC2DE of the nodes of depth d */
+int dc2de(kifmm_gpu* g, const GemmList& D, int d) {
+  LevelOp op{};
+  op.M = g->n_e; op.K = g->ld_e; op.A = g->DC2DE; op.lda = g->lda_e;
+  op.ncols = D.n; op.in_off = D.in_off; op.in = g->dchk; op.out_off = D.out_off; op.out = g->dden; op.e = -d;
+  return level_op(g, op, 1, 1);
+}
+
+/* L2L of the parents at depth d - 1, an octant of children per part, then
+ * DC2DE of the children */
+int l2l_dc2de_split(kifmm_gpu* g, const GemmList& L, const GemmList& D, int d) {
+  LevelOp op{};
+  op.M = g->n_e; op.K = g->ld_e; op.A = g->DE2DC; op.lda = g->lda_l2l; op.a_z = g->ld_e;
+  op.ncols = L.n; op.in_off = L.in_off; op.in = g->dden;
+  op.out_off = L.out_off; op.out_z = g->ld_e; op.out = g->dchk; op.e = d - 1; op.accumulate = 1;
+  TRY(level_op(g, op, 8, 1));
+  return dc2de(g, D, d);
 }
 
 int fill(kifmm_gpu* g, double* p, size_t n) {
@@ -1714,11 +1747,18 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
                          g->ld_surf, g->src4, g->chk, lduc);
     }
     LAUNCH_CHECK();
-    TRY(gemm(g, g->s2m_gemm, g->n_e, lduc, g->UC2UE, g->lda_e, g->chk, g->uden, 0));
+    /* below LEAF_SPLIT leaves the column GEMM splits K, with a reduction, or
+     * has few blocks: 21 -> 6 us at 4096 leaves NP 4, 57 -> 27 at 6592 NP 6
+     * (94 us at 32768 NP 6, where this would take about 130).  The mixed path keeps that order: another one flips FP32
+     * roundings further on (see k_x_surf) */
+    if (g->precision == KIFMM_PREC_FP64 && g->s2m_gemm.n < LEAF_SPLIT)
+      TRY(uc2ue(g, g->s2m_gemm, 1));
+    else
+      TRY(gemm(g, g->s2m_gemm, g->n_e, lduc, g->UC2UE, g->lda_e, g->chk, g->uden, 0));
   }
   for (int d = g->max_depth - 1; d >= 0 && (mask & KIFMM_PHASE_UP); d--) {
     if (g->lv[d].m2m_a.n == 0) continue;
-    if (fused_up(g)) {
+    if (!level_gemm_up(g)) {
       TRY(m2m(g, g->lv[d].m2m_a, g->lv[d].m2m_b, d));
     } else {
       TRY(gemm(g, g->lv[d].m2m_a, g->n_uc, 8 * lde, g->UE2UC, g->lda_uc, g->uden, g->chk, 0));
@@ -1745,8 +1785,13 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
   /* down: DC2DE at depth 2, then per level the fused L2L + DC2DE
    * (k_l2l_dc2de over the parents at depth d - 1), then L2T */
   for (int d = 2; d <= g->max_depth && (mask & KIFMM_PHASE_DOWN); d++) {
-    if (d >= 3 && fused_down(g)) {
-      TRY(l2l_dc2de(g, g->lv[d - 1].l2l, d));
+    if (d >= 3 && !level_gemm_down(g)) {
+      if (g->np == 6 && g->lv[d - 1].l2l.n <= L2L_SPLIT) TRY(l2l_dc2de_split(g, g->lv[d - 1].l2l, g->lv[d].dc2de, d));
+      else TRY(l2l_dc2de(g, g->lv[d - 1].l2l, d));
+      continue;
+    }
+    if (d == 2 && g->precision == KIFMM_PREC_FP64 && !level_gemm_down(g)) {
+      TRY(dc2de(g, g->lv[d].dc2de, d)); /* the mixed path keeps the split column GEMM's order */
       continue;
     }
     if (d >= 3) TRY(gemm(g, g->lv[d - 1].l2l, 8 * lde, lde, g->DE2DC, g->lda_l2l, g->dden, g->dchk, 1));
