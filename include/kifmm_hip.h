@@ -250,7 +250,7 @@ int kifmm_gpu_direct(kifmm_gpu* g, int nt, const double* tx, const double* ty, c
  * device memory (code under HIP graph capture, serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  The targets and sums
  * are staged in a file-scope device array of the library holding at most
- * KIFMM_DIRECT_NOALLOC_MAX points (512 KiB per device, kept until the
+ * KIFMM_DIRECT_NOALLOC_MAX points (1 MiB per device, kept until the
  * process ends); larger nt is rejected with KIFMM_EINVAL.  Every call on
  * one device shares that array: calls that overlap on one device (other
  * threads, other handles) race.  Blocks until the sums are in out. */

@@ -3136,46 +3136,128 @@ static __global__ __launch_bounds__(64) void k_l2t(const int4* __restrict__ item
   if (k < it.z) pot[it.y + k] += HALF_OOFP_R * ih * ((acc[0] + acc[1]) + (acc[2] + acc[3]));
 }
 
-/* Sampled direct sum for validation (validate, fmm/driver.cc:141-206, on
- * the GPU): one block per target point, 256 lanes stride over all sources,
- * FP64 w / sqrt(r^2) (IEEE division and square root, r = 0 excluded) with
- * Neumaier-compensated lane sums, combined by lane 0 in lane order (also
- * compensated): the result is independent of the source order to about
- * one rounding. */
-__device__ __forceinline__ void neumaier(double& s, double& c, double v) {
-  const double t = s + v;
-  c += fabs(s) >= fabs(v) ? (s - t) + v : (v - t) + s;
+/* Sampled direct sums for validation (validate, fmm/driver.cc:141-206, on
+ * the GPU): FP64 w / r over all sources, r = 0 excluded, compensated, so that
+ * the result is independent of the source order to about one rounding.
+ *
+ * Bound: the FP64 pipe.  A pair costs three differences, r^2 (3), v_rsq_f64
+ * (four slots), its third-order correction (4) and w / r into a run of DIR_RUN
+ * sources (1); the run's NaN test and compensated add (8) are shared by its
+ * sources: 17 slots, 0.57 ms for 1000 targets x 1M sources (a slot takes 5
+ * cycles, not 4, in a loop of FP64 FMAs alone, at 2.4 GHz).
+ * The correction has to be of third order: a Newton step leaves the one-sided
+ * error 3/2 e^2, up to 4e-15 of every term, which no summation averages out;
+ * with it a term is as close as division and square root give (about an ulp,
+ * either side).  r^2 = 0 and infinity make the run NaN (0 x infinity in the
+ * correction), and one test per run instead of one per pair then sends the
+ * wave through w / sqrt(r^2) itself, as a NaN of the inputs does.
+ *
+ * A block takes DIR_T targets (wave-uniform, so in scalar registers) and one
+ * chunk of the sources, which its lanes stride: a source record is read once
+ * for DIR_T pairs.  Chunk c is on the blocks b = c mod n_chunk, with n_chunk a
+ * multiple of 8 on XCD c mod 8 alone (direct_plan).  The chunks' sums are
+ * joined by k_direct_join.  1000 x 1M, the whole call: 2.65 ms with a block
+ * per target, division and square root, 0.62 now (error against long double
+ * 8.8e-17 rms both ways) */
+constexpr int DIR_T = 8, DIR_RUN = 4;
+/* (s, c) + v */
+__device__ __forceinline__ void two_sum(double& s, double& c, double v) {
+  const double t = s + v, b = t - s;
+  c += (s - (t - b)) + (v - b);
   s = t;
 }
+/* w / r for r^2 as it comes, 0 for r = 0 */
+__device__ __forceinline__ double pair_exact(double w, double r2) { return r2 != 0.0 ? w / sqrt(r2) : 0.0; }
 
+/* targets DIR_T i .. + DIR_T - 1 at tx, ty, tz[nt] (past the last one it is
+ * repeated) over the sources [c per, (c + 1) per): part[(c groups + i) DIR_T + k]
+ * = (s, c) */
 static __global__ __launch_bounds__(256) void k_direct(int nt, const double* __restrict__ tx,
                                                        const double* __restrict__ ty, const double* __restrict__ tz,
-                                                       const double4* __restrict__ src4, int n,
-                                                       double* __restrict__ out) {
-  __shared__ double ss[256], sc[256];
-  const int tid = threadIdx.x;
-  for (int t = blockIdx.x; t < nt; t += gridDim.x) {
-    const double x = tx[t], y = ty[t], z = tz[t];
-    double s = 0.0, c = 0.0;
-    for (int j = tid; j < n; j += 256) {
-      const double4 p = src4[j];
-      const double dx = x - p.x, dy = y - p.y, dz = z - p.z;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      if (r2 != 0.0) neumaier(s, c, p.w / sqrt(r2));
+                                                       const double4* __restrict__ src4, int n, int groups, int n_chunk,
+                                                       int per, double2* __restrict__ part) {
+  __shared__ double2 sh[4][DIR_T];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long items = (long)groups * n_chunk;
+  for (long b = blockIdx.x; b < items; b += gridDim.x) {
+    const int c = (int)(b % n_chunk), i = (int)(b / n_chunk);
+    const int lo = (int)min((long)n, (long)c * per);
+    const long hi = min((long)n, (long)lo + per);
+    double x[DIR_T], y[DIR_T], z[DIR_T], s[DIR_T], e[DIR_T];
+#pragma unroll
+    for (int k = 0; k < DIR_T; k++) {
+      const int t = min(i * DIR_T + k, nt - 1);
+      x[k] = tx[t], y[k] = ty[t], z[k] = tz[t];
+      s[k] = e[k] = 0.0;
     }
-    ss[tid] = s;
-    sc[tid] = c;
-    __syncthreads();
-    if (tid == 0) {
-      double S = 0.0, Cc = 0.0;
-      for (int k = 0; k < 256; k++) {
-        neumaier(S, Cc, ss[k]);
-        Cc += sc[k];
+    for (long j0 = (long)lo + threadIdx.x; j0 < hi; j0 += 256 * DIR_RUN) {
+      double4 p[DIR_RUN];
+#pragma unroll
+      for (int u = 0; u < DIR_RUN; u++) {
+        const long j = j0 + 256 * u;
+        p[u] = src4[j < hi ? j : hi - 1];
+        if (j >= hi) p[u] = make_double4(FAR, FAR, FAR, 0.0);
       }
-      out[t] = OOFP_R * (S + Cc);
+#pragma unroll
+      for (int k = 0; k < DIR_T; k++) {
+        double v = 0.0;
+#pragma unroll
+        for (int u = 0; u < DIR_RUN; u++) {
+          const double dx = x[k] - p[u].x, dy = y[k] - p[u].y, dz = z[k] - p[u].z;
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          const double q = __builtin_amdgcn_rsq(r2);
+          const double f = __builtin_fma(-(r2 * q), q, 1.0);
+          v = __builtin_fma(p[u].w, __builtin_fma(q * f, __builtin_fma(f, 0.375, 0.5), q), v);
+        }
+        if (__builtin_expect(__any(v != v), 0)) {
+          v = 0.0;
+#pragma unroll 1
+          for (long j = j0; j < min(hi, j0 + 256 * DIR_RUN); j += 256) {
+            const double4 o = src4[j];
+            const double dx = x[k] - o.x, dy = y[k] - o.y, dz = z[k] - o.z;
+            v += pair_exact(o.w, dx * dx + dy * dy + dz * dz);
+          }
+        }
+        two_sum(s[k], e[k], v);
+      }
+    }
+    /* lanes, then waves */
+#pragma unroll
+    for (int k = 0; k < DIR_T; k++) {
+      for (int m = 32; m > 0; m >>= 1) {
+        const double so = __shfl_xor(s[k], m), eo = __shfl_xor(e[k], m);
+        e[k] += eo;
+        two_sum(s[k], e[k], so);
+      }
+      if (lane == 0) sh[wave][k] = make_double2(s[k], e[k]);
+    }
+    __syncthreads();
+    if (threadIdx.x < DIR_T) {
+      double2 a = sh[0][threadIdx.x];
+      for (int w = 1; w < 4; w++) {
+        a.y += sh[w][threadIdx.x].y;
+        two_sum(a.x, a.y, sh[w][threadIdx.x].x);
+      }
+      part[((long)c * groups + i) * DIR_T + threadIdx.x] = a;
     }
     __syncthreads();
   }
+}
+
+/* out[t] = the sum of target t's chunks, in order; one lane per target */
+static __global__ __launch_bounds__(64) void k_direct_join(int nt, int groups, int n_chunk,
+                                                           const double2* __restrict__ part,
+                                                           double* __restrict__ out) {
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t >= nt) return;
+  double s = 0.0, e = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < n_chunk; c++) {
+    const double2 a = part[(long)c * groups * DIR_T + t];
+    e += a.y;
+    two_sum(s, e, a.x);
+  }
+  out[t] = OOFP_R * (s + e);
 }
 
 static __global__ void k_fill(double* __restrict__ p, size_t n, double v) {

@@ -41,12 +41,14 @@ using namespace kifmm_dev;
 using kifmm::set_error;
 
 /* Device scratch of kifmm_gpu_direct_noalloc: the staged coordinates of up
- * to KIFMM_DIRECT_NOALLOC_MAX points and their sums.  Every device the
+ * to KIFMM_DIRECT_NOALLOC_MAX points, their sums and the chunks' partial
+ * sums (direct_plan: at most DIR_ITEMS groups of them).  Every device the
  * library runs on holds its own copy until the process ends.  In host code
  * the array's name is not a device address: the per-device address comes
  * from hipGetSymbolAddress (scratch_address, called by kifmm_gpu_create with
  * the handle's device current) and only that address is passed on. */
-static __device__ __align__(256) double scratch[4 * KIFMM_DIRECT_NOALLOC_MAX];
+constexpr int DIR_ITEMS = 4096;
+static __device__ __align__(256) double scratch[4 * KIFMM_DIRECT_NOALLOC_MAX + 2 * DIR_T * DIR_ITEMS];
 
 namespace {
 
@@ -2132,34 +2134,71 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   return KIFMM_OK;
 }
 
+/* The split of nt targets over n sources: chunks of the sources until there
+ * are DIR_ITEMS work items (four per block slot of the chip at 4 blocks of 4
+ * waves per CU, so that the last round is a quarter of the work at most), a
+ * chunk being at least one run of every lane.  At 8 chunks or more a multiple
+ * of 8: a chunk then stays in one XCD's L2.  groups * n_chunk <= DIR_ITEMS,
+ * or one chunk. */
+struct DirectPlan {
+  int groups, n_chunk, per;
+  size_t part() const { return (size_t)groups * n_chunk * DIR_T; }
+};
+static DirectPlan direct_plan(int nt, int n) {
+  constexpr int run = 256 * DIR_RUN;
+  DirectPlan p;
+  p.groups = (int)(((long)nt + DIR_T - 1) / DIR_T);
+  const int most = std::max(1, (int)(((long)n + run - 1) / run));
+  int c = std::min(std::max(1, DIR_ITEMS / p.groups), most);
+  if (c >= 8) c &= ~7;
+  p.n_chunk = c;
+  p.per = (int)(((long)n + (long)c * run - 1) / ((long)c * run)) * run;
+  return p;
+}
+
+/* d: x, y, z, sums [nt] each, then plan.part() double2.  The targets go up
+ * in one copy, joined on the host first: three cost 8 us more each */
+static int direct_queue(kifmm_gpu* g, const DirectPlan& p, int nt, const double* xyz, double* out, double* d) {
+  const size_t b = sizeof(double) * (size_t)nt;
+  double* const sums = d + 3 * (size_t)nt;
+  double2* const part = reinterpret_cast<double2*>(d + 4 * (size_t)nt);
+  HIP_TRY(hipMemcpyAsync(d, xyz, 3 * b, hipMemcpyHostToDevice, g->stream));
+  const long items = (long)p.groups * p.n_chunk;
+  hipLaunchKernelGGL(k_direct, dim3((unsigned)std::min<long>(items, 1 << 20)), dim3(256), 0, g->stream, nt, d, d + nt,
+                     d + 2 * (size_t)nt, g->src4, g->n_src, p.groups, p.n_chunk, p.per, part);
+  hipLaunchKernelGGL(k_direct_join, dim3((unsigned)(((long)nt + 63) / 64)), dim3(64), 0, g->stream, nt, p.groups,
+                     p.n_chunk, part, sums);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(out, sums, b, hipMemcpyDeviceToHost, g->stream));
+  return KIFMM_OK;
+}
+static int direct_run(kifmm_gpu* g, const DirectPlan& p, int nt, const double* tx, const double* ty, const double* tz,
+                      double* out, double* d) {
+  const std::unique_ptr<double[]> xyz(new (std::nothrow) double[3 * (size_t)nt]);
+  if (!xyz) {
+    set_error("direct sums: out of host memory");
+    return KIFMM_ENOMEM;
+  }
+  std::copy(tx, tx + nt, xyz.get());
+  std::copy(ty, ty + nt, xyz.get() + nt);
+  std::copy(tz, tz + nt, xyz.get() + 2 * (size_t)nt);
+  const int r = direct_queue(g, p, nt, xyz.get(), out, d);
+  HIP_TRY(hipStreamSynchronize(g->stream));
+  return r;
+}
+
 int kifmm_gpu_direct(kifmm_gpu* g, int nt, const double* tx, const double* ty, const double* tz, double* out) {
   if (!g || nt <= 0 || !tx || !ty || !tz || !out) {
     set_error("kifmm_gpu_direct: invalid argument");
     return KIFMM_EINVAL;
   }
   HIP_TRY(hipSetDevice(g->dev));
+  const DirectPlan p = direct_plan(nt, g->n_src);
   double* d = nullptr;
-  HIP_TRY(hipMalloc(&d, sizeof(double) * 4 * (size_t)nt));
-  auto done = [&](int r) {
-    (void)hipFree(d);
-    return r;
-  };
-  const size_t b = sizeof(double) * nt;
-  if (hipMemcpyAsync(d, tx, b, hipMemcpyHostToDevice, g->stream) != hipSuccess ||
-      hipMemcpyAsync(d + nt, ty, b, hipMemcpyHostToDevice, g->stream) != hipSuccess ||
-      hipMemcpyAsync(d + 2 * (size_t)nt, tz, b, hipMemcpyHostToDevice, g->stream) != hipSuccess) {
-    set_error("kifmm_gpu_direct: upload failed");
-    return done(KIFMM_EDEVICE);
-  }
-  hipLaunchKernelGGL(k_direct, dim3(std::min(nt, 65535)), dim3(256), 0, g->stream, nt, d, d + nt, d + 2 * (size_t)nt,
-                     g->src4, g->n_src, d + 3 * (size_t)nt);
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(out, d + 3 * (size_t)nt, b, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-      hipStreamSynchronize(g->stream) != hipSuccess) {
-    set_error("kifmm_gpu_direct: kernel or copy failed");
-    return done(KIFMM_EDEVICE);
-  }
-  return done(KIFMM_OK);
+  HIP_TRY(hipMalloc(&d, sizeof(double) * (4 * (size_t)nt + 2 * p.part())));
+  const int r = direct_run(g, p, nt, tx, ty, tz, out, d);
+  (void)hipFree(d);
+  return r;
 }
 
 int kifmm_gpu_direct_noalloc(kifmm_gpu* g, int nt, const double* tx, const double* ty, const double* tz,
@@ -2178,19 +2217,11 @@ int kifmm_gpu_direct_noalloc(kifmm_gpu* g, int nt, const double* tx, const doubl
     return KIFMM_EDEVICE;
   }
   HIP_TRY(hipSetDevice(g->dev));
-  /* targets at d, d + nt, d + 2 nt, sums at d + 3 nt: inside 4 * MAX doubles;
-   * the kernel assigns every sum, so nothing needs clearing */
-  double* d = g->scratch;
-  const size_t b = sizeof(double) * nt;
-  HIP_TRY(hipMemcpyAsync(d, tx, b, hipMemcpyHostToDevice, g->stream));
-  HIP_TRY(hipMemcpyAsync(d + nt, ty, b, hipMemcpyHostToDevice, g->stream));
-  HIP_TRY(hipMemcpyAsync(d + 2 * (size_t)nt, tz, b, hipMemcpyHostToDevice, g->stream));
-  hipLaunchKernelGGL(k_direct, dim3(std::min(nt, 65535)), dim3(256), 0, g->stream, nt, d, d + nt, d + 2 * (size_t)nt,
-                     g->src4, g->n_src, d + 3 * (size_t)nt);
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(out, d + 3 * (size_t)nt, b, hipMemcpyDeviceToHost, g->stream));
-  HIP_TRY(hipStreamSynchronize(g->stream));
-  return KIFMM_OK;
+  /* 4 nt doubles and at most DIR_ITEMS groups of partial sums: MAX / DIR_T
+   * groups <= DIR_ITEMS.  The kernels assign every partial and every sum
+   * that is read, so nothing needs clearing */
+  static_assert(KIFMM_DIRECT_NOALLOC_MAX / DIR_T <= DIR_ITEMS, "one chunk of every group has to fit the scratch");
+  return direct_run(g, direct_plan(nt, g->n_src), nt, tx, ty, tz, out, g->scratch);
 }
 
 double kifmm_problem_validate_gpu(kifmm_problem* p, kifmm_gpu* g, const double* pot_orig, int nv, int* chk_ids,
