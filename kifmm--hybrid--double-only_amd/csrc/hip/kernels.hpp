@@ -3260,10 +3260,10 @@ static __global__ __launch_bounds__(64) void k_direct_join(int nt, int groups, i
   out[t] = OOFP_R * (s + e);
 }
 
-static __global__ void k_fill(double* __restrict__ p, size_t n, double v) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) p[i] = v;
+static __global__ void k_fill2(double* __restrict__ p, size_t n, double* __restrict__ q, size_t m) {
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = i0; i < n; i += stride) p[i] = 0.0;
+  for (size_t i = i0; i < m; i += stride) q[i] = 0.0;
 }
 
 /* pot = u + pot over [0, n): the U-list sums (u) written on the second

@@ -20,6 +20,7 @@
  *   T             translation spectra, frequency-major [f][343]
  *   operators     padded column-major, UE2UC and DE2DC stacked by octant
  */
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,7 +29,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -72,6 +75,12 @@ struct kifmm_gpu {
   int dev = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev[16] = {};
+  /* an event for the start of the next launch (null: none); the phase being
+   * launched (an index of ev) and how its last launch left
+   * that event; ev_at[i]: the event that stands for boundary i, an earlier
+   * one where a phase launched nothing (phase_end) */
+  hipEvent_t start_ev = nullptr;
+  int phase = 0, phase_state = 0, ev_at[16] = {};
   /* KIFMM_GPU_OVERLAP: the U-list on a second stream (default priority)
    * alongside up and V; fork / join events and the U-list's own timing */
   int overlap = 0;
@@ -1374,10 +1383,37 @@ int gram_setup(kifmm_gpu* g) {
     }                                                                            \
   } while (0)
 
-#define REC(e)                                                   \
-  do {                                                           \
-    if (!g->capturing) HIP_TRY(hipEventRecord((e), g->stream)); \
-  } while (0)
+/* Phase events (outside graph capture): E_START before the sequence, then
+ * one after each phase in launch order.  A phase's kernels are launched with
+ * its event as their stop event, so that the event ends up with the end of
+ * the last one: an event recorded between two kernels costs a marker packet
+ * and its drain, 2.4 us each, a stop event nothing measurable (ten 15 us kernels: 184
+ * us with an event recorded after each, 158 with stop events, 160 without). */
+enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_WX, E_DOWN, E_U, E_END };
+enum { PHASE_EMPTY, PHASE_STAMPED, PHASE_UNSTAMPED }; /* kifmm_gpu::phase_state */
+
+/* one launch on st; start and stop (stop, or both, may be null) take its start and end */
+template <typename... P, typename... A>
+void launch_on(hipStream_t st, hipEvent_t start, hipEvent_t stop, void (*kernel)(P...), dim3 grid, dim3 block,
+               A... args) {
+  if (stop) hipExtLaunchKernelGGL(kernel, grid, block, 0, st, start, stop, 0, static_cast<P>(args)...);
+  else hipLaunchKernelGGL(kernel, grid, block, 0, st, static_cast<P>(args)...);
+}
+/* one launch of the current phase on the main stream */
+template <typename... P, typename... A>
+void launch(kifmm_gpu* g, void (*kernel)(P...), dim3 grid, dim3 block, A... args) {
+  launch_on(g->stream, g->start_ev, g->capturing ? nullptr : g->ev[g->phase], kernel, grid, block, args...);
+  g->start_ev = nullptr;
+  g->phase_state = PHASE_STAMPED;
+}
+/* boundary e, after the current phase; the launches from here on are phase e + 1's */
+int phase_end(kifmm_gpu* g, int e) {
+  g->ev_at[e] = g->phase_state == PHASE_EMPTY ? g->ev_at[e - 1] : e;
+  if (!g->capturing && g->phase_state == PHASE_UNSTAMPED) HIP_TRY(hipEventRecord(g->ev[e], g->stream));
+  g->phase = e + 1;
+  g->phase_state = PHASE_EMPTY;
+  return KIFMM_OK;
+}
 
 int gemm(kifmm_gpu* g, const GemmList& L, int M, int K, const double* A, int lda, const double* in, double* out,
          int accumulate) {
@@ -1393,6 +1429,7 @@ int gemm(kifmm_gpu* g, const GemmList& L, int M, int K, const double* A, int lda
     set_error(std::string("GEMM launch: ") + hipGetErrorString(e));
     return KIFMM_EDEVICE;
   }
+  g->phase_state = PHASE_UNSTAMPED;
   return KIFMM_OK;
 }
 
@@ -1413,7 +1450,7 @@ int l2l_dc2de(kifmm_gpu* g, const GemmList& L, int d) {
   switch ((g->n_e + 15) / 16) {
 #define KIFMM_DOWN_CASE(R)                                                                                        \
   case R:                                                                                                         \
-    hipLaunchKernelGGL(k_l2l_dc2de<R>, grid, dim3(256), 0, g->stream, g->n_e, g->ld_e, g->DE2DC, g->lda_l2l,       \
+    launch(g, k_l2l_dc2de<R>, grid, dim3(256), g->n_e, g->ld_e, g->DE2DC, g->lda_l2l,       \
                        g->DC2DE, g->lda_e, L.n, L.in_off, L.out_off, g->tag, d, g->dchk, g->dden);                 \
     break;
     KIFMM_DOWN_CASE(2)
@@ -1431,8 +1468,8 @@ int l2l_dc2de(kifmm_gpu* g, const GemmList& L, int d) {
 int level_op(kifmm_gpu* g, const LevelOp& op, int parts, int nin) {
   if (op.ncols == 0) return KIFMM_OK;
   const dim3 grid((op.ncols + 15) / 16, (op.M + 63) / 64, parts);
-  if (nin == 1) hipLaunchKernelGGL(k_level_op<1>, grid, dim3(256), 0, g->stream, op);
-  else hipLaunchKernelGGL(k_level_op<M2M_PARTS>, grid, dim3(256), 0, g->stream, op);
+  if (nin == 1) launch(g, k_level_op<1>, grid, dim3(256), op);
+  else launch(g, k_level_op<M2M_PARTS>, grid, dim3(256), op);
   LAUNCH_CHECK();
   return KIFMM_OK;
 }
@@ -1478,9 +1515,10 @@ int l2l_dc2de_split(kifmm_gpu* g, const GemmList& L, const GemmList& D, int d) {
   return dc2de(g, D, d);
 }
 
-int fill(kifmm_gpu* g, double* p, size_t n) {
-  const int blocks = (int)std::min<size_t>(4096, (n + 255) / 256);
-  hipLaunchKernelGGL(k_fill, dim3(std::max(blocks, 1)), dim3(256), 0, g->stream, p, n, 0.0);
+/* zeros over p[0 .. n) and q[0 .. m) */
+int fill(kifmm_gpu* g, double* p, size_t n, double* q = nullptr, size_t m = 0) {
+  const int blocks = (int)std::min<size_t>(4096, (std::max(n, m) + 255) / 256);
+  launch(g, k_fill2, dim3(std::max(blocks, 1)), dim3(256), p, n, q, m);
   LAUNCH_CHECK();
   return KIFMM_OK;
 }
@@ -1499,23 +1537,23 @@ int had_block_size(const kifmm_gpu* g) {
 /* The V-list's four sub-phases; had launches the Hadamard in 8 per_xcd blocks
  * of fb frequencies in XCD-contiguous order (had_block). */
 template <int NP, typename ST, typename HAD>
-int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3, HAD had) {
+int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, HAD had) {
   if (g->n_vblocks > 0)
-    hipLaunchKernelGGL((k_dft_fwd<NP, ST>), dim3(g->n_vblocks), dim3(512), 0, g->stream, g->vblocks, g->vslot,
+    launch(g, (k_dft_fwd<NP, ST>), dim3(g->n_vblocks), dim3(512), g->vblocks, g->vslot,
                        g->depth, g->uden, g->ld_e, g->tw, g->cube2surf, X);
   LAUNCH_CHECK();
-  REC(e1);
+  TRY(phase_end(g, E_FFT));
   /* the translation spectra T depend only on NP: computed once at create
    * time (trans_setup), so this sub-phase is empty */
-  REC(e2);
+  TRY(phase_end(g, E_TRANS));
   if (g->n_hgroups > 0) {
     const int fb = had_block_size(g);
     TRY(had(fb, (int)(((long)g->n_hgroups * (g->F / fb) + 7) / 8)));
     LAUNCH_CHECK();
   }
-  REC(e3);
+  TRY(phase_end(g, E_HAD));
   if (g->n_vblocks > 0)
-    hipLaunchKernelGGL((k_dft_inv<NP, ST>), dim3(g->n_vblocks), dim3(512), 0, g->stream, g->vblocks, g->vslot, Y,
+    launch(g, (k_dft_inv<NP, ST>), dim3(g->n_vblocks), dim3(512), g->vblocks, g->vslot, Y,
                        g->tw, g->surf2cube, g->dchk, g->ld_e);
   LAUNCH_CHECK();
   return KIFMM_OK;
@@ -1525,13 +1563,13 @@ int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, hipEvent_t e1, hipEvent_t e2, hipEve
  * its translation values */
 #define KIFMM_HAD_LAUNCH(KERNEL, THREADS, T, X, Y)                                                                 \
   switch (fb) {                                                                                                    \
-    case 2: hipLaunchKernelGGL(KERNEL(2), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+    case 2: launch(g, KERNEL(2), dim3(8 * per), dim3(THREADS), g->hgroups, g->huslots,       \
                                g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
-    case 4: hipLaunchKernelGGL(KERNEL(4), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+    case 4: launch(g, KERNEL(4), dim3(8 * per), dim3(THREADS), g->hgroups, g->huslots,       \
                                g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
-    case 8: hipLaunchKernelGGL(KERNEL(8), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,       \
+    case 8: launch(g, KERNEL(8), dim3(8 * per), dim3(THREADS), g->hgroups, g->huslots,       \
                                g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                              \
-    case 16: hipLaunchKernelGGL(KERNEL(16), dim3(8 * per), dim3(THREADS), 0, g->stream, g->hgroups, g->huslots,     \
+    case 16: launch(g, KERNEL(16), dim3(8 * per), dim3(THREADS), g->hgroups, g->huslots,     \
                                 g->hloc, g->hslot, T, X, Y, g->n_hgroups, per); break;                             \
     default: set_error("internal: unknown Hadamard shape"); return KIFMM_EINVAL;                                   \
   }
@@ -1540,16 +1578,16 @@ int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, hipEvent_t e1, hipEvent_t e2, hipEve
 #define HAD_M32(FB) (k_hadamard_mfma<NP, FB>)
 #define HAD_F64(FB) (k_hadamard_fact<NP, FB>)
 template <int NP>
-int vlist_phase(kifmm_gpu* g, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3) {
+int vlist_phase(kifmm_gpu* g) {
   if constexpr (NP <= 4) {
     if (g->precision == KIFMM_PREC_MIXED)
-      return vlist_phase<NP>(g, g->Xf, g->Yf, e1, e2, e3, [&](int fb, int per) {
+      return vlist_phase<NP>(g, g->Xf, g->Yf, [&](int fb, int per) {
         if (g->had_form == KIFMM_HAD_VALU) KIFMM_HAD_LAUNCH(HAD_V32, 128, g->Tf, g->Xf, g->Yf)
         else KIFMM_HAD_LAUNCH(HAD_M32, 256, g->Tf, g->Xf, g->Yf)
         return KIFMM_OK;
       });
   }
-  return vlist_phase<NP>(g, g->X, g->Y, e1, e2, e3, [&](int fb, int per) {
+  return vlist_phase<NP>(g, g->X, g->Y, [&](int fb, int per) {
     if (g->had_form == KIFMM_HAD_VALU) KIFMM_HAD_LAUNCH(HAD_V64, 128, g->T, g->X, g->Y)
     else KIFMM_HAD_LAUNCH(HAD_F64, 512, g->That, g->X, g->Y)
     return KIFMM_OK;
@@ -1586,7 +1624,7 @@ int u_list_index(const kifmm_gpu* g) {
  * (device address of the pinned buffer) when host is set.  The
  * persistent form's per-XCD counters of the launch are slot c0. */
 template <bool MASK>
-int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum) {
+int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum, hipEvent_t stop) {
   const int l = u_list_index(g);
   const int4* list = l == 0 ? g->p2p_items : l == 1 ? g->p2p_items64 : l == 2 ? g->p2p_items5 : g->p2p_itemsP;
   const int beg = g->chunk_beg[l][c0], end = g->chunk_beg[l][c1];
@@ -1598,47 +1636,47 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
   const int4* items = list;
   if (g->precision == KIFMM_PREC_MIXED) {
     if (g->close_listed && g->p2p_form == KIFMM_P2P_SPLIT)
-      hipLaunchKernelGGL(k_p2p_ulist_mixed_split<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+      launch_on(st, nullptr, stop, k_p2p_ulist_mixed_split<MASK>, dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
                          g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, host, accum);
     else if (g->close_listed)
-      hipLaunchKernelGGL(k_p2p_ulist_mixed_tau<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+      launch_on(st, nullptr, stop, k_p2p_ulist_mixed_tau<MASK>, dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
                          g->rng, g->geo, g->src4, g->trg4, g->cptr, g->cidx, out, host, accum);
     else
-      hipLaunchKernelGGL(k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr, g->rng,
+      launch_on(st, nullptr, stop, k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), items, runs, g->rng_ptr, g->rng,
                          g->geo, g->src4, g->trg4, out, host, accum);
   } else if (l == 1) {
     if (g->gram_u)
-      hipLaunchKernelGGL((k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+      launch_on(st, nullptr, stop, (k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
                          g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
-      hipLaunchKernelGGL((k_p2p_ulist64<MASK, false>), dim3(8 * per), dim3(256), 0, st, items, runs, g->rng_ptr,
+      launch_on(st, nullptr, stop, (k_p2p_ulist64<MASK, false>), dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
                          g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
   } else if (g->p2p_form == KIFMM_P2P_PERSISTENT) {
     int* counters = g->p2p_counters + 8 * std::max(chunk, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, counters, 8, 0);
+    launch_on(st, nullptr, nullptr, k_fill_int, dim3(1), dim3(64), counters, 8, 0);
     if (g->gram_u)
-      hipLaunchKernelGGL((k_p2p_ulist_persist<MASK, P2P_G5, true>), dim3(g->persist_grid[1]), dim3(256), 0, st, items,
+      launch_on(st, nullptr, stop, (k_p2p_ulist_persist<MASK, P2P_G5, true>), dim3(g->persist_grid[1]), dim3(256), items,
                          runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
     else
-      hipLaunchKernelGGL((k_p2p_ulist_persist<MASK, P2P_G, false>), dim3(g->persist_grid[0]), dim3(256), 0, st, items,
+      launch_on(st, nullptr, stop, (k_p2p_ulist_persist<MASK, P2P_G, false>), dim3(g->persist_grid[0]), dim3(256), items,
                          runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, counters, g->geo, g->trg_gram, g->cptr,
                          g->cidx, accum);
   } else {
     if (g->gram_u)
-      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G5, true>), dim3(8 * per), dim3(256), 0, st, items, runs,
+      launch_on(st, nullptr, stop, (k_p2p_ulist<MASK, P2P_G5, true>), dim3(8 * per), dim3(256), items, runs,
                          g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
     else
-      hipLaunchKernelGGL((k_p2p_ulist<MASK, P2P_G, false>), dim3(8 * per), dim3(256), 0, st, items, runs,
+      launch_on(st, nullptr, stop, (k_p2p_ulist<MASK, P2P_G, false>), dim3(8 * per), dim3(256), items, runs,
                          g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
   }
   LAUNCH_CHECK();
   return KIFMM_OK;
 }
 
-int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum) {
-  return g->coincident ? launch_u<true>(g, st, c0, c1, out, host, accum)
-                       : launch_u<false>(g, st, c0, c1, out, host, accum);
+int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum, hipEvent_t stop) {
+  return g->coincident ? launch_u<true>(g, st, c0, c1, out, host, accum, stop)
+                       : launch_u<false>(g, st, c0, c1, out, host, accum, stop);
 }
 
 /* Copy-out chunks whose U-list runs on the second stream from the start of
@@ -1662,28 +1700,24 @@ int early_chunks(const kifmm_gpu* g, unsigned mask) {
 int wx_phase(kifmm_gpu* g, unsigned mask) {
   const int lists = (mask & KIFMM_PHASE_W ? WX_W : 0) | (mask & KIFMM_PHASE_X ? WX_X : 0);
   if (lists && g->n_wx > 0) {
-    hipLaunchKernelGGL(k_wx, dim3(g->n_wx), dim3(64), 0, g->stream, g->wx_items, g->wx_rng, lists, g->geo, g->surf_ue,
+    launch(g, k_wx, dim3(g->n_wx), dim3(64), g->wx_items, g->wx_rng, lists, g->geo, g->surf_ue,
                        g->surf_dc, g->ld_surf, g->uden, g->ld_e, g->src4, g->trg4, g->trg_gram, g->dc_gram, g->wxpart);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_wx_reduce, dim3((g->n_wxred + 1) / 2), dim3(64), 0, g->stream, g->wx_red, g->n_wxred, lists,
+    launch(g, k_wx_reduce, dim3((g->n_wxred + 1) / 2), dim3(64), g->wx_red, g->n_wxred, lists,
                        g->wxpart, g->pot, g->dchk);
     LAUNCH_CHECK();
   }
   if ((lists & WX_X) && g->n_xs > 0) {
-    hipLaunchKernelGGL(k_x_surf, dim3(g->n_xs), dim3(64), 0, g->stream, g->xs_items, g->wx_rng, g->geo, g->surf_dc,
+    launch(g, k_x_surf, dim3(g->n_xs), dim3(64), g->xs_items, g->wx_rng, g->geo, g->surf_dc,
                        g->ld_surf, g->src4, g->dchk, g->ld_e, g->wxpart);
     LAUNCH_CHECK();
     if (g->n_xsred > 0)
-      hipLaunchKernelGGL(k_x_surf_reduce, dim3(g->n_xsred), dim3(64), 0, g->stream, g->xs_red, g->ld_e, g->wxpart,
+      launch(g, k_x_surf_reduce, dim3(g->n_xsred), dim3(64), g->xs_red, g->ld_e, g->wxpart,
                          g->dchk);
     LAUNCH_CHECK();
   }
   return KIFMM_OK;
 }
-
-/* Phase events (recorded outside graph capture): E_START before the
- * sequence, then one after each phase in launch order. */
-enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_WX, E_DOWN, E_U, E_END };
 
 /* One evaluation is three launch sequences on the handle's streams:
  *   enqueue_side  the U-list of the early copy-out chunks (early_chunks) on
@@ -1706,22 +1740,20 @@ int enqueue_side(kifmm_gpu* g, unsigned mask) {
   HIP_TRY(hipEventRecord(g->fork_ev, g->stream)); /* after the previous evaluation's join read potU */
   HIP_TRY(hipStreamWaitEvent(g->side, g->fork_ev, 0));
   HIP_TRY(hipEventRecord(g->su0, g->side));
-  TRY(launch_u(g, g->side, 0, e, g->potU, nullptr, 0));
+  TRY(launch_u(g, g->side, 0, e, g->potU, nullptr, 0, nullptr));
   HIP_TRY(hipEventRecord(g->su1, g->side));
   HIP_TRY(hipEventRecord(g->join_ev, g->side));
   return KIFMM_OK;
 }
 
 int enqueue_far(kifmm_gpu* g, unsigned mask) {
-  hipEvent_t* ev = g->ev;
   const int lde = g->ld_e, lduc = g->ld_uc;
   /* zero what this call accumulates into (fill kernels, so the sequence
    * stays capturable): pot (W, X, L2T and the U-list add into it) and dchk
    * (V, X, L2L) always; uden and dden only when their phase, which assigns
    * every entry that is read, is left out */
-  TRY(fill(g, g->pot, (size_t)g->n_trg));
+  TRY(fill(g, g->pot, (size_t)g->n_trg, g->dchk, (size_t)g->n_nodes * lde));
   if (!(mask & KIFMM_PHASE_UP)) TRY(fill(g, g->uden, (size_t)g->n_nodes * lde));
-  TRY(fill(g, g->dchk, (size_t)g->n_nodes * lde));
   if (!(mask & KIFMM_PHASE_DOWN)) TRY(fill(g, g->dden, (size_t)g->n_nodes * lde));
   /* up: S2M check potentials, UC2UE, then M2M bottom-up */
   if ((mask & KIFMM_PHASE_UP) && g->n_s2m > 0) {
@@ -1736,7 +1768,7 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
       const bool small = g->n_uc <= 112;
       auto s2m = g->mix_lpb == 4 ? (small ? k_s2m_mixed<4, 4, 7> : k_s2m_mixed<4, 2, 5>)
                                  : (small ? k_s2m_mixed<1, 4, 7> : k_s2m_mixed<1, 2, 5>);
-      hipLaunchKernelGGL(s2m, dim3((g->n_s2m + g->mix_lpb - 1) / g->mix_lpb), dim3(64), 0, g->stream, g->s2m_items,
+      launch(g, s2m, dim3((g->n_s2m + g->mix_lpb - 1) / g->mix_lpb), dim3(64), g->s2m_items,
                          g->n_s2m, g->geo, g->surf_uc32, g->n_uc, g->ld_surf, g->src32, g->chk, lduc);
     } else {
       /* (phases, check points per lane) by the check surface size: 98, 152, 296 for NP 3, 4, 6 */
@@ -1745,7 +1777,7 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
         set_error("S2M: more than 320 check points");
         return KIFMM_EUNSUP;
       }
-      hipLaunchKernelGGL(s2m, dim3(g->n_s2m), dim3(64), 0, g->stream, g->s2m_items, g->geo, g->surf_uc, g->n_uc,
+      launch(g, s2m, dim3(g->n_s2m), dim3(64), g->s2m_items, g->geo, g->surf_uc, g->n_uc,
                          g->ld_surf, g->src4, g->chk, lduc);
     }
     LAUNCH_CHECK();
@@ -1767,23 +1799,21 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
       TRY(gemm(g, g->lv[d].m2m_b, g->n_e, lduc, g->UC2UE, g->lda_e, g->chk, g->uden, 0));
     }
   }
-  REC(ev[E_UP]);
+  TRY(phase_end(g, E_UP));
   /* V-list */
   if (mask & KIFMM_PHASE_V) switch (g->np) {
-    case 3: TRY(vlist_phase<3>(g, ev[E_FFT], ev[E_TRANS], ev[E_HAD])); break;
-    case 4: TRY(vlist_phase<4>(g, ev[E_FFT], ev[E_TRANS], ev[E_HAD])); break;
-    case 6: TRY(vlist_phase<6>(g, ev[E_FFT], ev[E_TRANS], ev[E_HAD])); break;
+    case 3: TRY(vlist_phase<3>(g)); break;
+    case 4: TRY(vlist_phase<4>(g)); break;
+    case 6: TRY(vlist_phase<6>(g)); break;
     default: set_error("NP must be 3, 4 or 6 on the GPU"); return KIFMM_EUNSUP;
   }
   else {
-    REC(ev[E_FFT]);
-    REC(ev[E_TRANS]);
-    REC(ev[E_HAD]);
+    for (int e : {E_FFT, E_TRANS, E_HAD}) TRY(phase_end(g, e));
   }
-  REC(ev[E_IFFT]);
+  TRY(phase_end(g, E_IFFT));
   /* W and X */
   TRY(wx_phase(g, mask));
-  REC(ev[E_WX]);
+  TRY(phase_end(g, E_WX));
   /* down: DC2DE at depth 2, then per level the fused L2L + DC2DE
    * (k_l2l_dc2de over the parents at depth d - 1), then L2T */
   for (int d = 2; d <= g->max_depth && (mask & KIFMM_PHASE_DOWN); d++) {
@@ -1801,21 +1831,21 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
   }
   if ((mask & KIFMM_PHASE_DOWN) && g->n_l2t > 0) {
     if (g->precision == KIFMM_PREC_MIXED)
-      hipLaunchKernelGGL(g->mix_lpb == 4 ? k_l2t_mixed<4> : k_l2t_mixed<1>, dim3((g->n_l2t + g->mix_lpb - 1) / g->mix_lpb),
-                         dim3(64), 0, g->stream, g->l2t_items, g->n_l2t, g->geo, g->surf_de32,
-                         g->ld_surf, g->n_e, g->dden, lde, g->trg4, g->pot);
+      launch(g, g->mix_lpb == 4 ? k_l2t_mixed<4> : k_l2t_mixed<1>, dim3((g->n_l2t + g->mix_lpb - 1) / g->mix_lpb),
+             dim3(64), g->l2t_items, g->n_l2t, g->geo, g->surf_de32, g->ld_surf, g->n_e, g->dden, lde, g->trg4, g->pot);
     else
-      hipLaunchKernelGGL(k_l2t, dim3(g->n_l2t), dim3(64), 0, g->stream, g->l2t_items, g->geo, g->surf_de, g->ld_surf,
+      launch(g, k_l2t, dim3(g->n_l2t), dim3(64), g->l2t_items, g->geo, g->surf_de, g->ld_surf,
                          g->n_e, g->dden, lde, g->trg4, g->pot);
   }
   LAUNCH_CHECK();
-  REC(ev[E_DOWN]);
+  TRY(phase_end(g, E_DOWN));
   return KIFMM_OK;
 }
 
 int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
   const int nch = (int)g->cuts.size() - 1, e = early_chunks(g, mask);
   if (e > 0) { /* the early chunks: join */
+    g->phase_state = PHASE_UNSTAMPED;
     const int m = g->cuts[e];
     HIP_TRY(hipStreamWaitEvent(g->stream, g->join_ev, 0));
     const int blocks = std::min(4096, (m + 255) / 256);
@@ -1827,6 +1857,8 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
   }
   if ((mask & KIFMM_PHASE_U) && e < nch) { /* the other chunks after the far field */
     const int late = chunked ? nch - e : 1;
+    const int l = u_list_index(g);
+    g->phase_state = late == 1 && g->chunk_beg[l][nch] > g->chunk_beg[l][e] ? PHASE_STAMPED : PHASE_UNSTAMPED;
     /* chunk launches on the two streams in turn (one chunk's last blocks run
      * beside the next chunk's first), or in layouts 4 - 6 one after another
      * on the main stream */
@@ -1838,7 +1870,7 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
     for (int k = 0; k < late; k++) {
       const int c = e + k;
       hipStream_t st = (pairs && (k & 1)) ? g->side : g->stream;
-      TRY(launch_u(g, st, c, chunked ? c + 1 : nch, g->pot, host, 1));
+      TRY(launch_u(g, st, c, chunked ? c + 1 : nch, g->pot, host, 1, late == 1 ? g->ev[E_U] : nullptr));
       if (chunked) HIP_TRY(hipEventRecord(g->cd_ev[c], st));
     }
     if (pairs) {
@@ -1846,8 +1878,7 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
       HIP_TRY(hipStreamWaitEvent(g->stream, g->sdone_ev, 0));
     }
   }
-  HIP_TRY(hipEventRecord(g->ev[E_U], g->stream));
-  return KIFMM_OK;
+  return phase_end(g, E_U);
 }
 
 /* pinned potentials -> the caller's buffer, a few host threads */
@@ -1898,11 +1929,20 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
     g->graph[0] = gr;
     HIP_TRY(hipGraphInstantiate(&g->gexec[0], gr, nullptr, nullptr, 0));
   }
-  HIP_TRY(hipEventRecord(ev[E_START], g->stream));
+  /* E_START: the start of the first fill, unless that is inside the graph or
+   * the second stream starts before it */
+  g->phase = E_UP;
+  g->phase_state = PHASE_EMPTY;
+  g->ev_at[E_START] = E_START;
+  g->start_ev = nullptr;
+  if (graph || early_chunks(g, mask) > 0) HIP_TRY(hipEventRecord(ev[E_START], g->stream));
+  else g->start_ev = ev[E_START];
   TRY(enqueue_side(g, mask));
-  if (graph) {
+  if (graph) { /* the far field's phases are not told apart */
     HIP_TRY(hipGraphLaunch(g->gexec[0], g->stream));
-    for (int i = E_UP; i <= E_DOWN; i++) HIP_TRY(hipEventRecord(ev[i], g->stream));
+    for (int i = E_UP; i < E_DOWN; i++) g->ev_at[i] = E_START;
+    g->phase_state = PHASE_UNSTAMPED;
+    TRY(phase_end(g, E_DOWN));
   } else {
     TRY(enqueue_far(g, mask));
   }
@@ -1930,7 +1970,10 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
   HIP_TRY(hipEventSynchronize(ev[E_END]));
   if (times) {
     float ms[E_END + 1] = {0};
-    for (int i = E_UP; i <= E_END; i++) HIP_TRY(hipEventElapsedTime(&ms[i], ev[i - 1], ev[i]));
+    g->ev_at[E_END] = E_END;
+    for (int i = E_UP; i <= E_END; i++)
+      if (g->ev_at[i] != g->ev_at[i - 1])
+        HIP_TRY(hipEventElapsedTime(&ms[i], ev[g->ev_at[i - 1]], ev[g->ev_at[i]]));
     float tot = 0;
     HIP_TRY(hipEventElapsedTime(&tot, ev[E_START], ev[E_END]));
     std::memset(times, 0, sizeof *times);
