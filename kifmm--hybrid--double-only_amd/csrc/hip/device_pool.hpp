@@ -1,0 +1,205 @@
+/*
+ * device_pool.hpp -- what handles and tree builds take from the device: idle
+ * streams, and memory carved from few allocations.
+ *
+ * A program that rebuilds its tree every step creates and destroys both each
+ * time, and at 131 thousand points that cost more than the work: 283 hipMallocs
+ * (each new 2 MB of the runtime's own pool takes 0.3 ms, 4.8 ms in all; the
+ * frees take as long, when the last event that refers to the memory goes) and
+ * three streams whose hardware queue went with the last of them (3 ms to take
+ * down, in stream and event destruction, and set up again).  With both kept,
+ * uploads staged (dev_upload) and downloads queued (Down, kifmm_gpu_tree.hip)
+ * a step of that size, tree to potentials, went from 18.0 to 10.5 ms.
+ */
+#ifndef KIFMM_DEVICE_POOL_HPP
+#define KIFMM_DEVICE_POOL_HPP
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <mutex>
+#include <new>
+#include <utility>
+#include <vector>
+
+namespace kifmm_dev {
+
+/* Idle non-blocking streams of default priority.  At most STREAMS_KEPT stay,
+ * in the whole process and over all devices (the hardware has four queues per process);
+ * a stream beyond those, or one that did not end its work cleanly, is
+ * destroyed.  An idle stream holds no user data. */
+constexpr size_t STREAMS_KEPT = 4;
+struct StreamPool {
+  std::mutex m;
+  std::vector<std::pair<int, hipStream_t>> idle;
+};
+inline StreamPool& stream_pool() {
+  alignas(StreamPool) static char at[sizeof(StreamPool)];
+  static StreamPool* const p = new (at) StreamPool; /* never destroyed: the runtime may be gone by then */
+  return *p;
+}
+/* a stream of device dev, the current one */
+inline hipError_t take_stream(int dev, hipStream_t* s) {
+  *s = nullptr;
+  {
+    StreamPool& p = stream_pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    for (size_t k = 0; k < p.idle.size(); k++)
+      if (p.idle[k].first == dev) {
+        *s = p.idle[k].second;
+        p.idle.erase(p.idle.begin() + (long)k);
+        break;
+      }
+  }
+  return *s ? hipSuccess : hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+}
+/* waits for the stream's work first */
+inline void give_stream(int dev, hipStream_t s) {
+  if (!s) return;
+  if (hipStreamSynchronize(s) == hipSuccess) {
+    StreamPool& p = stream_pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    if (p.idle.size() < STREAMS_KEPT) try {
+        p.idle.emplace_back(dev, s);
+        return;
+      } catch (const std::bad_alloc&) {
+      }
+  }
+  (void)hipStreamDestroy(s);
+}
+
+/* Idle blocks of device arenas, BLOCKS_KEPT bytes at most in the whole process.
+ * They go back to the runtime when an arena's allocation fails. */
+constexpr size_t BLOCKS_KEPT = (size_t)128 << 20;
+struct Block {
+  int dev;
+  void* p;
+  size_t bytes;
+};
+struct BlockPool {
+  std::mutex m;
+  std::vector<Block> idle;
+  size_t bytes = 0;
+};
+inline BlockPool& block_pool() {
+  alignas(BlockPool) static char at[sizeof(BlockPool)];
+  static BlockPool* const p = new (at) BlockPool; /* as stream_pool */
+  return *p;
+}
+inline void* take_block(int dev, size_t bytes) {
+  BlockPool& p = block_pool();
+  std::lock_guard<std::mutex> lock(p.m);
+  for (size_t k = 0; k < p.idle.size(); k++)
+    if (p.idle[k].dev == dev && p.idle[k].bytes == bytes) {
+      void* const q = p.idle[k].p;
+      p.idle.erase(p.idle.begin() + (long)k);
+      p.bytes -= bytes;
+      return q;
+    }
+  return nullptr;
+}
+/* false: not kept */
+inline bool give_block(const Block& b) {
+  BlockPool& p = block_pool();
+  std::lock_guard<std::mutex> lock(p.m);
+  if (p.bytes + b.bytes > BLOCKS_KEPT) return false;
+  try {
+    p.idle.push_back(b);
+  } catch (const std::bad_alloc&) {
+    return false;
+  }
+  p.bytes += b.bytes;
+  return true;
+}
+inline void drop_blocks() {
+  BlockPool& p = block_pool();
+  std::lock_guard<std::mutex> lock(p.m);
+  for (const Block& b : p.idle) (void)hipFree(b.p);
+  p.idle.clear();
+  p.bytes = 0;
+}
+
+/* Device memory of one owner: pieces of up to OWN bytes are cut from blocks of
+ * 8, 16, 32, then 64 MB, larger ones are allocations of their own.  No two
+ * owners share a block at a time; a block changes hands only when its owner's
+ * work has ended (stream, or the owner's word for it), with what the owner wrote
+ * in it. */
+class DeviceArena {
+ public:
+  static constexpr size_t OWN = (size_t)8 << 20, MOST = (size_t)64 << 20, ALIGN = 256;
+
+  /* st: the stream whose work uses the memory; null when the owner waits for
+   * it before free() */
+  explicit DeviceArena(hipStream_t st = nullptr) : st_(st) {}
+  DeviceArena(const DeviceArena&) = delete;
+  DeviceArena& operator=(const DeviceArena&) = delete;
+  ~DeviceArena() { free(); }
+
+  /* of the current device; null when there is no memory; aligned to ALIGN */
+  void* get(size_t bytes) {
+    bytes = (std::max<size_t>(bytes, 1) + ALIGN - 1) / ALIGN * ALIGN;
+    if (bytes > OWN) {
+      own_.reserve(own_.size() + 1); /* a throw here loses nothing */
+      void* const p = allocate(bytes);
+      if (p) own_.push_back(p);
+      return p;
+    }
+    if (bytes > left_) {
+      int dev = 0;
+      if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+      blocks_.reserve(blocks_.size() + 1);
+      size_t size = next_;
+      void* p = take_block(dev, size);
+      if (!p) p = allocate(size);
+      if (!p) p = allocate(size = bytes); /* the last of the memory */
+      if (!p) return nullptr;
+      blocks_.push_back({dev, p, size});
+      at_ = (char*)p;
+      left_ = size;
+      next_ = std::min(2 * next_, MOST);
+    }
+    void* const p = at_;
+    at_ += bytes;
+    left_ -= bytes;
+    return p;
+  }
+  /* a piece that no queued work uses: an allocation of its own is freed, a
+   * cut piece stays with its block */
+  void release(void* p) {
+    const auto it = std::find(own_.begin(), own_.end(), p);
+    if (it == own_.end()) return;
+    (void)hipFree(p);
+    own_.erase(it);
+  }
+  bool is_own(const void* p) const { return std::find(own_.begin(), own_.end(), p) != own_.end(); }
+  /* ended: the work that used the memory has, as far as the owner knows */
+  void free(bool ended = true) {
+    if (own_.empty() && blocks_.empty()) return;
+    if (st_ && hipStreamSynchronize(st_) != hipSuccess) ended = false;
+    for (void* p : own_) (void)hipFree(p);
+    for (const Block& b : blocks_)
+      if (!ended || b.bytes < OWN || !give_block(b)) (void)hipFree(b.p);
+    own_.clear();
+    blocks_.clear();
+    at_ = nullptr;
+    left_ = 0;
+  }
+
+ private:
+  static void* allocate(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    drop_blocks();
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  hipStream_t st_;
+  std::vector<void*> own_;
+  std::vector<Block> blocks_;
+  char* at_ = nullptr;
+  size_t left_ = 0, next_ = OWN;
+};
+
+}  // namespace kifmm_dev
+
+#endif

@@ -24,7 +24,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -38,6 +37,7 @@
 
 #include "kifmm_hip.h"
 #include "../host/kifmm_internal.h"
+#include "device_pool.hpp"
 #include "kernels.hpp"
 
 using namespace kifmm_dev;
@@ -89,7 +89,11 @@ struct kifmm_gpu {
   int np = 0, n_e = 0, n_uc = 0, ld_e = 0, ld_uc = 0, lda_e = 0, lda_uc = 0, lda_l2l = 0, ld_surf = 0;
   int N = 0, H = 0, F = 0;
   int n_nodes = 0, n_src = 0, n_trg = 0, coincident = 0, max_depth = 0, precision = 0;
-  std::vector<void*> allocs;
+  DeviceArena mem;
+  /* create time only: pinned staging of the uploads, and how much of it
+   * copies not yet waited for use (null: straight from the caller's memory) */
+  char* up_pin = nullptr;
+  size_t up_used = 0;
   /* device data */
   double4 *src4 = nullptr, *trg4 = nullptr, *geo = nullptr;
   double *pot = nullptr, *uden = nullptr, *dchk = nullptr, *dden = nullptr, *chk = nullptr;
@@ -169,6 +173,8 @@ struct kifmm_gpu {
   double* potU = nullptr;
   /* staging of kifmm_gpu_set_densities */
   double* den_stage = nullptr;
+  double *den_pin = nullptr, *den_pin_dev = nullptr; /* pinned, and its device address: kifmm_gpu_set_densities */
+  bool den_queued = false; /* a kernel that reads den_pin may not have run */
   /* this device's address of the file-scope scratch array */
   double* scratch = nullptr;
 };
@@ -184,23 +190,41 @@ namespace {
     }                                                                                      \
   } while (0)
 
+/* Uploads of up to UP_STAGED bytes are staged through pinned memory and not
+ * waited for: a copy from the caller's memory that is waited for, since the
+ * source may be a temporary, took 12 us at 1 KB and 47 at 100 KB, staged 2 and 6.
+ * From 1 MB both are bound by the copy. */
+constexpr size_t UP_PIN = (size_t)1 << 20, UP_STAGED = (size_t)256 << 10;
+
 template <typename T>
 int dev_upload(kifmm_gpu* g, T** dst, const T* src, size_t n) {
   *dst = nullptr;
   const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-  void* p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
+  void* const p = g->mem.get(bytes);
+  if (!p) {
     set_error("hipMalloc of " + std::to_string(bytes) + " bytes failed");
     return KIFMM_ENOMEM;
   }
-  g->allocs.push_back(p);
   *dst = (T*)p;
   /* on the handle's (non-blocking) stream, so that the kernels that fill
    * the buffer at create time run after the clear: a null-stream memset is
    * not ordered with them */
-  if (src && n) HIP_TRY(hipMemcpyAsync(p, src, n * sizeof(T), hipMemcpyHostToDevice, g->stream));
-  else HIP_TRY(hipMemsetAsync(p, 0, bytes, g->stream));
-  if (src && n) HIP_TRY(hipStreamSynchronize(g->stream)); /* src may be a temporary */
+  if (!src || !n) {
+    HIP_TRY(hipMemsetAsync(p, 0, bytes, g->stream));
+  } else if (g->up_pin && bytes <= UP_STAGED) {
+    if (g->up_used + bytes > UP_PIN) {
+      HIP_TRY(hipStreamSynchronize(g->stream));
+      g->up_used = 0;
+    }
+    char* const stage = g->up_pin + g->up_used;
+    g->up_used += (bytes + 63) / 64 * 64;
+    std::memcpy(stage, src, bytes);
+    HIP_TRY(hipMemcpyAsync(p, stage, bytes, hipMemcpyHostToDevice, g->stream));
+  } else {
+    HIP_TRY(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, g->stream));
+    HIP_TRY(hipStreamSynchronize(g->stream)); /* src may be a temporary */
+    g->up_used = 0;
+  }
   return KIFMM_OK;
 }
 
@@ -295,11 +319,11 @@ int check_view(const kifmm_tree_view* t) {
   const int* idxs[4] = {t->u_idx, t->v_idx, t->w_idx, t->x_idx};
   for (int L = 0; L < 4; L++) {
     if (ptrs[L][0] != 0) return bad("list pointer");
-    for (int i = 0; i < nn; i++) {
+    for (int i = 0; i < nn; i++)
       if (ptrs[L][i + 1] < ptrs[L][i]) return bad("list pointer order");
-      for (int k = ptrs[L][i]; k < ptrs[L][i + 1]; k++)
-        if (idxs[L][k] < 0 || idxs[L][k] >= nn) return bad("list entry");
-    }
+    unsigned out = 0; /* no early exit: the loop vectorises */
+    for (int k = 0; k < ptrs[L][nn]; k++) out |= (unsigned)((unsigned)idxs[L][k] >= (unsigned)nn);
+    if (out) return bad("list entry");
   }
   return KIFMM_OK;
 }
@@ -510,12 +534,22 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
   };
   std::vector<Chunk> chunks;
   std::vector<int2> lists[2]; /* far, near */
-  std::vector<std::pair<long, std::array<int4, 2>>> work, xs_work;
-  auto sorted = [](std::vector<std::pair<long, std::array<int4, 2>>>& w, std::vector<int4>& out) {
-    std::stable_sort(w.begin(), w.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
-    for (const auto& e : w) {
-      out.push_back(e.second[0]);
-      out.push_back(e.second[1]);
+  struct Work {
+    int cost; /* in steps of 64 sources */
+    int4 a, b;
+  };
+  std::vector<Work> work, xs_work;
+  auto sorted = [](const std::vector<Work>& w, std::vector<int4>& out) { /* largest first, stable */
+    int most = 0;
+    for (const Work& e : w) most = std::max(most, e.cost);
+    std::vector<size_t> at((size_t)most + 2, 0);
+    for (const Work& e : w) at[most - e.cost + 1]++;
+    for (int c = 0; c <= most; c++) at[c + 1] += at[c];
+    out.resize(2 * w.size());
+    for (const Work& e : w) {
+      const size_t k = at[most - e.cost]++;
+      out[2 * k] = e.a;
+      out[2 * k + 1] = e.b;
     }
   };
   for (int i = 0; i < nn; i++) {
@@ -546,7 +580,7 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
         for (int p = 0; p < npts && nch > 0; p += 64) {
           const int4 a = make_int4(i, p, std::min(64, npts - p), 0);
           for (int h = 0; h < nch; h++)
-            xs_work.push_back({chunks[h].n, {a, make_int4(chunks[h].rb, chunks[h].re, nch > 1 ? P.xs_slots + h : -1, 0)}});
+            xs_work.push_back({(chunks[h].n + 63) / 64, a, make_int4(chunks[h].rb, chunks[h].re, nch > 1 ? P.xs_slots + h : -1, 0)});
           if (nch > 1) {
             P.xs_red.push_back(a);
             P.xs_red.push_back(make_int4(P.xs_slots, nch, 0, 0));
@@ -604,9 +638,9 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
       for (int p = 0, m = 0; p < npts; p += WX_T, m++) {
         const int cnt = std::min(WX_T, npts - p), slot0 = P.wx_slots;
         for (const Chunk& c : chunks)
-          work.push_back({(long)((c.n + 63) / 64) * ((cnt + 7) / 8),
-                          {make_int4(c.rb, c.re, surf ? p : t->trg_beg[i] + p, cnt),
-                           make_int4(i, P.wx_slots++, c.flags | (surf ? WX_SURF : 0) | (xl ? WX_X : WX_W), c.n)}});
+          work.push_back({((c.n + 63) / 64) * ((cnt + 7) / 8),
+                          make_int4(c.rb, c.re, surf ? p : t->trg_beg[i] + p, cnt),
+                          make_int4(i, P.wx_slots++, c.flags | (surf ? WX_SURF : 0) | (xl ? WX_X : WX_W), c.n)});
         const int nch = P.wx_slots - slot0;
         if (join) {
           int4& b = P.wx_red[wred_at + 2 * m + 1];
@@ -1062,15 +1096,12 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
     TRY(dev_zero(g, &g->trg4, (size_t)t->n_trg));
     TRY(dev_zero(g, &g->pot, (size_t)t->n_trg));
     const size_t m = (size_t)std::max(std::max(t->n_src, t->n_trg), 1);
-    double* stage = nullptr;
-    if (hipMalloc(&stage, 4 * m * sizeof(double)) != hipSuccess) {
+    DeviceArena tmp(g->stream);
+    double* const stage = (double*)tmp.get(4 * m * sizeof(double));
+    if (!stage) {
       set_error("hipMalloc of the point staging buffer failed");
       return KIFMM_ENOMEM;
     }
-    struct Free {
-      double* p;
-      ~Free() { (void)hipFree(p); }
-    } free_stage{stage};
     const int blocks = (int)std::min<size_t>(4096, (m + 255) / 256);
     const double* srcs[4] = {t->sx, t->sy, t->sz, t->sden};
     const double* trgs[3] = {t->tx, t->ty, t->tz};
@@ -1288,20 +1319,9 @@ int close_list(kifmm_gpu* g) {
   const long long n = g->n_trg;
   const int nb = (int)std::max<long long>(1, (n + SCAN_PER - 1) / SCAN_PER);
   if (nb > SCAN_PER) return KIFMM_OK; /* beyond the scan's reach: not listed */
-  struct Tmp {
-    std::vector<void*> p;
-    ~Tmp() {
-      for (void* q : p) (void)hipFree(q);
-    }
-  } tmp;
-  auto tmp_alloc = [&](size_t bytes) -> void* {
-    void* q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(bytes, 8)) != hipSuccess) return nullptr;
-    tmp.p.push_back(q);
-    return q;
-  };
-  int* cnt = (int*)tmp_alloc(sizeof(int) * std::max<long long>(n, 1));
-  long long* bsum = (long long*)tmp_alloc(sizeof(long long) * (nb + 1));
+  DeviceArena tmp(g->stream);
+  int* cnt = (int*)tmp.get(sizeof(int) * std::max<long long>(n, 1));
+  long long* bsum = (long long*)tmp.get(sizeof(long long) * (nb + 1));
   if (!cnt || !bsum) {
     set_error("hipMalloc failed for the close-pair search");
     return KIFMM_ENOMEM;
@@ -1968,6 +1988,7 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
     host_copy_ms = (kifmm::wall_seconds() - t0) * 1e3; /* what is left after the device work */
   }
   HIP_TRY(hipEventSynchronize(ev[E_END]));
+  g->den_queued = false;
   if (times) {
     float ms[E_END + 1] = {0};
     g->ev_at[E_END] = E_END;
@@ -2066,7 +2087,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
     delete g;
     return KIFMM_EDEVICE;
   }
-  if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (take_stream(g->dev, &g->stream) != hipSuccess) {
     set_error("hipStreamCreate failed");
     delete g;
     return KIFMM_EDEVICE;
@@ -2080,7 +2101,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
   }
   g->overlap = opts ? (opts->flags & KIFMM_GPU_OVERLAP) != 0 : 0;
   /* the second stream exists on every handle: the layout is a tuning choice */
-  if (hipStreamCreateWithFlags(&g->side, hipStreamNonBlocking) != hipSuccess ||
+  if (take_stream(g->dev, &g->side) != hipSuccess ||
       hipEventCreateWithFlags(&g->fork_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->join_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->far_ev, hipEventDisableTiming) != hipSuccess ||
@@ -2101,6 +2122,10 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
       kifmm_gpu_destroy(g);
       return KIFMM_EDEVICE;
     }
+  if (hipHostMalloc((void**)&g->up_pin, UP_PIN, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    g->up_pin = nullptr;
+  }
   try {
     const double t0 = kifmm::wall_seconds();
     r = build(g, tree, ops, P);
@@ -2119,6 +2144,9 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
     set_error("host allocation failed in kifmm_gpu_create");
     r = KIFMM_ENOMEM;
   }
+  (void)hipStreamSynchronize(g->stream); /* staged uploads */
+  if (g->up_pin) (void)hipHostFree(g->up_pin);
+  g->up_pin = nullptr;
   if (r != KIFMM_OK) {
     kifmm_gpu_destroy(g);
     return r;
@@ -2157,22 +2185,24 @@ int kifmm_gpu_evaluate_phases(kifmm_gpu* g, unsigned phases, double* pot_leaf, k
 int kifmm_gpu_destroy(kifmm_gpu* g) {
   if (!g) return KIFMM_OK;
   (void)hipSetDevice(g->dev);
-  if (g->stream) (void)hipStreamSynchronize(g->stream);
+  bool ended = true;
+  for (hipStream_t s : {g->stream, g->side})
+    if (s && hipStreamSynchronize(s) != hipSuccess) ended = false;
   if (g->pinned) (void)hipHostFree(g->pinned);
-  if (g->side) (void)hipStreamSynchronize(g->side);
+  if (g->den_pin) (void)hipHostFree(g->den_pin);
   for (int k = 0; k < 2; k++) {
     if (g->gexec[k]) (void)hipGraphExecDestroy(g->gexec[k]);
     if (g->graph[k]) (void)hipGraphDestroy(g->graph[k]);
   }
-  for (void* p : g->allocs) (void)hipFree(p);
+  g->mem.free(ended);
   for (auto& e : g->ev)
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : {g->fork_ev, g->join_ev, g->su0, g->su1, g->far_ev, g->sdone_ev})
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : g->cd_ev)
     if (e) (void)hipEventDestroy(e);
-  if (g->side) (void)hipStreamDestroy(g->side);
-  if (g->stream) (void)hipStreamDestroy(g->stream);
+  give_stream(g->dev, g->side);
+  give_stream(g->dev, g->stream);
   delete g;
   return KIFMM_OK;
 }
@@ -2474,6 +2504,13 @@ int kifmm_gpu_work_counts(const kifmm_gpu* g, kifmm_work_counts* out) {
 
 double* kifmm_gpu_output(kifmm_gpu* g) { return g ? g->pinned : nullptr; }
 
+/* Densities of up to DEN_PINNED bytes are copied to pinned memory that the
+ * packing kernel reads, and not waited for (the evaluation follows on the same
+ * stream): this call with 16 thousand points 31 -> 7 us, 131 thousand 75 -> 30,
+ * 1M 272 -> 134, 2M 625 -> 240.  The line is where pinning a second copy of
+ * the densities gets large; above, the runtime's copy, waited for. */
+constexpr size_t DEN_PINNED = (size_t)16 << 20;
+
 int kifmm_gpu_set_densities(kifmm_gpu* g, const double* den_leaf) {
   if (!g || (!den_leaf && g->n_src > 0)) {
     set_error("kifmm_gpu_set_densities: invalid argument");
@@ -2481,13 +2518,27 @@ int kifmm_gpu_set_densities(kifmm_gpu* g, const double* den_leaf) {
   }
   if (g->n_src == 0) return KIFMM_OK;
   HIP_TRY(hipSetDevice(g->dev));
-  HIP_TRY(hipMemcpyAsync(g->den_stage, den_leaf, sizeof(double) * (size_t)g->n_src, hipMemcpyHostToDevice,
-                         g->stream));
+  const size_t bytes = sizeof(double) * (size_t)g->n_src;
+  if (bytes <= DEN_PINNED && !g->den_pin) {
+    if (hipHostMalloc((void**)&g->den_pin, bytes, hipHostMallocDefault) != hipSuccess) g->den_pin = nullptr;
+    else if (hipHostGetDevicePointer((void**)&g->den_pin_dev, g->den_pin, 0) != hipSuccess) g->den_pin_dev = nullptr;
+    (void)hipGetLastError();
+  }
+  const double* den = g->den_stage;
+  const bool pinned = bytes <= DEN_PINNED && g->den_pin_dev;
+  if (pinned) {
+    if (g->den_queued) HIP_TRY(hipStreamSynchronize(g->stream)); /* the previous densities are not read yet */
+    g->den_queued = true;
+    std::memcpy(g->den_pin, den_leaf, bytes);
+    den = g->den_pin_dev;
+  } else {
+    HIP_TRY(hipMemcpyAsync(g->den_stage, den_leaf, bytes, hipMemcpyHostToDevice, g->stream));
+  }
   const int blocks = (int)std::min<size_t>(4096, ((size_t)g->n_src + 255) / 256);
-  hipLaunchKernelGGL(k_set_w, dim3(blocks), dim3(256), 0, g->stream, g->src4, g->den_stage, (size_t)g->n_src);
+  hipLaunchKernelGGL(k_set_w, dim3(blocks), dim3(256), 0, g->stream, g->src4, den, (size_t)g->n_src);
   HIP_TRY(hipGetLastError());
   if (g->precision == KIFMM_PREC_MIXED) TRY(mixed_sources(g));
-  HIP_TRY(hipStreamSynchronize(g->stream)); /* den_leaf may be released on return */
+  if (!pinned) HIP_TRY(hipStreamSynchronize(g->stream)); /* den_leaf may be released on return */
   return KIFMM_OK;
 }
 
