@@ -59,7 +59,8 @@ enum {
  * blocking knobs BS and UPBS (fmm/util.c:118-163, read by the up pass at
  * fmm/omp_sse_block.cc:203): chosen per input by kifmm_gpu_autotune. */
 enum {
-  KIFMM_P2P_STATIC = 0,     /* one block per U-list item of <= 128 targets (default) */
+  KIFMM_P2P_STATIC = 0,     /* one block per U-list item of up to 160 targets, or on small FP64
+                               inputs one wave per item of 8 or 16 (default) */
   KIFMM_P2P_PERSISTENT = 1, /* a few blocks per CU drawing the same items from per-XCD queues */
   KIFMM_P2P_STATIC64 = 2,   /* one block per item of <= 64 targets */
   KIFMM_P2P_SPLIT = 3       /* mixed path only: items of <= 128 targets, up to 2 groups of 16

@@ -62,33 +62,48 @@ __device__ __forceinline__ double inv_r(double r2) {
 }
 constexpr double HALF_OOFP_R = 0.5 * OOFP_R; /* scales sums of 2 w / r */
 
+/* x from lane l ^ 8, ^ 4, ^ 2, ^ 1 (M) of the same 16 lanes, by DPP */
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double dpp64(double old, double x) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, 0xf, BANKS, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, 0xf, BANKS, false);
+  return __hiloint2double(hi, lo);
+}
+template <int M>
+__device__ __forceinline__ double lane_xor(double x) {
+  if constexpr (M == 8) return dpp64<0x128, 0xf>(x, x); /* row_ror:8 */
+  else if constexpr (M == 4) return dpp64<0x114, 0xa>(dpp64<0x104, 0x5>(x, x), x); /* row_shl:4 | row_shr:4 */
+  else if constexpr (M == 2) return dpp64<0x4e, 0xf>(x, x); /* quad_perm 2 3 0 1 */
+  else return dpp64<0xb1, 0xf>(x, x); /* quad_perm 1 0 3 2 */
+}
+/* swaps the upper half (W = 32), or the odd rows of 16 lanes (W = 16), of a
+ * with the lower half or even rows of b, and adds the two: the lower lanes
+ * hold a's pair sums, the upper ones b's */
+template <int W>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  auto swap = [](unsigned x, unsigned y) {
+    if constexpr (W == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  };
+  const auto lo = swap(__double2loint(a), __double2loint(b)), hi = swap(__double2hiint(a), __double2hiint(b));
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
 /* 8 partial sums per lane -> lane l holds the wave total of target (l >> 3)
- * in lanes with (l & 7) == 0.  Fixed order, deterministic. */
+ * in lanes with (l & 7) == 0.  Fixed order, deterministic: halving across
+ * lane distances 32, 16, 8, then 4, 2, 1.  Row swaps and DPP, 36 VALU
+ * instructions: as shuffles through the LDS crossbar with a select on either
+ * side it was twice that and 26 LDS instructions, once per 8 targets. */
 __device__ __forceinline__ double wave_reduce8(const double acc[8], int lane) {
-  double a[4], b[2], c;
+  double a[4], b[2];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const bool hi = lane & 32;
-    double send = hi ? acc[i] : acc[i + 4];
-    double keep = hi ? acc[i + 4] : acc[i];
-    a[i] = keep + __shfl_xor(send, 32);
-  }
+  for (int i = 0; i < 4; i++) a[i] = swap_add<32>(acc[i], acc[i + 4]);
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const bool hi = lane & 16;
-    double send = hi ? a[i] : a[i + 2];
-    double keep = hi ? a[i + 2] : a[i];
-    b[i] = keep + __shfl_xor(send, 16);
-  }
-  {
-    const bool hi = lane & 8;
-    double send = hi ? b[0] : b[1];
-    double keep = hi ? b[1] : b[0];
-    c = keep + __shfl_xor(send, 8);
-  }
-  c += __shfl_xor(c, 4);
-  c += __shfl_xor(c, 2);
-  c += __shfl_xor(c, 1);
+  for (int i = 0; i < 2; i++) b[i] = swap_add<16>(a[i], a[i + 2]);
+  double c = (lane & 8 ? b[1] : b[0]) + dpp64<0x128, 0xc>(dpp64<0x128, 0x3>(b[0], b[0]), b[1]);
+  c += lane_xor<4>(c);
+  c += lane_xor<2>(c);
+  c += lane_xor<1>(c);
   return c;
 }
 
@@ -244,6 +259,46 @@ __device__ __forceinline__ void eval8_gram(const double4* __restrict__ src, cons
   }
 }
 
+/* The close-pair terms of the nt <= 16 targets from tg0: the sum of target
+ * tg0 + t on the lanes l with l % 16 = t.  Four lanes take a target's pairs in
+ * turn; a target with more than CLOSE_FEW of them takes the whole wave.  Both
+ * orders are fixed and depend on the target alone: deterministic, and the
+ * same for every launch form.  (A segmented scan over the run of all pairs of 8
+ * targets, mostly 8 to 20 pairs, spent 6 exchange steps on each.)  isc = 1 / sc,
+ * exact. */
+constexpr int CLOSE_FEW = 16;
+template <bool MASK>
+__device__ __forceinline__ double close_sums(int tg0, int nt, int lane, double isc, double sc, const double4& g,
+                                             const double4* __restrict__ src4, const double4* __restrict__ trg4,
+                                             const double4* __restrict__ trg_gram, const int* __restrict__ cptr,
+                                             const int* __restrict__ cidx) {
+  auto term = [&](const double4& tp, const double4& a, int j) {
+    const double4 q = src4[j];
+    const double dx = tp.x - q.x, dy = tp.y - q.y, dz = tp.z - q.z;
+    const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+    return q.w * (inv_r2<MASK>(r2) * isc - gram_pair(a, gram_src(q, g, sc)));
+  };
+  const int t = lane & 15, tt = tg0 + min(t, nt - 1);
+  const int beg = cptr[tt], n = t < nt ? cptr[tt + 1] - beg : 0;
+  double v = 0.0;
+  if (__any(n > 0)) {
+    const double4 tp = trg4[tt], a = trg_gram[tt];
+    for (int k = lane >> 4; n <= CLOSE_FEW && k < n; k += 4) v += term(tp, a, cidx[beg + k]);
+    v += __shfl_xor(v, 16);
+    v += __shfl_xor(v, 32);
+    for (unsigned many = (unsigned)__ballot(n > CLOSE_FEW) & 0xffffu; many; many &= many - 1) {
+      const int o = __builtin_ctz(many), b = __builtin_amdgcn_readlane(beg, o), e = b + __builtin_amdgcn_readlane(n, o);
+      const double4 op = trg4[tg0 + o], oa = trg_gram[tg0 + o];
+      double u = 0.0;
+      for (int k = b + lane; k < e; k += 64) u += term(op, oa, cidx[k]);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) u += __shfl_xor(u, off);
+      if (t == o) v = u;
+    }
+  }
+  return v;
+}
+
 /* The item's potentials on their way out, in the Gram form first its close-
  * pair sums (sc_sum, LDS); and for the Gram form the scaled source weights of
  * a tile (LDS) and the per-target records (-2t', |t'|^2) with the close-pair
@@ -339,60 +394,29 @@ __device__ __forceinline__ void p2p_item(double4* tile, const int4 it, int rot, 
       }
     }
   }
-  if constexpr (GRAM) {
-    /* close-pair terms: a group's pairs are one contiguous run of cidx
-     * (targets in order), spread over the 64 lanes and summed per target by
-     * a segmented scan over the lanes (fixed order: deterministic) */
-    const double isc = g.w / GRAM_SC; /* 1 / sc, exact */
-#pragma unroll
-    for (int k = 0; k < G; k++) {
-      const int grp = wave + 4 * k;
-      if (grp < ngroups) {
-        const int t0 = 8 * grp, nt = min(8, it.z - t0), tg0 = it.y + t0;
-        if (lane < 8) ga.sc_sum[t0 + lane] = 0.0;
-        const int kbeg = ga.cptr[tg0], kend = ga.cptr[tg0 + nt];
-        const int ej = ga.cptr[tg0 + min(lane & 7, nt - 1) + 1]; /* end of target lane&7's run */
-        for (int kb = kbeg; kb < kend; kb += 64) {
-          const int kk = kb + lane;
-          const bool live = kk < kend;
-          int tl = 0; /* the target of pair kk: the number of runs that end at or before kk */
-#pragma unroll
-          for (int j = 0; j < 8; j++) tl += __builtin_amdgcn_readlane(ej, j) <= kk;
-          tl = live ? tl : 8;
-          double v = 0.0;
-          if (live) {
-            const double4 q = src4[ga.cidx[kk]];
-            const double4 tp = trg4[tg0 + tl];
-            const double dx = tp.x - q.x, dy = tp.y - q.y, dz = tp.z - q.z;
-            const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-            v = q.w * (inv_r2<MASK>(r2) * isc - gram_pair(ga.trg_gram[tg0 + tl], gram_src(q, g, sc)));
-          }
-#pragma unroll
-          for (int off = 1; off < 64; off <<= 1) {
-            const double u = __shfl_up(v, off, 64);
-            const int ut = __shfl_up(tl, off, 64);
-            if (lane >= off && ut == tl) v += u;
-          }
-          const int nx = __shfl_down(tl, 1, 64);
-          if (live && (lane == 63 || nx != tl)) ga.sc_sum[t0 + tl] += v; /* one writer per target and chunk */
-        }
-      }
-    }
-  }
 #pragma unroll
   for (int k = 0; k < G; k++) {
     const int grp = wave + 4 * k;
     if (grp < ngroups) {
       const double sum = wave_reduce8(acc[k], lane);
       const int t = 8 * grp + (lane >> 3);
-      if ((lane & 7) == 0 && t < it.z)
-        ga.sc_sum[t] = GRAM ? (HALF_OOFP_R * sc) * (sum + ga.sc_sum[t]) : HALF_OOFP_R * sum;
+      if ((lane & 7) == 0 && t < it.z) ga.sc_sum[t] = sum;
     }
+  }
+  const double scale = GRAM ? HALF_OOFP_R * sc : HALF_OOFP_R;
+  __syncthreads();
+  if constexpr (GRAM) {
+    const double isc = g.w / GRAM_SC;
+    for (int t0 = 16 * wave; t0 < it.z; t0 += 64) {
+      const double v = close_sums<MASK>(it.y + t0, min(16, it.z - t0), lane, isc, sc, g, src4, trg4, ga.trg_gram,
+                                        ga.cptr, ga.cidx);
+      if (lane < 16 && t0 + lane < it.z) ga.sc_sum[t0 + lane] += v;
+    }
+    __syncthreads();
   }
   /* the item's potentials leave as one run (and writing them here, with the
    * accumulators dead, keeps the kernel's registers free of spills) */
-  __syncthreads();
-  for (int t = tid; t < it.z; t += 256) put_pot(pot, host, it.y + t, ga.sc_sum[t], accum);
+  for (int t = tid; t < it.z; t += 256) put_pot(pot, host, it.y + t, scale * ga.sc_sum[t], accum);
 }
 
 /* One block per item of at most 32 G targets. */
@@ -433,6 +457,142 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   if (item < 0) return; /* whole block, before any barrier */
   const GramArgs ga{sw, sc_sum, geo, trg_gram, cptr, cidx};
   p2p_item<MASK, P2P_G / 2, GRAM>(tile, items[item], item, rng_ptr, rng, src4, trg4, pot, host, ga, accum);
+}
+
+/* U-list of small inputs, Gram form: a wave per item of at most 8 G targets
+ * (G = 1 or 2).  With some thousand items the block kernels are bound by their
+ * blocks' serial chain (item, ranges, one source wait per range, barriers, close
+ * pairs, reduction; 20 us for 1.7M pairs) and by waves that have no group of a
+ * 14- to 40-target leaf.  Here nothing is staged or waited for across waves:
+ * the lanes hold the next 64 ranges, two rows of 64 sources are on their way
+ * while two are computed, and every wave has all of its item's groups.  A row's
+ * conversion (gram_src, 9 instructions) is not shared, which costs G = 2
+ * 6 % of its loop and G = 1 12 %, and is why larger inputs stay with blocks
+ * (u_wave_groups).  Lanes, rows and reductions are those of the block
+ * kernels: the same bits.  Block kernel -> here: 21.3 -> 12 us at 4 thousand
+ * points, 24.3 -> 16.5 at 16 thousand, 61 -> 53 at 100 thousand, 138 -> 136 at 300
+ * thousand. */
+struct RowWalk {
+  int ri, ro, rlast, base;
+  int2 mine; /* lane l: range base + l */
+};
+__device__ __forceinline__ RowWalk row_walk(const int* __restrict__ rng_ptr, const int2* __restrict__ rng, int set,
+                                            int lane) {
+  RowWalk w;
+  w.ri = w.base = rng_ptr[set];
+  w.rlast = rng_ptr[set + 1];
+  w.ro = 0;
+  w.mine = w.ri < w.rlast ? rng[min(w.ri + lane, w.rlast - 1)] : make_int2(0, 0);
+  return w;
+}
+/* the next R x 64 sources: lane's source of row m in idx[m], -1 past the
+ * count, which is returned */
+template <int R>
+__device__ __forceinline__ int walk_rows(RowWalk& w, const int2* __restrict__ rng, int lane, int (&idx)[R]) {
+  int fill = 0;
+#pragma unroll
+  for (int m = 0; m < R; m++) {
+    /* the row's ranges in turn, each overwriting the lanes from its first
+     * slot on: three VALU instructions a range */
+    int at = 0;
+    idx[m] = 0;
+    while (at < 64 && w.ri < w.rlast) {
+      if (w.ri - w.base == 64) {
+        w.base = w.ri;
+        w.mine = rng[min(w.ri + lane, w.rlast - 1)];
+      }
+      const int beg = __builtin_amdgcn_readlane(w.mine.x, w.ri - w.base);
+      const int num = __builtin_amdgcn_readlane(w.mine.y, w.ri - w.base);
+      const int take = min(num - w.ro, 64 - at), from = beg + w.ro - at;
+      idx[m] = lane >= at ? from + lane : idx[m];
+      at += take;
+      w.ro += take;
+      if (w.ro == num) {
+        w.ri++;
+        w.ro = 0;
+      }
+    }
+    fill += at;
+    idx[m] = lane < at ? idx[m] : -1;
+  }
+  return fill;
+}
+
+template <bool MASK, int G>
+__global__ __launch_bounds__(64) void k_p2p_wave(const int4* __restrict__ items, const XcdRuns runs,
+                                                 const int* __restrict__ rng_ptr, const int2* __restrict__ rng,
+                                                 const double4* __restrict__ src4, const double4* __restrict__ trg4,
+                                                 double* __restrict__ pot, double* __restrict__ host,
+                                                 const double4* __restrict__ geo, const double4* __restrict__ trg_gram,
+                                                 const int* __restrict__ cptr, const int* __restrict__ cidx, int accum) {
+  constexpr int R = 2; /* rows of 64 sources at a time */
+  __shared__ double sc_sum[8 * G];
+  const int item = xcd_item(runs);
+  if (item < 0) return;
+  const int4 it = items[item];
+  const int lane = threadIdx.x, ngroups = (it.z + 7) >> 3;
+  RowWalk walk = row_walk(rng_ptr, rng, it.x, lane);
+  const double4 g = geo[it.w];
+  const double sc = GRAM_SC / g.w;
+  double acc[G][8];
+#pragma unroll
+  for (int k = 0; k < G; k++)
+#pragma unroll
+    for (int t = 0; t < 8; t++) acc[k][t] = 0.0;
+  int idx[R];
+  double4 q[R];
+  int fill = walk_rows(walk, rng, lane, idx);
+#pragma unroll
+  for (int m = 0; m < R; m++)
+    if (idx[m] >= 0) q[m] = src4[idx[m]];
+  while (fill > 0) {
+    double4 p[R];
+    double w[R];
+#pragma unroll
+    for (int m = 0; m < R; m++) {
+      p[m] = gram_src(q[m], g, sc);
+      w[m] = q[m].w;
+    }
+    if (fill < 64 * R) { /* the last rows */
+#pragma unroll
+      for (int m = 0; m < R; m++)
+        if (idx[m] < 0) {
+          p[m] = make_double4(GRAM_FAR, GRAM_FAR, GRAM_FAR, 3.0 * GRAM_FAR * GRAM_FAR);
+          w[m] = 0.0;
+        }
+    }
+    const int next = walk_rows(walk, rng, lane, idx);
+#pragma unroll
+    for (int m = 0; m < R; m++)
+      if (idx[m] >= 0) q[m] = src4[idx[m]];
+#pragma unroll
+    for (int k = 0; k < G; k++)
+      if (k < ngroups) {
+        double4 a[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) a[t] = trg_gram[it.y + min(8 * k + t, it.z - 1)];
+#pragma unroll
+        for (int t = 0; t < 8; t++) acc[k][t] = __builtin_fma(w[0], gram_pair(a[t], p[0]), acc[k][t]);
+        if (fill > 64) {
+#pragma unroll
+          for (int t = 0; t < 8; t++) acc[k][t] = __builtin_fma(w[1], gram_pair(a[t], p[1]), acc[k][t]);
+        }
+      }
+    fill = next;
+  }
+#pragma unroll
+  for (int k = 0; k < G; k++)
+    if (k < ngroups) {
+      const double sum = wave_reduce8(acc[k], lane);
+      if ((lane & 7) == 0) sc_sum[8 * k + (lane >> 3)] = sum;
+    }
+  __syncthreads();
+  const double isc = g.w / GRAM_SC;
+  for (int t0 = 0; t0 < it.z; t0 += 16) {
+    const double v = close_sums<MASK>(it.y + t0, min(16, it.z - t0), lane, isc, sc, g, src4, trg4, trg_gram, cptr, cidx);
+    if (lane < 16 && t0 + lane < it.z)
+      put_pot(pot, host, it.y + t0 + lane, (HALF_OOFP_R * sc) * (sc_sum[t0 + lane] + v), accum);
+  }
 }
 
 /* Persistent form over the same items (<= 32 G targets): a fixed grid

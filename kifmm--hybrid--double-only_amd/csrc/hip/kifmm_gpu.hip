@@ -111,6 +111,7 @@ struct kifmm_gpu {
   int4* p2p_items = nullptr; int n_p2p = 0;
   int4* p2p_items64 = nullptr; int n_p2p64 = 0;
   int4* p2p_items5 = nullptr; int n_p2p5 = 0; /* <= P2P_MAXT5 targets: the FP64 Gram-form kernels */
+  int4* p2p_itemsW = nullptr; int n_p2pW = 0, wave_g = 0; /* <= 8 wave_g targets (none: 0): k_p2p_wave */
   int4* p2p_itemsP = nullptr; int n_p2pP = 0; /* sibling pairs and single leaves: the mixed tau kernel */
   int* rng_ptr = nullptr; int2* rng = nullptr;
   int* p2p_counters = nullptr; /* 8, one per XCD: persistent U-list */
@@ -164,8 +165,8 @@ struct kifmm_gpu {
    * the first item of each chunk per item list, whether the items cover every
    * target, and the events that mark a chunk's potentials as on the host */
   std::vector<int> cuts;
-  std::vector<int> chunk_beg[4];
-  std::vector<double> u_cost[4]; /* prefix sums of the items' costs, per list */
+  std::vector<int> chunk_beg[5];
+  std::vector<double> u_cost[5]; /* prefix sums of the items' costs, per list */
   bool tiled = false;
   std::vector<hipEvent_t> cd_ev;
   hipEvent_t far_ev = nullptr, sdone_ev = nullptr;
@@ -346,13 +347,14 @@ struct HostLevel {
 struct Plan {
   int np = 0, n_e = 0, n_uc = 0, ld_e = 0, ld_uc = 0, lda_e = 0, lda_uc = 0, lda_l2l = 0, ld_surf = 0;
   int N = 0, H = 0, F = 0, nblk = 0, max_depth = 0;
-  std::vector<int4> p2p_items, p2p_items64, p2p_items5, p2p_itemsP;
+  std::vector<int4> p2p_items, p2p_items64, p2p_items5, p2p_itemsP, p2p_itemsW;
+  int wave_g = 0;
   /* copy-out chunks: target cut points (leaf starts, 0 .. n_trg) and, per
    * item list (<= P2P_MAXT, <= P2P_MAXT / 2, <= P2P_MAXT5, pairs), the
    * first item of each chunk */
   std::vector<int> cuts;
-  std::vector<int> chunk_beg[4];
-  std::vector<double> u_cost[4];
+  std::vector<int> chunk_beg[5];
+  std::vector<double> u_cost[5];
   bool tiled = false;
   std::vector<int> rng_ptr;
   std::vector<int2> rng;
@@ -468,6 +470,23 @@ double item_cost(const int4& it, int group, const std::vector<int>& set_src) {
   double src = set_src[it.x];
   if (it.z >> 16) src += 0.5 * ((double)set_src[it.x + 1] + set_src[it.x + 2]); /* of a pair: half the groups each */
   return (groups + 3) / 4 * (src / 64.0 + 1.0) + 4.0;
+}
+
+double wave_cost(const int4& it, const std::vector<int>& set_src) { /* of k_p2p_wave's */
+  return (it.z + 7) / 8 * (set_src[it.x] / 64.0 + 1.0) + 4.0;
+}
+
+/* 8-target groups per wave of the U-list's wave kernel (k_p2p_wave), 0: the
+ * block kernels.  One up to 8 groups per SIMD of the chip, so that few items
+ * spread (16 thousand points, 2752 groups: 16.5 us with one, 20 with two); then two,
+ * which share a row's conversion (100 thousand, 14504 groups: 55 and 53); from 65536 on
+ * the blocks' shared conversion is as good (300 thousand, 47776: 136 against 138; 1M
+ * ellipsoid, 180072: 472 - 495 and 482 - 492; 16M: 12950 and 12770). */
+int u_wave_groups(const kifmm_tree_view* t) {
+  long groups = 0;
+  for (int i = 0; i < t->n_nodes; i++)
+    if (t->child[i] == -1) groups += (t->trg_num[i] + 7) / 8;
+  return groups < 8192 ? 1 : groups < 65536 ? 2 : 0;
 }
 
 /* Items [b, e) of a list cut into 8 runs of about equal cost. */
@@ -858,6 +877,17 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
           (long)it.y + it.z > t->n_trg || it.w < 0 || it.w >= nn)
         return fail("U-list work item out of range");
   TRY(pair_items(t, P));
+  if (!mixed) P.wave_g = u_wave_groups(t);
+  for (int i = 0, set = 0; P.wave_g > 0 && i < nn; i++) {
+    if (t->child[i] != -1 || t->trg_num[i] <= 0) continue;
+    const int n = t->trg_num[i], cap = 8 * P.wave_g, nit = (n + cap - 1) / cap, per = (((n + nit - 1) / nit) + 7) & ~7;
+    for (int c = 0; c < n; c += per) P.p2p_itemsW.push_back(make_int4(set, t->trg_beg[i] + c, std::min(per, n - c), i));
+    set++;
+  }
+  for (const int4& it : P.p2p_itemsW)
+    if (it.x < 0 || it.x + 1 >= (int)P.rng_ptr.size() || it.z < 1 || it.z > 8 * P.wave_g || it.y < 0 ||
+        (long)it.y + it.z > t->n_trg || it.w < 0 || it.w >= nn)
+      return fail("U-list wave item out of range");
   for (const int2& r : P.rng)
     if (r.x < 0 || r.y < 1 || (long)r.x + r.y > t->n_src) return fail("U-list source range out of range");
   /* Copy-out chunks.  The U-list runs last, chunk by chunk, and each
@@ -868,9 +898,10 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
    * chunks shrink towards the end so that the copy left after the last
    * chunk is short.  Small inputs are one chunk. */
   {
-    const std::vector<int4>* lists[4] = {&P.p2p_items, &P.p2p_items64, &P.p2p_items5, &P.p2p_itemsP};
+    const std::vector<int4>* lists[5] = {&P.p2p_items, &P.p2p_items64, &P.p2p_items5, &P.p2p_itemsP, &P.p2p_itemsW};
     bool tiled = t->n_trg > 0;
     for (const std::vector<int4>* L : lists) {
+      if (L == &P.p2p_itemsW && P.wave_g == 0) continue; /* not in use */
       long next = 0;
       for (const int4& it : *L) {
         if (it.y != next) tiled = false;
@@ -899,11 +930,12 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
     std::vector<int> set_src(P.rng_ptr.size(), 0); /* sources of each range set */
     for (size_t k = 0; k + 1 < P.rng_ptr.size(); k++)
       for (int r = P.rng_ptr[k]; r < P.rng_ptr[k + 1]; r++) set_src[k] += P.rng[r].y;
-    for (int l = 0; l < 4; l++) {
+    for (int l = 0; l < 5; l++) {
       const std::vector<int4>& L = *lists[l];
       std::vector<double>& cost = P.u_cost[l];
       cost.assign(1, 0.0);
-      for (const int4& it : L) cost.push_back(cost.back() + item_cost(it, l == 3 ? 16 : 8, set_src));
+      for (const int4& it : L)
+        cost.push_back(cost.back() + (l == 4 ? wave_cost(it, set_src) : item_cost(it, l == 3 ? 16 : 8, set_src)));
       P.chunk_beg[l].clear();
       size_t k = 0;
       for (size_t c = 0; c + 1 < P.cuts.size(); c++) {
@@ -1216,12 +1248,15 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
   TRY(dev_upload(g, &g->p2p_items64, P.p2p_items64.data(), P.p2p_items64.size()));
   g->n_p2p5 = (int)P.p2p_items5.size();
   TRY(dev_upload(g, &g->p2p_items5, P.p2p_items5.data(), P.p2p_items5.size()));
+  g->n_p2pW = (int)P.p2p_itemsW.size();
+  g->wave_g = P.wave_g;
+  TRY(dev_upload(g, &g->p2p_itemsW, P.p2p_itemsW.data(), P.p2p_itemsW.size()));
   g->n_p2pP = (int)P.p2p_itemsP.size();
   TRY(dev_upload(g, &g->p2p_itemsP, P.p2p_itemsP.data(), P.p2p_itemsP.size()));
   TRY(dev_zero(g, &g->p2p_counters, 8 * std::max<size_t>(P.cuts.size(), 1)));
   g->cuts = P.cuts;
   g->tiled = P.tiled;
-  for (int l = 0; l < 4; l++) {
+  for (int l = 0; l < 5; l++) {
     g->chunk_beg[l] = P.chunk_beg[l];
     g->u_cost[l] = P.u_cost[l];
   }
@@ -1623,8 +1658,8 @@ int vlist_phase(kifmm_gpu* g) {
  * pairs and single leaves (list 3), the FP64 Gram-form kernels items of
  * <= P2P_MAXT5 targets (list 2), the STATIC64 shape items of <= 64 (list
  * 1), the difference form, the mixed source-split form and the mixed
- * in-loop test items of <= P2P_MAXT (list 0).  The STATIC Gram form also
- * takes the <= 64 list where leaves are small, U_SMALL targets or fewer per
+ * in-loop test items of <= P2P_MAXT (list 0).  The STATIC Gram form takes
+ * a wave per item on small inputs (list 4, u_wave_groups) and the <= 64 list where leaves are small, U_SMALL targets or fewer per
  * item of list 2: its kernel holds 6 waves per SIMD instead of 4, which on
  * short items outweighs the second source walk of the few large leaves.
  * Measured, list 2 -> list 1: 0.503 -> 0.455 ms at 50 targets per item (1M
@@ -1635,6 +1670,7 @@ constexpr double U_SMALL = 96.0;
 int u_list_index(const kifmm_gpu* g) {
   if (g->precision == KIFMM_PREC_MIXED) return g->close_listed && g->p2p_form != KIFMM_P2P_SPLIT ? 3 : 0;
   if (g->p2p_form == KIFMM_P2P_STATIC64) return 1;
+  if (g->p2p_form == KIFMM_P2P_STATIC && g->gram_u && g->wave_g > 0) return 4;
   if (g->p2p_form == KIFMM_P2P_STATIC && g->gram_u && g->n_trg <= U_SMALL * g->n_p2p5) return 1;
   return g->gram_u ? 2 : 0;
 }
@@ -1646,7 +1682,7 @@ int u_list_index(const kifmm_gpu* g) {
 template <bool MASK>
 int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* host, int accum, hipEvent_t stop) {
   const int l = u_list_index(g);
-  const int4* list = l == 0 ? g->p2p_items : l == 1 ? g->p2p_items64 : l == 2 ? g->p2p_items5 : g->p2p_itemsP;
+  const int4* list = l == 0 ? g->p2p_items : l == 1 ? g->p2p_items64 : l == 2 ? g->p2p_items5 : l == 3 ? g->p2p_itemsP : g->p2p_itemsW;
   const int beg = g->chunk_beg[l][c0], end = g->chunk_beg[l][c1];
   const int chunk = c0;
   if (end <= beg) return KIFMM_OK;
@@ -1664,6 +1700,9 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
     else
       launch_on(st, nullptr, stop, k_p2p_ulist_mixed<MASK>, dim3(8 * per), dim3(256), items, runs, g->rng_ptr, g->rng,
                          g->geo, g->src4, g->trg4, out, host, accum);
+  } else if (l == 4) {
+    launch_on(st, nullptr, stop, g->wave_g == 1 ? k_p2p_wave<MASK, 1> : k_p2p_wave<MASK, 2>, dim3(8 * per), dim3(64),
+              items, runs, g->rng_ptr, g->rng, g->src4, g->trg4, out, host, g->geo, g->trg_gram, g->cptr, g->cidx, accum);
   } else if (l == 1) {
     if (g->gram_u)
       launch_on(st, nullptr, stop, (k_p2p_ulist64<MASK, true>), dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
