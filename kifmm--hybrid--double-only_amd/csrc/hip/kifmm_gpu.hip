@@ -166,6 +166,9 @@ struct kifmm_gpu {
    * target, and the events that mark a chunk's potentials as on the host */
   std::vector<int> cuts;
   std::vector<int> chunk_beg[5];
+  /* the items of list u_order_list over the whole range, in launch order (u_launch_order) */
+  int4* u_order = nullptr;
+  int u_order_list = -1;
   std::vector<double> u_cost[5]; /* prefix sums of the items' costs, per list */
   bool tiled = false;
   std::vector<hipEvent_t> cd_ev;
@@ -355,6 +358,8 @@ struct Plan {
   std::vector<int> cuts;
   std::vector<int> chunk_beg[5];
   std::vector<double> u_cost[5];
+  std::vector<int4> u_order;
+  int u_order_list = -1;
   bool tiled = false;
   std::vector<int> rng_ptr;
   std::vector<int2> rng;
@@ -476,6 +481,8 @@ double wave_cost(const int4& it, const std::vector<int>& set_src) { /* of k_p2p_
   return (it.z + 7) / 8 * (set_src[it.x] / 64.0 + 1.0) + 4.0;
 }
 
+constexpr double U_SMALL = 96.0; /* u_list_index */
+
 /* 8-target groups per wave of the U-list's wave kernel (k_p2p_wave), 0: the
  * block kernels.  One up to 8 groups per SIMD of the chip, so that few items
  * spread (16 thousand points, 2752 groups: 16.5 us with one, 20 with two); then two,
@@ -500,6 +507,35 @@ XcdRuns xcd_runs(const std::vector<double>& cost, int b, int e) {
   }
   r.beg[8] = e;
   return r;
+}
+
+/* The items of a list for a launch over all of them: within an XCD's run those
+ * of more than the mean cost first, in classes of falling cost (factor 1.25),
+ * then the others in their order, in which neighbours share sources.  An
+ * uneven list otherwise ends with its long items on an emptying chip.  U-list
+ * kernel: 53 -> 50.5 us at 100 thousand points, 136 -> 128 at 300 thousand, 482 -> 465 at 1M
+ * ellipsoid, 5.36 -> 5.28 ms at 4M.  Not on the mixed path, whose kernel was slower
+ * for it (465 thousand points 0.315 -> 0.40 ms). */
+std::vector<int4> u_launch_order(const std::vector<int4>& items, const std::vector<double>& cost) {
+  const int n = (int)items.size();
+  std::vector<int4> out(items);
+  if (n == 0) return out;
+  const XcdRuns runs = xcd_runs(cost, 0, n);
+  const double mean = cost[n] / n;
+  std::vector<std::vector<int>> cls;
+  for (int x = 0; x < 8; x++) {
+    for (auto& c : cls) c.clear();
+    for (int k = runs.beg[x]; k < runs.beg[x + 1]; k++) {
+      const double r = (cost[k + 1] - cost[k]) / mean;
+      const size_t c = r <= 1.0 ? 0 : std::min<size_t>(30, 1 + (size_t)(std::log(r) / std::log(1.25)));
+      if (c >= cls.size()) cls.resize(c + 1);
+      cls[c].push_back(k);
+    }
+    int at = runs.beg[x];
+    for (size_t c = cls.size(); c-- > 0;)
+      for (int k : cls[c]) out[at++] = items[k];
+  }
+  return out;
 }
 
 /* The W / X items (k_wx) and their reductions.  Per target node and list,
@@ -945,6 +981,11 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
       }
       P.chunk_beg[l].push_back((int)L.size());
     }
+    /* the list that the default form launches, FP64 */
+    if (!mixed) {
+      P.u_order_list = P.wave_g > 0 ? 4 : t->n_trg <= U_SMALL * P.p2p_items5.size() ? 1 : 2;
+      P.u_order = u_launch_order(*lists[P.u_order_list], P.u_cost[P.u_order_list]);
+    }
   }
 
   /* S2M + UC2UE over source leaves */
@@ -1248,6 +1289,8 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
   TRY(dev_upload(g, &g->p2p_items64, P.p2p_items64.data(), P.p2p_items64.size()));
   g->n_p2p5 = (int)P.p2p_items5.size();
   TRY(dev_upload(g, &g->p2p_items5, P.p2p_items5.data(), P.p2p_items5.size()));
+  g->u_order_list = P.u_order_list;
+  TRY(dev_upload(g, &g->u_order, P.u_order.data(), P.u_order.size()));
   g->n_p2pW = (int)P.p2p_itemsW.size();
   g->wave_g = P.wave_g;
   TRY(dev_upload(g, &g->p2p_itemsW, P.p2p_itemsW.data(), P.p2p_itemsW.size()));
@@ -1666,7 +1709,6 @@ int vlist_phase(kifmm_gpu* g) {
  * ellipsoid), 0.160 -> 0.137 at 37 (300 thousand, NP 6), 13.16 -> 12.89 at
  * 64 (16M uniform); 5.36 -> 5.59 at 128 (4M uniform).  The sums are the same
  * bit for bit. */
-constexpr double U_SMALL = 96.0;
 int u_list_index(const kifmm_gpu* g) {
   if (g->precision == KIFMM_PREC_MIXED) return g->close_listed && g->p2p_form != KIFMM_P2P_SPLIT ? 3 : 0;
   if (g->p2p_form == KIFMM_P2P_STATIC64) return 1;
@@ -1689,7 +1731,7 @@ int launch_u(kifmm_gpu* g, hipStream_t st, int c0, int c1, double* out, double* 
   const XcdRuns runs = xcd_runs(g->u_cost[l], beg, end);
   int per = 0;
   for (int x = 0; x < 8; x++) per = std::max(per, runs.beg[x + 1] - runs.beg[x]);
-  const int4* items = list;
+  const int4* items = l == g->u_order_list && beg == 0 && end == g->chunk_beg[l].back() ? g->u_order : list;
   if (g->precision == KIFMM_PREC_MIXED) {
     if (g->close_listed && g->p2p_form == KIFMM_P2P_SPLIT)
       launch_on(st, nullptr, stop, k_p2p_ulist_mixed_split<MASK>, dim3(8 * per), dim3(256), items, runs, g->rng_ptr,
