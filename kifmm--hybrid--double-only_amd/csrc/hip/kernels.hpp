@@ -2272,7 +2272,25 @@ template <int NP>
 struct Grid {
   static constexpr int N = 2 * NP, H = NP + 1, F = N * N * H, OFF = NP / 2;
   static constexpr int NE = NP * NP * NP - (NP - 2) * (NP - 2) * (NP - 2);
+  /* octants per block of the DFTs: all 8 siblings, or half of them at NP 6,
+   * whose planes of 8 take 100 KB of LDS, one block per CU, so that memory
+   * idles while it computes (300 thousand points NP 6, 14 thousand boxes: forward 59 ->
+   * 49 us, inverse 73 -> 55; their spectra take 47 at the copy rate).  At NP 4 and 3
+   * four and more blocks share a CU, and both are at that rate. */
+  static constexpr int OC = NP == 6 ? 4 : 8, OC_SHIFT = OC == 4 ? 2 : 3, THREADS = 64 * OC;
 };
+/* a DFT block's child block and first octant; the halves of a child block
+ * share 128-byte lines and go to one XCD, 8 blocks apart */
+template <int NP>
+__device__ __forceinline__ int2 dft_block() {
+  const int b = blockIdx.x;
+  if constexpr (Grid<NP>::OC == 8) return make_int2(b, 0);
+  return make_int2((b >> 4) * 8 + (b & 7), (b >> 3 & 1) * 4);
+}
+template <int NP>
+int dft_blocks(int n) {
+  return Grid<NP>::OC == 8 ? n : 2 * ((n + 7) & ~7);
+}
 
 /* Forward transform of the 8 sibling equivalent densities of one child
  * block: scatter 2^depth * uden onto the (2NP)^3 grid (only the NP^3 cube
@@ -2286,7 +2304,7 @@ struct Grid {
  * entries, and the z pass writes each kz plane of X contiguously.  Per
  * output the sum runs over the input index in increasing order. */
 template <int NP, typename ST = double2>
-__global__ __launch_bounds__(512) void k_dft_fwd(const int* __restrict__ blocks, /* first child node per block */
+__global__ __launch_bounds__(Grid<NP>::THREADS) void k_dft_fwd(const int* __restrict__ blocks, int n_blocks, /* first child node per block */
                                                  const int* __restrict__ xslot,  /* X slot per block */
                                                  const int* __restrict__ depth,
                                                  const double* __restrict__ uden, int ld_e,
@@ -2294,25 +2312,28 @@ __global__ __launch_bounds__(512) void k_dft_fwd(const int* __restrict__ blocks,
                                                  const int* __restrict__ cube2surf, /* NP^3: sample id or -1 */
                                                  ST* __restrict__ X) {
   using G = Grid<NP>;
-  constexpr int N = G::N, H = G::H, F = G::F, NE = G::NE, OFF = G::OFF;
-  __shared__ double gs[NE][8];
-  __shared__ double2 A[NP][NP][H][8]; /* [iz][iy][kx][oct] */
-  __shared__ double2 B[NP][N][H][8];  /* [iz][ky][kx][oct] */
+  constexpr int N = G::N, H = G::H, F = G::F, NE = G::NE, OFF = G::OFF, OC = G::OC, OS = G::OC_SHIFT;
+  __shared__ double2 A[NP][NP][H][OC]; /* [iz][iy][kx][oct] */
+  __shared__ double2 B[NP][N][H][OC];  /* [iz][ky][kx][oct] */
+  static_assert(sizeof(B) >= sizeof(double) * NE * OC, "the densities in B, which the y pass writes");
+  double(*const gs)[OC] = reinterpret_cast<double(*)[OC]>(&B[0][0][0][0]);
   __shared__ int c2s[NP * NP * NP];
   const int tid = threadIdx.x;
-  const int first = blocks[blockIdx.x];
+  const int2 bo = dft_block<NP>();
+  if (bo.x >= n_blocks) return; /* whole block */
+  const int first = blocks[bo.x] + bo.y;
   double2 w[N];
 #pragma unroll
   for (int m = 0; m < N; m++) w[m] = tw[m];
   for (int e = tid; e < NP * NP * NP; e += blockDim.x) c2s[e] = cube2surf[e];
-  for (int e = tid; e < 8 * NE; e += blockDim.x) {
+  for (int e = tid; e < OC * NE; e += blockDim.x) {
     const int o = e / NE, j = e % NE, node = first + o;
     gs[j][o] = ldexp(uden[(size_t)node * ld_e + j], depth[node]);
   }
   __syncthreads();
   /* x pass: column (iz, iy, oct), real input x in [OFF, OFF + NP) -> kx <= N/2 */
-  for (int e = tid; e < NP * NP * 8; e += blockDim.x) {
-    const int o = e & 7, iy = (e >> 3) % NP, iz = (e >> 3) / NP;
+  for (int e = tid; e < NP * NP * OC; e += blockDim.x) {
+    const int o = e & (OC - 1), iy = (e >> OS) % NP, iz = (e >> OS) / NP;
     double v[NP];
 #pragma unroll
     for (int ix = 0; ix < NP; ix++) {
@@ -2333,8 +2354,8 @@ __global__ __launch_bounds__(512) void k_dft_fwd(const int* __restrict__ blocks,
   }
   __syncthreads();
   /* y pass: column (iz, kx, oct) */
-  for (int e = tid; e < NP * H * 8; e += blockDim.x) {
-    const int o = e & 7, kx = (e >> 3) % H, iz = (e >> 3) / H;
+  for (int e = tid; e < NP * H * OC; e += blockDim.x) {
+    const int o = e & (OC - 1), kx = (e >> OS) % H, iz = (e >> OS) / H;
     double2 a[NP];
 #pragma unroll
     for (int iy = 0; iy < NP; iy++) a[iy] = A[iz][iy][kx][o];
@@ -2351,11 +2372,11 @@ __global__ __launch_bounds__(512) void k_dft_fwd(const int* __restrict__ blocks,
     }
   }
   __syncthreads();
-  /* z pass: column (ky, kx, oct) = thread e; output (kz, ky, kx, oct) at
-   * X[slot][kz * N * H * 8 + e] */
-  ST* out = X + (size_t)xslot[blockIdx.x] * F * 8;
-  for (int e = tid; e < N * H * 8; e += blockDim.x) {
-    const int o = e & 7, kk = e >> 3; /* kk = ky * H + kx */
+  /* z pass: column (ky, kx, oct); output (kz, ky, kx, oct) at
+   * X[slot][(kz * N * H + ky * H + kx) * 8 + oct] */
+  ST* out = X + (size_t)xslot[bo.x] * F * 8 + bo.y;
+  for (int e = tid; e < N * H * OC; e += blockDim.x) {
+    const int o = e & (OC - 1), kk = e >> OS; /* kk = ky * H + kx */
     double2 b[NP];
 #pragma unroll
     for (int iz = 0; iz < NP; iz++) b[iz] = B[iz][kk / H][kk % H][o];
@@ -2368,7 +2389,7 @@ __global__ __launch_bounds__(512) void k_dft_fwd(const int* __restrict__ blocks,
         re = __builtin_fma(b[iz].x, t.x, __builtin_fma(-b[iz].y, t.y, re));
         im = __builtin_fma(b[iz].x, t.y, __builtin_fma(b[iz].y, t.x, im));
       }
-      out[(size_t)kz * N * H * 8 + e] = Spec<ST>::mk(re, im);
+      out[((size_t)kz * N * H + kk) * 8 + o] = Spec<ST>::mk(re, im);
     }
   }
 }
@@ -2918,31 +2939,33 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
  * octant-fastest.  Per output the sum runs over the input index in
  * increasing order. */
 template <int NP, typename ST = double2>
-__global__ __launch_bounds__(512) void k_dft_inv(const int* __restrict__ blocks, const int* __restrict__ yslot,
+__global__ __launch_bounds__(Grid<NP>::THREADS) void k_dft_inv(const int* __restrict__ blocks, int n_blocks, const int* __restrict__ yslot,
                                                  const ST* __restrict__ Y, const double2* __restrict__ tw,
                                                  const int* __restrict__ surf2cube, /* NE: (ix*NP+iy)*NP+iz */
                                                  double* __restrict__ dchk, int ld_e) {
   using G = Grid<NP>;
-  constexpr int N = G::N, H = G::H, F = G::F, NE = G::NE, OFF = G::OFF;
-  __shared__ double2 B[NP][N][H][8];  /* [iz][ky][kx][oct] */
-  __shared__ double2 A[NP][NP][H][8]; /* [iz][iy][kx][oct] */
+  constexpr int N = G::N, H = G::H, F = G::F, NE = G::NE, OFF = G::OFF, OC = G::OC, OS = G::OC_SHIFT;
+  __shared__ double2 B[NP][N][H][OC];  /* [iz][ky][kx][oct] */
+  __shared__ double2 A[NP][NP][H][OC]; /* [iz][iy][kx][oct] */
   __shared__ double2 ws[N];           /* for the x pass, whose twiddle index is not a constant */
   const int tid = threadIdx.x;
-  const int first = blocks[blockIdx.x];
+  const int2 bo = dft_block<NP>();
+  if (bo.x >= n_blocks) return; /* whole block */
+  const int first = blocks[bo.x] + bo.y;
   double2 w[N];
 #pragma unroll
   for (int m = 0; m < N; m++) w[m] = tw[m];
   if (tid < N) ws[tid] = tw[tid];
-  const ST* in = Y + (size_t)yslot[blockIdx.x] * F * 8;
-  /* z pass: column (ky, kx, oct) = thread e, reading Y[slot][kz * N * H * 8 + e] */
-  for (int e = tid; e < N * H * 8; e += blockDim.x) {
-    const int o = e & 7, kk = e >> 3; /* kk = ky*H + kx */
+  const ST* in = Y + (size_t)yslot[bo.x] * F * 8 + bo.y;
+  /* z pass: column (ky, kx, oct), reading Y[slot][(kz * N * H + ky * H + kx) * 8 + oct] */
+  for (int e = tid; e < N * H * OC; e += blockDim.x) {
+    const int o = e & (OC - 1), kk = e >> OS; /* kk = ky*H + kx */
     double re[NP], im[NP];
 #pragma unroll
     for (int iz = 0; iz < NP; iz++) { re[iz] = 0.0; im[iz] = 0.0; }
 #pragma unroll
     for (int kz = 0; kz < N; kz++) {
-      const ST vs = in[(size_t)kz * N * H * 8 + e];
+      const ST vs = in[((size_t)kz * N * H + kk) * 8 + o];
       const double2 v = make_double2(vs.x, vs.y);
 #pragma unroll
       for (int iz = 0; iz < NP; iz++) {
@@ -2957,8 +2980,8 @@ __global__ __launch_bounds__(512) void k_dft_inv(const int* __restrict__ blocks,
   }
   __syncthreads();
   /* y pass: column (iz, kx, oct) */
-  for (int e = tid; e < NP * H * 8; e += blockDim.x) {
-    const int o = e & 7, kx = (e >> 3) % H, iz = (e >> 3) / H;
+  for (int e = tid; e < NP * H * OC; e += blockDim.x) {
+    const int o = e & (OC - 1), kx = (e >> OS) % H, iz = (e >> OS) / H;
     double2 v[N];
 #pragma unroll
     for (int ky = 0; ky < N; ky++) v[ky] = B[iz][ky][kx][o];
@@ -2977,11 +3000,11 @@ __global__ __launch_bounds__(512) void k_dft_inv(const int* __restrict__ blocks,
   __syncthreads();
   /* x pass (c2r) at the surface samples */
   const double nrm = 1.0 / (double)(N * N * N);
-  for (int e = tid; e < 8 * NE; e += blockDim.x) {
+  for (int e = tid; e < OC * NE; e += blockDim.x) {
     const int o = e / NE, j = e % NE;
     const int cube = surf2cube[j];
     const int ix = cube / (NP * NP), iy = (cube / NP) % NP, iz = cube % NP;
-    const double2 (*r)[8] = A[iz][iy];
+    const double2 (*r)[OC] = A[iz][iy];
     const int xg = ix + OFF;
     double s = r[0][o].x + ((xg & 1) ? -r[N / 2][o].x : r[N / 2][o].x);
     double acc = 0.0;

@@ -1637,7 +1637,7 @@ int had_block_size(const kifmm_gpu* g) {
 template <int NP, typename ST, typename HAD>
 int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, HAD had) {
   if (g->n_vblocks > 0)
-    launch(g, (k_dft_fwd<NP, ST>), dim3(g->n_vblocks), dim3(512), g->vblocks, g->vslot,
+    launch(g, (k_dft_fwd<NP, ST>), dim3(dft_blocks<NP>(g->n_vblocks)), dim3(Grid<NP>::THREADS), g->vblocks, g->n_vblocks, g->vslot,
                        g->depth, g->uden, g->ld_e, g->tw, g->cube2surf, X);
   LAUNCH_CHECK();
   TRY(phase_end(g, E_FFT));
@@ -1651,7 +1651,7 @@ int vlist_phase(kifmm_gpu* g, ST* X, ST* Y, HAD had) {
   }
   TRY(phase_end(g, E_HAD));
   if (g->n_vblocks > 0)
-    launch(g, (k_dft_inv<NP, ST>), dim3(g->n_vblocks), dim3(512), g->vblocks, g->vslot, Y,
+    launch(g, (k_dft_inv<NP, ST>), dim3(dft_blocks<NP>(g->n_vblocks)), dim3(Grid<NP>::THREADS), g->vblocks, g->n_vblocks, g->vslot, Y,
                        g->tw, g->surf2cube, g->dchk, g->ld_e);
   LAUNCH_CHECK();
   return KIFMM_OK;

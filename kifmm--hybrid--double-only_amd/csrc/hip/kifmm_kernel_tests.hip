@@ -122,7 +122,7 @@ int dft_fwd_np(int nblocks, const double* den, const int* depth, double* out) {
     set_error("device allocation failed");
     return KIFMM_ENOMEM;
   }
-  hipLaunchKernelGGL(k_dft_fwd<NP>, dim3(nblocks), dim3(512), 0, 0, dblk, dslot, ddep, du, lde, dtw, dc2s, dX);
+  hipLaunchKernelGGL(k_dft_fwd<NP>, dim3(dft_blocks<NP>(nblocks)), dim3(Grid<NP>::THREADS), 0, 0, dblk, nblocks, dslot, ddep, du, lde, dtw, dc2s, dX);
   int r = finish("k_dft_fwd");
   if (r != KIFMM_OK) return r;
   return down((double2*)out, dX + (size_t)F * 8, (size_t)nblocks * F * 8);
@@ -160,7 +160,7 @@ int dft_inv_np(int nblocks, const double* spec, double* out) {
     set_error("device allocation failed");
     return KIFMM_ENOMEM;
   }
-  hipLaunchKernelGGL(k_dft_inv<NP>, dim3(nblocks), dim3(512), 0, 0, dblk, dslot, dY, dtw, ds2c, dchk, lde);
+  hipLaunchKernelGGL(k_dft_inv<NP>, dim3(dft_blocks<NP>(nblocks)), dim3(Grid<NP>::THREADS), 0, 0, dblk, nblocks, dslot, dY, dtw, ds2c, dchk, lde);
   int r = finish("k_dft_inv");
   if (r != KIFMM_OK) return r;
   std::vector<double> h((size_t)(1 + 8 * nblocks) * lde);

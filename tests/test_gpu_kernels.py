@@ -176,3 +176,23 @@ def test_rsq_clamp_f32():
     exact = np.minimum(1.0, 1.0 / np.sqrt(np.abs(x.astype(np.float64))))
     assert np.max(np.abs(y - exact) / exact) < 2.0 ** -22
     assert KL.rsq_clamp_f32(np.array([np.inf], dtype=np.float32))[0] == 0.0
+
+
+@pytest.mark.parametrize("nb", [1, 7, 8, 9, 17])
+def test_dft_blocks_of_half_the_octants(nb):
+    """NP 6 runs a child block as two blocks of four octants, 8 blocks apart:
+    counts around the multiples of 8, every octant against numpy (bounds as
+    above)."""
+    rng = np.random.default_rng(60 + nb)
+    ne, N = K.n_e(6), 12
+    den, depth = rng.standard_normal((8 * nb, ne)), rng.integers(2, 6, 8 * nb)
+    got = KL.dft_fwd(6, den, depth)
+    for k in range(8 * nb):
+        ref = np.fft.rfftn(_grid_from_surface(6, den[k] * 2.0 ** depth[k])).reshape(-1)
+        assert np.max(np.abs(got[k // 8, :, k % 8] - ref)) <= 1e-14 * np.max(np.abs(ref)), k
+    grids = rng.standard_normal((nb * 8, N, N, N))
+    spec = np.stack([np.fft.rfftn(x).reshape(-1) for x in grids]).reshape(nb, 8, -1).transpose(0, 2, 1).copy()
+    back = KL.dft_inv(6, spec)
+    for k in range(8 * nb):
+        ref = _surface_from_grid(6, grids[k])
+        assert np.max(np.abs(back[k] - ref)) <= 1e-13 * np.max(np.abs(ref)), k
