@@ -332,11 +332,13 @@ int check_view(const kifmm_tree_view* t) {
   return KIFMM_OK;
 }
 
-/* Parts along K of a level's UE2UC stack: at NP 6 (304 MFMA steps, FP64 only)
- * short levels split it over more blocks; at NP <= 4, where the mixed path
- * needs one order of summation, never. */
+/* Parts along K of a level's UE2UC stack: on the FP64 path short levels split
+ * it over more blocks, whose waves otherwise run 304 (NP 6) or 112 (NP 4) MFMA
+ * steps one after another: with the sum over the parts in UC2UE a level of 64
+ * parents takes 11.2 us at NP 4 instead of 14.8.  The mixed path keeps one order of
+ * summation. */
 constexpr int M2M_PARTS = 4;
-inline int m2m_parts(int np, int ncols) { return np == 6 && ncols < 1024 ? M2M_PARTS : 1; }
+inline int m2m_parts(int np, int ncols, bool mixed) { return (np == 6 || !mixed) && ncols < 1024 ? M2M_PARTS : 1; }
 constexpr int LEAF_SPLIT = 8192; /* leaves below which the FP64 leaf UC2UE is a k_level_op */
 
 /* Everything the device needs, derived on the host from the tree view.
@@ -509,32 +511,34 @@ XcdRuns xcd_runs(const std::vector<double>& cost, int b, int e) {
   return r;
 }
 
-/* The items of a list for a launch over all of them: within an XCD's run those
- * of more than the mean cost first, in classes of falling cost (factor 1.25),
- * then the others in their order, in which neighbours share sources.  An
- * uneven list otherwise ends with its long items on an emptying chip.  U-list
- * kernel: 53 -> 50.5 us at 100 thousand points, 136 -> 128 at 300 thousand, 482 -> 465 at 1M
- * ellipsoid, 5.36 -> 5.28 ms at 4M.  Not on the mixed path, whose kernel was slower
- * for it (465 thousand points 0.315 -> 0.40 ms). */
+/* The indices [b, e) of items, those of more than the mean cost first, in
+ * classes of falling cost (factor 1.25), then the others in their order, in
+ * which neighbours share data.  An uneven list otherwise ends with its long
+ * items on an emptying chip. */
+template <typename Cost>
+void long_first(int b, int e, double mean, Cost cost, std::vector<int>& out) {
+  std::vector<std::vector<int>> cls(1);
+  for (int k = b; k < e; k++) {
+    const double r = cost(k) / mean;
+    const size_t c = r <= 1.0 ? 0 : std::min<size_t>(30, 1 + (size_t)(std::log(r) / std::log(1.25)));
+    if (c >= cls.size()) cls.resize(c + 1);
+    cls[c].push_back(k);
+  }
+  for (size_t c = cls.size(); c-- > 0;) out.insert(out.end(), cls[c].begin(), cls[c].end());
+}
+/* The U-list items of a launch over all of them, long ones first within each
+ * XCD's run.  U-list kernel: 53 -> 50.5 us at 100 thousand points, 136 -> 128 at 300
+ * thousand, 482 -> 465 at 1M ellipsoid, 5.36 -> 5.28 ms at 4M.  Not on the mixed
+ * path, whose kernel was slower for it (465 thousand points 0.315 -> 0.40 ms). */
 std::vector<int4> u_launch_order(const std::vector<int4>& items, const std::vector<double>& cost) {
   const int n = (int)items.size();
-  std::vector<int4> out(items);
-  if (n == 0) return out;
+  if (n == 0) return {};
   const XcdRuns runs = xcd_runs(cost, 0, n);
-  const double mean = cost[n] / n;
-  std::vector<std::vector<int>> cls;
-  for (int x = 0; x < 8; x++) {
-    for (auto& c : cls) c.clear();
-    for (int k = runs.beg[x]; k < runs.beg[x + 1]; k++) {
-      const double r = (cost[k + 1] - cost[k]) / mean;
-      const size_t c = r <= 1.0 ? 0 : std::min<size_t>(30, 1 + (size_t)(std::log(r) / std::log(1.25)));
-      if (c >= cls.size()) cls.resize(c + 1);
-      cls[c].push_back(k);
-    }
-    int at = runs.beg[x];
-    for (size_t c = cls.size(); c-- > 0;)
-      for (int k : cls[c]) out[at++] = items[k];
-  }
+  std::vector<int> order;
+  for (int x = 0; x < 8; x++)
+    long_first(runs.beg[x], runs.beg[x + 1], cost[n] / n, [&](int k) { return cost[k + 1] - cost[k]; }, order);
+  std::vector<int4> out;
+  for (int k : order) out.push_back(items[k]);
   return out;
 }
 
@@ -1002,6 +1006,16 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
   P.chk_cols = P.s2m_items.size();
   for (const int4& it : P.s2m_items)
     if (it.y < 0 || it.z < 1 || (long)it.y + it.z > t->n_src) return fail("S2M source range out of range");
+  /* FP64: long leaves first, 60 -> 50 us at 300 thousand points NP 6, 14.2 -> 12.8 at 100
+   * thousand NP 4, no change at 4M; the mixed kernel, four leaves a block, was
+   * slower for it (65 thousand points 16.6 -> 18.1).  The columns stay in leaf order */
+  if (!mixed) {
+    const int n = (int)P.s2m_items.size();
+    const std::vector<int4> by_leaf(P.s2m_items);
+    std::vector<int> order;
+    long_first(0, n, (double)t->n_src / std::max(n, 1), [&](int k) { return (double)by_leaf[k].z; }, order);
+    for (int k = 0; k < n; k++) P.s2m_items[k] = by_leaf[order[k]];
+  }
 
   /* per-level M2M, L2L and DC2DE column lists */
   P.lv.assign(maxd + 1, HostLevel());
@@ -1027,7 +1041,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
         wc.gemm_flops += 2.0 * ne * ne;
       }
     }
-    P.chk_cols = std::max(P.chk_cols, (size_t)col * m2m_parts(np, col));
+    P.chk_cols = std::max(P.chk_cols, (size_t)col * m2m_parts(np, col, mixed));
   }
   /* the fused downward kernel (k_l2l_dc2de) of depth d >= 3 runs over the
    * L2L parents at d - 1 and writes the densities of their target
@@ -1584,7 +1598,7 @@ int uc2ue(kifmm_gpu* g, const GemmList& B, int nin) {
 /* M2M of one level in two launches: the UE2UC stack into check values, in
  * m2m_parts slices along K, then UC2UE */
 int m2m(kifmm_gpu* g, const GemmList& A, const GemmList& B, int d) {
-  const int parts = m2m_parts(g->np, A.n);
+  const int parts = m2m_parts(g->np, A.n, g->precision == KIFMM_PREC_MIXED);
   LevelOp op{};
   op.M = g->n_uc; op.K = 8 * g->ld_e / parts; op.A = g->UE2UC; op.lda = g->lda_uc;
   op.a_z = (size_t)op.K * g->lda_uc; op.in_z = op.K;
