@@ -259,44 +259,62 @@ __device__ __forceinline__ void eval8_gram(const double4* __restrict__ src, cons
   }
 }
 
-/* The close-pair terms of the nt <= 16 targets from tg0: the sum of target
- * tg0 + t on the lanes l with l % 16 = t.  Four lanes take a target's pairs in
- * turn; a target with more than CLOSE_FEW of them takes the whole wave.  Both
- * orders are fixed and depend on the target alone: deterministic, and the
- * same for every launch form.  (A segmented scan over the run of all pairs of 8
- * targets, mostly 8 to 20 pairs, spent 6 exchange steps on each.)  isc = 1 / sc,
- * exact. */
+/* Sums over the close pairs of 16 targets: that of target t on the lanes l
+ * with l % 16 = t, whose n pairs are cidx[beg ..] (n = 0 past the last
+ * target); term(t, source) is a pair's.  Four lanes take a target's pairs in
+ * turn; a target with more than CLOSE_FEW of them takes the whole wave.  Four
+ * pairs of a lane are under way at a time.  Both orders are fixed and depend
+ * on the target alone: deterministic, and the same for every launch form.  (A
+ * segmented scan over the run of all pairs of the targets, mostly 8 to 20
+ * pairs, spent 6 exchange steps on each 64.) */
 constexpr int CLOSE_FEW = 16;
+template <typename Term>
+__device__ __forceinline__ double pair_sums(int beg, int n, int lane, const int* __restrict__ cidx,
+                                            const double4* __restrict__ src4, Term term) {
+  /* pairs k, k + step, .. + 3 step, before end, added to v in order */
+  auto four = [&](double& v, int t, int k, int step, int end) {
+    int j[4];
+    double4 q[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) j[u] = k + step * u < end ? cidx[k + step * u] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (j[u] >= 0) q[u] = src4[j[u]];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (j[u] >= 0) v += term(t, q[u]);
+  };
+  double v = 0.0;
+  if (!__any(n > 0)) return v;
+  static_assert(CLOSE_FEW == 16, "four pairs on each of four lanes");
+  if (n <= CLOSE_FEW) four(v, lane & 15, beg + (lane >> 4), 4, beg + n);
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  for (unsigned many = (unsigned)__ballot(n > CLOSE_FEW) & 0xffffu; many; many &= many - 1) {
+    const int o = __builtin_ctz(many), b = __builtin_amdgcn_readlane(beg, o), e = b + __builtin_amdgcn_readlane(n, o);
+    double u = 0.0;
+    for (int k = b + lane; k < e; k += 256) four(u, o, k, 64, e);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) u += __shfl_xor(u, off);
+    if ((lane & 15) == o) v = u;
+  }
+  return v;
+}
+/* The close-pair terms of the nt <= 16 targets from tg0 (pair_sums).  isc = 1 /
+ * sc, exact. */
 template <bool MASK>
 __device__ __forceinline__ double close_sums(int tg0, int nt, int lane, double isc, double sc, const double4& g,
                                              const double4* __restrict__ src4, const double4* __restrict__ trg4,
                                              const double4* __restrict__ trg_gram, const int* __restrict__ cptr,
                                              const int* __restrict__ cidx) {
-  auto term = [&](const double4& tp, const double4& a, int j) {
-    const double4 q = src4[j];
-    const double dx = tp.x - q.x, dy = tp.y - q.y, dz = tp.z - q.z;
-    const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-    return q.w * (inv_r2<MASK>(r2) * isc - gram_pair(a, gram_src(q, g, sc)));
-  };
   const int t = lane & 15, tt = tg0 + min(t, nt - 1);
   const int beg = cptr[tt], n = t < nt ? cptr[tt + 1] - beg : 0;
-  double v = 0.0;
-  if (__any(n > 0)) {
-    const double4 tp = trg4[tt], a = trg_gram[tt];
-    for (int k = lane >> 4; n <= CLOSE_FEW && k < n; k += 4) v += term(tp, a, cidx[beg + k]);
-    v += __shfl_xor(v, 16);
-    v += __shfl_xor(v, 32);
-    for (unsigned many = (unsigned)__ballot(n > CLOSE_FEW) & 0xffffu; many; many &= many - 1) {
-      const int o = __builtin_ctz(many), b = __builtin_amdgcn_readlane(beg, o), e = b + __builtin_amdgcn_readlane(n, o);
-      const double4 op = trg4[tg0 + o], oa = trg_gram[tg0 + o];
-      double u = 0.0;
-      for (int k = b + lane; k < e; k += 64) u += term(op, oa, cidx[k]);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) u += __shfl_xor(u, off);
-      if (t == o) v = u;
-    }
-  }
-  return v;
+  return pair_sums(beg, n, lane, cidx, src4, [&](int tl, const double4& q) {
+    const double4 tp = trg4[tg0 + tl];
+    const double dx = tp.x - q.x, dy = tp.y - q.y, dz = tp.z - q.z;
+    const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+    return q.w * (inv_r2<MASK>(r2) * isc - gram_pair(trg_gram[tg0 + tl], gram_src(q, g, sc)));
+  });
 }
 
 /* The item's potentials on their way out, in the Gram form first its close-
@@ -940,72 +958,29 @@ __device__ __forceinline__ void mixed_tau_chunks(const v8bf (*sB)[P2P_TILE], con
     for (int e = 0; e < 4; e++) acc[q][e] += (double)part[q][e];
 }
 
-/* close pairs per target up to which the per-target form sums them */
-constexpr int MIX_FEW = 16;
-
 /* FP64 close-pair terms of one 16-target group (slots t0 .. t0 + 15 of sT,
  * nt of them real, the first at target index tg0): sC[t0 + t] = sum over
  * the listed pairs of target t of w (1 / r' - 1), in the scaled frame (g,
- * sc).  A group's pairs are one contiguous run of cidx (targets in order).
- * When no target of the group has more than MIX_FEW of them, four lanes
- * serve each target (pairs s, s + 4, ... of its run on lane 16 s + t) and
- * add their sums by two lane exchanges; otherwise the pairs are spread over
- * the 64 lanes whatever their distribution over the 16 targets and summed
- * per target by a segmented scan over the lanes.  Both orders are fixed:
- * deterministic.  One wave. */
+ * sc).  One wave; the lanes as in close_sums (a target's few pairs on four
+ * lanes, many on the whole wave): deterministic.  Many are what matters: on
+ * clustered inputs a leaf's targets have a thousand close pairs each, and their
+ * block is the launch's last.  A segmented scan per 64 pairs of a group, a
+ * round trip for the indices and one for the sources in front of it, made the
+ * kernel 0.315 ms at 465 thousand points, 0.25 now. */
 template <bool MASK>
 __device__ __forceinline__ void mixed_close_group(const double4* __restrict__ sT, double* __restrict__ sC, int t0,
                                                   int nt, int tg0, const int* __restrict__ cptr,
                                                   const int* __restrict__ cidx, const double4* __restrict__ src4,
                                                   double4 g, double sc, int lane) {
-  const int tj = lane & 15;
-  const int sj = cptr[tg0 + min(tj, nt - 1)];
-  const int ej = cptr[tg0 + min(tj, nt - 1) + 1]; /* end of target lane&15's run */
-  int most = tj < nt ? ej - sj : 0;
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) most = max(most, __shfl_xor(most, off, 64));
-  if (__builtin_amdgcn_readfirstlane(most) <= MIX_FEW) {
-    double v = 0.0;
-    if (tj < nt) {
-      const double4 tp = sT[t0 + tj];
-      for (int k = sj + (lane >> 4); k < ej; k += 4) {
-        const double4 sp = src4[cidx[k]];
-        const double dx = tp.x - (sp.x - g.x) * sc, dy = tp.y - (sp.y - g.y) * sc, dz = tp.z - (sp.z - g.z) * sc;
-        const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-        v += sp.w * (inv_r<MASK>(r2) - 1.0);
-      }
-    }
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    if (lane < 16) sC[t0 + lane] = v;
-    return;
-  }
-  if (lane < 16) sC[t0 + lane] = 0.0;
-  const int kbeg = cptr[tg0], kend = cptr[tg0 + nt];
-  for (int kb = kbeg; kb < kend; kb += 64) {
-    const int k = kb + lane;
-    const bool live = k < kend;
-    int tl = 0; /* the target of pair k: the number of runs that end at or before k */
-#pragma unroll
-    for (int j = 0; j < 16; j++) tl += __builtin_amdgcn_readlane(ej, j) <= k;
-    tl = live ? tl : 16;
-    double v = 0.0;
-    if (live) {
-      const double4 sp = src4[cidx[k]];
-      const double4 tp = sT[t0 + tl];
-      const double dx = tp.x - (sp.x - g.x) * sc, dy = tp.y - (sp.y - g.y) * sc, dz = tp.z - (sp.z - g.z) * sc;
-      const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-      v = sp.w * (inv_r<MASK>(r2) - 1.0);
-    }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const double u = __shfl_up(v, off, 64);
-      const int ut = __shfl_up(tl, off, 64);
-      if (lane >= off && ut == tl) v += u;
-    }
-    const int nx = __shfl_down(tl, 1, 64);
-    if (live && (lane == 63 || nx != tl)) sC[t0 + tl] += v; /* one writer per target and chunk */
-  }
+  const int t = lane & 15, tt = tg0 + min(t, nt - 1);
+  const int beg = cptr[tt], n = t < nt ? cptr[tt + 1] - beg : 0;
+  const double v = pair_sums(beg, n, lane, cidx, src4, [&](int tl, const double4& sp) {
+    const double4 tp = sT[t0 + tl];
+    const double dx = tp.x - (sp.x - g.x) * sc, dy = tp.y - (sp.y - g.y) * sc, dz = tp.z - (sp.z - g.z) * sc;
+    const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+    return sp.w * (inv_r<MASK>(r2) - 1.0);
+  });
+  if (lane < 16) sC[t0 + lane] = v;
 }
 
 /* Groups of 16 targets per wave: items of up to P2P_MAXT5 targets (10
