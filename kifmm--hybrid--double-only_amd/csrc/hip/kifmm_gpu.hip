@@ -528,8 +528,8 @@ void long_first(int b, int e, double mean, Cost cost, std::vector<int>& out) {
 }
 /* The U-list items of a launch over all of them, long ones first within each
  * XCD's run.  U-list kernel: 53 -> 50.5 us at 100 thousand points, 136 -> 128 at 300
- * thousand, 482 -> 465 at 1M ellipsoid, 5.36 -> 5.28 ms at 4M.  Not on the mixed
- * path, whose kernel was slower for it (465 thousand points 0.315 -> 0.40 ms). */
+ * thousand, 482 -> 465 at 1M ellipsoid, 5.36 -> 5.28 ms at 4M; mixed 258 -> 238 us at
+ * 465 thousand, 32.8 -> 31.8 at 65 thousand, 1.96 -> 1.93 ms at 4M. */
 std::vector<int4> u_launch_order(const std::vector<int4>& items, const std::vector<double>& cost) {
   const int n = (int)items.size();
   if (n == 0) return {};
@@ -985,11 +985,9 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
       }
       P.chunk_beg[l].push_back((int)L.size());
     }
-    /* the list that the default form launches, FP64 */
-    if (!mixed) {
-      P.u_order_list = P.wave_g > 0 ? 4 : t->n_trg <= U_SMALL * P.p2p_items5.size() ? 1 : 2;
-      P.u_order = u_launch_order(*lists[P.u_order_list], P.u_cost[P.u_order_list]);
-    }
+    /* the list that the default form launches */
+    P.u_order_list = mixed ? 3 : P.wave_g > 0 ? 4 : t->n_trg <= U_SMALL * P.p2p_items5.size() ? 1 : 2;
+    P.u_order = u_launch_order(*lists[P.u_order_list], P.u_cost[P.u_order_list]);
   }
 
   /* S2M + UC2UE over source leaves */
