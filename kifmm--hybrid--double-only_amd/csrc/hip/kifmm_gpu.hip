@@ -1633,14 +1633,17 @@ int fill(kifmm_gpu* g, double* p, size_t n, double* q = nullptr, size_t m = 0) {
   return KIFMM_OK;
 }
 
-/* Frequencies per Hadamard block: had_fb, halved (to 2 at least) while the
- * launch has fewer than two blocks per CU.  A block runs its frequencies one
- * after another: 4 thousand points NP 3 took 29 us in blocks of 8, 17 of 4
- * and 12 of 2; above that the prefetch across frequencies pays (4M NP 6: 0.88
- * ms in blocks of 4, 0.87 of 8).  The sums are the same. */
+/* Frequencies per Hadamard block: had_fb, halved down to 4 while the launch has
+ * fewer than two blocks per CU and to 2 below four.  A block runs its
+ * frequencies one after another: 4 thousand points NP 3 took 29 us in blocks
+ * of 8, 17 of 4 and 12 of 2; 100 thousand NP 4 57 in 800 blocks of 4 and 53 in
+ * 1600 of 2, 65 thousand mixed 44 and 41, 16 thousand NP 6 the same.  Above that
+ * the prefetch across frequencies pays (465 thousand mixed: 61 us in 680 blocks of
+ * 8, 62.5 in 1360 of 4; 4M NP 6: 0.87 ms in blocks of 8, 0.88 of 4).  The sums are
+ * the same. */
 int had_block_size(const kifmm_gpu* g) {
   int fb = g->had_fb;
-  while (fb > 2 && (long)g->n_hgroups * (g->F / fb) < 512) fb /= 2;
+  while (fb > 2 && (long)g->n_hgroups * (g->F / fb) < (fb > 4 ? 512 : 1024)) fb /= 2;
   return fb;
 }
 
