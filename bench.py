@@ -6,8 +6,8 @@ Headline workload: 4,194,304 points i.i.d. uniform in [0,1]^3 (mapped to the
 reference root box by x' = 2x - 1), separate targets, densities in [0,1),
 seed 1, NP = 4.  A step is one kifmm_gpu_evaluate over inputs already
 resident in HBM: up, V, W, X, down and the U-list, and the device -> host
-copy of the potentials into host memory (the handle's pinned buffer; the
-copies of early U-list chunks overlap the later chunks).  `value` is the
+copy of the potentials into host memory (the handle's pinned buffer, which
+the U-list writes as it runs).  `value` is the
 mixed-precision, batched, model-tuned path (the cost model picks points per
 box and the precision path, kifmm_gpu_autotune the launch shapes and the
 stream layout, one HIP graph per step); `mixed_vs_fp64` holds it beside the

@@ -2,11 +2,11 @@
  * kernels.hpp -- gfx950 kernels of the KIFMM evaluation path (FP64 plain path).
  *
  * Stage map (reference kernel it replaces, fmm/cuda.cu):
- *   k_p2p_ulist ....... ulist_eval__gpu             (604-663)   U-list P2P
+ *   k_p2p_ulist, k_p2p_wave  ulist_eval__gpu        (604-663)   U-list P2P
  *   k_s2m ............. up_eval__gpu, first half    (108-190)   sources -> UC check potential
- *   k_gemm_cols ....... the dgemv loops of up_eval__gpu, up_eval__gpu_non_leaf,
+ *   k_gemm_cols, k_level_op  the dgemv loops of up_eval__gpu, up_eval__gpu_non_leaf,
  *                       down_eval__gpu_depth_2 / _non_leaves    (430-528, 1682-1801)
- *                       as FP64 MFMA GEMMs over a column list
+ *                       as FP64 MFMA applies over a column list
  *   k_dft_fwd ......... compute_fft_src__gpu_eval + cuFFT D2Z   (718-871)
  *   k_trans ........... compute_fft_trans__gpu_eval + D2Z x343  (874-963)
  *   k_hadamard ........ vlist_calc__gpu_eval                    (1200-1240)
