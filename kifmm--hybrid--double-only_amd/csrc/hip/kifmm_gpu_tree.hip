@@ -320,6 +320,7 @@ struct Down {
   };
   hipStream_t st = nullptr;
   char* pin = nullptr;
+  bool tried = false;
   size_t used = 0;
   std::vector<Piece> queued;
   ~Down() {
@@ -333,7 +334,17 @@ struct Down {
     return true;
   }
   bool bytes(void* to, const void* from, size_t n) {
-    if (!pin) GT_TRY(hipHostMalloc((void**)&pin, PIN, hipHostMallocDefault));
+    if (!pin && !tried) {
+      tried = true;
+      if (hipHostMalloc((void**)&pin, PIN, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        pin = nullptr;
+      }
+    }
+    if (!pin) { /* no pinned memory: the runtime's own copy */
+      if (n) GT_TRY(hipMemcpyAsync(to, from, n, hipMemcpyDeviceToHost, st));
+      return true;
+    }
     for (size_t at = 0; at < n;) {
       const size_t m = std::min(n - at, PIN);
       if (used + m > PIN && !wait()) return false;
