@@ -243,6 +243,7 @@ inline int blocks(long long n, int t) { return (int)std::max<long long>(1, (n + 
 
 struct Dev {
   kifmm_dev::DeviceArena mem;
+  explicit Dev(hipStream_t st) : mem(st) {}
   template <typename T>
   T* alloc(size_t n) {
     return (T*)mem.get(sizeof(T) * std::max<size_t>(n, 1));
@@ -371,14 +372,14 @@ bool build(int device, kifmm_problem* p, double* seconds) {
   GT_TRY(hipSetDevice(device));
   hipStream_t st = nullptr;
   GT_TRY(kifmm_dev::take_stream(device, &st));
-  Dev D; /* freed after sg has waited for the stream */
-  Down host;
-  host.st = st;
-  struct StreamGuard { /* goes before the memory does: the stream's work ends first */
+  struct StreamGuard {
     int dev;
     hipStream_t s;
     ~StreamGuard() { kifmm_dev::give_stream(dev, s); }
   } sg{device, st};
+  Down host;
+  host.st = st;
+  Dev D(st); /* goes first: waits for the stream, and keeps no block for a next owner if that fails */
   double* xyz[6];
   for (int a = 0; a < 6; a++) {
     xyz[a] = D.alloc<double>(n);

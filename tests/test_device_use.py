@@ -1,0 +1,34 @@
+"""What the library's host code takes from the HIP runtime and gives back, and
+what it makes of the runtime's errors, on the fake runtime (fake_device.py)."""
+import pytest
+
+import fake_device
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = fake_device.build(tmp_path_factory.mktemp("fake"))
+    return lambda code: fake_device.run(so, code)
+
+
+def test_tree_build_that_did_not_end_keeps_nothing(fake):
+    """A tree build whose stream cannot be waited for, from any of its waits
+    on: its memory and stream are freed, not handed to the next owner."""
+    fake("""
+    for skip in range(100):
+        n0 = fake.fake_calls(b"hipStreamSynchronize")
+        fail("hipStreamSynchronize", skip, 1 << 30)
+        try:
+            K.Problem.create(500, "uniform", 40, np_=3, seed=1, device=0)
+        except K.KifmmError:
+            pass
+        fail("hipStreamSynchronize", 0, 0)
+        fake.hipGetLastError()
+        failed = fake.fake_calls(b"hipStreamSynchronize") - n0 - skip
+        if failed <= 0:
+            break  # it has no more waits
+        assert fake.fake_streams() == 0, skip
+        # (the last wait of all is the stream's own, after one that ended the work on the memory)
+        assert fake.fake_used() == 0 or (failed == 1 and skip > 3), (skip, failed, fake.fake_used())
+    assert 3 < skip < 99
+    """)
