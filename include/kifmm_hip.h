@@ -7,7 +7,8 @@
  * kifmm_gpu_create replaces preproc (flatten + upload, library-owned device
  * memory); kifmm_gpu_evaluate replaces run (up, U, V, W, X, down, copy;
  * phase timing as fmm/run--cuda.cu:323-340 with the copy actually timed);
- * kifmm_gpu_destroy frees what create allocated (the reference never frees).
+ * kifmm_gpu_destroy frees what create allocated (the reference never frees), but
+ * for idle memory and streams kept for the next handle (kifmm_gpu_release_idle).
  *
  * All entry points return 0 on success or a negative KIFMM_E* code, never
  * exit.  A handle is not thread-safe; several handles may coexist.  Each
@@ -161,6 +162,13 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops,
  * NULL. */
 int kifmm_gpu_evaluate(kifmm_gpu* g, double* pot_leaf, kifmm_phase_times* times);
 int kifmm_gpu_destroy(kifmm_gpu* g);
+/* Gives idle device memory and streams back to the runtime: destroyed handles
+ * and finished tree builds leave up to 128 MB of memory blocks and four streams
+ * of the process for the next ones to take.  Live handles keep what is theirs.
+ * An allocation of this library that fails gives the memory back by itself;
+ * other allocators of the process (another library, hipMalloc) need this call.
+ * No counterpart in the reference, which never frees. */
+int kifmm_gpu_release_idle(void);
 
 /* The handle's pinned host buffer of n_trg potentials (gathered target
  * order), valid until kifmm_gpu_destroy; NULL if pinned memory could not be

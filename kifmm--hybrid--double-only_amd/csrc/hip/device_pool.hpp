@@ -52,6 +52,12 @@ inline hipError_t take_stream(int dev, hipStream_t* s) {
   }
   return *s ? hipSuccess : hipStreamCreateWithFlags(s, hipStreamNonBlocking);
 }
+inline void drop_streams() {
+  StreamPool& p = stream_pool();
+  std::lock_guard<std::mutex> lock(p.m);
+  for (const auto& s : p.idle) (void)hipStreamDestroy(s.second);
+  p.idle.clear();
+}
 /* waits for the stream's work first */
 inline void give_stream(int dev, hipStream_t s) {
   if (!s) return;
@@ -68,7 +74,8 @@ inline void give_stream(int dev, hipStream_t s) {
 }
 
 /* Idle blocks of device arenas, BLOCKS_KEPT bytes at most in the whole process.
- * They go back to the runtime when an arena's allocation fails. */
+ * They go back to the runtime when an arena's allocation fails, and with the
+ * idle streams by kifmm_gpu_release_idle. */
 constexpr size_t BLOCKS_KEPT = (size_t)128 << 20;
 struct Block {
   int dev;

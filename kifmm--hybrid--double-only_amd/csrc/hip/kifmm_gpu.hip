@@ -2303,6 +2303,12 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   return KIFMM_OK;
 }
 
+int kifmm_gpu_release_idle(void) {
+  drop_blocks();
+  drop_streams();
+  return KIFMM_OK;
+}
+
 /* The split of nt targets over n sources: chunks of the sources until there
  * are DIR_ITEMS work items (four per block slot of the chip at 4 blocks of 4
  * waves per CU, so that the last round is a quarter of the work at most), a

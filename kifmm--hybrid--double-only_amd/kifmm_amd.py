@@ -134,6 +134,7 @@ _sig("kifmm_gpu_create", C.c_int, [C.POINTER(TreeView), C.POINTER(Operators), C.
                                    C.POINTER(C.c_void_p)])
 _sig("kifmm_gpu_evaluate", C.c_int, [C.c_void_p, _dp, C.POINTER(PhaseTimes)])
 _sig("kifmm_gpu_destroy", C.c_int, [C.c_void_p])
+_sig("kifmm_gpu_release_idle", C.c_int, [])
 _sig("kifmm_gpu_evaluate_phases", C.c_int, [C.c_void_p, C.c_uint, _dp, C.POINTER(PhaseTimes)])
 _sig("kifmm_gpu_work_counts", C.c_int, [C.c_void_p, C.POINTER(WorkCounts)])
 _sig("kifmm_gpu_copy_intermediate", C.c_int, [C.c_void_p, C.c_int, _dp, C.c_long])
@@ -335,6 +336,13 @@ def write_points(path, sx, sy, sz, den, tx=None, ty=None, tz=None):
 
 def gpu_available() -> bool:
     return bool(lib.kifmm_gpu_available())
+
+
+def release_idle():
+    """Give the device memory and streams that closed evaluators and finished
+    tree builds left for the next ones back to the runtime
+    (kifmm_gpu_release_idle)."""
+    _check(lib.kifmm_gpu_release_idle())
 
 
 class GpuEvaluator:

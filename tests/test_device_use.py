@@ -32,3 +32,26 @@ def test_tree_build_that_did_not_end_keeps_nothing(fake):
         assert fake.fake_used() == 0 or (failed == 1 and skip > 3), (skip, failed, fake.fake_used())
     assert 3 < skip < 99
     """)
+
+
+def test_idle_memory_and_streams_are_given_back(fake):
+    """What handles and tree builds leave for the next ones goes back to the
+    runtime on request, whatever handles live; they work on afterwards."""
+    fake("""
+    prob = K.Problem.create(5000, "ellipsoid", 40, np_=4, seed=1, device=None)
+    ops = prob.operators()
+    live = K.GpuEvaluator(prob, operators=ops)
+    K.release_idle()  # its set-up leaves idle memory too
+    used, streams = fake.fake_used(), fake.fake_streams()
+    K.Problem.create(5000, "ellipsoid", 40, np_=4, seed=1, device=0)
+    K.GpuEvaluator(prob, operators=ops).close()
+    assert fake.fake_used() > used and fake.fake_streams() > streams, (fake.fake_used(), used, fake.fake_streams(), streams)
+    K.release_idle()
+    assert fake.fake_used() == used and fake.fake_streams() == streams, (fake.fake_used(), used, fake.fake_streams(), streams)
+    K.release_idle()
+    live.evaluate()
+    K.GpuEvaluator(prob, operators=ops).close()
+    live.close()
+    K.release_idle()
+    assert fake.fake_used() == 0 and fake.fake_streams() == 0 and fake.fake_events() == 0
+    """)
