@@ -23,82 +23,132 @@
 
 namespace kifmm_dev {
 
-/* Idle non-blocking streams of default priority.  At most STREAMS_KEPT stay,
- * in the whole process and over all devices (the hardware has four queues per process);
- * a stream beyond those, or one that did not end its work cleanly, is
- * destroyed.  An idle stream holds no user data. */
+/* What is idle between owners: non-blocking streams of default priority, at
+ * most STREAMS_KEPT in the whole process and over all devices (the hardware has
+ * four queues per process), and blocks of device arenas, BLOCKS_KEPT bytes at
+ * most.  A stream beyond those, or one that did not end its work cleanly, is
+ * destroyed.  An idle stream holds no user data.  The blocks go back to the
+ * runtime when an arena's allocation fails, and with the streams by
+ * kifmm_gpu_release_idle.
+ * hipDeviceReset destroys all of it.  So a device's idle things count as long
+ * as its mark does, a small allocation made with the first of them: an
+ * allocation's buffer id names no other one later, whatever its address.
+ * After a reset they are forgotten, not used and not freed. */
 constexpr size_t STREAMS_KEPT = 4;
-struct StreamPool {
-  std::mutex m;
-  std::vector<std::pair<int, hipStream_t>> idle;
-};
-inline StreamPool& stream_pool() {
-  alignas(StreamPool) static char at[sizeof(StreamPool)];
-  static StreamPool* const p = new (at) StreamPool; /* never destroyed: the runtime may be gone by then */
-  return *p;
-}
-/* a stream of device dev, the current one */
-inline hipError_t take_stream(int dev, hipStream_t* s) {
-  *s = nullptr;
-  {
-    StreamPool& p = stream_pool();
-    std::lock_guard<std::mutex> lock(p.m);
-    for (size_t k = 0; k < p.idle.size(); k++)
-      if (p.idle[k].first == dev) {
-        *s = p.idle[k].second;
-        p.idle.erase(p.idle.begin() + (long)k);
-        break;
-      }
-  }
-  return *s ? hipSuccess : hipStreamCreateWithFlags(s, hipStreamNonBlocking);
-}
-inline void drop_streams() {
-  StreamPool& p = stream_pool();
-  std::lock_guard<std::mutex> lock(p.m);
-  for (const auto& s : p.idle) (void)hipStreamDestroy(s.second);
-  p.idle.clear();
-}
-/* waits for the stream's work first */
-inline void give_stream(int dev, hipStream_t s) {
-  if (!s) return;
-  if (hipStreamSynchronize(s) == hipSuccess) {
-    StreamPool& p = stream_pool();
-    std::lock_guard<std::mutex> lock(p.m);
-    if (p.idle.size() < STREAMS_KEPT) try {
-        p.idle.emplace_back(dev, s);
-        return;
-      } catch (const std::bad_alloc&) {
-      }
-  }
-  (void)hipStreamDestroy(s);
-}
-
-/* Idle blocks of device arenas, BLOCKS_KEPT bytes at most in the whole process.
- * They go back to the runtime when an arena's allocation fails, and with the
- * idle streams by kifmm_gpu_release_idle. */
 constexpr size_t BLOCKS_KEPT = (size_t)128 << 20;
 struct Block {
   int dev;
   void* p;
   size_t bytes;
 };
-struct BlockPool {
+struct IdlePool {
+  struct Mark {
+    int dev;
+    void* p;
+    unsigned long long id;
+  };
   std::mutex m;
-  std::vector<Block> idle;
-  size_t bytes = 0;
+  std::vector<std::pair<int, hipStream_t>> streams;
+  std::vector<Block> blocks;
+  size_t bytes = 0; /* of blocks */
+  std::vector<Mark> marks;
+
+  static bool buffer_id(void* p, unsigned long long* id) {
+    *id = 0;
+    if (hipPointerGetAttribute(id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, (hipDeviceptr_t)p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  /* whether what is idle of dev can be used; m is held, here and below */
+  bool alive(int dev) {
+    for (size_t k = 0; k < marks.size(); k++) {
+      if (marks[k].dev != dev) continue;
+      unsigned long long id;
+      if (buffer_id(marks[k].p, &id) && id == marks[k].id) return true;
+      forget(dev);
+      return false;
+    }
+    return false; /* nothing of dev is idle */
+  }
+  /* before something of dev is put away; false: it cannot be kept */
+  bool mark(int dev) {
+    if (alive(dev)) return true;
+    int cur = -1;
+    Mark k{dev, nullptr, 0};
+    if (hipGetDevice(&cur) != hipSuccess || cur != dev) return false;
+    if (hipMalloc(&k.p, 1) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (buffer_id(k.p, &k.id)) try {
+        marks.push_back(k);
+        return true;
+      } catch (const std::bad_alloc&) {
+      }
+    (void)hipFree(k.p);
+    return false;
+  }
+  void forget(int dev) {
+    streams.erase(std::remove_if(streams.begin(), streams.end(), [&](const auto& e) { return e.first == dev; }),
+                  streams.end());
+    for (const Block& b : blocks)
+      if (b.dev == dev) bytes -= b.bytes;
+    blocks.erase(std::remove_if(blocks.begin(), blocks.end(), [&](const Block& b) { return b.dev == dev; }),
+                 blocks.end());
+    marks.erase(std::remove_if(marks.begin(), marks.end(), [&](const Mark& k) { return k.dev == dev; }), marks.end());
+  }
+  void free_blocks() {
+    for (size_t k = blocks.size(); k-- > 0;) {
+      if (k >= blocks.size() || !alive(blocks[k].dev)) continue; /* forgotten */
+      (void)hipFree(blocks[k].p);
+      bytes -= blocks[k].bytes;
+      blocks.erase(blocks.begin() + (long)k);
+    }
+  }
 };
-inline BlockPool& block_pool() {
-  alignas(BlockPool) static char at[sizeof(BlockPool)];
-  static BlockPool* const p = new (at) BlockPool; /* as stream_pool */
+inline IdlePool& idle_pool() {
+  alignas(IdlePool) static char at[sizeof(IdlePool)];
+  static IdlePool* const p = new (at) IdlePool; /* never destroyed: the runtime may be gone by then */
   return *p;
 }
+/* a stream of device dev, the current one */
+inline hipError_t take_stream(int dev, hipStream_t* s) {
+  *s = nullptr;
+  {
+    IdlePool& p = idle_pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    if (p.alive(dev))
+      for (size_t k = 0; k < p.streams.size(); k++)
+        if (p.streams[k].first == dev) {
+          *s = p.streams[k].second;
+          p.streams.erase(p.streams.begin() + (long)k);
+          break;
+        }
+  }
+  return *s ? hipSuccess : hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+}
+/* waits for the stream's work first */
+inline void give_stream(int dev, hipStream_t s) {
+  if (!s) return;
+  if (hipStreamSynchronize(s) == hipSuccess) {
+    IdlePool& p = idle_pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    if (p.streams.size() < STREAMS_KEPT && p.mark(dev)) try {
+        p.streams.emplace_back(dev, s);
+        return;
+      } catch (const std::bad_alloc&) {
+      }
+  }
+  (void)hipStreamDestroy(s);
+}
 inline void* take_block(int dev, size_t bytes) {
-  BlockPool& p = block_pool();
+  IdlePool& p = idle_pool();
   std::lock_guard<std::mutex> lock(p.m);
-  for (size_t k = 0; k < p.idle.size(); k++)
-    if (p.idle[k].dev == dev && p.idle[k].bytes == bytes) {
-      void* const q = p.idle[k].p;
-      p.idle.erase(p.idle.begin() + (long)k);
+  if (!p.alive(dev)) return nullptr;
+  for (size_t k = 0; k < p.blocks.size(); k++)
+    if (p.blocks[k].dev == dev && p.blocks[k].bytes == bytes) {
+      void* const q = p.blocks[k].p;
+      p.blocks.erase(p.blocks.begin() + (long)k);
       p.bytes -= bytes;
       return q;
     }
@@ -106,11 +156,11 @@ inline void* take_block(int dev, size_t bytes) {
 }
 /* false: not kept */
 inline bool give_block(const Block& b) {
-  BlockPool& p = block_pool();
+  IdlePool& p = idle_pool();
   std::lock_guard<std::mutex> lock(p.m);
-  if (p.bytes + b.bytes > BLOCKS_KEPT) return false;
+  if (p.bytes + b.bytes > BLOCKS_KEPT || !p.mark(b.dev)) return false;
   try {
-    p.idle.push_back(b);
+    p.blocks.push_back(b);
   } catch (const std::bad_alloc&) {
     return false;
   }
@@ -118,11 +168,22 @@ inline bool give_block(const Block& b) {
   return true;
 }
 inline void drop_blocks() {
-  BlockPool& p = block_pool();
+  IdlePool& p = idle_pool();
   std::lock_guard<std::mutex> lock(p.m);
-  for (const Block& b : p.idle) (void)hipFree(b.p);
-  p.idle.clear();
-  p.bytes = 0;
+  p.free_blocks();
+}
+inline void drop_idle() {
+  IdlePool& p = idle_pool();
+  std::lock_guard<std::mutex> lock(p.m);
+  p.free_blocks();
+  while (!p.marks.empty()) {
+    const IdlePool::Mark k = p.marks.back();
+    if (!p.alive(k.dev)) continue; /* forgotten, the mark with it */
+    for (const auto& s : p.streams)
+      if (s.first == k.dev) (void)hipStreamDestroy(s.second);
+    (void)hipFree(k.p);
+    p.forget(k.dev);
+  }
 }
 
 /* Device memory of one owner: pieces of up to OWN bytes are cut from blocks of

@@ -2304,8 +2304,7 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
 }
 
 int kifmm_gpu_release_idle(void) {
-  drop_blocks();
-  drop_streams();
+  drop_idle();
   return KIFMM_OK;
 }
 

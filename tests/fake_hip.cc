@@ -148,6 +148,7 @@ void fake_reset() {
     for (auto& p : *m) F().dead.push_back(p.first);
     m->clear();
   }
+  for (auto& v : F().var_mem) F().pin[(char*)v.second] = {F().var_bytes[v.first], 0}; /* the program's own variables stay */
   F().used = 0;
   F().streams.clear();
   F().events.clear();

@@ -55,3 +55,35 @@ def test_idle_memory_and_streams_are_given_back(fake):
     K.release_idle()
     assert fake.fake_used() == 0 and fake.fake_streams() == 0 and fake.fake_events() == 0
     """)
+
+
+@pytest.mark.parametrize("then", ["K.GpuEvaluator(prob, operators=ops).close()", "build()", "K.release_idle()",
+                                  "fake.fake_limit(1 << 14); out_of_memory()"])
+def test_device_reset_between_owners(fake, then):
+    """hipDeviceReset with no handle alive destroys what is idle: a handle or a
+    tree build after it takes nothing of that, and nothing of it is freed
+    (runs on the fake runtime only, which lists each use of what is gone)."""
+    fake(f"""
+    prob = K.Problem.create(5000, "ellipsoid", 40, np_=4, seed=1)
+    ops = prob.operators()
+    def build():
+        K.Problem.create(5000, "ellipsoid", 40, np_=4, seed=1, device=0)
+    def out_of_memory():
+        try:
+            build()
+            assert False
+        except K.KifmmError:
+            pass
+    build()
+    K.GpuEvaluator(prob, operators=ops).close()
+    assert fake.fake_used() > 0 and fake.fake_streams() > 0
+    fake.fake_reset()
+    {then}
+    fake.fake_limit(1 << 40)
+    fake.hipGetLastError()
+    ev = K.GpuEvaluator(prob, operators=ops)
+    ev.evaluate()
+    ev.close()
+    K.release_idle()
+    assert fake.fake_used() == 0 and fake.fake_streams() == 0
+    """)
