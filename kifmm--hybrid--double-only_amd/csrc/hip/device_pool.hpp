@@ -256,6 +256,7 @@ class DeviceArena {
   static void* allocate(size_t bytes) {
     void* p = nullptr;
     if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError(); /* handled here: not for a later launch check to find */
     drop_blocks();
     if (hipMalloc(&p, bytes) == hipSuccess) return p;
     (void)hipGetLastError();

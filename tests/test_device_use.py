@@ -87,3 +87,24 @@ def test_device_reset_between_owners(fake, then):
     K.release_idle()
     assert fake.fake_used() == 0 and fake.fake_streams() == 0
     """)
+
+
+def test_allocation_that_needs_the_idle_memory_leaves_no_error(fake):
+    """An allocation that fails until the idle blocks are given back succeeds
+    as if it had at once: the runtime's error does not stay for a later launch
+    to find."""
+    fake("""
+    prob = K.Problem.create(60000, "uniform", 64, np_=4, seed=1)
+    ops = prob.operators()
+    ev = K.GpuEvaluator(prob, operators=ops)
+    room = fake.fake_used() + (1 << 20)
+    second = K.GpuEvaluator(prob, operators=ops)
+    ev.close()
+    second.close()
+    idle = fake.fake_used()  # of two handles: more than one takes
+    fake.fake_limit(room)
+    n0 = fake.fake_calls(b"hipFree")
+    ev = K.GpuEvaluator(prob, operators=ops)
+    assert fake.fake_calls(b"hipFree") > n0, (room, idle, fake.fake_used())  # idle blocks were given back
+    ev.evaluate()
+    """)
