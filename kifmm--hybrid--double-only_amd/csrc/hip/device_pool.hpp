@@ -186,6 +186,20 @@ inline void drop_idle() {
   }
 }
 
+/* hipMalloc, with the idle blocks given back if it needs their memory; what
+ * failed is returned and not left for a later launch check to find */
+inline hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < 2; k++) {
+    *p = nullptr;
+    if ((e = hipMalloc(p, bytes)) == hipSuccess) return e;
+    (void)hipGetLastError();
+    if (k == 0) drop_blocks();
+  }
+  *p = nullptr;
+  return e;
+}
+
 /* Device memory of one owner: pieces of up to OWN bytes are cut from blocks of
  * 8, 16, 32, then 64 MB, larger ones are allocations of their own.  No two
  * owners share a block at a time; a block changes hands only when its owner's
@@ -207,8 +221,8 @@ class DeviceArena {
     bytes = (std::max<size_t>(bytes, 1) + ALIGN - 1) / ALIGN * ALIGN;
     if (bytes > OWN) {
       own_.reserve(own_.size() + 1); /* a throw here loses nothing */
-      void* const p = allocate(bytes);
-      if (p) own_.push_back(p);
+      void* p;
+      if (device_malloc(&p, bytes) == hipSuccess) own_.push_back(p);
       return p;
     }
     if (bytes > left_) {
@@ -217,9 +231,8 @@ class DeviceArena {
       blocks_.reserve(blocks_.size() + 1);
       size_t size = next_;
       void* p = take_block(dev, size);
-      if (!p) p = allocate(size);
-      if (!p) p = allocate(size = bytes); /* the last of the memory */
-      if (!p) return nullptr;
+      if (!p && device_malloc(&p, size) != hipSuccess && device_malloc(&p, size = bytes) != hipSuccess)
+        return nullptr; /* (the second: the last of the memory) */
       blocks_.push_back({dev, p, size});
       at_ = (char*)p;
       left_ = size;
@@ -253,15 +266,6 @@ class DeviceArena {
   }
 
  private:
-  static void* allocate(size_t bytes) {
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError(); /* handled here: not for a later launch check to find */
-    drop_blocks();
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError();
-    return nullptr;
-  }
   hipStream_t st_;
   std::vector<void*> own_;
   std::vector<Block> blocks_;

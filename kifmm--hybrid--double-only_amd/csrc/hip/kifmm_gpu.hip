@@ -2368,9 +2368,9 @@ int kifmm_gpu_direct(kifmm_gpu* g, int nt, const double* tx, const double* ty, c
   }
   HIP_TRY(hipSetDevice(g->dev));
   const DirectPlan p = direct_plan(nt, g->n_src);
-  double* d = nullptr;
-  HIP_TRY(hipMalloc(&d, sizeof(double) * (4 * (size_t)nt + 2 * p.part())));
-  const int r = direct_run(g, p, nt, tx, ty, tz, out, d);
+  void* d = nullptr;
+  HIP_TRY(device_malloc(&d, sizeof(double) * (4 * (size_t)nt + 2 * p.part())));
+  const int r = direct_run(g, p, nt, tx, ty, tz, out, (double*)d);
   (void)hipFree(d);
   return r;
 }

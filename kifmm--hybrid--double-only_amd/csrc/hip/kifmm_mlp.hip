@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "kifmm_mlp.h"
+#include "device_pool.hpp"
 #include "../host/kifmm_internal.h"
 
 using kifmm::set_error;
@@ -148,7 +149,7 @@ int reserve(kifmm_mlp* h, int n) {
               {&h->a2, (long)c * D2}, {&h->h2, (long)c * D2}, {&h->y, (long)c * D3}, {&h->gy, (long)c * D3},
               {&h->g2, (long)c * D2}, {&h->g1, (long)c * D1}, {&h->rl, (long)c}};
   for (auto& w : want)
-    if (hipMalloc((void**)w.p, sizeof(float) * w.n) != hipSuccess) {
+    if (kifmm_dev::device_malloc((void**)w.p, sizeof(float) * w.n) != hipSuccess) {
       release(h);
       set_error("kifmm_mlp: device allocation failed");
       return KIFMM_ENOMEM;
@@ -231,7 +232,8 @@ int kifmm_mlp_create(int device, const float* params, kifmm_mlp** out) {
   }
   float** arrs[] = {&h->p, &h->g, &h->m, &h->v};
   for (float** a : arrs)
-    if (hipMalloc((void**)a, sizeof(float) * NPAR) != hipSuccess || hipMemset(*a, 0, sizeof(float) * NPAR) != hipSuccess) {
+    if (kifmm_dev::device_malloc((void**)a, sizeof(float) * NPAR) != hipSuccess ||
+        hipMemset(*a, 0, sizeof(float) * NPAR) != hipSuccess) {
       set_error("kifmm_mlp_create: device allocation failed");
       return fail(KIFMM_ENOMEM);
     }

@@ -108,3 +108,35 @@ def test_allocation_that_needs_the_idle_memory_leaves_no_error(fake):
     assert fake.fake_calls(b"hipFree") > n0, (room, idle, fake.fake_used())  # idle blocks were given back
     ev.evaluate()
     """)
+
+
+def test_every_allocation_can_have_the_idle_memory(fake):
+    """Direct sums and the cost model's network need device memory that only
+    the idle blocks hold: they get it."""
+    fake("""
+    prob = K.Problem.create(60000, "uniform", 64, np_=4, seed=1)
+    ops = prob.operators()
+    ev = K.GpuEvaluator(prob, operators=ops)
+    others = [K.GpuEvaluator(prob, operators=ops) for _ in range(2)]
+    t = np.zeros((3, 100000))
+    def leave_idle():
+        for e in others:
+            e.close()
+        fake.fake_limit(fake.fake_used())
+    leave_idle()
+    n0 = fake.fake_calls(b"hipFree")
+    ev.direct(*t)
+    assert fake.fake_calls(b"hipFree") > n0 + 1
+    ev.evaluate()
+    fake.fake_limit(1 << 40)
+    others = [K.GpuEvaluator(prob, operators=ops) for _ in range(2)]
+    leave_idle()
+    h, w = C.c_void_p(), (C.c_float * 8192)()
+    assert K.lib.kifmm_mlp_create(0, w, C.byref(h)) == 0, K.last_error()
+    fake.fake_limit(1 << 40)
+    others = [K.GpuEvaluator(prob, operators=ops) for _ in range(2)]
+    leave_idle()
+    n = 10000
+    assert K.lib.kifmm_mlp_predict(h, (C.c_float * (16 * n))(), n, (C.c_float * (4 * n))()) == 0, K.last_error()
+    assert K.lib.kifmm_mlp_destroy(h) == 0
+    """)
