@@ -2252,6 +2252,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
   if (hipHostMalloc((void**)&g->pinned, sizeof(double) * std::max(g->n_trg, 1), hipHostMallocDefault) != hipSuccess)
     g->pinned = nullptr;
   if (g->pinned && hipHostGetDevicePointer((void**)&g->pinned_dev, g->pinned, 0) != hipSuccess) g->pinned_dev = nullptr;
+  (void)hipGetLastError(); /* of either: done without, and not for the next launch check to find */
   if (hipDeviceSynchronize() != hipSuccess) {
     set_error("device synchronisation failed after upload");
     kifmm_gpu_destroy(g);

@@ -140,3 +140,23 @@ def test_every_allocation_can_have_the_idle_memory(fake):
     assert K.lib.kifmm_mlp_predict(h, (C.c_float * (16 * n))(), n, (C.c_float * (4 * n))()) == 0, K.last_error()
     assert K.lib.kifmm_mlp_destroy(h) == 0
     """)
+
+
+@pytest.mark.parametrize("what", ["hipHostMalloc", "hipHostGetDevicePointer"])
+@pytest.mark.parametrize("prec", ["K.PREC_FP64", "K.PREC_MIXED"])
+def test_no_pinned_memory_leaves_no_error(fake, what, prec):
+    """Without pinned memory, or its device address, a handle is created and
+    evaluates, takes densities and sums directly all the same: the runtime's
+    error is not left for the next launch check to find."""
+    fake(f"""
+    prob = K.Problem.create(3000, "ellipsoid", 20, np_=4, seed=1)
+    fail({what!r}, 0, 1 << 30, OUT_OF_MEMORY)
+    ev = K.GpuEvaluator(prob, precision={prec})
+    ev.evaluate()
+    assert (ev.output() is None) == ({what!r} == "hipHostMalloc")
+    ev.set_densities(prob.tree()["sden"])
+    ev.evaluate()
+    ev.direct(*np.zeros((3, 5)))
+    ev.close()
+    K.Problem.create(3000, "ellipsoid", 20, np_=4, seed=1, device=0)
+    """)
