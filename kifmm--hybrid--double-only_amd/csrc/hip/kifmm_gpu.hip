@@ -2031,8 +2031,8 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
   const bool host_pass = pot_leaf && g->pinned && pot_leaf != g->pinned;
   const bool pipelined = direct && host_pass && g->cuts.size() > 2; /* the host pass chunk by chunk */
   if (graph && !g->gexec[0]) {
-    g->capturing = true;
     HIP_TRY(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
+    g->capturing = true;
     const int r = enqueue_far(g, mask);
     hipGraph_t gr = nullptr;
     const hipError_t e = hipStreamEndCapture(g->stream, &gr);

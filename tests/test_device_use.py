@@ -160,3 +160,24 @@ def test_no_pinned_memory_leaves_no_error(fake, what, prec):
     ev.close()
     K.Problem.create(3000, "ellipsoid", 20, np_=4, seed=1, device=0)
     """)
+
+
+def test_capture_that_does_not_begin(fake):
+    """A graph handle whose capture cannot begin reports it, and is an eager
+    handle as before until a later capture succeeds: phase times included."""
+    fake("""
+    prob = K.Problem.create(3000, "ellipsoid", 20, np_=4, seed=1)
+    ev = K.GpuEvaluator(prob, graph=True)
+    fail("hipStreamBeginCapture")
+    try:
+        ev.evaluate()
+        assert False
+    except K.KifmmError as e:
+        assert e.code == -3, e
+    fake.hipGetLastError()
+    _, t = ev.evaluate_phases(K.PHASE_UP | K.PHASE_V)
+    assert t["up"] > 0 and t["v_hadamard"] > 0 and t["total"] >= t["up"] + t["vlist"]
+    log()
+    _, t = ev.evaluate()
+    assert any(ln.startswith("graph") for ln in log()) and t["ulist"] > 0
+    """)
