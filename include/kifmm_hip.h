@@ -71,8 +71,7 @@ enum {
 typedef struct kifmm_gpu_tuning {
   int p2p_form;      /* KIFMM_P2P_*: STATIC, PERSISTENT or STATIC64 on the FP64 path;
                         STATIC or SPLIT on the mixed path */
-  int hadamard_fb;   /* frequencies per V-list Hadamard block: 4, 8 (default) or 16; fewer
-                        where that many leave CUs without a block */
+  int hadamard_fb;   /* frequencies per V-list Hadamard block: 2, 4, 8 (default) or 16 */
   int hadamard_form; /* KIFMM_HAD_*: how the V-list Hadamard forms its products */
   int overlap;       /* stream layout of the U-list: 0 all of it last, after the far field;
                         1 all of it on the handle's second stream from the start, alongside
@@ -83,7 +82,9 @@ typedef struct kifmm_gpu_tuning {
                         stream instead of on the two streams in turn */
   int up_form;       /* KIFMM_LEVEL_*: how each level's M2M (UE2UC stack, then UC2UE) runs */
   int down_form;     /* KIFMM_LEVEL_*: how each level's L2L + DC2DE runs */
-  int reserved[2];
+  int hadamard_auto; /* 0: hadamard_fb exactly; 1 (initially): at most, fewer where that many
+                        leave CUs without a block (kifmm_work_counts.hadamard_block) */
+  int reserved[1];
 } kifmm_gpu_tuning;
 enum {
   KIFMM_LEVEL_AUTO = 0,  /* default: as FUSED, the faster form measured at every NP on
@@ -148,7 +149,8 @@ typedef struct kifmm_work_counts {
                           or too many) */
   double copy_chunks;  /* U-list chunks whose host passes into a caller buffer overlap the later chunks */
   double pair_items;   /* sibling-leaf pairs among the mixed U-list's work items */
-  double reserved[2];
+  double hadamard_block; /* frequencies per V-list Hadamard block as launched (kifmm_gpu_plan: 0) */
+  double reserved[1];
 } kifmm_work_counts;
 
 int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops,
@@ -239,7 +241,8 @@ int kifmm_gpu_get_tuning(const kifmm_gpu* g, kifmm_gpu_tuning* t);
  * and on the down phase, then the stream layouts on whole (eager)
  * evaluations with the copy back of this handle's own input, reps timed
  * runs each after one warm-up, keep the fastest of each (minimum over runs)
- * and set it.  best (may be NULL) receives the choice; ms (may be NULL, n_ms
+ * and set it (Hadamard blocks of 2 are tried, outside ms, where the handle
+ * would pick them by itself).  best (may be NULL) receives the choice; ms (may be NULL, n_ms
  * entries, up to 21) receives the times in the order STATIC, PERSISTENT,
  * STATIC64, VALU fb 4, 8, 16, MFMA fb 4, 8, 16, layout 0, layout 1, SPLIT,
  * layout 2, layout 3, up as column GEMMs, up fused, down as column GEMMs,

@@ -119,7 +119,7 @@ struct kifmm_gpu {
   /* launch shapes (kifmm_gpu_set_tuning / kifmm_gpu_autotune) */
   int mix_lpb = 1; /* leaves per block of the mixed S2M / L2T */
   int p2p_form = KIFMM_P2P_STATIC;
-  int had_fb = 8;
+  int had_fb = 8, had_auto = 1; /* kifmm_gpu_tuning.hadamard_fb, .hadamard_auto */
   int had_form = KIFMM_HAD_MFMA;
   int up_form = KIFMM_LEVEL_AUTO, down_form = KIFMM_LEVEL_AUTO;
   /* mixed path: per target, the U-list sources closer than MIX_CLOSE h */
@@ -1633,8 +1633,9 @@ int fill(kifmm_gpu* g, double* p, size_t n, double* q = nullptr, size_t m = 0) {
   return KIFMM_OK;
 }
 
-/* Frequencies per Hadamard block: had_fb, halved down to 4 while the launch has
- * fewer than two blocks per CU and to 2 below four.  A block runs its
+/* Frequencies per Hadamard block: had_fb as the caller set it; by default
+ * (had_auto) it is halved down to 4 while the launch has fewer than two blocks
+ * per CU and to 2 below four.  A block runs its
  * frequencies one after another: 4 thousand points NP 3 took 29 us in blocks
  * of 8, 17 of 4 and 12 of 2; 100 thousand NP 4 57 in 800 blocks of 4 and 53 in
  * 1600 of 2, 65 thousand mixed 44 and 41, 16 thousand NP 6 the same.  Above that
@@ -1643,7 +1644,7 @@ int fill(kifmm_gpu* g, double* p, size_t n, double* q = nullptr, size_t m = 0) {
  * the same. */
 int had_block_size(const kifmm_gpu* g) {
   int fb = g->had_fb;
-  while (fb > 2 && (long)g->n_hgroups * (g->F / fb) < (fb > 4 ? 512 : 1024)) fb /= 2;
+  while (g->had_auto && fb > 2 && (long)g->n_hgroups * (g->F / fb) < (fb > 4 ? 512 : 1024)) fb /= 2;
   return fb;
 }
 
@@ -2448,12 +2449,13 @@ int kifmm_gpu_set_tuning(kifmm_gpu* g, const kifmm_gpu_tuning* t) {
     return KIFMM_EINVAL;
   }
   if (t->p2p_form < KIFMM_P2P_STATIC || t->p2p_form > KIFMM_P2P_SPLIT ||
-      (t->hadamard_fb != 4 && t->hadamard_fb != 8 && t->hadamard_fb != 16) ||
+      (t->hadamard_fb != 2 && t->hadamard_fb != 4 && t->hadamard_fb != 8 && t->hadamard_fb != 16) ||
+      t->hadamard_auto < 0 || t->hadamard_auto > 1 ||
       (t->hadamard_form != KIFMM_HAD_VALU && t->hadamard_form != KIFMM_HAD_MFMA) ||
       t->overlap < 0 || t->overlap > 6 || t->up_form < KIFMM_LEVEL_AUTO || t->up_form > KIFMM_LEVEL_FUSED ||
       t->down_form < KIFMM_LEVEL_AUTO || t->down_form > KIFMM_LEVEL_FUSED) {
-    set_error("kifmm_gpu_set_tuning: p2p_form must be a KIFMM_P2P_* value, hadamard_fb 4, 8 or 16, "
-              "hadamard_form a KIFMM_HAD_* value, overlap 0 to 6 and up_form / down_form KIFMM_LEVEL_* "
+    set_error("kifmm_gpu_set_tuning: p2p_form must be a KIFMM_P2P_* value, hadamard_fb 2, 4, 8 or 16, "
+              "hadamard_auto 0 or 1, hadamard_form a KIFMM_HAD_* value, overlap 0 to 6 and up_form / down_form KIFMM_LEVEL_* "
               "values");
     return KIFMM_EINVAL;
   }
@@ -2467,11 +2469,13 @@ int kifmm_gpu_set_tuning(kifmm_gpu* g, const kifmm_gpu_tuning* t) {
     set_error("kifmm_gpu_set_tuning: the SPLIT U-list form is the mixed path's");
     return KIFMM_EUNSUP;
   }
-  if (t->p2p_form == g->p2p_form && t->hadamard_fb == g->had_fb && t->hadamard_form == g->had_form &&
+  if (t->p2p_form == g->p2p_form && t->hadamard_fb == g->had_fb && t->hadamard_auto == g->had_auto &&
+      t->hadamard_form == g->had_form &&
       t->overlap == g->overlap && t->up_form == g->up_form && t->down_form == g->down_form)
     return KIFMM_OK;
   g->p2p_form = t->p2p_form;
   g->had_fb = t->hadamard_fb;
+  g->had_auto = t->hadamard_auto;
   g->had_form = t->hadamard_form;
   g->overlap = t->overlap;
   g->up_form = t->up_form;
@@ -2493,6 +2497,7 @@ int kifmm_gpu_get_tuning(const kifmm_gpu* g, kifmm_gpu_tuning* t) {
   std::memset(t, 0, sizeof *t);
   t->p2p_form = g->p2p_form;
   t->hadamard_fb = g->had_fb;
+  t->hadamard_auto = g->had_auto;
   t->hadamard_form = g->had_form;
   t->overlap = g->overlap;
   t->up_form = g->up_form;
@@ -2546,8 +2551,13 @@ int kifmm_gpu_autotune(kifmm_gpu* g, int reps, kifmm_gpu_tuning* best, double* m
     }
   }
   c.p2p_form = best_form;
+  c.hadamard_fb = 8;
+  c.hadamard_auto = 1;
+  TRY(kifmm_gpu_set_tuning(g, &c));
+  const int own_fb = had_block_size(g);
   const int fbs[3] = {4, 8, 16};
   int best_v = 0;
+  c.hadamard_auto = 0;
   for (int k = 0; k < 6; k++) { /* VALU fb 4, 8, 16, then MFMA fb 4, 8, 16 */
     c.hadamard_form = k / 3;
     c.hadamard_fb = fbs[k % 3];
@@ -2555,8 +2565,21 @@ int kifmm_gpu_autotune(kifmm_gpu* g, int reps, kifmm_gpu_tuning* best, double* m
     TRY(time_phase(KIFMM_PHASE_V, &t[3 + k]));
     if (t[3 + k] < t[3 + best_v]) best_v = k;
   }
+  double t_v = t[3 + best_v];
   c.hadamard_form = best_v / 3;
   c.hadamard_fb = fbs[best_v % 3];
+  if (own_fb < fbs[0] && g->n_hgroups > 0) { /* where the handle picks fewer by itself, they are tried too */
+    kifmm_gpu_tuning f = c;
+    f.hadamard_fb = own_fb;
+    for (f.hadamard_form = 0; f.hadamard_form < 2; f.hadamard_form++) {
+      double t_f;
+      TRY(kifmm_gpu_set_tuning(g, &f));
+      TRY(time_phase(KIFMM_PHASE_V, &t_f));
+      if (t_f >= t_v) continue;
+      t_v = t_f;
+      c = f;
+    }
+  }
   /* up and down: the column GEMMs against the fused kernels, each phase on
    * its own (slots 14, 15: up; 16, 17: down) */
   for (int k = 0; k < 2; k++) {
@@ -2601,6 +2624,7 @@ int kifmm_gpu_work_counts(const kifmm_gpu* g, kifmm_work_counts* out) {
   *out = g->counts;
   out->close_pairs = g->close_listed ? (double)g->n_close : -1.0;
   out->copy_chunks = (double)std::max<size_t>(g->cuts.size(), 2) - 1.0;
+  out->hadamard_block = had_block_size(g);
   return KIFMM_OK;
 }
 

@@ -74,7 +74,8 @@ class GpuOptions(C.Structure):
 
 class GpuTuning(C.Structure):
     _fields_ = [("p2p_form", C.c_int), ("hadamard_fb", C.c_int), ("hadamard_form", C.c_int),
-                ("overlap", C.c_int), ("up_form", C.c_int), ("down_form", C.c_int), ("reserved", C.c_int * 2)]
+                ("overlap", C.c_int), ("up_form", C.c_int), ("down_form", C.c_int),
+                ("hadamard_auto", C.c_int), ("reserved", C.c_int * 1)]
 
 
 P2P_STATIC, P2P_PERSISTENT, P2P_STATIC64, P2P_SPLIT = 0, 1, 2, 3
@@ -93,8 +94,9 @@ class PhaseTimes(C.Structure):
 class WorkCounts(C.Structure):
     _fields_ = [(n, C.c_double) for n in (
         "u_pairs", "s2m_pairs", "l2t_pairs", "w_pairs", "x_pairs", "v_entries", "v_cmac", "v_cmac_ref",
-        "gemm_flops", "fft_bytes", "hadamard_bytes", "close_pairs", "copy_chunks", "pair_items")] + \
-        [("reserved", C.c_double * 2)]
+        "gemm_flops", "fft_bytes", "hadamard_bytes", "close_pairs", "copy_chunks", "pair_items",
+        "hadamard_block")] + \
+        [("reserved", C.c_double * 1)]
 
     def as_dict(self):
         return {n: getattr(self, n) for n, _ in self._fields_ if n != "reserved"}
@@ -460,15 +462,18 @@ class GpuEvaluator:
         return {"p2p_form": t.p2p_form, "hadamard_fb": t.hadamard_fb, "hadamard_form": t.hadamard_form,
                 "overlap": t.overlap, "up_form": t.up_form, "down_form": t.down_form}
 
-    def set_tuning(self, p2p_form=P2P_STATIC, hadamard_fb=8, hadamard_form=HAD_MFMA, overlap=None, up_form=None,
+    def set_tuning(self, p2p_form=P2P_STATIC, hadamard_fb=None, hadamard_form=HAD_MFMA, overlap=None, up_form=None,
                    down_form=None):
-        """overlap / up_form / down_form None keep the handle's current
+        """hadamard_fb None: 8, or fewer where that leaves CUs without a
+        block (work_counts()["hadamard_block"]); a number: exactly that.
+        overlap / up_form / down_form None keep the handle's current
         stream layout / level forms."""
         cur = self.tuning()
         overlap = cur["overlap"] if overlap is None else overlap
         up_form = cur["up_form"] if up_form is None else up_form
         down_form = cur["down_form"] if down_form is None else down_form
-        t = GpuTuning(p2p_form, hadamard_fb, hadamard_form, int(overlap), int(up_form), int(down_form))
+        t = GpuTuning(p2p_form, 8 if hadamard_fb is None else hadamard_fb, hadamard_form, int(overlap), int(up_form),
+                      int(down_form), int(hadamard_fb is None))
         _check(lib.kifmm_gpu_set_tuning(self._h, C.byref(t)))
 
     def autotune(self, reps=3):

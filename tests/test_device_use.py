@@ -181,3 +181,56 @@ def test_capture_that_does_not_begin(fake):
     _, t = ev.evaluate()
     assert any(ln.startswith("graph") for ln in log()) and t["ulist"] > 0
     """)
+
+
+@pytest.mark.parametrize("np_,prec", [(3, "K.PREC_FP64"), (4, "K.PREC_FP64"), (6, "K.PREC_FP64"),
+                                      (3, "K.PREC_MIXED"), (4, "K.PREC_MIXED")])
+def test_hadamard_block_size_that_was_set_is_launched(fake, np_, prec):
+    """A block size given to set_tuning is the launched kernel's, on an input
+    too small to fill the chip with it; without one the handle picks (2
+    here), and a C caller's round trip through get_tuning keeps that."""
+    fake(f"""
+    ev = K.GpuEvaluator(K.Problem.create(3000, "uniform", 20, np_={np_}, seed=1), precision={prec})
+    def launched():
+        log()
+        ev.evaluate()
+        names = [k[4] for k in kernels() if "k_hadamard" in k[4]]
+        assert len(names) == 1
+        return int(names[0].split(">(")[0].split(",")[-1])
+    def auto():
+        t = K.GpuTuning()
+        K._check(K.lib.kifmm_gpu_get_tuning(ev._h, C.byref(t)))
+        return t, (t.hadamard_fb, t.hadamard_auto)
+    assert launched() == ev.work_counts()["hadamard_block"] == 2 and auto()[1] == (8, 1)
+    for form in (K.HAD_VALU, K.HAD_MFMA):
+        for fb in (2, 4, 8, 16):
+            ev.set_tuning(K.P2P_STATIC, fb, form)
+            assert launched() == ev.work_counts()["hadamard_block"] == fb == ev.tuning()["hadamard_fb"], (form, fb)
+            assert auto()[1] == (fb, 0)
+    ev.set_tuning(overlap=4)
+    t, a = auto()
+    assert launched() == 2 and a == (8, 1)
+    t.overlap = 0
+    K._check(K.lib.kifmm_gpu_set_tuning(ev._h, C.byref(t)))
+    assert launched() == 2 and auto()[1] == (8, 1)
+    for bad in (K.GpuTuning(0, 8, 1, 0, 0, 0, 2), K.GpuTuning(0, 8, 1, 0, 0, 0, -1), K.GpuTuning(0, 3, 1), K.GpuTuning(0, 1, 1)):
+        assert K.lib.kifmm_gpu_set_tuning(ev._h, C.byref(bad)) == -1
+    # the autotuner times 2 where the handle would pick it by itself
+    fake.fake_kernel_ms(b"k_hadamard", 5.0)
+    fake.fake_kernel_ms(b"k_hadamard_{"mfma" if "MIXED" in prec else "fact"}<{np_}, 2>", 0.5)
+    best, ms = ev.autotune(reps=1)
+    assert (best["hadamard_fb"], best["hadamard_form"]) == (2, K.HAD_MFMA) and launched() == 2 and np.all(ms[3:9] == 5.0)
+    """)
+
+
+def test_hadamard_block_size_on_inputs_that_fill_the_chip(fake):
+    """... where the handle picks 8, and the autotuner chooses from 4, 8, 16."""
+    fake("""
+    ev = K.GpuEvaluator(K.Problem.create(300000, "uniform", 8, np_=4, seed=1))
+    assert ev.work_counts()["hadamard_block"] == 8
+    fake.fake_kernel_ms(b"k_hadamard", 5.0)
+    fake.fake_kernel_ms(b"k_hadamard_fact<4, 2>", 0.5)
+    fake.fake_kernel_ms(b"k_hadamard_fact<4, 16>", 4.0)
+    best, ms = ev.autotune(reps=1)
+    assert best["hadamard_fb"] == 16 == ev.work_counts()["hadamard_block"]
+    """)

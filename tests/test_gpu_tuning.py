@@ -209,3 +209,25 @@ def test_hadamard_groups_and_forms(n, q, np_, kind):
     r = rel(first, ref)
     print(f"  {kind} n={n} q={q} NP={np_}: {r:.2e}", flush=True)
     assert r <= O.PARITY_RTOL[np_]
+
+
+@pytest.mark.parametrize("n,dist,q,np_,prec", [(400, "gaussmix", 2, 3, K.PREC_FP64), (60000, "uniform", 64, 4, K.PREC_FP64),
+                                               (20000, "ellipsoid", 16, 6, K.PREC_FP64),
+                                               (3000, "ellipsoid", 8, 3, K.PREC_MIXED),
+                                               (40000, "uniform", 64, 4, K.PREC_MIXED)])
+def test_every_block_size_runs_and_gives_the_same_bits(n, dist, q, np_, prec):
+    """Hadamard blocks of 2, 4, 8 and 16 frequencies as set, on inputs where
+    the handle picks 2 by itself and, at NP 6, 8: the same potentials bit for
+    bit within a form."""
+    print(f"case n={n} dist={dist} q={q} NP={np_} prec={prec}", flush=True)
+    ev = K.GpuEvaluator(K.Problem.create(n, dist, q, np_=np_, seed=11), precision=prec)
+    assert ev.work_counts()["hadamard_block"] == (8 if np_ == 6 else 2)
+    own, _ = ev.evaluate()
+    for form in (K.HAD_VALU, K.HAD_MFMA):
+        ref = own if form == K.HAD_MFMA else None
+        for fb in (2, 4, 8, 16):
+            ev.set_tuning(K.P2P_STATIC, fb, form)
+            assert ev.work_counts()["hadamard_block"] == fb
+            got, _ = ev.evaluate()
+            ref = got if ref is None else ref
+            assert np.all(np.isfinite(got)) and np.array_equal(got, ref), (form, fb)
