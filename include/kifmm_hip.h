@@ -120,7 +120,9 @@ typedef struct kifmm_phase_times {
                        create time, so ~0 here               */
   double v_hadamard;/* spectral multiply-accumulate       */
   double v_ifft;    /* inverse DFT + check-surface gather */
-  double wlist;     /* W and X run in one launch, whose time is split by their pair counts */
+  double wlist;     /* W and X run in one launch, whose time is split by what their work
+                       items cost (kifmm_gpu_evaluate_phases with one of them times it
+                       alone); the mixed path's X sums onto check surfaces are timed */
   double xlist;
   double down;      /* L2L + DC2DE + L2T                  */
   double copy;      /* device -> host potentials: the part left after the last

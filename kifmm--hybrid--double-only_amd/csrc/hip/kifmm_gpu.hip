@@ -144,6 +144,7 @@ struct kifmm_gpu {
   int4* xs_red = nullptr; int n_xsred = 0;  /* and the reductions of split ones */
   double* wxpart = nullptr;                 /* chunk sums, WX_T per slot (k_x_surf: 64) */
   bool wx_targets = false;                  /* some item's points are targets */
+  double wx_cost[2] = {0.0, 0.0};           /* of the W and of the X items (wx_plan) */
   int4* l2t_items = nullptr; int n_l2t = 0;
   size_t chk_cols = 0;
   double* ws = nullptr;
@@ -375,6 +376,7 @@ struct Plan {
   std::vector<int2> wx_rng;
   int wx_slots = 0, xs_slots = 0;
   bool wx_targets = false; /* some W / X item's points are targets */
+  double wx_cost[2] = {0.0, 0.0};
   std::vector<int4> l2t_items;
   std::vector<int4> hgroups;
   std::vector<int> huslots;
@@ -549,7 +551,12 @@ std::vector<int4> u_launch_order(const std::vector<int4>& items, const std::vect
  * Chunks hold WX_CAP sources on inputs with plenty of work; below, as many
  * as leave about WX_ITEMS items (16 waves on each of 256 CUs), at least 128:
  * a 4 thousand point input has 33 W blocks, and walking 1024 sources each
- * took 82 us on an otherwise idle chip.  Items run largest first.  On the
+ * took 82 us on an otherwise idle chip.  Items run largest first.
+ * wx_cost, which splits the launch's time between the lists: in passes of 64
+ * sources over 8 points (96 issue slots, twice that on differences), 0.4 for
+ * the conversion of 64 sources and 1 for the rest of an item.  W's share by
+ * that, and of the two lists run alone: 0.476 and 0.474 at 1M ellipsoid points
+ * NP 4, 0.474 and 0.51 at 300 thousand NP 6 (by pairs alone 0.512 and 0.51).  On the
  * mixed path the X sums onto check surfaces are k_x_surf's: blocks of 64
  * points, chunks of XS_CHUNK sources cut at entry boundaries. */
 int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
@@ -696,10 +703,13 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
       }
       for (int p = 0, m = 0; p < npts; p += WX_T, m++) {
         const int cnt = std::min(WX_T, npts - p), slot0 = P.wx_slots;
-        for (const Chunk& c : chunks)
-          work.push_back({((c.n + 63) / 64) * ((cnt + 7) / 8),
+        for (const Chunk& c : chunks) {
+          const int steps = (c.n + 63) / 64, groups = (cnt + 7) / 8;
+          P.wx_cost[xl] += 1.0 + steps * (0.4 + groups * (c.flags & WX_DIFF ? 2.0 : 1.0));
+          work.push_back({steps * groups,
                           make_int4(c.rb, c.re, surf ? p : t->trg_beg[i] + p, cnt),
                           make_int4(i, P.wx_slots++, c.flags | (surf ? WX_SURF : 0) | (xl ? WX_X : WX_W), c.n)});
+        }
         const int nch = P.wx_slots - slot0;
         if (join) {
           int4& b = P.wx_red[wred_at + 2 * m + 1];
@@ -1365,6 +1375,7 @@ int build(kifmm_gpu* g, const kifmm_tree_view* t, const kifmm_operators* ops, co
   g->n_wx = (int)P.wx_items.size() / 2;
   g->n_wxred = (int)P.wx_red.size() / 2;
   g->wx_targets = P.wx_targets;
+  for (int xl = 0; xl < 2; xl++) g->wx_cost[xl] = P.wx_cost[xl];
   g->n_xs = (int)P.xs_items.size() / 2;
   g->n_xsred = (int)P.xs_red.size() / 2;
   g->n_l2t = (int)P.l2t_items.size();
@@ -1499,7 +1510,7 @@ int gram_setup(kifmm_gpu* g) {
  * the last one: an event recorded between two kernels costs a marker packet
  * and its drain, 2.4 us each, a stop event nothing measurable (ten 15 us kernels: 184
  * us with an event recorded after each, 158 with stop events, 160 without). */
-enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_WX, E_DOWN, E_U, E_END };
+enum { E_START = 0, E_UP, E_FFT, E_TRANS, E_HAD, E_IFFT, E_WX, E_XSURF, E_DOWN, E_U, E_END };
 enum { PHASE_EMPTY, PHASE_STAMPED, PHASE_UNSTAMPED }; /* kifmm_gpu::phase_state */
 
 /* one launch on st; start and stop (stop, or both, may be null) take its start and end */
@@ -1824,6 +1835,7 @@ int wx_phase(kifmm_gpu* g, unsigned mask) {
                        g->wxpart, g->pot, g->dchk);
     LAUNCH_CHECK();
   }
+  TRY(phase_end(g, E_WX));
   if ((lists & WX_X) && g->n_xs > 0) {
     launch(g, k_x_surf, dim3(g->n_xs), dim3(64), g->xs_items, g->wx_rng, g->geo, g->surf_dc,
                        g->ld_surf, g->src4, g->dchk, g->ld_e, g->wxpart);
@@ -1833,7 +1845,7 @@ int wx_phase(kifmm_gpu* g, unsigned mask) {
                          g->dchk);
     LAUNCH_CHECK();
   }
-  return KIFMM_OK;
+  return phase_end(g, E_XSURF);
 }
 
 /* One evaluation is three launch sequences on the handle's streams:
@@ -1930,7 +1942,6 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
   TRY(phase_end(g, E_IFFT));
   /* W and X */
   TRY(wx_phase(g, mask));
-  TRY(phase_end(g, E_WX));
   /* down: DC2DE at depth 2, then per level the fused L2L + DC2DE
    * (k_l2l_dc2de over the parents at depth d - 1), then L2T */
   for (int d = 2; d <= g->max_depth && (mask & KIFMM_PHASE_DOWN); d++) {
@@ -2102,10 +2113,10 @@ int evaluate(kifmm_gpu* g, unsigned mask, double* pot_leaf, kifmm_phase_times* t
       times->v_hadamard = ms[E_HAD];
       times->v_ifft = ms[E_IFFT];
       times->vlist = ms[E_FFT] + ms[E_TRANS] + ms[E_HAD] + ms[E_IFFT];
-      /* one launch: its time split by the lists' pairs */
-      const double w = mask & KIFMM_PHASE_W ? g->counts.w_pairs : 0.0, x = mask & KIFMM_PHASE_X ? g->counts.x_pairs : 0.0;
-      times->wlist = w + x > 0.0 ? ms[E_WX] * w / (w + x) : ms[E_WX];
-      times->xlist = ms[E_WX] - times->wlist;
+      /* k_wx is one launch, its time split by what the lists' items cost; k_x_surf is X alone */
+      const double w = mask & KIFMM_PHASE_W ? g->wx_cost[0] : 0.0, x = mask & KIFMM_PHASE_X ? g->wx_cost[1] : 0.0;
+      times->wlist = w > 0.0 ? ms[E_WX] * (w / (w + x)) : 0.0;
+      times->xlist = ms[E_WX] - times->wlist + ms[E_XSURF];
       times->down = ms[E_DOWN];
     }
     /* the U-list: its chunks after the far field, plus the span of the

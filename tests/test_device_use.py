@@ -234,3 +234,25 @@ def test_hadamard_block_size_on_inputs_that_fill_the_chip(fake):
     best, ms = ev.autotune(reps=1)
     assert best["hadamard_fb"] == 16 == ev.work_counts()["hadamard_block"]
     """)
+
+
+def test_x_sums_of_their_own_launch_are_xlist_time(fake):
+    """Mixed path: the time of the X sums onto check surfaces, launches of
+    their own, is X's, not shared out to W; one list alone has all of its time."""
+    fake("""
+    for n, d in (b"k_wx(", 4.0), (b"k_wx_reduce(", 2.0), (b"k_x_surf(", 1000.0), (b"k_x_surf_reduce(", 500.0):
+        fake.fake_kernel_ms(n, d)
+    prob = K.Problem.create(20000, "gaussmix", 100, np_=4, seed=1)
+    ev = K.GpuEvaluator(prob, precision=K.PREC_MIXED)
+    log()
+    _, t = ev.evaluate()
+    names = " ".join(k[4] for k in kernels())
+    surf = 1000.0 + (500.0 if "k_x_surf_reduce" in names else 0.0)
+    assert "k_x_surf(" in names and "k_wx(" in names
+    assert surf <= t["xlist"] <= surf + 6.0 and 0.0 < t["wlist"] < 6.0, t
+    assert t["wlist"] + t["xlist"] == surf + 6.0
+    _, t = ev.evaluate_phases(K.PHASE_UP | K.PHASE_W)
+    assert (t["wlist"], t["xlist"]) == (6.0, 0.0)
+    _, t = ev.evaluate_phases(K.PHASE_UP | K.PHASE_X)
+    assert (t["wlist"], t["xlist"]) == (0.0, surf + 6.0)
+    """)
