@@ -12,8 +12,9 @@
  *
  * All entry points return 0 on success or a negative KIFMM_E* code, never
  * exit.  A handle is not thread-safe; several handles may coexist.  Each
- * handle owns two HIP streams at default priority on its device: the main
- * one and a second compute stream.
+ * handle owns two HIP streams at default priority on its device, the main
+ * one and a second compute stream, and a third for copies once it has run a
+ * stream layout with large early U-list chunks and later ones.
  */
 #ifndef KIFMM_HIP_H
 #define KIFMM_HIP_H

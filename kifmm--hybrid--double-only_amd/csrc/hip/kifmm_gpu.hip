@@ -174,6 +174,8 @@ struct kifmm_gpu {
   bool tiled = false;
   std::vector<hipEvent_t> cd_ev;
   hipEvent_t far_ev = nullptr, sdone_ev = nullptr;
+  hipStream_t cstream = nullptr; /* copies of early chunks; taken by the first evaluation with some */
+  hipEvent_t copied_ev = nullptr;
   /* the U-list's own sums when it runs on the second stream (overlap layout) */
   double* potU = nullptr;
   /* staging of kifmm_gpu_set_densities */
@@ -1972,16 +1974,36 @@ int enqueue_far(kifmm_gpu* g, unsigned mask) {
 
 int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
   const int nch = (int)g->cuts.size() - 1, e = early_chunks(g, mask);
+  /* The early chunks' potentials go to the host from the join itself, or from
+   * EARLY_COPY targets on, with others to come, by copies on a stream of their
+   * own beside those: the join would hold the main stream for as long as PCIe
+   * takes.  Two chunks early, join -> copies, into the handle's and a caller's
+   * buffer: 2.96 -> 2.63 and 3.15 -> 2.90 ms at 4M points mixed (2.3M targets
+   * early), 8.05 -> 7.73 and 8.20 -> 7.89 at 4M NP 6; but 1.55 -> 1.53 and 1.72 ->
+   * 1.76 at 1M ellipsoid (0.6M), 1.13 -> 1.16 and 1.20 -> 1.20 at 300 thousand. */
+  constexpr int EARLY_COPY = 1 << 20;
+  const bool early_copy = e > 0 && e < nch && host && g->cuts[e] >= EARLY_COPY;
   if (e > 0) { /* the early chunks: join */
     g->phase_state = PHASE_UNSTAMPED;
     const int m = g->cuts[e];
     HIP_TRY(hipStreamWaitEvent(g->stream, g->join_ev, 0));
     const int blocks = std::min(4096, (m + 255) / 256);
     if (m > 0)
-      hipLaunchKernelGGL(k_join_pot, dim3(std::max(blocks, 1)), dim3(256), 0, g->stream, g->pot, host, g->potU, m);
+      hipLaunchKernelGGL(k_join_pot, dim3(std::max(blocks, 1)), dim3(256), 0, g->stream, g->pot,
+                         early_copy ? nullptr : host, g->potU, m);
     LAUNCH_CHECK();
-    if (chunked)
-      for (int c = 0; c < e; c++) HIP_TRY(hipEventRecord(g->cd_ev[c], g->stream));
+    if (early_copy) {
+      if (!g->cstream) HIP_TRY(take_stream(g->dev, &g->cstream));
+      HIP_TRY(hipEventRecord(g->far_ev, g->stream));
+      HIP_TRY(hipStreamWaitEvent(g->cstream, g->far_ev, 0));
+    }
+    for (int c = 0; c < e && (early_copy || chunked); c++) {
+      const int b = g->cuts[c], n = g->cuts[c + 1] - b;
+      if (early_copy && n > 0)
+        HIP_TRY(hipMemcpyAsync(g->pinned + b, g->pot + b, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, g->cstream));
+      if (chunked) HIP_TRY(hipEventRecord(g->cd_ev[c], early_copy ? g->cstream : g->stream));
+    }
+    if (early_copy) HIP_TRY(hipEventRecord(g->copied_ev, g->cstream));
   }
   if ((mask & KIFMM_PHASE_U) && e < nch) { /* the other chunks after the far field */
     const int late = chunked ? nch - e : 1;
@@ -2006,7 +2028,9 @@ int enqueue_near(kifmm_gpu* g, unsigned mask, double* host, bool chunked) {
       HIP_TRY(hipStreamWaitEvent(g->stream, g->sdone_ev, 0));
     }
   }
-  return phase_end(g, E_U);
+  TRY(phase_end(g, E_U));
+  if (early_copy) HIP_TRY(hipStreamWaitEvent(g->stream, g->copied_ev, 0));
+  return KIFMM_OK;
 }
 
 /* pinned potentials -> the caller's buffer, a few host threads */
@@ -2214,6 +2238,7 @@ int kifmm_gpu_create(const kifmm_tree_view* tree, const kifmm_operators* ops, co
       hipEventCreateWithFlags(&g->join_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->far_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&g->sdone_ev, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&g->copied_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&g->su0) != hipSuccess || hipEventCreate(&g->su1) != hipSuccess) {
     set_error("kifmm_gpu_create: second stream or its events could not be created");
     kifmm_gpu_destroy(g);
@@ -2295,7 +2320,7 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   if (!g) return KIFMM_OK;
   (void)hipSetDevice(g->dev);
   bool ended = true;
-  for (hipStream_t s : {g->stream, g->side})
+  for (hipStream_t s : {g->stream, g->side, g->cstream})
     if (s && hipStreamSynchronize(s) != hipSuccess) ended = false;
   if (g->pinned) (void)hipHostFree(g->pinned);
   if (g->den_pin) (void)hipHostFree(g->den_pin);
@@ -2306,12 +2331,11 @@ int kifmm_gpu_destroy(kifmm_gpu* g) {
   g->mem.free(ended);
   for (auto& e : g->ev)
     if (e) (void)hipEventDestroy(e);
-  for (hipEvent_t e : {g->fork_ev, g->join_ev, g->su0, g->su1, g->far_ev, g->sdone_ev})
+  for (hipEvent_t e : {g->fork_ev, g->join_ev, g->su0, g->su1, g->far_ev, g->sdone_ev, g->copied_ev})
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : g->cd_ev)
     if (e) (void)hipEventDestroy(e);
-  give_stream(g->dev, g->side);
-  give_stream(g->dev, g->stream);
+  for (hipStream_t s : {g->cstream, g->side, g->stream}) give_stream(g->dev, s);
   delete g;
   return KIFMM_OK;
 }

@@ -28,7 +28,11 @@ struct Fake {
   };
   std::map<char*, Mem> dev, pin;                /* live allocations */
   std::vector<void*> dead;                      /* freed ones, kept mapped so that a stray access is a fault entry, not a crash */
-  std::map<hipStream_t, bool> streams;          /* live; capturing */
+  struct Stream {
+    int id;
+    bool capturing;
+  };
+  std::map<hipStream_t, Stream> streams;        /* live ones */
   std::map<hipEvent_t, double> events;          /* live; time recorded, < 0: none */
   std::map<const void*, std::string> kernels, vars;
   std::map<const void*, size_t> var_bytes;
@@ -45,6 +49,7 @@ struct Fake {
   double clock = 0.0;
   size_t limit = (size_t)1 << 40, used = 0;
   unsigned next_id = 1;
+  int next_stream = 0;
   struct {
     dim3 grid, block;
     size_t shmem;
@@ -91,7 +96,7 @@ bool stream_ok(hipStream_t s, const char* fn) {
   F().faults += std::string(fn) + " on a stream that is not live\n";
   return false;
 }
-std::string id(hipStream_t s) { return s ? std::to_string((long)(std::distance(F().streams.begin(), F().streams.find(s)))) : "null"; }
+std::string id(hipStream_t s) { return s ? std::to_string(F().streams[s].id) : "null"; }
 hipError_t alloc(std::map<char*, Fake::Mem>& m, void** p, size_t n) {
   char* const q = (char*)std::calloc(1, n ? n : 1);
   if (!q) return done(hipErrorOutOfMemory);
@@ -253,7 +258,7 @@ hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t s) {
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   ENTER("hipStreamCreate");
   *s = (hipStream_t)std::malloc(16);
-  F().streams[*s] = false;
+  F().streams[*s] = {F().next_stream++, false};
   return hipSuccess;
 }
 hipError_t hipStreamCreate(hipStream_t* s) { return hipStreamCreateWithFlags(s, 0); }
@@ -275,13 +280,13 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   ENTER("hipStreamBeginCapture");
   if (!stream_ok(s, "hipStreamBeginCapture")) return hipErrorInvalidValue;
-  F().streams[s] = true;
+  F().streams[s].capturing = true;
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
   ENTER("hipStreamEndCapture");
-  if (!F().streams.count(s) || !F().streams[s]) return fault("hipStreamEndCapture of a stream that does not capture");
-  F().streams[s] = false;
+  if (!F().streams.count(s) || !F().streams[s].capturing) return fault("hipStreamEndCapture of a stream that does not capture");
+  F().streams[s].capturing = false;
   *g = (hipGraph_t)std::malloc(16);
   return hipSuccess;
 }

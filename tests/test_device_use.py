@@ -256,3 +256,37 @@ def test_x_sums_of_their_own_launch_are_xlist_time(fake):
     _, t = ev.evaluate_phases(K.PHASE_UP | K.PHASE_X)
     assert (t["wlist"], t["xlist"]) == (0.0, surf + 6.0)
     """)
+
+
+@pytest.mark.parametrize("prec", ["K.PREC_FP64", "K.PREC_MIXED"])
+def test_large_early_chunks_are_copied_beside_the_later_ones(fake, prec):
+    """Stream layouts with some U-list chunks early, a million targets or more
+    of them: their potentials go to the host on a stream that runs no U-list,
+    so that the later chunks do not wait for PCIe; whole and once, whatever
+    buffer the caller gave.  Fewer: the join writes them, and no copy is made."""
+    fake(f"""
+    for n, large in ((3600000, (2, 3, 5, 6)), (2200000, (3, 6)), (280000, ())):
+        prob = K.Problem.create(n, "uniform", 512, np_=3, seed=1)
+        ev = K.GpuEvaluator(prob, precision={prec})
+        own = np.zeros(ev.n_trg)
+        for layout in range(7):
+            ev.set_tuning(overlap=layout)
+            for into in (False, True):
+                log()
+                ev.evaluate_into(own) if into else ev.evaluate(copy="view")
+                lines = log()
+                copies = [ln.split() for ln in lines if ln.startswith("copy")]
+                if layout not in large:
+                    assert not copies, (layout, copies)
+                    continue
+                early = sum(int(c[3]) for c in copies)
+                assert len(copies) == (1 if layout in (2, 5) else 2) and all(c[2] == "d2h" for c in copies), copies
+                assert 8 << 20 <= early < 8 * ev.n_trg
+                u = [ln.split()[1] for ln in lines if "k_p2p" in ln or "k_join_pot" in ln]
+                assert len(u) >= 3 and all(c[1] not in u for c in copies), (u, copies)
+                at = [ln for ln in lines if "k_join_pot" in ln or " d2h " in ln or "k_p2p" in ln]
+                assert "k_join_pot" in at[1] and all(" d2h " in ln for ln in at[2 : 2 + len(copies)])  # before the later chunks
+        ev.close()
+    K.release_idle()
+    assert fake.fake_streams() == 0 and fake.fake_events() == 0
+    """)

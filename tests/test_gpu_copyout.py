@@ -169,3 +169,26 @@ def test_close_list_is_the_brute_force_list(n, dist, q, c):
     ms = ev.create_times()
     print(f"  {checked} close pairs; create ms {ms}", flush=True)
     assert all(v >= 0 for v in ms.values()) and ms["total"] >= ms["close_pairs"]
+
+
+@pytest.mark.parametrize("n,prec", [(3600000, K.PREC_MIXED), (2200000, K.PREC_FP64)], ids=["mixed", "fp64"])
+def test_large_early_chunks(n, prec):
+    """Early U-list chunks of a million targets and more, copied beside the
+    later ones: the device's potentials, in either buffer, whatever was there
+    before, and the same in every layout."""
+    prob = K.Problem.create(n, "uniform", 512, np_=3, seed=13, device=0)
+    ev = K.GpuEvaluator(prob, precision=prec)
+    ev.evaluate(copy=False)
+    dev = ev.intermediate("pot")
+    own = np.empty(ev.n_trg)
+    for ov in (0, 2, 3, 5, 6, 1):
+        print(f"case n={n} layout {ov}", flush=True)
+        ev.set_tuning(overlap=ov)
+        for _ in range(2):
+            ev.output()[:] = np.nan
+            view, _ = ev.evaluate(copy="view")
+            assert np.array_equal(view, dev), ov
+            own[:] = np.nan
+            ev.output()[:] = np.nan
+            ev.evaluate_into(own)
+            assert np.array_equal(own, dev), ov
