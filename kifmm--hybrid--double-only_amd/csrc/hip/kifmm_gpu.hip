@@ -2667,10 +2667,13 @@ double* kifmm_gpu_output(kifmm_gpu* g) { return g ? g->pinned : nullptr; }
 
 /* Densities of up to DEN_PINNED bytes are copied to pinned memory that the
  * packing kernel reads, and not waited for (the evaluation follows on the same
- * stream): this call with 16 thousand points 31 -> 7 us, 131 thousand 75 -> 30,
- * 1M 272 -> 134, 2M 625 -> 240.  The line is where pinning a second copy of
- * the densities gets large; above, the runtime's copy, waited for. */
-constexpr size_t DEN_PINNED = (size_t)16 << 20;
+ * stream); above, the runtime's copy, waited for.  The line is where the two
+ * routes meet, by the time of this call and an evaluation (the call alone
+ * returns sooner up to 2M points, but one thread fills the pinned memory and
+ * the evaluation waits for the kernel to read it): runtime's copy -> pinned at
+ * 131 thousand points 530 -> 493 us, 500 thousand 958 -> 940, 700 thousand 1493 ->
+ * 1488, 1M 2643 -> 2642, but 1.4M 4770 -> 4915, 2M 8373 -> 8636, 4M 7134 -> 7647. */
+constexpr size_t DEN_PINNED = (size_t)8 << 20;
 
 int kifmm_gpu_set_densities(kifmm_gpu* g, const double* den_leaf) {
   if (!g || (!den_leaf && g->n_src > 0)) {

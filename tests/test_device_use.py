@@ -290,3 +290,20 @@ def test_large_early_chunks_are_copied_beside_the_later_ones(fake, prec):
     K.release_idle()
     assert fake.fake_streams() == 0 and fake.fake_events() == 0
     """)
+
+
+@pytest.mark.parametrize("n,pinned", [(1000, True), (1 << 20, True), ((1 << 20) + 1, False), (2000000, False)])
+def test_route_of_new_densities(fake, n, pinned):
+    """Up to a million sources the packing kernel reads pinned memory; beyond,
+    the runtime's copy, waited for: there the pinned route is the slower one."""
+    fake(f"""
+    prob = K.Problem.create({n}, "uniform", 512, np_=3, seed=1, coincide=1)
+    ev = K.GpuEvaluator(prob)
+    den = np.zeros({n})
+    ev.set_densities(den)
+    log()
+    ev.set_densities(den)
+    lines = log()
+    assert sum("k_set_w" in ln for ln in lines) == 1
+    assert [ln.split()[2:] for ln in lines if ln.startswith("copy")] == ([] if {pinned} else [["h2d", "{8 * n}"]]), lines
+    """)
