@@ -188,7 +188,10 @@ double* kifmm_gpu_output(kifmm_gpu* g);
  * densities (in the reference a new AllNodes and preproc).  Everything
  * create derives ahead of time (lists, close pairs, Gram records,
  * translation spectra) depends on the points only; evaluations read the
- * densities afresh.  Blocks until the upload is done. */
+ * densities afresh.  den_leaf may be reused or released on return.  Up to a
+ * million sources the transfer may still run then: it comes before the work of
+ * every later call on the handle, and such a call (or destroy) waits for it and
+ * reports its errors.  Above, the call blocks until it is done. */
 int kifmm_gpu_set_densities(kifmm_gpu* g, const double* den_leaf);
 
 /* Wall milliseconds of the handle's kifmm_gpu_create: [0] the host plan

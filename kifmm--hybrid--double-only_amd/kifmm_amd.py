@@ -425,7 +425,9 @@ class GpuEvaluator:
         return out
 
     def set_densities(self, den_leaf):
-        """New source densities in gathered source order (kifmm_gpu_set_densities)."""
+        """New source densities in gathered source order (kifmm_gpu_set_densities).
+        The array may be reused at once; up to a million sources the transfer
+        itself may end, and its errors show, in the next call."""
         den = np.ascontiguousarray(den_leaf, dtype=np.float64)
         assert den.size == self._view.n_src
         _check(lib.kifmm_gpu_set_densities(self._h, _dptr(den)))

@@ -192,3 +192,29 @@ def test_large_early_chunks(n, prec):
             ev.output()[:] = np.nan
             ev.evaluate_into(own)
             assert np.array_equal(own, dev), ov
+
+
+@pytest.mark.parametrize("prec", [K.PREC_FP64, K.PREC_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("n", [20000, 1 << 20, (1 << 20) + 1, 1500000])
+def test_densities_array_may_be_reused_at_once(n, prec):
+    """On both sides of the line between the two transfers (a million
+    sources): the caller's array overwritten right after the call, a second
+    call before any evaluation, direct sums as the next call."""
+    print(f"case n={n} prec={prec}", flush=True)
+    prob = K.Problem.create(n, "uniform", 512, np_=3, seed=15, coincide=1, device=0)
+    den = prob.tree()["sden"]
+    ev = K.GpuEvaluator(prob, precision=prec)
+    first, _ = ev.evaluate()
+    t = np.random.default_rng(2).uniform(-1.0, 1.0, (3, 20))
+    sums = ev.direct(*t)
+    buf = 3.0 * den
+    ev.set_densities(buf)
+    buf[:] = 2.0 * den
+    ev.set_densities(buf)
+    buf[:] = np.nan
+    assert np.array_equal(ev.direct(*t), 2.0 * sums)
+    assert np.array_equal(ev.evaluate()[0], 2.0 * first)  # a power of two: exact
+    buf[:] = den
+    ev.set_densities(buf)
+    buf[:] = np.nan
+    assert np.array_equal(ev.evaluate()[0], first)
