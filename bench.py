@@ -46,21 +46,26 @@ P2P_FLOPS_PER_PAIR = 11.0  # the reference's convention, fmm/driver.cc:60
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 (vector and dense matrix)
 FP32_PEAK_TFLOPS = 157.3   # MI355X FP32 vector
 HBM_PEAK_GBS = 8000.0
-# Instruction-issue ceilings of the U-list kernels' inner loops (gfx950
-# assembly of this build; packed FP32 is off, transcendentals are quarter
-# rate, and MFMA issue adds to VALU issue rather than overlapping it):
-#   mixed: per 1024 pairs 4 v_mfma_f32_16x16x32_bf16 (16 cycles each),
-#          16 v_rsq_f32 (16) and 16 v_fmac_f32 (4): 384 cycles per SIMD;
+# Ceilings of the U-list kernels' inner loops by instruction issue (gfx950
+# assembly of this build, packed FP32 off), at 2.4 GHz:
+#   mixed: per 1024 pairs 4 v_mfma_f32_16x16x32_bf16, 16 v_rsq_f32 and 16
+#          v_fmac_f32, which take 288 cycles per SIMD where nothing else runs
+#          (measured, independent operands, 4 waves per SIMD on every CU; by
+#          themselves 29, 9.7 and 2.9 cycles each);
 #   FP64 Gram form: per 64 pairs 8 full-rate FP64 instructions (4 cycles each)
-#          and one v_rsq_f64 (16): 48 cycles per SIMD.
+#          and one quarter-rate v_rsq_f64 (16): 48 cycles per SIMD.
 SIMDS, CLOCK_GHZ = 1024, 2.4
-ISSUE_PAIRS_PER_CYCLE = {"mixed": 1024 / 384, "fp64": 64 / 48}
+ISSUE_PAIRS_PER_CYCLE = {"mixed": 1024 / 288, "fp64": 64 / 48}
+ISSUE_MODEL = {"mixed": "the inner loop's instructions alone, as measured",
+               "fp64": "inner-loop instruction issue, quarter-rate rsq"}
 
 
 def issue_bound(kind, achieved_tflops):
     t = P2P_FLOPS_PER_PAIR * ISSUE_PAIRS_PER_CYCLE[kind] * SIMDS * CLOCK_GHZ * 1e9 / 1e12
     return {"tflops": t, "frac": achieved_tflops / t, "pairs_per_cycle_per_simd": ISSUE_PAIRS_PER_CYCLE[kind],
-            "model": "inner-loop instruction issue at 2.4 GHz on 1024 SIMDs (quarter-rate rsq, no packed FP32)"}
+            "model": ISSUE_MODEL[kind] + " (2.4 GHz, 1024 SIMDs, no packed FP32)"}
+
+
 METRIC = "Mpoints/s per FMM eval (4M uniform), mixed vs FP64 GPU at matched sampled rel err"
 
 
