@@ -341,7 +341,7 @@ int check_view(const kifmm_tree_view* t) {
  * parents takes 11.2 us at NP 4 instead of 14.8.  The mixed path keeps one order of
  * summation. */
 constexpr int M2M_PARTS = 4;
-inline int m2m_parts(int np, int ncols, bool mixed) { return (np == 6 || !mixed) && ncols < 1024 ? M2M_PARTS : 1; }
+inline int m2m_parts(int ncols, bool mixed) { return !mixed && ncols < 1024 ? M2M_PARTS : 1; }
 constexpr int LEAF_SPLIT = 8192; /* leaves below which the FP64 leaf UC2UE is a k_level_op */
 
 /* Everything the device needs, derived on the host from the tree view.
@@ -1051,7 +1051,7 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
         wc.gemm_flops += 2.0 * ne * ne;
       }
     }
-    P.chk_cols = std::max(P.chk_cols, (size_t)col * m2m_parts(np, col, mixed));
+    P.chk_cols = std::max(P.chk_cols, (size_t)col * m2m_parts(col, mixed));
   }
   /* the fused downward kernel (k_l2l_dc2de) of depth d >= 3 runs over the
    * L2L parents at d - 1 and writes the densities of their target
@@ -1609,7 +1609,7 @@ int uc2ue(kifmm_gpu* g, const GemmList& B, int nin) {
 /* M2M of one level in two launches: the UE2UC stack into check values, in
  * m2m_parts slices along K, then UC2UE */
 int m2m(kifmm_gpu* g, const GemmList& A, const GemmList& B, int d) {
-  const int parts = m2m_parts(g->np, A.n, g->precision == KIFMM_PREC_MIXED);
+  const int parts = m2m_parts(A.n, g->precision == KIFMM_PREC_MIXED);
   LevelOp op{};
   op.M = g->n_uc; op.K = 8 * g->ld_e / parts; op.A = g->UE2UC; op.lda = g->lda_uc;
   op.a_z = (size_t)op.K * g->lda_uc; op.in_z = op.K;
