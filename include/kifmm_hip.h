@@ -177,9 +177,9 @@ int kifmm_gpu_release_idle(void);
 
 /* The handle's pinned host buffer of n_trg potentials (gathered target
  * order), valid until kifmm_gpu_destroy; NULL if pinned memory could not be
- * allocated.  Passing it to kifmm_gpu_evaluate copies the result at PCIe
- * rate with no host pass: the counterpart of the host array that
- * copy_trg_val__gpu fills (fmm/cuda.cu:2543-2565).  Each evaluation
+ * allocated.  Passing it to kifmm_gpu_evaluate leaves the result there, where
+ * the U-list writes it, with no host pass: the counterpart of the host array
+ * that copy_trg_val__gpu fills (fmm/cuda.cu:2543-2565).  Each evaluation
  * overwrites it. */
 double* kifmm_gpu_output(kifmm_gpu* g);
 

@@ -33,14 +33,11 @@ constexpr double FAR = 1.0e8; /* coordinate of padding sources */
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-/* x^(-1/2): the hardware estimate (v_rsq_f64, relative error below 2^-24,
- * measured max 5.2e-8) refined by one Newton step, e = 1 - x y^2,
- * y <- y + y e / 2, which leaves a relative error of (3/2) e0^2 <= 2e-14
- * (4e-15 for the measured estimate): far below the 1e-12 parity bar, and
- * one instruction per pair cheaper than a third-order step. */
-/* 2 / sqrt(x): the v_rsq_f64 estimate y (relative error <= 2^-24.2 on this
- * chip) and one Newton step written as y (3 - x y^2) = (2 / sqrt(x)) (1 -
- * 3e^2/2 + ...): three VALU instructions after the rsq.  The factor 2 is
+/* 2 / sqrt(x): the v_rsq_f64 estimate y (relative error e below 2^-24,
+ * measured max 5.2e-8) and one Newton step written as y (3 - x y^2) = (2 /
+ * sqrt(x)) (1 - 3e^2/2 + ...): three VALU instructions after the rsq, one
+ * fewer than a third-order step, and a relative error of at most 2e-14 (4e-15
+ * for the measured estimate), far below the 1e-12 parity bar.  The factor 2 is
  * left in; pair sums built from it are halved once at the end (an exact
  * power-of-two scale), which saves a multiply per pair. */
 __device__ __forceinline__ double rsqrt2_fp64(double x) {

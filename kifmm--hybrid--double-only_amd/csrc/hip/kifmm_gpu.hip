@@ -4,9 +4,10 @@
  * kifmm_gpu_create is the counterpart of preproc() (fmm/evaluate--cuda.cu:1441-2239):
  * it derives the device work lists from the flattened tree and uploads
  * everything once.  kifmm_gpu_evaluate is the counterpart of run()
- * (fmm/run--cuda.cu:27-345): up (S2M + M2M), U, V (forward DFT,
+ * (fmm/run--cuda.cu:27-345): up (S2M + M2M), V (forward DFT,
  * translation spectra, spectral multiply-add, inverse DFT), W, X, down
- * (L2L + DC2DE + L2T) and the copy back, in that order, on one stream.
+ * (L2L + DC2DE + L2T) and the U-list, which writes the potentials to the
+ * host as well, in that order on one stream (by default; enqueue_side).
  *
  * Device layout (HBM):
  *   src4 / trg4   gathered points as (x, y, z, w) double4 records
@@ -942,13 +943,15 @@ int make_plan(const kifmm_tree_view* t, const kifmm_operators* ops, bool mixed, 
       return fail("U-list wave item out of range");
   for (const int2& r : P.rng)
     if (r.x < 0 || r.y < 1 || (long)r.x + r.y > t->n_src) return fail("U-list source range out of range");
-  /* Copy-out chunks.  The U-list runs last, chunk by chunk, and each
-   * chunk's potentials go to the host while the next chunks compute.  A
-   * chunk is a run of whole leaves whose targets are one contiguous range:
-   * the item lists cover [0, n_trg) in item order with no gap (checked), and
-   * cuts fall at leaf starts, where every list has an item boundary.  The
-   * chunks shrink towards the end so that the copy left after the last
-   * chunk is short.  Small inputs are one chunk. */
+  /* Copy-out chunks.  The U-list runs last, as one launch that writes the
+   * device's and the pinned host potentials; it runs chunk by chunk only where
+   * the host copies each chunk to a caller's own buffer while the next ones
+   * compute, and where some chunks run early on the second stream
+   * (early_chunks).  A chunk is a run of whole leaves whose targets are one
+   * contiguous range: the item lists cover [0, n_trg) in item order with no
+   * gap (checked), and cuts fall at leaf starts, where every list has an item
+   * boundary.  The chunks shrink towards the end so that the host's pass left
+   * after the last chunk is short.  Small inputs are one chunk. */
   {
     const std::vector<int4>* lists[5] = {&P.p2p_items, &P.p2p_items64, &P.p2p_items5, &P.p2p_itemsP, &P.p2p_itemsW};
     bool tiled = t->n_trg > 0;

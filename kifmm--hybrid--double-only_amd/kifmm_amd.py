@@ -392,8 +392,8 @@ class GpuEvaluator:
     def evaluate(self, copy=True):
         """Returns (potentials in gathered order or None, phase times in ms).
         copy=True: the potentials come back into the handle's pinned buffer
-        (chunk by chunk while the U-list still runs) and a numpy copy of them
-        is returned; copy="view": the pinned buffer itself is returned (no
+        (written by the U-list as it runs) and a numpy copy of them is
+        returned; copy="view": the pinned buffer itself is returned (no
         host pass; the next evaluation overwrites it); copy=False: they stay
         on the device."""
         t = PhaseTimes()
