@@ -56,3 +56,28 @@ def test_on_several_threads():
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def test_release_between_and_beside_others():
+    """Idle memory and streams given back between handles, and while handles on
+    other threads are built and evaluate: the same bits."""
+    first = [once(*s) for s in SIZES]
+    K.release_idle()
+    errors = []
+
+    def work(k):
+        try:
+            for _ in range(3):
+                same(once(*SIZES[k]), first[k])
+                K.release_idle()
+        except BaseException as e:  # noqa: BLE001
+            errors.append((k, e))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(SIZES))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    K.release_idle()
+    same(once(*SIZES[0]), first[0])
