@@ -3026,6 +3026,7 @@ __global__ __launch_bounds__(Grid<NP>::THREADS) void k_dft_inv(const int* __rest
 constexpr int WX_T = 32, WX_G = WX_T / 8; /* points per item, groups of 8 */
 constexpr int WX_P = 4;                   /* sources per lane and pass */
 constexpr int WX_CAP = 1024;              /* sources per chunk at most */
+constexpr double WX_FAR = 0.5;            /* of the target box's half-width: from there on, the Gram form */
 enum { WX_SURF = 1, WX_DIFF = 2, WX_W = 4, WX_X = 8 }; /* item flags; WX_W / WX_X also select lists in a launch */
 
 static __global__ __launch_bounds__(64) void k_wx(const int4* __restrict__ items, /* {first range, end range, first point, points}, {node, slot, flags, sources} */

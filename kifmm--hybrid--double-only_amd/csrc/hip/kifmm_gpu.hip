@@ -577,7 +577,7 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
     surf = xl && !(t->child[i] == -1 && t->trg_num[i] < ne);
     return surf ? ne : t->trg_num[i];
   };
-  /* whether box s stays CLOSE_FRAC h away from box i (h = i's half-width) */
+  /* whether box s stays WX_FAR h away from box i (h = i's half-width) */
   auto far = [&](int i, int s) {
     const double hi = 1.0 / (1 << t->depth[i]), hs = 1.0 / (1 << t->depth[s]);
     double d2 = 0.0;
@@ -585,7 +585,7 @@ int wx_plan(const kifmm_tree_view* t, int ne, int lde, bool mixed, Plan& P) {
       const double gap = std::fabs((2 * t->path[3 * i + k] + 1) * hi - (2 * t->path[3 * s + k] + 1) * hs) - (hi + hs);
       if (gap > 0.0) d2 += gap * gap;
     }
-    return d2 >= CLOSE_FRAC * CLOSE_FRAC * hi * hi;
+    return d2 >= WX_FAR * WX_FAR * hi * hi;
   };
   long total = 0; /* sources x blocks */
   for (int i = 0; i < nn; i++)

@@ -78,3 +78,39 @@ def test_lists_together_and_apart(n, dist, q, np_, c, prec):
     for k in range(2):
         both = got["w"][k] + got["x"][k]
         assert np.all(np.abs(got["wx"][k] - both) <= 4e-16 * (np.abs(got["w"][k]) + np.abs(got["x"][k])))
+
+
+@pytest.mark.parametrize("n,seed", [(500, 0), (700, 2), (900, 1), (900, 3)])
+def test_near_pairs_are_as_exact_as_by_differences(n, seed):
+    """One source in a W-list leaf closer than h/2 to targets in a corner of
+    their leaf: each pair within 6e-15 of long double, the bound of the difference
+    form ((3/2) e^2 = 5.3e-15 for an estimate e of 2^-24, and the roundings of
+    r^2 and the scale, 4 x 1.1e-16).  In Gram form the roundings of |t|^2 + |s|^2 -
+    2 t.s alone are 3e-14 at h/8."""
+    rng = np.random.default_rng(seed)
+    s = rng.uniform(-1.0, 1.0, (3, n))
+    s[:, :200] = rng.uniform([[0.001], [0.47], [0.47]], [[0.03], [0.499], [0.499]], (3, 200))
+    s[:, 200:206] = rng.uniform([[0.0313], [0.47], [0.47]], [[0.036], [0.499], [0.499]], (3, 6))
+    t = rng.uniform([[-0.005], [0.46], [0.46]], [[0.0], [0.4999], [0.4999]], (3, n))
+    prob = K.Problem.from_points(*s, rng.uniform(0.5, 1.0, n), *t, pts_max=8, np_=3)
+    tree = prob.tree()
+    ev = K.GpuEvaluator(prob)
+    h = 2.0 ** -tree["depth"].astype(float)
+    c = (2.0 * tree["path"] + 1.0) * h[:, None]
+    pairs, worst = 0, 0.0
+    for i in np.flatnonzero((tree["child"] == -1) & (tree["trg_num"] > 0)):
+        for b in tree["w_idx"][tree["w_ptr"][i] : tree["w_ptr"][i + 1]]:
+            gap = np.maximum(np.abs(c[i] - c[b]) - (h[i] + h[b]), 0.0)
+            if tree["child"][b] != -1 or not 0 < tree["src_num"][b] < K.n_e(3) or np.sqrt(np.sum(gap * gap)) >= 0.5 * h[i]:
+                continue
+            j, k = tree["src_beg"][b], slice(tree["trg_beg"][i], tree["trg_beg"][i] + tree["trg_num"][i])
+            den = np.zeros(n)
+            den[j] = 1.0
+            ev.set_densities(den)
+            got = ev.evaluate_phases(K.PHASE_UP | K.PHASE_W)[0][k]
+            x = [tree[a][k].astype(np.longdouble) - np.longdouble(tree[b_][j]) for a, b_ in (("tx", "sx"), ("ty", "sy"), ("tz", "sz"))]
+            want = 1 / np.sqrt(x[0] ** 2 + x[1] ** 2 + x[2] ** 2) / (4 * np.arccos(np.longdouble(-1)))
+            pairs += got.size
+            worst = max(worst, float(np.max(np.abs(got / want - 1))))
+    print(f"  {pairs} pairs, worst {worst:.2e}", flush=True)
+    assert pairs > 0 and worst <= 6e-15
