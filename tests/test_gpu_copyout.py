@@ -2,8 +2,9 @@
 
 The potentials come back to the host as part of every evaluation (the
 reference's copy_trg_val__gpu, fmm/cuda.cu:2543-2565, inside run(),
-fmm/run--cuda.cu:319-324).  The U-list runs last, in chunks whose copies
-overlap the later chunks; whatever the route (pinned buffer, caller buffer,
+fmm/run--cuda.cu:319-324).  The U-list runs last and writes them to the
+pinned buffer itself, as one launch, or in chunks for a caller's buffer and in
+the layouts with early chunks; whatever the route (pinned buffer, caller buffer,
 graph replay, either stream layout, any U-list form) the host must receive
 bit for bit what the device holds.  New densities on an existing handle must
 give bit for bit what a fresh handle built with them gives.  The close-pair
